@@ -381,7 +381,7 @@ int StageToDevice(mi355x_search_ctx* ctx, hipStream_t s, void* dst, const void* 
 int SampleImpl(mi355x_search_ctx* ctx, hipStream_t s, const void* logits, const void* const* row_ptrs, int dtype,
                int64_t row_stride, int rows, int vocab, const mi355x_logits_xform* xf, mi355x_sample_params params,
                const mi355x_sample_params* per_row_params, const double* uniforms, int32_t* out_tokens,
-               int32_t* kept_count, int32_t* kept_ids, float* kept_probs, int kept_capacity) {
+               int32_t* kept_count, int32_t* kept_ids, float* kept_probs, int kept_capacity, bool kept_pad) {
   ms::SampleArgs a{};
   if (int r = MakeXform(ctx, xf, rows, vocab, s, &a.xf)) return r;
   bool any_nucleus = false, any_other = false, any_large_k = false, any_exact = false;
@@ -430,6 +430,7 @@ int SampleImpl(mi355x_search_ctx* ctx, hipStream_t s, const void* logits, const 
   a.kept_ids = kept_ids;
   a.kept_probs = kept_probs;
   a.kept_capacity = kept_capacity;
+  a.kept_pad = kept_pad ? 1 : 0;
   a.cand_small = ctx->cand_small;
   a.chunk_cnt = ctx->chunk_cnt;
   a.chunk_max = ctx->chunk_max;
@@ -462,24 +463,22 @@ int CheckSampleArgs(int dtype, const double* uniforms, const int32_t* out_tokens
   return MI355X_OK;
 }
 
-}  // namespace
-
-int mi355x_sample_typed(mi355x_search_ctx* ctx, void* stream, const void* logits, int dtype, int64_t row_stride,
-                        int rows, int vocab, const mi355x_logits_xform* xf, mi355x_sample_params params,
-                        const mi355x_sample_params* per_row_params, const double* uniforms, int32_t* out_tokens,
-                        int32_t* kept_count, int32_t* kept_ids, float* kept_probs, int kept_capacity) {
+int SampleRows(mi355x_search_ctx* ctx, void* stream, const void* logits, int dtype, int64_t row_stride, int rows, int vocab,
+               const mi355x_logits_xform* xf, mi355x_sample_params params, const mi355x_sample_params* per_row_params,
+               const double* uniforms, int32_t* out_tokens, int32_t* kept_count, int32_t* kept_ids, float* kept_probs,
+               int kept_capacity, bool kept_pad) {
   if (int r = CheckRows(ctx, rows, vocab)) return r;
   if (!logits) return Fail(MI355X_E_INVALID, "null logits, uniforms or output");
   if (int r = CheckSampleArgs(dtype, uniforms, out_tokens, kept_ids, kept_probs, kept_capacity)) return r;
   if (row_stride < vocab) return Fail(MI355X_E_INVALID, "row_stride smaller than vocab");
   return SampleImpl(ctx, static_cast<hipStream_t>(stream), logits, nullptr, dtype, row_stride, rows, vocab, xf, params,
-                    per_row_params, uniforms, out_tokens, kept_count, kept_ids, kept_probs, kept_capacity);
+                    per_row_params, uniforms, out_tokens, kept_count, kept_ids, kept_probs, kept_capacity, kept_pad);
 }
 
-int mi355x_sample_scattered(mi355x_search_ctx* ctx, void* stream, const void* const* row_ptrs, int dtype, int rows,
-                            int vocab, const mi355x_logits_xform* xf, mi355x_sample_params params,
-                            const mi355x_sample_params* per_row_params, const double* uniforms, int32_t* out_tokens,
-                            int32_t* kept_count, int32_t* kept_ids, float* kept_probs, int kept_capacity) {
+int SampleScattered(mi355x_search_ctx* ctx, void* stream, const void* const* row_ptrs, int dtype, int rows, int vocab,
+                    const mi355x_logits_xform* xf, mi355x_sample_params params, const mi355x_sample_params* per_row_params,
+                    const double* uniforms, int32_t* out_tokens, int32_t* kept_count, int32_t* kept_ids, float* kept_probs,
+                    int kept_capacity, bool kept_pad) {
   if (int r = CheckRows(ctx, rows, vocab)) return r;
   if (!row_ptrs) return Fail(MI355X_E_INVALID, "null row pointer array");
   for (int r = 0; r < rows; ++r)
@@ -500,9 +499,46 @@ int mi355x_sample_scattered(mi355x_search_ctx* ctx, void* stream, const void* co
                             xf ? &part : nullptr, params, per_row_params ? per_row_params + r0 : nullptr, uniforms + r0,
                             out_tokens + r0, kept_count ? kept_count + r0 : nullptr,
                             kept_ids ? kept_ids + static_cast<size_t>(r0) * kept_capacity : nullptr,
-                            kept_probs ? kept_probs + static_cast<size_t>(r0) * kept_capacity : nullptr, kept_capacity))
+                            kept_probs ? kept_probs + static_cast<size_t>(r0) * kept_capacity : nullptr, kept_capacity, kept_pad))
       return rc;
   }
+  return MI355X_OK;
+}
+
+}  // namespace
+
+int mi355x_sample_typed(mi355x_search_ctx* ctx, void* stream, const void* logits, int dtype, int64_t row_stride,
+                        int rows, int vocab, const mi355x_logits_xform* xf, mi355x_sample_params params,
+                        const mi355x_sample_params* per_row_params, const double* uniforms, int32_t* out_tokens,
+                        int32_t* kept_count, int32_t* kept_ids, float* kept_probs, int kept_capacity) {
+  return SampleRows(ctx, stream, logits, dtype, row_stride, rows, vocab, xf, params, per_row_params, uniforms, out_tokens,
+                    kept_count, kept_ids, kept_probs, kept_capacity, false);
+}
+
+int mi355x_sample_scattered(mi355x_search_ctx* ctx, void* stream, const void* const* row_ptrs, int dtype, int rows,
+                            int vocab, const mi355x_logits_xform* xf, mi355x_sample_params params,
+                            const mi355x_sample_params* per_row_params, const double* uniforms, int32_t* out_tokens,
+                            int32_t* kept_count, int32_t* kept_ids, float* kept_probs, int kept_capacity) {
+  return SampleScattered(ctx, stream, row_ptrs, dtype, rows, vocab, xf, params, per_row_params, uniforms, out_tokens, kept_count,
+                         kept_ids, kept_probs, kept_capacity, false);
+}
+
+// mi355x_sample_typed, or mi355x_sample_scattered where row_ptrs is given, whose kept ids and probabilities are padded
+// with -1 and 0 up to the capacity (the Python binding's form: a fill of each by launches of their own costs two).
+int ms_sample_padded(mi355x_search_ctx* ctx, void* stream, const void* logits, const void* const* row_ptrs, int dtype,
+                     int64_t row_stride, int rows, int vocab, const mi355x_logits_xform* xf, mi355x_sample_params params,
+                     const mi355x_sample_params* per_row_params, const double* uniforms, int32_t* out_tokens, int32_t* kept_count,
+                     int32_t* kept_ids, float* kept_probs, int kept_capacity) {
+  if (row_ptrs)
+    return SampleScattered(ctx, stream, row_ptrs, dtype, rows, vocab, xf, params, per_row_params, uniforms, out_tokens, kept_count,
+                           kept_ids, kept_probs, kept_capacity, true);
+  return SampleRows(ctx, stream, logits, dtype, row_stride, rows, vocab, xf, params, per_row_params, uniforms, out_tokens, kept_count,
+                    kept_ids, kept_probs, kept_capacity, true);
+}
+
+// Device-to-device copy in stream order.
+int ms_copy_on_stream(void* stream, void* dst, const void* src, size_t bytes) {
+  HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, static_cast<hipStream_t>(stream)));
   return MI355X_OK;
 }
 

@@ -647,6 +647,7 @@ struct RowOutputs {
   int32_t* kept_ids;
   float* kept_probs;
   int kept_capacity;
+  int pad;  // non-zero: entries from the kept count to the capacity get id -1 and probability 0
 };
 
 // The reference's ComputeSampledCategorical + SampleCategoricalToken
@@ -739,10 +740,12 @@ __device__ __forceinline__ bool block_sample_epilogue(Sorted sorted, Exps exps, 
   };
   if (out.kept_count && threadIdx.x == 0) *out.kept_count = keep;
   if (out.kept_ids) {
-    const int lim = keep < out.kept_capacity ? keep : out.kept_capacity;
+    const int kept = keep < out.kept_capacity ? keep : out.kept_capacity;
+    const int lim = out.pad ? out.kept_capacity : kept;
     for (int i = threadIdx.x; i < lim; i += blockDim.x) {
-      out.kept_ids[i] = static_cast<int32_t>(key64_index(sorted(i)));
-      if (out.kept_probs) out.kept_probs[i] = q(i);
+      const bool in = i < kept;
+      out.kept_ids[i] = in ? static_cast<int32_t>(key64_index(sorted(i))) : -1;
+      if (out.kept_probs) out.kept_probs[i] = in ? q(i) : 0.0f;
     }
   }
   const int pos = block_discrete_draw<ITEMS>(keep, q, u, sh);

@@ -62,6 +62,7 @@ struct SampleArgs {
   int32_t* kept_ids;
   float* kept_probs;
   int kept_capacity;
+  int kept_pad;           // non-zero: kept ids / probs beyond the kept count are written as -1 / 0 up to the capacity
   // workspace
   u64* cand_small;        // [rows][chunks][kSmallCap]; zero between launches (published, then cleared by the finisher)
   uint32_t* chunk_cnt;    // [rows][chunks]

@@ -66,7 +66,7 @@ __device__ __forceinline__ RowOutputs row_outputs(const SampleArgs& a, int row) 
   return RowOutputs{a.out_tokens + row, a.kept_count ? a.kept_count + row : nullptr,
                     a.kept_ids ? a.kept_ids + static_cast<size_t>(row) * a.kept_capacity : nullptr,
                     a.kept_probs ? a.kept_probs + static_cast<size_t>(row) * a.kept_capacity : nullptr,
-                    a.kept_capacity};
+                    a.kept_capacity, a.kept_pad};
 }
 
 // A row of the logits as fp32 values, whatever it is stored as: InT float, uint16_t (fp16 bits) or bf16_t,
@@ -439,9 +439,16 @@ __device__ __forceinline__ void wave_topk_epilogue(u64 key, int m, mi355x_sample
     *out.token = tok;
     if (out.kept_count) *out.kept_count = keep;
   }
-  if (out.kept_ids && lane < keep && lane < out.kept_capacity) {
-    out.kept_ids[lane] = static_cast<int32_t>(idx);
-    if (out.kept_probs) out.kept_probs[lane] = q;
+  if (out.kept_ids) {
+    if (lane < keep && lane < out.kept_capacity) {
+      out.kept_ids[lane] = static_cast<int32_t>(idx);
+      if (out.kept_probs) out.kept_probs[lane] = q;
+    }
+    if (out.pad)
+      for (int i = lane < keep ? lane + 64 : lane; i < out.kept_capacity; i += 64) {
+        out.kept_ids[i] = -1;
+        if (out.kept_probs) out.kept_probs[i] = 0.0f;
+      }
   }
 }
 
@@ -882,7 +889,8 @@ __device__ __forceinline__ bool stream_row(const SampleArgs& a, int row, const v
                               arg_now(a.kept_count),
                               arg_now(a.kept_ids),
                               arg_now(a.kept_probs),
-                              arg_now(a.kept_capacity)};
+                              arg_now(a.kept_capacity),
+                              a.kept_pad};
   if constexpr (XFORM) {
     // fp32 rows: the registers past the row's end, see the loads above
     if constexpr (kOneRun) {
