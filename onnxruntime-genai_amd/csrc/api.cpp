@@ -81,6 +81,8 @@ struct mi355x_search_ctx {
   int* sub_se{};
   float* row_max{};
   float* row_sum{};
+  ms::WideRow* wide_rows{};
+  uint32_t* wide_tile_start{};
   int32_t* row_index{};  // device copy of per-row host indices (logits hand-off)
   int32_t* beam_row_tokens{};
   // Pinned host staging for the calls that take a table from a caller's HOST array (per-row parameters of more
@@ -215,7 +217,11 @@ int mi355x_search_create(int device, int max_rows, int max_vocab, mi355x_search_
   ok(c->Alloc(&c->params_dev, static_cast<size_t>(max_rows), false));
   ok(c->Alloc(&c->beam_row_scores, static_cast<size_t>(max_rows) * ms::kBeamMaxCand, false));
   ok(c->Alloc(&c->beam_row_tokens, static_cast<size_t>(max_rows) * ms::kBeamMaxCand, false));
-  c->max_segs = (max_vocab + ms::kSegElems - 1) / ms::kSegElems;
+  // (segments of the exact sums; the tiles of rows sampled from the whole vocabulary are shorter and share the arrays)
+  c->max_segs = (max_vocab + ms::kWideTile - 1) / ms::kWideTile;
+  static_assert(ms::kWideTile <= ms::kSegElems, "room for either");
+  ok(c->Alloc(&c->wide_rows, static_cast<size_t>(max_rows), false));
+  ok(c->Alloc(&c->wide_tile_start, static_cast<size_t>(max_rows) * (c->max_segs + 1), false));
   ok(c->Alloc(&c->seg_max, static_cast<size_t>(max_rows) * c->max_segs, false));
   ok(c->Alloc(&c->seg_sum, static_cast<size_t>(max_rows) * c->max_segs, false));
   // "not written yet" everywhere (all bits set): the state the exact-sum kernels expect and leave behind
@@ -316,7 +322,7 @@ int mi355x_argmax(mi355x_search_ctx* ctx, void* stream, const void* logits, int 
     f.big_stride = ctx->big_stride;
     f.fallback_rows = ctx->fallback_rows;
     f.poll_limit = ctx->poll_limit;
-    HIP_TRY(ms_launch_sample(&f, nullptr, true, false, false, s, nullptr));
+    HIP_TRY(ms_launch_sample(&f, nullptr, true, false, false, s, nullptr, nullptr));
     return MI355X_OK;
   }
   ms::ArgmaxArgs a{};
@@ -384,10 +390,14 @@ int SampleImpl(mi355x_search_ctx* ctx, hipStream_t s, const void* logits, const 
                int32_t* kept_count, int32_t* kept_ids, float* kept_probs, int kept_capacity, bool kept_pad) {
   ms::SampleArgs a{};
   if (int r = MakeXform(ctx, xf, rows, vocab, s, &a.xf)) return r;
-  bool any_nucleus = false, any_other = false, any_large_k = false, any_exact = false;
+  bool any_nucleus = false, any_other = false, any_large_k = false, any_exact = false, any_wide = false;
   const int chunks = (vocab + ms::kSChunk - 1) / ms::kSChunk;
   ms::InlineParams table{};
   bool use_table = false;
+  // Sampling from the whole vocabulary is spread over the GPU wherever its kernels can take the row as it lies: no
+  // logits processing, a row long enough to cut up, no more tiles than the finishing workgroup holds.
+  const int tiles = (vocab + ms::kWideTile - 1) / ms::kWideTile;
+  const bool wide_fits = vocab >= ms::kWideMinVocab && tiles <= ms::kWideMaxTiles && chunks * ms::kSmallCap <= ms::kAllCap && !a.xf.active();
   auto check = [&](const mi355x_sample_params& p) -> int {
     if (!(p.temperature > 0.0f)) return Fail(MI355X_E_INVALID, "temperature must be positive (got %g)", p.temperature);
     // the kernels' own rule (row_mode) decides; these flags only have to cover it
@@ -397,7 +407,8 @@ int SampleImpl(mi355x_search_ctx* ctx, hipStream_t s, const void* logits, const 
     const bool nucleus = p.k <= 1 && !whole, large_k = p.k > 1 && kk > 64 && kk <= ms::kLargeKMax;
     if (nucleus && vocab > 64) any_nucleus = true;
     if (large_k && vocab > 64) any_large_k = true;
-    if (vocab > 64 && (!fits || whole || (p.k > 1 && kk > ms::kLargeKMax))) any_exact = true;
+    if (whole && wide_fits) any_wide = true;
+    else if (vocab > 64 && (!fits || whole || (p.k > 1 && kk > ms::kLargeKMax))) any_exact = true;
     else if (!((nucleus || large_k) && fits)) any_other = true;
     return MI355X_OK;
   };
@@ -442,14 +453,16 @@ int SampleImpl(mi355x_search_ctx* ctx, hipStream_t s, const void* logits, const 
   a.fallback_rows = ctx->fallback_rows;
   a.poll_limit = ctx->poll_limit;
   a.row_done = ctx->row_done;
-  a.exact_kernel = any_exact ? 1 : 0;
+  a.exact_kernel = (any_exact ? ms::kExactRows : 0) | (any_wide ? ms::kWideRows : 0);
+  const ms::WideArgs wide{(vocab + ms::kWideChunk - 1) / ms::kWideChunk, tiles, ctx->wide_rows, ctx->wide_tile_start, ctx->seg_sum,
+                          ctx->seg_step, ctx->sub_step, ctx->sub_se, ctx->chunk_next};
   // a caller that bounds the number of allowed ids per row lets the sparse-mask kernel work alone
   if (xf && xf->mask && xf->mask_allowed_max > 0) {
     const int hist = a.xf.history_lens ? a.xf.history_stride : a.xf.history_len;
     const int64_t listed = static_cast<int64_t>(xf->mask_allowed_max) + (a.xf.use_penalty() ? hist : 0) + 2;
     a.sparse_only = listed <= ms::kNucleusCap && hist <= 2048;  // (what the kernel can list; beyond, all three kernels)
   }
-  HIP_TRY(ms_launch_sample(&a, use_table ? &table : nullptr, any_other, any_nucleus, any_large_k, s, &ctx->sides));
+  HIP_TRY(ms_launch_sample(&a, use_table ? &table : nullptr, any_other, any_nucleus, any_large_k, s, &ctx->sides, &wide));
   return MI355X_OK;
 }
 
@@ -581,8 +594,8 @@ int mi355x_topk_scores(mi355x_search_ctx* ctx, void* stream, const void* logits,
   const bool fits = vocab > 64 && a.chunks * ms::kSmallCap <= ms::kAllCap;
   const bool large_k = fits && k > 64 && k <= ms::kLargeKMax;
   const bool exact = vocab > 64 && (!fits || k > ms::kLargeKMax);
-  a.exact_kernel = exact ? 1 : 0;
-  HIP_TRY(ms_launch_sample(&a, nullptr, !large_k && !exact, false, large_k, s, nullptr));
+  a.exact_kernel = exact ? ms::kExactRows : 0;
+  HIP_TRY(ms_launch_sample(&a, nullptr, !large_k && !exact, false, large_k, s, nullptr, nullptr));
   return MI355X_OK;
 }
 

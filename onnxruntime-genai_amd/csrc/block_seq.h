@@ -99,6 +99,13 @@ __device__ __forceinline__ Step quad_scan_steps(Step x) {
   return x;
 }
 
+// The same over groups of eight lanes: lanes 7, 15, 23, ... end with the composition of their group.
+__device__ __forceinline__ Step oct_scan_steps(Step x) {
+  x = quad_scan_steps(x);
+  x = step_compose(step_from_below<0x114, 0xf>(x), x);  // row_shr:4
+  return x;
+}
+
 __device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) { return ~wave_max<uint32_t>(~v); }
 
 // Fetches the ITEMS consecutive addends thread t owns in the window [w0, wend): indices
@@ -186,8 +193,8 @@ struct StopAtMass {
 // FindNucleus' stop (src/sampling_distribution.h:164-174) over addends in descending order: the prefix reaches
 // p times (prefix + the bound (vocab - i - 1) * addend on what follows).  In exact arithmetic prefix - p * (prefix +
 // bound) does not decrease along the row (prefixes do not decrease, addends and counts do not increase); the
-// float evaluation is within a few 2^-24 of it, so a run whose last element misses the stop by more than 2^-18 of
-// the right-hand side holds none.
+// float evaluation is within three roundings of 2^-24 of the right-hand side wherever it turns true, and this test's
+// own within four, so a run whose last element misses the stop by more than 2^-21 of the right-hand side holds none.
 struct StopAtNucleus {
   float p;
   int vocab, offset;  // the addend's rank in the row is its index + offset
@@ -197,7 +204,7 @@ struct StopAtNucleus {
   }
   __device__ __forceinline__ bool nowhere_in_run_ending(float pf, float e, int i) const {
     const float tail = static_cast<float>(vocab - (i + offset) - 1) * e;
-    return pf < (p * (pf + tail)) * 0.99999619f;  // 1 - 2^-18
+    return pf < (p * (pf + tail)) * 0.99999952f;  // 1 - 2^-21
   }
 };
 

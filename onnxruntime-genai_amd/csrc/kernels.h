@@ -24,6 +24,7 @@ constexpr int kFinishBlock = 1024;
 
 constexpr int kEmitArgmax = 2;
 constexpr int kArgmaxFusedMinBlocks = 1;  // rows x 32768-id chunks from which mi355x_argmax uses the fused kernel
+constexpr int kExactRows = 1, kWideRows = 2;  // SampleArgs::exact_kernel: the one-workgroup kernel / the kernels of wide_rows.h
 constexpr int kModeTopkSmall = 0;
 constexpr int kModeNucleus = 1;
 constexpr int kModeGeneral = 2;
@@ -80,7 +81,38 @@ struct SampleArgs {
   uint32_t* row_done;       // [rows] or null: nucleus rows under a grammar mask that the sparse-mask kernel finished
   int sparse_only;          // the sparse-mask kernel is the only one launched for nucleus rows: a row it cannot
                             // finish goes to the exact path inside it
-  int exact_kernel;         // rows whose parameters alone send them to the exact path have a kernel of their own
+  int exact_kernel;         // rows whose parameters alone send them to the exact path have kernels of their own (kExact*)
+};
+
+// Rows of the exact path that are spread over the GPU (wide_rows.h): sampling from the whole vocabulary.
+constexpr int kWideChunk = 8192;      // logits per workgroup of the passes over the row
+constexpr int kWideBuckets = 2048;    // buckets of the row's histogram
+constexpr int kWideTile = 3072;       // keys after which a new tile begins, with the next bucket
+constexpr int kWideBucketMax = 1024;  // keys of a bucket
+constexpr int kWideMaxTiles = 192;    // tiles of the longest row (589824 logits)
+constexpr int kWideMinVocab = 4096;   // shorter rows are a single workgroup's work anyway
+struct WideRow {
+  uint32_t n, tiles, declined;  // listed keys, their tiles; declined: the row is not one for this path
+  float top;                    // the row's maximum
+};
+struct WideArgs {
+  int chunks, max_tiles;
+  WideRow* rows;         // [rows]
+  uint32_t* tile_start;  // [rows][max_tiles + 1]
+  double* tile_sum;      // [rows][max_tiles]
+  int4* tile_step;       // [rows][max_tiles]: see SeqSumArgs::seg_step, and sub_step / sub_se
+  int4* sub_step;
+  int* sub_se;
+  u64* best_below;       // [rows]: the best element past the list, 0: none
+};
+struct NoTable {};
+template <bool INLINE>
+struct WideTable {  // the second argument of the kernels that come with and without a table in their arguments
+  typedef NoTable type;
+};
+template <>
+struct WideTable<true> {
+  typedef InlineParams type;
 };
 
 struct ArgmaxArgs {
@@ -193,13 +225,13 @@ extern "C" {
 hipError_t ms_sample_init();
 // `table`, when not null, holds the parameters of rows 0 .. a->rows-1 (a->rows <= kInlineParamRows).
 // any_nucleus / any_large_k / any_other: some row may be in nucleus mode / a top-k row with
-// 64 < k <= kLargeKMax / in another mode (each mode has kernels of its own); a->exact_kernel: some row's
-// parameters send it to the exact path.
+// 64 < k <= kLargeKMax / in another mode (each mode has kernels of its own); a->exact_kernel: which kernels of the
+// exact path some row's parameters ask for (kWideRows: `wide` holds their arguments).
 // sides, when not null: streams and events of the context on which the kernels of a call whose rows are in several
 // modes run side by side (each mode's kernels skip the other modes' rows and share no state with them): they fork
 // from `stream` behind an event, and `stream` waits for them before the exact rows' kernel and before the call returns.
 hipError_t ms_launch_sample(const ms::SampleArgs* a, const ms::InlineParams* table, bool any_other, bool any_nucleus,
-                            bool any_large_k, hipStream_t stream, const ms::SideStreams* sides);
+                            bool any_large_k, hipStream_t stream, const ms::SideStreams* sides, const ms::WideArgs* wide);
 hipError_t ms_launch_argmax(const ms::ArgmaxArgs* a, int dtype, hipStream_t stream);
 hipError_t ms_launch_process_logits(float* logits, int64_t row_stride, int rows, int vocab,
                                     const ms::Xform* xf, hipStream_t stream);

@@ -367,6 +367,12 @@ struct SortWithTile {
 // (i ^ (i >> 4)) & 7, which spreads those reads over all banks.
 __device__ __forceinline__ uint32_t exp_slot(uint32_t i) { return (i & ~7u) | ((i ^ (i >> 4)) & 7u); }
 
+}  // namespace ms
+
+#include "wide_rows.h"
+
+namespace ms {
+
 // Where DeviceInterface::TopKScores wants a row's k best: ids and raw scores, best first (tokens null: not asked for).
 struct EmitTopk {
   int32_t* tokens = nullptr;
@@ -1677,7 +1683,7 @@ __global__ __launch_bounds__(kFinishBlock) void nucleus_sparse_rows_kernel(const
 }
 
 // Rows whose parameters alone put them on the exact path (k above kLargeKMax, more chunks than a finishing
-// workgroup ranks): one workgroup per row with the finish kernels' LDS, so that the row is sorted by the radix
+// workgroup ranks; sampling from the whole vocabulary where wide_rows.h does not serve): one workgroup per row with the finish kernels' LDS, so that the row is sorted by the radix
 // sort instead of a sorting network in global memory.
 template <bool INLINE>
 __device__ __forceinline__ void exact_rows_body(const SampleArgs& a) {
@@ -1688,6 +1694,7 @@ __device__ __forceinline__ void exact_rows_body(const SampleArgs& a) {
   const int row = blockIdx.x;
   const mi355x_sample_params prm = row_params<INLINE>(a, row);
   if (row_mode(prm, a.vocab, a.chunks, a.emit_topk) != kModeGeneral) return;
+  if ((a.exact_kernel & kWideRows) && wide_row(prm)) return;
   general_row<AnyDtype, SortWithTile, 8>(a, row, row_start<INLINE>(a, row, dtype_bytes(a.dtype)), prm, a.big + static_cast<size_t>(row) * a.big_stride,
                         seqsh,
                         SortWithTile{a.big2 ? a.big2 + static_cast<size_t>(row) * a.big_stride : nullptr, lds_keys, red32, red64});
@@ -1701,7 +1708,7 @@ MS_STREAM_KERNELS(, float)  // the fp32 streaming kernels live here, next to the
 
 extern "C" hipError_t ms_launch_sample(const ms::SampleArgs* a, const ms::InlineParams* table, bool any_other,
                                        bool any_nucleus, bool any_large_k, hipStream_t stream,
-                                       const ms::SideStreams* sides) {
+                                       const ms::SideStreams* sides, const ms::WideArgs* wide) {
   const dim3 fgrid(a->rows), fblock(ms::kFinishBlock);
   auto launch_stream = a->dtype == MI355X_F16 ? ms_launch_stream_f16 : a->dtype == MI355X_BF16 ? ms_launch_stream_bf16 : ms_launch_stream;
   // A call whose rows are in several modes launches the kernels of every mode present; one after the other their
@@ -1757,7 +1764,11 @@ extern "C" hipError_t ms_launch_sample(const ms::SampleArgs* a, const ms::Inline
     if (e == hipSuccess) e = j;
   }
   if (e != hipSuccess) return e;
-  if (a->exact_kernel) {
+  if (a->exact_kernel & ms::kWideRows) {
+    e = table ? ms::launch_wide<true>(*a, *table, *wide, stream) : ms::launch_wide<false>(*a, ms::NoTable{}, *wide, stream);
+    if (e != hipSuccess) return e;
+  }
+  if (a->exact_kernel & ms::kExactRows) {
     if (table) hipLaunchKernelGGL(ms::exact_rows_rows_kernel, fgrid, fblock, ms::kFinishLds, stream, *a, *table);
     else hipLaunchKernelGGL(ms::exact_rows_kernel, fgrid, fblock, ms::kFinishLds, stream, *a);
     e = hipGetLastError();
@@ -1773,7 +1784,16 @@ extern "C" hipError_t ms_sample_init() {
                           reinterpret_cast<const void*>(ms::nucleus_sparse_kernel),
                           reinterpret_cast<const void*>(ms::nucleus_sparse_rows_kernel),
                           reinterpret_cast<const void*>(ms::exact_rows_kernel),
-                          reinterpret_cast<const void*>(ms::exact_rows_rows_kernel)};
+                          reinterpret_cast<const void*>(ms::exact_rows_rows_kernel),
+                          reinterpret_cast<const void*>(ms::wide_finish_kernel<false>),
+                          reinterpret_cast<const void*>(ms::wide_finish_kernel<true>),
+                          reinterpret_cast<const void*>(ms::wide_scatter_kernel<float, false>),
+                          reinterpret_cast<const void*>(ms::wide_scatter_kernel<float, true>),
+                          reinterpret_cast<const void*>(ms::wide_scatter_kernel<uint16_t, false>),
+                          reinterpret_cast<const void*>(ms::wide_scatter_kernel<uint16_t, true>),
+                          reinterpret_cast<const void*>(ms::wide_scatter_kernel<ms::bf16_t, false>),
+                          reinterpret_cast<const void*>(ms::wide_scatter_kernel<ms::bf16_t, true>)};
+  static_assert(sizeof(ms::WideScatterShared) <= ms::kFinishLds, "one limit for all");
   for (const void* f : finish) {
     const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, ms::kFinishLds);
     if (e != hipSuccess) return e;

@@ -1,0 +1,755 @@
+// Rows that need most of their vocabulary in rank order: sampling from the whole vocabulary (k <= 1 with p >= 1).
+//
+// The reference sorts such a row, adds the exponentials of all of it one after the other and draws from the result.
+// One workgroup per row (exact_rows_kernel) spends 0.55 ms on that however few rows there are: its sort moves every
+// key three times at the memory rate of a single CU, and its sums run over 128 K exponentials in one workgroup.  Here
+// every step but the last is spread over the GPU, in five launches (16 x 128256 fp16: 557 -> WIDE_US us per step):
+//   1. wide_max:     the maximum of every 16384-logit chunk.
+//   2. wide_count:   a histogram per chunk over kWideBuckets buckets, linear in the score below the row's maximum down
+//                    to the depth past which no element can lie inside the kept set.
+//   3. wide_scatter: every workgroup scans the row's histograms, gives its chunk's keys their places, bucket by
+//                    bucket, in the row's key buffer, and the first chunk's cuts the list into tiles of whole buckets
+//                    (kWideTile keys and at most one bucket more).
+//   4. wide_rank:    a workgroup per tile sorts it in LDS (a counting sort with buckets linear between the tile's own
+//                    extremes), writes (exponential, id) entries in rank order, and composes the tile's step record
+//                    for the exact sequential sum under the binade the double sums of the tiles before it predict (a
+//                    look-back at sums that lower workgroup indices of the same launch publish, as in
+//                    seqsum_exp_step).
+//   5. wide_finish:  a workgroup per row walks the records (the exact sum behind every tile), searches the one tile
+//                    in which the stop of FindNucleus can lie, and draws from the double sums of the tiles.
+// Elements of equal score need not be told apart before the draw: a run of ties weighs the same in any order.  Large
+// runs of ties (bf16 logits have hundreds per value) stay in arrival order, and the one run the draw falls into is
+// ordered by id then.  A call that asks for the kept ids has its ties ordered by wide_rank.
+// A row this does not fit (a bucket of more than kWideBucketMax keys, a maximum that is not finite, a stop beyond the
+// listed elements) is finished by the exact path inside wide_finish.
+#pragma once
+#include "sample_stream.h"
+#include "seqsum_exp_step.h"
+#include "seq_walk.h"
+
+namespace ms {
+
+constexpr int kWideBlock = 1024;
+constexpr int kWidePer = kWideChunk / kWideBlock;  // logits per thread
+constexpr int kWideRankBlock = 512;
+constexpr int kWideRankPer = kSegElems / kWideRankBlock;
+static_assert(kWideTile + kWideBucketMax <= kSegElems, "a tile fits the segment its step record describes");
+
+// Rows of this kind: every element counts, whatever k says (k <= 1) and however large p is.
+__device__ __forceinline__ bool wide_row(mi355x_sample_params prm) { return prm.k <= 1 && !(prm.p < 1.0f); }
+
+// How far below the maximum (in score units) the list reaches: an element past ln V + 18 exponent units below the
+// maximum satisfies the stop of FindNucleus for p = 1, (V - i - 1) * e_i < prefix * 2^-25, wherever it ranks, so the
+// stop lies at or before the first such element (which follows the list, wide_best).
+__device__ __forceinline__ float wide_depth(mi355x_sample_params prm, int vocab) {
+  return (logf(static_cast<float>(vocab)) + 18.0f) * prm.temperature;
+}
+
+// Which row, and which of its `per_row` shares of the work, a workgroup has.  Workgroups go round-robin over the eight
+// XCDs; all shares of a row get indices of one remainder, so what they hand over -- every launch reads what the one
+// before it wrote, scattered all over the row's buffers -- stays in one L2 (scattered from all XCDs, the keys' 8-byte
+// writes reach memory one partial line each: 18.2 us of the scatter at 16 x 128256).  Rows past the last have no work.
+struct WideShare {
+  int row, item;
+};
+__device__ __forceinline__ WideShare wide_share(int per_row) {
+  const int xcd = static_cast<int>(blockIdx.x) & 7, slot = static_cast<int>(blockIdx.x) >> 3;
+  return WideShare{xcd + 8 * (slot / per_row), slot % per_row};
+}
+
+// The 16 logits of thread t in a chunk, in loads of 16 bytes; ids past the vocabulary are NaN.
+template <typename InT>
+__device__ __forceinline__ void wide_load(const InT* row, int V, int chunk, float (&v)[kWidePer]) {
+  constexpr int VEC = 16 / static_cast<int>(sizeof(InT));
+#pragma unroll
+  for (int j = 0; j < kWidePer / VEC; ++j) {
+    const int i0 = chunk * kWideChunk + (j * kWideBlock + static_cast<int>(threadIdx.x)) * VEC;
+    if (i0 + VEC <= V) {
+      if constexpr (VEC == 4) {
+        const v4f_any q = *reinterpret_cast<const v4f_any*>(row + i0);
+        v[j * 4] = q.x, v[j * 4 + 1] = q.y, v[j * 4 + 2] = q.z, v[j * 4 + 3] = q.w;
+      } else {
+        const v4u q = *reinterpret_cast<const v4u_any*>(row + i0);
+        if constexpr (__is_same(InT, uint16_t)) widen_half8(q, &v[j * 8]);
+        else widen_bf16x8(q, &v[j * 8]);
+      }
+    } else {
+#pragma unroll
+      for (int c = 0; c < VEC; ++c) v[j * VEC + c] = i0 + c < V ? load_one<InT>(row, i0 + c) : __uint_as_float(0x7fc00000u);
+    }
+  }
+}
+template <typename InT>
+__device__ __forceinline__ int wide_index(int chunk, int e) {
+  constexpr int VEC = 16 / static_cast<int>(sizeof(InT));
+  return chunk * kWideChunk + ((e / VEC) * kWideBlock + static_cast<int>(threadIdx.x)) * VEC + e % VEC;
+}
+
+// The row's maximum as the chunks left it (0xffffffff where the row is not one for this path).
+__device__ __forceinline__ uint32_t wide_row_max(const SampleArgs& a, const WideArgs& w, int row) {
+  const int lane = lane_id();
+  uint32_t m = 0u;
+  for (int c = lane; c < w.chunks; c += 64) {
+    const uint32_t k = a.chunk_max[static_cast<size_t>(row) * w.chunks + c];
+    m = k > m ? k : m;
+  }
+  m = wave_max<uint32_t>(m);
+  return (m <= order_key(-1e30f) || m >= order_key(1e30f)) ? 0xffffffffu : m;
+}
+
+template <typename InT, bool INLINE>
+__global__ __launch_bounds__(kWideBlock) void wide_max_kernel(const SampleArgs a, const typename WideTable<INLINE>::type, const WideArgs w) {
+  __shared__ uint32_t red[16];
+  const WideShare mine = wide_share(w.chunks);
+  const int chunk = mine.item, row = mine.row, tid = threadIdx.x;
+  if (row >= a.rows || !wide_row(row_params<INLINE>(a, row))) return;
+  float v[kWidePer];
+  wide_load<InT>(static_cast<const InT*>(row_start<INLINE>(a, row, sizeof(InT))), a.vocab, chunk, v);
+  // (this launch is the first of its sequence: it also marks the sums of the row's tiles as not written)
+  if (chunk == 0) {
+    for (int t = tid; t < w.max_tiles; t += kWideBlock) store_sum_bits(w.tile_sum + static_cast<size_t>(row) * w.max_tiles + t, kSumNotReady);
+    if (tid == 0) w.best_below[row] = 0;
+  }
+  float m = -__builtin_inff();
+#pragma unroll
+  for (int e = 0; e < kWidePer; ++e) m = fmaxf(m, v[e]);
+  const uint32_t k = block_max<uint32_t>(order_key(m), red, false);
+  if (tid == 0) a.chunk_max[static_cast<size_t>(row) * w.chunks + chunk] = k;
+}
+
+// Bucket of a score: a non-increasing function of it (every operation is monotone), kWideBuckets and up for what lies
+// past the depth and for NaN.
+struct WideBuckets {
+  float top, scale;
+  __device__ __forceinline__ WideBuckets(float max_score, float depth) : top(max_score), scale(static_cast<float>(kWideBuckets) / depth) {}
+  __device__ __forceinline__ uint32_t operator()(float x) const {
+    const float b = (top - x) * scale;
+    return b < static_cast<float>(kWideBuckets) ? static_cast<uint32_t>(b) : static_cast<uint32_t>(kWideBuckets);
+  }
+};
+
+template <typename InT, bool INLINE>
+__global__ __launch_bounds__(kWideBlock) void wide_count_kernel(const SampleArgs a, const typename WideTable<INLINE>::type, const WideArgs w) {
+  __shared__ uint32_t hist[kWideBuckets + 1];
+  const WideShare mine = wide_share(w.chunks);
+  const int chunk = mine.item, row = mine.row, tid = threadIdx.x;
+  if (row >= a.rows) return;
+  const mi355x_sample_params prm = row_params<INLINE>(a, row);
+  if (!wide_row(prm)) return;
+  const uint32_t rmax = wide_row_max(a, w, row);
+  if (rmax == 0xffffffffu) return;
+  float v[kWidePer];
+  wide_load<InT>(static_cast<const InT*>(row_start<INLINE>(a, row, sizeof(InT))), a.vocab, chunk, v);
+  for (int b = tid; b <= kWideBuckets; b += kWideBlock) hist[b] = 0u;
+  __syncthreads();
+  const WideBuckets bucket_of(key_to_float(rmax), wide_depth(prm, a.vocab));
+#pragma unroll
+  for (int e = 0; e < kWidePer; ++e) {
+    const uint32_t b = bucket_of(v[e]);
+    if (b < static_cast<uint32_t>(kWideBuckets)) atomicAdd(&hist[b], 1u);
+  }
+  __syncthreads();
+  // two buckets a thread, packed: a chunk holds at most 16384 keys
+  static_assert(kWideBuckets == 2 * kWideBlock, "a pair of buckets per thread");
+  uint32_t* out = reinterpret_cast<uint32_t*>(a.big + static_cast<size_t>(row) * a.big_stride) + static_cast<size_t>(chunk) * kWideBlock;
+  out[tid] = hist[2 * tid] | (hist[2 * tid + 1] << 16);
+}
+
+// The keys go to LDS in bucket order first and from there to memory, so that neighbouring lanes write neighbouring
+// places (eight keys a bucket and chunk at 128256 logits).  Written straight from the registers every lane's 8 bytes
+// are a line of their own: 8.3 of the 17.9 us the launch took at 16 x 128256.
+struct WideScatterShared {
+  u64 keys[kWideChunk];
+  uint32_t place[kWideBuckets];  // the bucket's next place in keys
+  uint32_t shift[kWideBuckets];  // what takes a place in keys to one in the row's buffer
+};
+template <typename InT, bool INLINE>
+__global__ __launch_bounds__(kWideBlock) void wide_scatter_kernel(const SampleArgs a, const typename WideTable<INLINE>::type, const WideArgs w) {
+  extern __shared__ u64 lds_keys[];
+  WideScatterShared& sh = *reinterpret_cast<WideScatterShared*>(lds_keys);
+  __shared__ uint32_t wave_sums[16], wave_own[16], red[16];
+  __shared__ u64 red64[16];
+  const WideShare mine = wide_share(w.chunks);
+  const int chunk = mine.item, row = mine.row, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  if (row >= a.rows) return;
+  const mi355x_sample_params prm = row_params<INLINE>(a, row);
+  if (!wide_row(prm)) return;
+  WideRow* const info = w.rows + row;
+  const uint32_t rmax = wide_row_max(a, w, row);
+  if (rmax == 0xffffffffu) {
+    if (chunk == 0 && tid == 0) *info = WideRow{0u, 0u, 1u, 0.0f};
+    return;
+  }
+  float v[kWidePer];
+  wide_load<InT>(static_cast<const InT*>(row_start<INLINE>(a, row, sizeof(InT))), a.vocab, chunk, v);
+  // the thread's two buckets: keys in the whole row, in the chunks before this one, and in this one
+  uint32_t all0 = 0u, all1 = 0u, before0 = 0u, before1 = 0u, own = 0u;
+  const uint32_t* h = reinterpret_cast<const uint32_t*>(a.big + static_cast<size_t>(row) * a.big_stride) + tid;
+  for (int c0 = 0; c0 < w.chunks; c0 += 8) {
+    uint32_t pair[8];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) pair[c] = c0 + c < w.chunks ? h[static_cast<size_t>(c0 + c) * kWideBlock] : 0u;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      all0 += pair[c] & 0xffffu;
+      all1 += pair[c] >> 16;
+      if (c0 + c < chunk) {
+        before0 += pair[c] & 0xffffu;
+        before1 += pair[c] >> 16;
+      }
+      own = c0 + c == chunk ? pair[c] : own;
+    }
+  }
+  const uint32_t own0 = own & 0xffffu, own1 = own >> 16;
+  const uint32_t inc = wave_prefix_sum<uint32_t>(all0 + all1), own_inc = wave_prefix_sum<uint32_t>(own0 + own1);
+  if (lane == 63) {
+    wave_sums[wave] = inc;
+    wave_own[wave] = own_inc;
+  }
+  const uint32_t widest = block_max<uint32_t>(all0 > all1 ? all0 : all1, red, false);  // (its barrier publishes the waves' sums)
+  const uint32_t ws = wave_prefix_sum<uint32_t>(lane < 16 ? wave_sums[lane] : 0u), wo = wave_prefix_sum<uint32_t>(lane < 16 ? wave_own[lane] : 0u);
+  const uint32_t n = wave_read_lane(ws, 15), n_own = wave_read_lane(wo, 15);
+  const uint32_t start0 = (wave > 0 ? wave_read_lane(ws, wave - 1) : 0u) + inc - (all0 + all1), start1 = start0 + all0;
+  const uint32_t here0 = (wave > 0 ? wave_read_lane(wo, wave - 1) : 0u) + own_inc - (own0 + own1), here1 = here0 + own0;
+  if (widest > static_cast<uint32_t>(kWideBucketMax)) {
+    if (chunk == 0 && tid == 0) *info = WideRow{0u, 0u, 1u, 0.0f};
+    return;
+  }
+  sh.place[2 * tid] = here0;
+  sh.place[2 * tid + 1] = here1;
+  sh.shift[2 * tid] = start0 + before0 - here0;
+  sh.shift[2 * tid + 1] = start1 + before1 - here1;
+  if (chunk == 0) {
+    // Tile t begins with the first bucket that starts at or after t * kWideTile: a bucket's start and the one before
+    // it enclose the multiples it is the first after.  (The first bucket starts tile 0; an empty tile begins where
+    // the next one does.)
+    uint32_t* const tile = w.tile_start + static_cast<size_t>(row) * (w.max_tiles + 1);
+    auto enclose = [&](uint32_t prev, uint32_t at) {
+      for (uint32_t t = prev / kWideTile + 1u; t <= at / kWideTile; ++t) tile[t] = at;
+    };
+    if (tid == 0) tile[0] = 0u;
+    enclose(start0, start1);  // (the start after the last bucket's is n)
+    enclose(start1, start1 + all1);
+    const uint32_t tiles = (n + kWideTile - 1u) / kWideTile;
+    if (tid == 0) {
+      if (n % kWideTile != 0u) tile[tiles] = n;  // (where n is a multiple itself, it is enclosed above)
+      *info = WideRow{n, tiles, 0u, key_to_float(rmax)};
+    }
+  }
+  __syncthreads();
+  const WideBuckets bucket_of(key_to_float(rmax), wide_depth(prm, a.vocab));
+  u64 below = 0;
+#pragma unroll
+  for (int e = 0; e < kWidePer; ++e) {
+    const uint32_t b = bucket_of(v[e]);
+    const u64 k = make_key64(order_key(v[e]), static_cast<uint32_t>(wide_index<InT>(chunk, e)));
+    if (b < static_cast<uint32_t>(kWideBuckets)) sh.keys[atomicAdd(&sh.place[b], 1u)] = k;
+    else if (v[e] == v[e]) below = k > below ? k : below;
+  }
+  below = block_max<u64>(below, red64, false);  // (its barrier: the keys are in their places)
+  if (tid == 0 && below != 0) atomicMax(reinterpret_cast<unsigned long long*>(w.best_below + row), static_cast<unsigned long long>(below));
+  u64* const keys = a.big2 + static_cast<size_t>(row) * a.big_stride;
+#pragma unroll
+  for (int e = 0; e < kWidePer; ++e) {
+    const uint32_t p = static_cast<uint32_t>(e * kWideBlock + tid);
+    if (p < n_own) {
+      const u64 k = sh.keys[p];
+      keys[p + sh.shift[bucket_of(key_to_float(key64_okey(k)))]] = k;
+    }
+  }
+}
+
+constexpr int kWideSubBuckets = 4096;
+
+struct WideRankShared {  // 50 KB: three workgroups a CU
+  union {
+    u64 keys[kSegElems];                  // by bucket, then in rank order with the exponentials in the score half
+    uint32_t first_key[kWideSubBuckets];  // while the keys are counted: the score of the first key of a bucket
+  };
+  uint32_t start[kWideSubBuckets + 1];
+  uint32_t mixed[kWideSubBuckets / 32];  // buckets that hold more than one score
+  uint64_t exp_tab[32];
+  uint32_t red[8], red2[8];
+  double dred[8];
+  Step wave_tot[8];
+};
+
+template <bool INLINE>
+__global__ __launch_bounds__(kWideRankBlock) void wide_rank_kernel(const SampleArgs a, const typename WideTable<INLINE>::type, const WideArgs w) {
+  __shared__ WideRankShared sh;
+  const WideShare mine_of_rows = wide_share(w.max_tiles);
+  const int t = mine_of_rows.item, row = mine_of_rows.row, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  if (row >= a.rows) return;
+  const mi355x_sample_params prm = row_params<INLINE>(a, row);
+  if (!wide_row(prm)) return;
+  const WideRow info = w.rows[row];
+  if (info.declined != 0u || static_cast<uint32_t>(t) >= info.tiles) return;
+  const uint32_t* const tile = w.tile_start + static_cast<size_t>(row) * (w.max_tiles + 1) + t;
+  const uint32_t first = tile[0], n = tile[1] - first;
+  const u64* const src = a.big2 + static_cast<size_t>(row) * a.big_stride + first;
+  u64 k[kWideRankPer];
+#pragma unroll
+  for (int r = 0; r < kWideRankPer; ++r) {
+    const uint32_t i = static_cast<uint32_t>(r * kWideRankBlock + tid);
+    k[r] = i < n ? src[i] : 0;
+  }
+  for (int b = tid; b <= kWideSubBuckets; b += kWideRankBlock) sh.start[b] = 0u;
+  if (tid < kWideSubBuckets / 32) sh.mixed[tid] = 0u;
+  if (tid >= 64 && tid < 96) sh.exp_tab[tid - 64] = em::exp2_tab(static_cast<uint32_t>(tid - 64));
+  uint32_t hi = 0u, lo = 0xffffffffu;
+#pragma unroll
+  for (int r = 0; r < kWideRankPer; ++r) {
+    const uint32_t o = key64_okey(k[r]);
+    hi = o > hi ? o : hi;
+    if (k[r] != 0) lo = o < lo ? o : lo;
+  }
+  hi = wave_max<uint32_t>(hi);
+  lo = wave_min_u32(lo);
+  if (lane == 0) {
+    sh.red[wave] = hi;
+    sh.red2[wave] = lo;
+  }
+  __syncthreads();
+  hi = row16_max<uint32_t>(lane < kWideRankBlock / 64 ? sh.red[lane] : 0u);
+  lo = ~row16_max<uint32_t>(lane < kWideRankBlock / 64 ? ~sh.red2[lane] : 0u);
+  const float top = key_to_float(hi), span = top - key_to_float(lo);
+  const float scale = span > 0.0f ? static_cast<float>(kWideSubBuckets) / span : 0.0f;
+  auto bucket_of = [=](u64 key) {
+    float bf = (top - key_to_float(key64_okey(key))) * scale;
+    bf = bf < static_cast<float>(kWideSubBuckets - 1) ? bf : static_cast<float>(kWideSubBuckets - 1);
+    return bf > 0.0f ? static_cast<uint32_t>(bf) : 0u;
+  };
+  uint32_t slot[kWideRankPer];
+#pragma unroll
+  for (int r = 0; r < kWideRankPer; ++r) {
+    if (k[r] != 0) {
+      const uint32_t b = bucket_of(k[r]);
+      slot[r] = atomicAdd(&sh.start[b], 1u);
+      if (slot[r] == 0u) sh.first_key[b] = key64_okey(k[r]);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < kWideRankPer; ++r) {
+    if (k[r] != 0 && slot[r] != 0u) {
+      const uint32_t b = bucket_of(k[r]);
+      if (sh.first_key[b] != key64_okey(k[r])) atomicOr(&sh.mixed[b >> 5], 1u << (b & 31u));
+    }
+  }
+  {  // the buckets' first places: eight consecutive buckets per thread
+    constexpr int kPer = kWideSubBuckets / kWideRankBlock;
+    uint32_t cnt[kPer], local = 0u;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      cnt[i] = sh.start[tid * kPer + i];
+      local += cnt[i];
+    }
+    const uint32_t inc = wave_prefix_sum<uint32_t>(local);
+    if (lane == 63) sh.red[wave] = inc;
+    __syncthreads();
+    const uint32_t ws = wave_prefix_sum<uint32_t>(lane < kWideRankBlock / 64 ? sh.red[lane] : 0u);
+    uint32_t c = (wave > 0 ? wave_read_lane(ws, wave - 1) : 0u) + inc - local;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      sh.start[tid * kPer + i] = c;
+      c += cnt[i];
+    }
+    if (tid == kWideRankBlock - 1) sh.start[kWideSubBuckets] = c;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < kWideRankPer; ++r)
+    if (k[r] != 0) sh.keys[sh.start[bucket_of(k[r])] + slot[r]] = k[r];
+  __syncthreads();
+  // Ranks, place by place (the lanes of a wave then look at the same few buckets).  A bucket of one score is in order
+  // as it lies unless the ids are asked for; so are its exponentials.
+  const bool order_ties = a.kept_ids != nullptr;
+  uint32_t fin[kWideRankPer];
+#pragma unroll
+  for (int r = 0; r < kWideRankPer; ++r) {
+    const uint32_t p = static_cast<uint32_t>(r * kWideRankBlock + tid);
+    k[r] = 0;
+    fin[r] = p;
+    if (p < n) {
+      k[r] = sh.keys[p];
+      const uint32_t b = bucket_of(k[r]);
+      const uint32_t s0 = sh.start[b], s1 = sh.start[b + 1u];
+      if (s1 - s0 > 1u && (order_ties || ((sh.mixed[b >> 5] >> (b & 31u)) & 1u))) {
+        uint32_t rank = 0u;
+        for (uint32_t j = s0; j < s1; ++j) rank += sh.keys[j] > k[r] ? 1u : 0u;
+        fin[r] = s0 + rank;
+      }
+    }
+  }
+  __syncthreads();
+  const float inv_temp = 1.0f / prm.temperature;
+  const uint64_t* const tab = sh.exp_tab;
+  auto lds_tab = [=](uint32_t i) { return tab[i]; };
+  double part = 0.0;
+#pragma unroll
+  for (int r = 0; r < kWideRankPer; ++r) {
+    const float e = k[r] != 0 ? em::expf_core((key_to_float(key64_okey(k[r])) - info.top) * inv_temp, lds_tab) : 0.0f;
+    part += static_cast<double>(e);
+    sh.keys[exp_slot(fin[r])] = (static_cast<u64>(__float_as_uint(e)) << 32) | (k[r] & 0xffffffffull);  // (zeros past the tile's end)
+  }
+  part = wave_sum<double>(part);
+  if (lane == 0) sh.dred[wave] = part;
+  __syncthreads();
+  const double own = wave_read_lane(row_scan_add(lane < kWideRankBlock / 64 ? sh.dred[lane] : 0.0), kWideRankBlock / 64 - 1);
+  double* const sums = w.tile_sum + static_cast<size_t>(row) * w.max_tiles;
+  if (tid == 0) store_sum_bits(sums + t, static_cast<unsigned long long>(__double_as_longlong(own)));
+  u64* const dst = a.big + static_cast<size_t>(row) * a.big_stride + first;
+#pragma unroll
+  for (int r = 0; r < kWideRankPer; ++r) {
+    const uint32_t p = static_cast<uint32_t>(r * kWideRankBlock + tid);
+    if (p < n) dst[p] = sh.keys[exp_slot(p)];
+  }
+  // the exact sum's step record, as in seqsum_exp_step_body: the sums of the tiles before this one tell the binade
+  double before = 0.0;
+  bool gave_up = false;
+  for (int s = tid; s < t; s += kWideRankBlock) {
+    unsigned long long bits = load_sum_bits(sums + s);
+    for (int spins = 0; bits == kSumNotReady && spins < a.poll_limit; ++spins) {
+      __builtin_amdgcn_s_sleep(1);
+      bits = load_sum_bits(sums + s);
+    }
+    if (bits == kSumNotReady) gave_up = true;
+    else before += __longlong_as_double(static_cast<long long>(bits));
+  }
+  gave_up = __syncthreads_or(gave_up ? 1 : 0) != 0;
+  before = wave_sum<double>(before);
+  if (lane == 0) sh.dred[wave] = before;
+  __syncthreads();
+  before = wave_read_lane(row_scan_add(lane < kWideRankBlock / 64 ? sh.dred[lane] : 0.0), kWideRankBlock / 64 - 1);
+  const size_t rec_at = static_cast<size_t>(row) * w.max_tiles + t;
+  int4* const rec = w.tile_step + rec_at;
+  if (gave_up) {
+    if (tid < kSegSubs) w.sub_se[rec_at * kSegSubs + tid] = -1;
+    if (tid == 0) {
+      *rec = make_int4(0, 0, -2, 0);
+      atomicAdd(a.fallback_rows + 2, 1u);
+    }
+    return;
+  }
+  float ev[kWideRankPer];
+#pragma unroll
+  for (int j = 0; j < kWideRankPer; ++j)
+    ev[j] = __uint_as_float(static_cast<uint32_t>(sh.keys[exp_slot(static_cast<uint32_t>(tid * kWideRankPer + j))] >> 32));
+  const float lo_f = __double2float_rd(before * (1.0 - seq_drift(static_cast<int>(first))));
+  const float hi_f = __double2float_ru((before + own) * (1.0 + seq_drift(static_cast<int>(first + n))));
+  const int se = seq_decompose(lo_f).se;
+  const bool known = lo_f > 0.0f && hi_f < 3.0e38f && seq_decompose(hi_f).se == se;
+  if (!known) {
+    // powers of two may fall inside the tile: records per part of 64 elements, eight lanes each
+    constexpr int kPartLanes = kWalkPart / kWideRankPer;
+    static_assert(kPartLanes == 8 && kSegSubs * kPartLanes == kWideRankBlock, "a part is eight lanes");
+    double mine = 0.0;
+#pragma unroll
+    for (int j = 0; j < kWideRankPer; ++j) mine += static_cast<double>(ev[j]);
+    mine += __longlong_as_double(static_cast<long long>(lane_xor64<1>(static_cast<u64>(__double_as_longlong(mine)))));
+    mine += __longlong_as_double(static_cast<long long>(lane_xor64<2>(static_cast<u64>(__double_as_longlong(mine)))));
+    mine += __longlong_as_double(static_cast<long long>(lane_xor64<4>(static_cast<u64>(__double_as_longlong(mine)))));
+    const int part_i = tid / kPartLanes;
+    const double upto = wave_prefix_sum<double>((lane & (kPartLanes - 1)) == 0 ? mine : 0.0);
+    __syncthreads();
+    if (lane == 63) sh.dred[wave] = upto;
+    __syncthreads();
+    double start = before + upto - mine;
+    for (int w = 0; w < wave; ++w) start += sh.dred[w];
+    const int p_first = static_cast<int>(first) + part_i * kWalkPart;
+    const float plo = __double2float_rd(start * (1.0 - seq_drift(p_first)));
+    const float phi = __double2float_ru((start + mine) * (1.0 + seq_drift(p_first + kWalkPart)));
+    int pse = seq_decompose(plo).se;
+    if (!(plo > 0.0f && phi < 3.0e38f && seq_decompose(phi).se <= pse + 1)) pse = -1;  // the walk adds this part itself
+    Step lo_step{0u, 0u}, hi_step{0u, 0u};
+    if (pse >= 0) {
+      lo_step = seq_compose_run(ev, kWideRankPer, pse);
+      hi_step = seq_compose_run(ev, kWideRankPer, pse + 1);
+    }
+    lo_step = oct_scan_steps(lo_step);
+    hi_step = oct_scan_steps(hi_step);
+    if ((lane & (kPartLanes - 1)) == kPartLanes - 1) {
+      const size_t at = rec_at * kSegSubs + part_i;
+      w.sub_step[at] = make_int4(static_cast<int>(lo_step.d0), static_cast<int>(lo_step.d1), static_cast<int>(hi_step.d0),
+                                      static_cast<int>(hi_step.d1));
+      w.sub_se[at] = pse;
+    }
+    if (tid == 0) *rec = make_int4(0, 0, -2, 0);
+    return;
+  }
+  const Step inc = wave_scan_steps(seq_compose_run(ev, kWideRankPer, se));
+  if (lane == 63) sh.wave_tot[wave] = inc;
+  __syncthreads();
+  if (tid == 0) {
+    Step s = sh.wave_tot[0];
+    for (int w = 1; w < kWideRankBlock / 64; ++w) s = step_compose(s, sh.wave_tot[w]);
+    *rec = make_int4(static_cast<int>(s.d0), static_cast<int>(s.d1), se, 0);
+  }
+}
+
+// The tiles of a row as the walk reads them.
+struct WideSegments {
+  int segs;
+  const int4* seg_step;
+  const int4* sub_step;
+  const int* sub_se;
+  const u64* list;             // (exponential, ~id) entries in rank order
+  const uint32_t* tile_start;  // LDS
+  __device__ __forceinline__ int first(int sg) const { return static_cast<int>(tile_start[sg]); }
+  __device__ __forceinline__ int count(int sg) const { return static_cast<int>(tile_start[sg + 1] - tile_start[sg]); }
+  __device__ __forceinline__ float value(int i) const { return __uint_as_float(static_cast<uint32_t>(list[i] >> 32)); }
+};
+
+struct WideFinishShared {
+  WalkShared walk;
+  uint32_t tile_start[kWideMaxTiles + 1];
+  float ends[kWideMaxTiles];       // the exact sequential sum behind every tile
+  double weight[kWideMaxTiles];    // a tile's share of the kept weight ...
+  double upto[kWideMaxTiles];      // ... and the shares of all tiles up to it
+  u64 ties[kSegElems];
+};
+static_assert(sizeof(WideFinishShared) <= kFinishLds, "the finish runs in the finish kernels' LDS");
+
+// First position whose cumulative weight reaches u times the total, for weights w(0 .. keep) that the caller has
+// summed per tile into sh.weight[0 .. used) (double).  A comparison within `band` of the total decides nothing:
+// returns -1.  The last position's value is forced to one, as std::discrete_distribution forces it.
+template <typename W>
+__device__ __forceinline__ int wide_draw(W w, int keep, int used, double u, double band, WideFinishShared& sh, SeqShared& seqsh) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  if (wave == 0) {
+    constexpr int kPer = kWideMaxTiles / 64;
+    double s[kPer], loc = 0.0;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      loc += lane * kPer + i < used ? sh.weight[lane * kPer + i] : 0.0;
+      s[i] = loc;
+    }
+    const double before = wave_scan_add(loc) - loc;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) sh.upto[lane * kPer + i] = before + s[i];
+  }
+  __syncthreads();
+  const double total = sh.upto[used - 1];
+  const double target = u * total, guard = band * total;
+  // the tile the target falls into, the last one if none reaches it
+  int lo = 0, hi = used - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (sh.upto[mid] >= target) hi = mid;
+    else lo = mid + 1;
+  }
+  const int first = static_cast<int>(sh.tile_start[lo]);
+  const int end = keep < static_cast<int>(sh.tile_start[lo + 1]) || lo == used - 1 ? keep : static_cast<int>(sh.tile_start[lo + 1]);
+  const double base = lo > 0 ? sh.upto[lo - 1] : 0.0;
+  int risky = (lo > 0 && fabs(base - target) <= guard) ? 1 : 0, found = kIntMax;
+  constexpr int kPer = 5;  // a tile and the entry that may follow the last one
+  static_assert(kPer * kFinishBlock > kSegElems, "a tile in one window");
+  double pv[kPer], loc = 0.0;
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    const int i = first + tid * kPer + j;
+    pv[j] = i < end ? w(i) : 0.0;
+    loc += pv[j];
+  }
+  const double inc = wave_scan_add(loc);
+  if (lane == 63) seqsh.dscan[wave] = inc;
+  __syncthreads();
+  const double ws = row_scan_add(lane < 16 ? seqsh.dscan[lane] : 0.0);
+  double run = base + (wave > 0 ? wave_read_lane(ws, wave - 1) : 0.0) + (inc - loc);
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    const int i = first + tid * kPer + j;
+    run += pv[j];
+    if (i < end) {
+      if (i != keep - 1 && fabs(run - target) <= guard) risky = 1;
+      if ((i == keep - 1 || run >= target) && i < found) found = i;
+    }
+  }
+  int calm = risky ? 0 : 1;
+  block_min2(found, calm, seqsh);
+  return calm == 0 || found == kIntMax ? -1 : found;
+}
+
+// Runs by the whole workgroup; false: the row needs the exact path.
+template <bool INLINE>
+__device__ __forceinline__ bool wide_finish_row(const SampleArgs& a, const WideArgs& w, int row, mi355x_sample_params prm, WideFinishShared& sh, SeqShared& seqsh) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, V = a.vocab;
+  const WideRow info = w.rows[row];
+  if (info.declined != 0u || info.n == 0u) return false;
+  const int n = static_cast<int>(info.n), tiles = static_cast<int>(info.tiles);
+  const size_t rbase = static_cast<size_t>(row) * w.max_tiles;
+  for (int t = tid; t <= tiles; t += kFinishBlock) sh.tile_start[t] = w.tile_start[static_cast<size_t>(row) * (w.max_tiles + 1) + t];
+  for (int t = tid; t < tiles; t += kFinishBlock) sh.weight[t] = w.tile_sum[rbase + t];
+  const u64 below = w.best_below[row];  // the best element past the list; it follows the list's last
+  const u64* const list = a.big + static_cast<size_t>(row) * a.big_stride;
+  const double u = a.uniforms[row];
+  __syncthreads();
+  const WideSegments segments{tiles, w.tile_step + rbase, w.sub_step + rbase * kSegSubs, w.sub_se + rbase * kSegSubs, list, sh.tile_start};
+  walk_segments<true>(segments, sh.walk, sh.ends);
+  __syncthreads();
+  const float inv_temp = 1.0f / prm.temperature;
+  const int limit = n + (below != 0 ? 1 : 0);
+  const float e_below = below != 0 ? em::expf_exact((key_to_float(key64_okey(below)) - info.top) * inv_temp) : 0.0f;
+  auto exps = [=](int i) { return i < n ? __uint_as_float(static_cast<uint32_t>(list[i] >> 32)) : e_below; };
+  // the first tile the stop of FindNucleus may lie in: it lies in none whose last element misses it by a margin
+  const float p = prm.p;
+  const StopAtNucleus stop{p, V, 0};
+  int first_tile = tiles;
+  for (int t = tid; t < tiles; t += kFinishBlock) {
+    const int last = static_cast<int>(sh.tile_start[t + 1]) - 1;
+    const bool empty = sh.tile_start[t] == sh.tile_start[t + 1];
+    if (!empty && !stop.nowhere_in_run_ending(sh.ends[t], exps(last), last) && t < first_tile) first_tile = t;
+  }
+  int dummy = kIntMax;
+  block_min2(first_tile, dummy, seqsh);
+  int base = first_tile < tiles ? static_cast<int>(sh.tile_start[first_tile]) : n;
+  float prefix = first_tile > 0 ? sh.ends[first_tile - 1] : 0.0f;
+  int keep;
+  for (;;) {  // (the batches of the reference's search: see block_sample_epilogue)
+    const int b = base;
+    int si;
+    prefix = block_seq_sum<8>(prefix, limit - b, [=](int i) { return exps(i + b); }, StopAtNucleus{p, V, b}, &si, seqsh, nullptr, b == 0 ? kEpiHead : 0);
+    if (si < 0) {
+      if (limit != V) return false;
+      keep = V;
+      break;
+    }
+    keep = b + si + 1;
+    const bool batch_end = keep >= 16 && (keep & (keep - 1)) == 0 && ((__ffs(keep) - 1) & 1) == 0;
+    if (!batch_end || keep >= V) break;
+    if (keep >= limit) return false;
+    base = keep;
+  }
+  const float scale = prefix > 0.0f ? 1.0f / prefix : 0.0f;
+  // Where the draw falls.  The reference's weights are q_i = e_i * scale, rounded to fp32; the common factor cancels
+  // and the roundings move no cumulative share by more than 2^-23, so unless the target lies within 1.3e-7 of the total
+  // of a cumulative value, the exponentials' own double sums decide.  Otherwise the weights themselves are summed.
+  int used = 0;  // tiles that hold kept entries
+  {
+    int lo = 0, hi = tiles - 1;
+    while (lo < hi) {  // the tile of entry keep - 1 (the last one for the entry that follows the list)
+      const int mid = (lo + hi) >> 1;
+      if (static_cast<int>(sh.tile_start[mid + 1]) >= keep) hi = mid;
+      else lo = mid + 1;
+    }
+    used = lo + 1;
+  }
+  int pos = 0;
+  if (keep >= 2) {
+    {  // the last of these tiles counts only as far as it is kept
+      double part = 0.0;
+      for (int i = static_cast<int>(sh.tile_start[used - 1]) + tid; i < keep; i += kFinishBlock) part += static_cast<double>(exps(i));
+      part = wave_sum<double>(part);
+      if (lane == 0) seqsh.dred[wave] = part;
+      __syncthreads();
+      if (tid == 0) {
+        double s = 0.0;
+        for (int w = 0; w < kFinishBlock / 64; ++w) s += seqsh.dred[w];
+        sh.weight[used - 1] = s;
+      }
+      __syncthreads();
+    }
+    pos = wide_draw([=](int i) { return static_cast<double>(exps(i)); }, keep, used, u, 1.3e-7, sh, seqsh);
+    if (pos < 0) {
+      for (int t = wave; t < used; t += kFinishBlock / 64) {
+        const int end = t == used - 1 ? keep : static_cast<int>(sh.tile_start[t + 1]);
+        double s = 0.0;
+#pragma unroll 4
+        for (int i = static_cast<int>(sh.tile_start[t]) + lane; i < end; i += 64) s += static_cast<double>(exps(i) * scale);
+        s = wave_sum<double>(s);
+        if (lane == 0) sh.weight[t] = s;
+      }
+      __syncthreads();
+      pos = wide_draw([=](int i) { return static_cast<double>(exps(i) * scale); }, keep, used, u, 16.0 * keep * 1.1102230246251565e-16, sh, seqsh);
+      if (pos < 0) pos = block_discrete_draw<4>(keep, [=](int i) { return exps(i) * scale; }, u, seqsh);  // (replays the reference's own operations)
+    }
+  }
+  const RowOutputs out = row_outputs(a, row);
+  if (out.kept_count && tid == 0) *out.kept_count = keep;
+  if (out.kept_ids) {
+    const int kept = keep < out.kept_capacity ? keep : out.kept_capacity;
+    const int lim = out.pad ? out.kept_capacity : kept;
+    for (int i = tid; i < lim; i += kFinishBlock) {
+      const bool in = i < kept;
+      out.kept_ids[i] = in ? static_cast<int32_t>(key64_index(i < n ? list[i] : below)) : -1;
+      if (out.kept_probs) out.kept_probs[i] = in ? exps(i) * scale : 0.0f;
+    }
+  }
+  if (pos >= n) {
+    if (tid == 0) *out.token = static_cast<int32_t>(key64_index(below));
+    return true;
+  }
+  // entries of one exponential may be ties in arrival order: the run the draw fell into is ordered by whole keys
+  const uint32_t mine = static_cast<uint32_t>(list[pos] >> 32);
+  int lo = 0, hi = tiles - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (static_cast<int>(sh.tile_start[mid + 1]) > pos) hi = mid;
+    else lo = mid + 1;
+  }
+  const int t0 = static_cast<int>(sh.tile_start[lo]), t1 = static_cast<int>(sh.tile_start[lo + 1]);
+  int run_lo = kIntMax, run_hi = kIntMax;  // first entry of the run, and minus its last
+  for (int i = t0 + tid; i < t1; i += kFinishBlock) {
+    if (static_cast<uint32_t>(list[i] >> 32) == mine) {
+      run_lo = i < run_lo ? i : run_lo;
+      run_hi = -i < run_hi ? -i : run_hi;
+    }
+  }
+  block_min2(run_lo, run_hi, seqsh);
+  const int run = -run_hi - run_lo + 1;
+  if (run == 1) {
+    if (tid == 0) *out.token = static_cast<int32_t>(key64_index(list[pos]));
+    return true;
+  }
+  const RowPtr<AnyDtype> lrow(row_start<INLINE>(a, row, dtype_bytes(a.dtype)), a.dtype);
+  for (int i = tid; i < run; i += kFinishBlock) {
+    const uint32_t id = key64_index(list[run_lo + i]);
+    sh.ties[i] = make_key64(order_key(lrow[id]), id);
+  }
+  __syncthreads();
+  for (int i = tid; i < run; i += kFinishBlock) {
+    const u64 k = sh.ties[i];
+    int rank = 0;
+    for (int j = 0; j < run; ++j) rank += sh.ties[j] > k ? 1 : 0;
+    if (rank == pos - run_lo) *out.token = static_cast<int32_t>(key64_index(k));
+  }
+  return true;
+}
+
+template <bool INLINE>
+__global__ __launch_bounds__(kFinishBlock) void wide_finish_kernel(const SampleArgs a, const typename WideTable<INLINE>::type, const WideArgs w) {
+  extern __shared__ u64 lds_keys[];
+  __shared__ SeqShared seqsh;
+  __shared__ uint32_t red32[16];
+  __shared__ u64 red64[16];
+  const int row = blockIdx.x;
+  const mi355x_sample_params prm = row_params<INLINE>(a, row);
+  if (!wide_row(prm)) return;
+  if (wide_finish_row<INLINE>(a, w, row, prm, *reinterpret_cast<WideFinishShared*>(lds_keys), seqsh)) {
+    if (threadIdx.x == 0) atomicAdd(a.fallback_rows, 1u);  // (a row of the exact path, spread over the GPU)
+    return;
+  }
+  __syncthreads();
+  general_row<AnyDtype, SortWithTile, 8>(a, row, row_start<INLINE>(a, row, dtype_bytes(a.dtype)), prm, a.big + static_cast<size_t>(row) * a.big_stride, seqsh,
+                                         SortWithTile{a.big2 + static_cast<size_t>(row) * a.big_stride, lds_keys, red32, red64});
+}
+
+template <bool INLINE>
+hipError_t launch_wide(const SampleArgs& a, const typename WideTable<INLINE>::type& table, const WideArgs& w, hipStream_t stream) {
+  const int rows8 = (a.rows + 7) & ~7;  // (see wide_share)
+  const dim3 grid(w.chunks * rows8), block(kWideBlock);
+  auto passes = [&](auto elt) {
+    typedef decltype(elt) InT;
+    hipLaunchKernelGGL((wide_max_kernel<InT, INLINE>), grid, block, 0, stream, a, table, w);
+    hipLaunchKernelGGL((wide_count_kernel<InT, INLINE>), grid, block, 0, stream, a, table, w);
+    hipLaunchKernelGGL((wide_scatter_kernel<InT, INLINE>), grid, block, sizeof(WideScatterShared), stream, a, table, w);
+  };
+  if (a.dtype == MI355X_F16) passes(uint16_t{});
+  else if (a.dtype == MI355X_BF16) passes(bf16_t{});
+  else passes(float{});
+  hipLaunchKernelGGL(wide_rank_kernel<INLINE>, dim3(w.max_tiles * rows8), dim3(kWideRankBlock), 0, stream, a, table, w);
+  hipLaunchKernelGGL(wide_finish_kernel<INLINE>, dim3(a.rows), dim3(kFinishBlock), kFinishLds, stream, a, table, w);
+  return hipGetLastError();
+}
+
+}  // namespace ms
