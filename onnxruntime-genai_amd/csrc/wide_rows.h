@@ -1,9 +1,13 @@
 // Rows that need most of their vocabulary in rank order: sampling from the whole vocabulary (k <= 1 with p >= 1).
+// (Nuclei of p < 1 stay with the candidate lists of nucleus_stream_kernel: routed through here 64 x 128256 rows with
+// nuclei of 4000 tokens took 84 us per step instead of 41.)
 //
 // The reference sorts such a row, adds the exponentials of all of it one after the other and draws from the result.
 // One workgroup per row (exact_rows_kernel) spends 0.55 ms on that however few rows there are: its sort moves every
 // key three times at the memory rate of a single CU, and its sums run over 128 K exponentials in one workgroup.  Here
-// every step but the last is spread over the GPU, in five launches (16 x 128256 fp16: 557 -> WIDE_US us per step):
+// every step but the last is spread over the GPU, in five launches (16 x 128256 fp16: 557 -> 59 us per step:
+// 4.7 + 4.7 + 12 + 21 + 21 us by a trace; every one of them is a chain of dependent phases of a few barriers each, no
+// launch moves more than 33 MB):
 //   1. wide_max:     the maximum of every 16384-logit chunk.
 //   2. wide_count:   a histogram per chunk over kWideBuckets buckets, linear in the score below the row's maximum down
 //                    to the depth past which no element can lie inside the kept set.
@@ -48,7 +52,7 @@ __device__ __forceinline__ float wide_depth(mi355x_sample_params prm, int vocab)
 // Which row, and which of its `per_row` shares of the work, a workgroup has.  Workgroups go round-robin over the eight
 // XCDs; all shares of a row get indices of one remainder, so what they hand over -- every launch reads what the one
 // before it wrote, scattered all over the row's buffers -- stays in one L2 (scattered from all XCDs, the keys' 8-byte
-// writes reach memory one partial line each: 18.2 us of the scatter at 16 x 128256).  Rows past the last have no work.
+// writes would reach memory one partial line each).  Rows past the last have no work.
 struct WideShare {
   int row, item;
 };

@@ -1374,3 +1374,41 @@ def test_draw_in_order_follows_one_engine(ctx, orc, rows, cap):
     _, used = ctx.draw_in_order(torch.from_numpy(broken).cuda(), torch.from_numpy(ids).cuda(),
                                 torch.from_numpy(probs).cuda(), torch.from_numpy(pool).cuda(), None)
     assert used.item() == -1
+
+
+@pytest.mark.parametrize("vocab", [4095, 4096, 8191, 8193, 12289, 50257, 128256])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_whole_vocabulary_rows_spread_over_the_gpu(ctx, orc, vocab, dtype):
+    """Temperature-only sampling (k = 0, p >= 1): token-only calls, whose ties stay unordered until the draw, on rows
+    that end on and beside the edges of chunks and tiles; kept sets of a few entries; a batch of scattered rows of
+    which only some sample from the whole vocabulary; rows the spread path declines (one score for all, a maximum of
+    -1e38, a bucket too full) among the others."""
+    say("whole vocabulary", vocab, dtype)
+    rng = np.random.default_rng(vocab)
+    rows = 11
+    x = (rng.standard_normal((rows, vocab)) * np.linspace(0.5, 5.0, rows)[:, None]).astype(np.float32)
+    x[1, : vocab // 2] = np.round(x[1, : vocab // 2])  # runs of ties longer than a bucket holds
+    x[2, :] = 0.25
+    x[3, :] = -1e38
+    x[4, 7] = 90.0      # one token far above the rest
+    x[5, 11:400] = np.nan
+    x[6, vocab - 1] = np.inf
+    x[7, ::3] = -np.inf
+    xd = torch.from_numpy(x).cuda().to(dtype)
+    xw = x if dtype == torch.float32 else ctx.logits_handoff(xd.view(rows, 1, vocab)).cpu().numpy()
+    u = rng.random(rows)
+    u[0], u[8], u[9] = 0.0, 0.9999999999, 1e-12
+    ud = torch.from_numpy(u).cuda()
+    for p, t in ((1.0, 1.0), (1.0, 0.3), (2.0, 1.5)):
+        want = orc.sample_batch(xw, 0, p, t, u)
+        assert np.array_equal(ctx.sample(xd, ud, k=0, p=p, temperature=t).cpu().numpy(), want), (p, t)
+        tok, kc, ki, kp = [v.cpu().numpy() for v in ctx.sample(xd, ud, k=1, p=p, temperature=t, kept_capacity=300)]
+        assert np.array_equal(tok, want), (p, t)
+        for r in range(rows):
+            idx, probs = orc.sampled_categorical(xw[r], 1, p, t)
+            n = min(len(idx), 300)
+            assert kc[r] == len(idx) and np.array_equal(ki[r, :n], idx[:n]) and np.array_equal(bits(kp[r, :n]), bits(probs[:n])), (p, t, r)
+            assert (ki[r, n:] == -1).all() and (kp[r, n:] == 0).all()
+    params = [[(0, 1.0, 0.8), (20, 0.9, 1.0), (0, 0.7, 1.0)][r % 3] for r in range(rows)]
+    got = ctx.sample([row.clone() for row in xd], ud, per_row=params).cpu().numpy()
+    assert np.array_equal(got, [orc.sample_row(xw[r], *params[r], u[r]) for r in range(rows)])
