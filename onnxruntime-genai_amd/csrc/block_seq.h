@@ -662,11 +662,13 @@ struct RowOutputs {
 // sorted(i) returns the key64 of the i-th best element for i < n_sorted.  exps(i) must return
 // exp((score_i - score_0) * inv_temp) as a float (callers may cache it).  Returns false -- without
 // writing outputs -- when the nucleus does not end inside the n_sorted available elements.  synced: every thread
-// has passed a barrier since `sh` was last used, so the first sum need not begin with one.
-template <int ITEMS, typename Sorted, typename Exps>
+// has passed a barrier since `sh` was last used, so the first sum need not begin with one.  id_at(i), when given: the
+// id of the i-th best element, called by the whole block for the drawn position (the id in sorted(i) otherwise).
+struct IdAsSorted {};
+template <int ITEMS, typename Sorted, typename Exps, typename IdAt = IdAsSorted>
 __device__ __forceinline__ bool block_sample_epilogue(Sorted sorted, Exps exps, int n_sorted, int vocab,
                                       mi355x_sample_params prm, double u, const RowOutputs& out,
-                                      SeqShared& sh, bool synced = false) {
+                                      SeqShared& sh, bool synced = false, IdAt id_at = IdAt{}) {
   int keep;
   float scale;     // kept probability j = base_j * scale, base_j = exps(j) or exps(j)/sum
   float sum = 1.0f;
@@ -756,7 +758,10 @@ __device__ __forceinline__ bool block_sample_epilogue(Sorted sorted, Exps exps, 
     }
   }
   const int pos = block_discrete_draw<ITEMS>(keep, q, u, sh);
-  if (threadIdx.x == 0) *out.token = static_cast<int32_t>(key64_index(sorted(pos)));
+  uint32_t id;
+  if constexpr (std::is_same<IdAt, IdAsSorted>::value) id = key64_index(sorted(pos));
+  else id = id_at(pos);
+  if (threadIdx.x == 0) *out.token = static_cast<int32_t>(id);
   return true;
 }
 

@@ -389,11 +389,15 @@ struct EmitTopk {
 // the best and of (a bound below) the lowest candidate, which scale the buckets of the sort.  Returns false
 // when the row needs the exact path (the epilogue found no end of the nucleus among the elements given).
 // presorted: lds_keys[0 .. n_c) are sorted and hold their exponentials already (sort_gathered), only the epilogue is left.
+// TIES: ties_row0, when not null, says that entries of one score are in no particular order and where the row's logits
+// (of type ties_dtype) start: the run of entries that share the drawn one's exponential is ordered before its id is taken.
+template <bool TIES = false>
 __device__ __forceinline__ bool finish_candidates(u64* lds_keys, uint32_t* bucket_start, uint32_t n_c, u64 best_below,
                                                   uint32_t rmax, uint32_t thr, bool cut_at_best_below,
                                                   mi355x_sample_params prm, int V, double u, const RowOutputs& out,
                                                   SeqShared& seqsh, uint32_t* red32, EmitTopk emit = EmitTopk{},
-                                                  bool presorted = false, u64 second_below = 0) {
+                                                  bool presorted = false, u64 second_below = 0,
+                                                  const void* ties_row0 = nullptr, int ties_dtype = 0) {
   const int tid = threadIdx.x;
   const u64* lk = lds_keys;
   auto sorted = [=](int i) { return lk[exp_slot(static_cast<uint32_t>(i))]; };
@@ -471,7 +475,41 @@ __device__ __forceinline__ bool finish_candidates(u64* lds_keys, uint32_t* bucke
     }
     __syncthreads();
   }
-  return block_sample_epilogue<8>(sorted, exps, static_cast<int>(n_c), V, prm, u, out, seqsh, true);  // (a barrier has just passed)
+  if constexpr (TIES) {
+    const int n = static_cast<int>(n_c);
+    auto id_at = [&](int pos) __attribute__((always_inline)) -> uint32_t {
+      auto e_bits = [=](int i) { return static_cast<uint32_t>(lk[exp_slot(static_cast<uint32_t>(i))] >> 32); };
+      const uint32_t mine = e_bits(pos);
+      if (ties_row0 == nullptr || ((pos == 0 || e_bits(pos - 1) != mine) && (pos + 1 >= n || e_bits(pos + 1) != mine)))
+        return key64_index(sorted(pos));
+      int first = kIntMax, last = kIntMax;  // of the run; the last one negated
+      for (int i = tid; i < n; i += kFinishBlock) {
+        if (e_bits(i) == mine) {
+          first = i < first ? i : first;
+          last = -i < last ? -i : last;
+        }
+      }
+      block_min2(first, last, seqsh);  // (its barriers: every thread has read the list)
+      last = -last;
+      const RowPtr<AnyDtype> lrow(ties_row0, ties_dtype);
+      for (int i = first + tid; i <= last; i += kFinishBlock) {
+        const uint32_t id = key64_index(sorted(i));
+        lds_keys[exp_slot(static_cast<uint32_t>(i))] = make_key64(order_key(lrow[id]), id);
+      }
+      __syncthreads();
+      for (int i = first + tid; i <= last; i += kFinishBlock) {
+        const u64 k = sorted(i);
+        int rank = first;
+        for (int j = first; j <= last; ++j) rank += sorted(j) > k ? 1 : 0;
+        if (rank == pos) seqsh.bcast_i = static_cast<int>(key64_index(k));
+      }
+      __syncthreads();
+      return static_cast<uint32_t>(seqsh.bcast_i);
+    };
+    return block_sample_epilogue<8>(sorted, exps, n, V, prm, u, out, seqsh, true, id_at);  // (a barrier has just passed)
+  } else {
+    return block_sample_epilogue<8>(sorted, exps, static_cast<int>(n_c), V, prm, u, out, seqsh, true);  // (a barrier has just passed)
+  }
 }
 
 // Drops the candidates that certainly lie past the end of the nucleus, so that only the rest is sorted.
@@ -727,14 +765,37 @@ __device__ __forceinline__ TrimmedBuckets scan_buckets_and_trim(uint32_t* start,
 // caches exp((score - max) / T) in the score half of every entry, at exp_slot(rank), the way the epilogue reads the
 // list (rmax: order key of the row's maximum).  SHIFTED: the keys were placed by counting start[b] up, so bucket b
 // now lies between start[b - 1] and start[b]; otherwise between start[b] and start[b + 1].
+// mixed (one bit per bucket, zero), when given: a bucket whose keys all have one score keeps them in the order they
+// lie in.  Sixteen-bit logits have up to a few hundred ties per value, and a compare per pair of them buys nothing
+// that a draw needs: the exponentials are the same in any order (whoever needs the ids of ties orders them later).
+// Returns false, with the keys where they were, when a bucket of several scores holds more than kMixedCap keys.
+constexpr uint32_t kMixedCap = 256;
 template <bool SHIFTED>
-__device__ __forceinline__ void rank_and_cache_exps(u64* keys, const uint32_t* start, const ScoreBuckets& bucket_of,
-                                                    const TrimmedBuckets& kept, uint32_t rmax, float inv_temp) {
+__device__ __forceinline__ bool rank_and_cache_exps(u64* keys, const uint32_t* start, const ScoreBuckets& bucket_of,
+                                                    const TrimmedBuckets& kept, uint32_t rmax, float inv_temp, uint32_t* mixed = nullptr) {
   const int t = threadIdx.x;
   constexpr int R = kNucleusCap / kFinishBlock;
   const uint32_t n_pad = (kept.n + 7u) & ~7u;
   u64 k[R];
   uint32_t fin[R];
+  if (mixed != nullptr) {
+    int too_full = 0;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const uint32_t pos = static_cast<uint32_t>(r * kFinishBlock + t);
+      if (pos < kept.n_sorted) {
+        const uint32_t okey = key64_okey(keys[pos]);
+        const uint32_t b = bucket_of(okey);
+        const uint32_t lo = SHIFTED ? (b > 0u ? start[b - 1u] : 0u) : start[b];
+        const uint32_t hi = SHIFTED ? start[b] : start[b + 1u];
+        if (hi - lo > 1u && key64_okey(keys[lo]) != okey) {
+          atomicOr(&mixed[b >> 5], 1u << (b & 31u));
+          if (hi - lo > kMixedCap) too_full = 1;
+        }
+      }
+    }
+    if (__syncthreads_or(too_full)) return false;
+  }
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     if (static_cast<uint32_t>(r * kFinishBlock) < n_pad) {
@@ -747,9 +808,11 @@ __device__ __forceinline__ void rank_and_cache_exps(u64* keys, const uint32_t* s
         const uint32_t b = bucket_of(key64_okey(k[r]));
         const uint32_t lo = SHIFTED ? (b > 0u ? start[b - 1u] : 0u) : start[b];
         const uint32_t hi = SHIFTED ? start[b] : start[b + 1u];
-        uint32_t rank = 0u;
-        for (uint32_t j = lo; j < hi; ++j) rank += keys[j] > k[r] ? 1u : 0u;
-        fin[r] = lo + rank;
+        if (mixed == nullptr || ((mixed[b >> 5] >> (b & 31u)) & 1u)) {
+          uint32_t rank = 0u;
+          for (uint32_t j = lo; j < hi; ++j) rank += keys[j] > k[r] ? 1u : 0u;
+          fin[r] = lo + rank;
+        }
       }
     }
   }
@@ -767,6 +830,7 @@ __device__ __forceinline__ void rank_and_cache_exps(u64* keys, const uint32_t* s
     }
   }
   __syncthreads();
+  return true;
 }
 
 // Per-row finish of the nucleus path: gathers the candidates the streaming pass left in `big`,
@@ -780,6 +844,7 @@ __device__ __forceinline__ void nucleus_finish_body(const SampleArgs& a) {
   __shared__ uint32_t sh_count;
   __shared__ uint32_t red32[16];
   __shared__ u64 red64[16];
+  __shared__ uint32_t mixed_buckets[kSortBuckets / 32];
   const int row = blockIdx.x;
   const int V = a.vocab;
   const int tid = threadIdx.x;
@@ -805,6 +870,11 @@ __device__ __forceinline__ void nucleus_finish_body(const SampleArgs& a) {
     pre[q] = (a.chunks <= kAheadChunks && c < a.chunks) ? big_row[static_cast<size_t>(c) * kSChunk + u * kFinishBlock + tid] : 0;
   }
   for (int b = tid; b <= kSortBuckets; b += kFinishBlock) bucket_start[b] = 0u;  // the sort's table, while the loads are on their way
+  // Rows of sixteen-bit logits whose token alone is asked for keep ties as they come (see rank_and_cache_exps); the
+  // run of ties the draw falls into is ordered then.  (fp32 rows have few; rows whose logits are processed on the way
+  // in would need that processing there.)
+  const bool free_ties = a.dtype != MI355X_F32 && a.kept_ids == nullptr && a.emit_topk == 0 && !a.xf.active();
+  if (tid < kSortBuckets / 32) mixed_buckets[tid] = 0u;
   // Lane c of every wave reads what chunk c left behind (at most 16 chunks), so the row's maximum and threshold
   // are reductions inside the wave, with no exchange between the waves; wave 0 publishes the counts and where
   // every list's rows begin, behind the one barrier that follows.
@@ -959,7 +1029,8 @@ __device__ __forceinline__ void nucleus_finish_body(const SampleArgs& a) {
       }
     });
     __syncthreads();
-    TrimmedBuckets kept = scan_buckets_and_trim(bucket_start, bucket_of, below, prm, V, kNucleusCap, red32, red64, k_wanted);
+    TrimmedBuckets kept = scan_buckets_and_trim(bucket_start, bucket_of, below, prm, V, kNucleusCap, red32, red64, k_wanted,
+                                                free_ties ? kNucleusCap : kBucketCap);
     if constexpr (!LARGEK) {
       // The list ends with the one element below the candidates and has 16, 64, 256 ... entries: should the search
       // stop on that last element, the reference notices it one element later (src/sampling_distribution.h:166-181),
@@ -1025,8 +1096,8 @@ __device__ __forceinline__ void nucleus_finish_body(const SampleArgs& a) {
         }
       });
       __syncthreads();
-      rank_and_cache_exps<true>(lds_keys, bucket_start, bucket_of, kept, rmax, 1.0f / prm.temperature);
-      presorted = ok = true;
+      presorted = ok = rank_and_cache_exps<true>(lds_keys, bucket_start, bucket_of, kept, rmax, 1.0f / prm.temperature,
+                                                 free_ties ? mixed_buckets : nullptr);
       n_c = kept.n;
     }
   }
@@ -1231,8 +1302,9 @@ __device__ __forceinline__ void nucleus_finish_body(const SampleArgs& a) {
     EmitTopk target;  // (by value: a pointer to the kernel's arguments would put all of them on the stack)
     if (emit) target = EmitTopk{a.out_tokens + static_cast<size_t>(row) * prm.k, a.out_scores + static_cast<size_t>(row) * prm.k,
                                 row_start<INLINE>(a, row, dtype_bytes(a.dtype)), a.dtype};
-    ok = finish_candidates(lds_keys, bucket_start, n_c, presorted ? 0 : best_below, rmax, thr, false, prm, V,
-                           emit ? 0.0 : a.uniforms[row], row_outputs(a, row), seqsh, red32, target, presorted);
+    ok = finish_candidates<true>(lds_keys, bucket_start, n_c, presorted ? 0 : best_below, rmax, thr, false, prm, V,
+                                 emit ? 0.0 : a.uniforms[row], row_outputs(a, row), seqsh, red32, target, presorted, 0,
+                                 presorted && free_ties ? row_start<INLINE>(a, row, dtype_bytes(a.dtype)) : nullptr, a.dtype);
   }
   if (!ok && !wide_ok) {
     __syncthreads();

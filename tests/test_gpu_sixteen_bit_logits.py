@@ -297,3 +297,28 @@ def test_captured_calls_with_host_tables_use_up_staging_slots():
         c.kv_gather(present, past, idx)
     torch.cuda.synchronize()
     c.close()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("k,p,temp", [(0, 0.9, 1.0), (0, 0.97, 0.7), (0, 0.9, 1e6), (300, 0.0, 1.0), (1000, 0.95, 2.0)])
+def test_draws_that_fall_into_runs_of_ties(ctx, orc, dtype, k, p, temp):
+    """Token-only calls keep ties of sixteen-bit logits unordered until the draw falls into a run of them: runs of two
+    to thousands of equal scores, runs that the kept set ends inside, rows of few distinct values, a temperature at
+    which different scores share an exponential, and buckets that hold many keys of several scores."""
+    say("ties", dtype, k, p, temp)
+    rng = np.random.default_rng(int(k + 100 * p))
+    rows, vocab = 12, 60013
+    x = (rng.standard_normal((rows, vocab)) * 2).astype(np.float32)
+    x[1:4] += 16.0                                           # coarse steps: hundreds of ties per value
+    x[4, rng.integers(0, vocab, 500)] = 12.0                 # the best score itself is a run
+    x[5, rng.integers(0, vocab, 3000)] = 14.0
+    x[6] = np.round(x[6] * 2) / 2 + 8.0                      # a dozen distinct values
+    x[7, rng.integers(0, vocab, 6000)] = 0.001 * rng.standard_normal(6000)  # many scores close to zero
+    x[7, 9] = 6.0
+    x[8, :2] = 20.0
+    x16 = torch.from_numpy(x).cuda().to(dtype)
+    wide = widened(orc, x16)
+    for rep in range(3):
+        u = rng.random(rows)
+        got = ctx.sample(x16, torch.from_numpy(u).cuda(), k=k, p=p, temperature=temp).cpu().numpy()
+        assert np.array_equal(got, orc.sample_batch(wide, k, p, temp, u)), rep
