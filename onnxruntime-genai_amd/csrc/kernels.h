@@ -44,11 +44,6 @@ struct InlineParams {
   const void* row_ptr[kInlineParamRows];  // where each row starts, for rows scattered over memory; null: row_stride apart
 };
 
-struct SideStreams {
-  hipStream_t side[2];
-  hipEvent_t fork, join[2];
-};
-
 struct SampleArgs {
   const void* logits;   // rows of fp32, fp16 or bf16 values (dtype), row_stride elements apart
   int64_t row_stride;
@@ -227,11 +222,9 @@ hipError_t ms_sample_init();
 // any_nucleus / any_large_k / any_other: some row may be in nucleus mode / a top-k row with
 // 64 < k <= kLargeKMax / in another mode (each mode has kernels of its own); a->exact_kernel: which kernels of the
 // exact path some row's parameters ask for (kWideRows: `wide` holds their arguments).
-// sides, when not null: streams and events of the context on which the kernels of a call whose rows are in several
-// modes run side by side (each mode's kernels skip the other modes' rows and share no state with them): they fork
-// from `stream` behind an event, and `stream` waits for them before the exact rows' kernel and before the call returns.
+// Rows of several modes in one call are streamed and finished by one pair of launches.
 hipError_t ms_launch_sample(const ms::SampleArgs* a, const ms::InlineParams* table, bool any_other, bool any_nucleus,
-                            bool any_large_k, hipStream_t stream, const ms::SideStreams* sides, const ms::WideArgs* wide);
+                            bool any_large_k, hipStream_t stream, const ms::WideArgs* wide);
 hipError_t ms_launch_argmax(const ms::ArgmaxArgs* a, int dtype, hipStream_t stream);
 hipError_t ms_launch_process_logits(float* logits, int64_t row_stride, int rows, int vocab,
                                     const ms::Xform* xf, hipStream_t stream);

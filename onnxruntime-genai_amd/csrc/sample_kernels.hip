@@ -836,7 +836,10 @@ __device__ __forceinline__ bool rank_and_cache_exps(u64* keys, const uint32_t* s
 // Per-row finish of the nucleus path: gathers the candidates the streaming pass left in `big`,
 // sorts them in LDS and runs the exact epilogue.  One block of kFinishBlock threads per row;
 // dynamic LDS: kNucleusCap key64s + the bucket table of the sort.
-template <bool INLINE, bool LARGEK>
+// MODE: which rows it finishes: nucleus rows, large-k rows, or both (a call whose rows are in several modes; there a
+// top-k row of any k <= kLargeKMax counts as one of large k).
+enum FinishMode { kFinishNucleus, kFinishLargeK, kFinishMixed };
+template <bool INLINE, FinishMode MODE>
 __device__ __forceinline__ void nucleus_finish_body(const SampleArgs& a) {
   extern __shared__ u64 lds_keys[];
   uint32_t* bucket_start = reinterpret_cast<uint32_t*>(lds_keys + kNucleusCap);  // kSortBuckets + 1 entries
@@ -849,9 +852,12 @@ __device__ __forceinline__ void nucleus_finish_body(const SampleArgs& a) {
   const int V = a.vocab;
   const int tid = threadIdx.x;
   const mi355x_sample_params prm = row_params<INLINE>(a, row);
-  if (row_mode(prm, V, a.chunks, a.emit_topk) != (LARGEK ? kModeTopkLarge : kModeNucleus)) return;
-  if (!LARGEK && a.xf.mask && a.row_done && a.row_done[row] != 0u) return;  // finished by the sparse-mask kernel
-  constexpr bool large_k = LARGEK;  // then every listed element is a candidate and no element after them is needed
+  const int mode = MODE == kFinishMixed ? row_mode_of_mixed(prm, V, a.chunks) : row_mode(prm, V, a.chunks, a.emit_topk);
+  if (MODE == kFinishMixed ? mode != kModeTopkLarge && mode != kModeNucleus : mode != (MODE == kFinishLargeK ? kModeTopkLarge : kModeNucleus)) return;
+  // a large-k row: then every listed element is a candidate and no element after them is needed
+  const bool large_k = MODE == kFinishMixed ? mode == kModeTopkLarge : MODE == kFinishLargeK;
+  constexpr bool kMayBeNucleus = MODE != kFinishLargeK;
+  if (!large_k && a.xf.mask && a.row_done && a.row_done[row] != 0u) return;  // finished by the sparse-mask kernel
   u64* big_row = a.big + static_cast<size_t>(row) * a.big_stride;
   const size_t cbase = static_cast<size_t>(row) * a.chunks;
   // The head of every chunk's list (a few entries per thread) is requested before the counts are
@@ -1031,7 +1037,7 @@ __device__ __forceinline__ void nucleus_finish_body(const SampleArgs& a) {
     __syncthreads();
     TrimmedBuckets kept = scan_buckets_and_trim(bucket_start, bucket_of, below, prm, V, kNucleusCap, red32, red64, k_wanted,
                                                 free_ties ? kNucleusCap : kBucketCap);
-    if constexpr (!LARGEK) {
+    if (kMayBeNucleus && !large_k) {
       // The list ends with the one element below the candidates and has 16, 64, 256 ... entries: should the search
       // stop on that last element, the reference notices it one element later (src/sampling_distribution.h:166-181),
       // and that element is in no list.  Rare enough to look for it in the row itself: the best key below
@@ -1101,7 +1107,7 @@ __device__ __forceinline__ void nucleus_finish_body(const SampleArgs& a) {
       n_c = kept.n;
     }
   }
-  if constexpr (!LARGEK) {
+  if (kMayBeNucleus && !large_k) {
     __syncthreads();
     const uint32_t wide_end_t = sh_wide_end_t;
     if (wide_end_t != 0u) {  // (decided after the first scan; the table holds the buckets' first places)
@@ -1313,13 +1319,17 @@ __device__ __forceinline__ void nucleus_finish_body(const SampleArgs& a) {
   }
 }
 
-__global__ __launch_bounds__(kFinishBlock) void nucleus_finish_kernel(const SampleArgs a) { nucleus_finish_body<false, false>(a); }
+__global__ __launch_bounds__(kFinishBlock) void nucleus_finish_kernel(const SampleArgs a) { nucleus_finish_body<false, kFinishNucleus>(a); }
 __global__ __launch_bounds__(kFinishBlock) void nucleus_finish_rows_kernel(const SampleArgs a, const InlineParams) {
-  nucleus_finish_body<true, false>(a);
+  nucleus_finish_body<true, kFinishNucleus>(a);
 }
-__global__ __launch_bounds__(kFinishBlock) void largek_finish_kernel(const SampleArgs a) { nucleus_finish_body<false, true>(a); }
+__global__ __launch_bounds__(kFinishBlock) void largek_finish_kernel(const SampleArgs a) { nucleus_finish_body<false, kFinishLargeK>(a); }
 __global__ __launch_bounds__(kFinishBlock) void largek_finish_rows_kernel(const SampleArgs a, const InlineParams) {
-  nucleus_finish_body<true, true>(a);
+  nucleus_finish_body<true, kFinishLargeK>(a);
+}
+__global__ __launch_bounds__(kFinishBlock) void mixed_finish_kernel(const SampleArgs a) { nucleus_finish_body<false, kFinishMixed>(a); }
+__global__ __launch_bounds__(kFinishBlock) void mixed_finish_rows_kernel(const SampleArgs a, const InlineParams) {
+  nucleus_finish_body<true, kFinishMixed>(a);
 }
 
 // ---- nucleus rows under a sparse grammar mask ------------------------------------------------------------
@@ -1779,61 +1789,40 @@ __global__ __launch_bounds__(kFinishBlock) void exact_rows_rows_kernel(const Sam
 MS_STREAM_KERNELS(, float)  // the fp32 streaming kernels live here, next to the finish kernels
 
 extern "C" hipError_t ms_launch_sample(const ms::SampleArgs* a, const ms::InlineParams* table, bool any_other,
-                                       bool any_nucleus, bool any_large_k, hipStream_t stream,
-                                       const ms::SideStreams* sides, const ms::WideArgs* wide) {
+                                       bool any_nucleus, bool any_large_k, hipStream_t stream, const ms::WideArgs* wide) {
   const dim3 fgrid(a->rows), fblock(ms::kFinishBlock);
   auto launch_stream = a->dtype == MI355X_F16 ? ms_launch_stream_f16 : a->dtype == MI355X_BF16 ? ms_launch_stream_bf16 : ms_launch_stream;
-  // A call whose rows are in several modes launches the kernels of every mode present; one after the other their
-  // chains of dependent phases add up (12 + 42 + 39 us for top-k, nucleus and large-k rows in one batch of 64 x
-  // 128256), side by side the longest decides.  The nucleus rows' kernels, the longest chain, stay on the caller's
-  // stream.
-  const int modes = (any_other ? 1 : 0) + (any_nucleus ? 1 : 0) + (any_large_k ? 1 : 0);
-  const bool fork = sides != nullptr && modes > 1;
-  int forked = 0;
-  hipError_t e = hipSuccess;
-  auto stream_of_mode = [&](bool stays) -> hipStream_t {
-    if (!fork || stays) return stream;
-    hipStream_t s = sides->side[forked++];
-    if (e == hipSuccess) e = hipStreamWaitEvent(s, sides->fork, 0);
-    return s;
+  // which = 1, 2, 3: nucleus rows, large-k rows, rows of several modes
+  auto launch_finish = [&](int which) {
+    if (table) {
+      auto* f = which == 1 ? ms::nucleus_finish_rows_kernel : which == 2 ? ms::largek_finish_rows_kernel : ms::mixed_finish_rows_kernel;
+      hipLaunchKernelGGL(f, fgrid, fblock, ms::kFinishLds, stream, *a, *table);
+    } else {
+      auto* f = which == 1 ? ms::nucleus_finish_kernel : which == 2 ? ms::largek_finish_kernel : ms::mixed_finish_kernel;
+      hipLaunchKernelGGL(f, fgrid, fblock, ms::kFinishLds, stream, *a);
+    }
+    return hipGetLastError();
   };
-  if (fork) {
-    e = hipEventRecord(sides->fork, stream);
-    if (e != hipSuccess) return e;
+  hipError_t e = hipSuccess;
+  const bool sparse = any_nucleus && a->xf.mask && a->row_done;
+  if (sparse) {  // nucleus rows under a sparse grammar mask are finished here; the kernels after it skip them
+    if (table) hipLaunchKernelGGL(ms::nucleus_sparse_rows_kernel, fgrid, fblock, ms::kFinishLds, stream, *a, *table);
+    else hipLaunchKernelGGL(ms::nucleus_sparse_kernel, fgrid, fblock, ms::kFinishLds, stream, *a);
+    e = hipGetLastError();
+    if (a->sparse_only) any_nucleus = false;  // (and no kernel after it has any to do)
   }
-  if (any_other) {
-    const hipStream_t s = stream_of_mode(!any_nucleus && !any_large_k);
-    if (e == hipSuccess) e = launch_stream(a, table, 0, s);
-  }
-  if (any_large_k && e == hipSuccess) {
-    const hipStream_t s = stream_of_mode(!any_nucleus);
-    if (e == hipSuccess) e = launch_stream(a, table, 2, s);
-    if (e == hipSuccess) {
-      if (table) hipLaunchKernelGGL(ms::largek_finish_rows_kernel, fgrid, fblock, ms::kFinishLds, s, *a, *table);
-      else hipLaunchKernelGGL(ms::largek_finish_kernel, fgrid, fblock, ms::kFinishLds, s, *a);
-      e = hipGetLastError();
-    }
-  }
-  if (any_nucleus && e == hipSuccess) {
-    if (a->xf.mask && a->row_done) {  // rows under a sparse grammar mask are finished here; the next two kernels skip them
-      if (table) hipLaunchKernelGGL(ms::nucleus_sparse_rows_kernel, fgrid, fblock, ms::kFinishLds, stream, *a, *table);
-      else hipLaunchKernelGGL(ms::nucleus_sparse_kernel, fgrid, fblock, ms::kFinishLds, stream, *a);
-      e = hipGetLastError();
-    }
-    if (e == hipSuccess && !(a->xf.mask && a->row_done && a->sparse_only)) {
-      e = launch_stream(a, table, 1, stream);
-      if (e == hipSuccess) {
-        if (table) hipLaunchKernelGGL(ms::nucleus_finish_rows_kernel, fgrid, fblock, ms::kFinishLds, stream, *a, *table);
-        else hipLaunchKernelGGL(ms::nucleus_finish_kernel, fgrid, fblock, ms::kFinishLds, stream, *a);
-        e = hipGetLastError();
+  const int modes = (any_other ? 1 : 0) + (any_nucleus ? 1 : 0) + (any_large_k ? 1 : 0);
+  if (modes > 1) {
+    if (e == hipSuccess) e = launch_stream(a, table, 3, stream);
+    if (e == hipSuccess) e = launch_finish(3);
+  } else {
+    if (any_other && e == hipSuccess) e = launch_stream(a, table, 0, stream);
+    for (int which = 1; which <= 2; ++which) {
+      if (which == 1 ? any_nucleus : any_large_k) {
+        if (e == hipSuccess) e = launch_stream(a, table, which, stream);
+        if (e == hipSuccess) e = launch_finish(which);
       }
     }
-  }
-  // (the forked streams join even after an error: a stream left forked would poison a capture)
-  for (int i = 0; i < forked; ++i) {
-    hipError_t j = hipEventRecord(sides->join[i], sides->side[i]);
-    if (j == hipSuccess) j = hipStreamWaitEvent(stream, sides->join[i], 0);
-    if (e == hipSuccess) e = j;
   }
   if (e != hipSuccess) return e;
   if (a->exact_kernel & ms::kWideRows) {
@@ -1853,6 +1842,8 @@ extern "C" hipError_t ms_sample_init() {
                           reinterpret_cast<const void*>(ms::nucleus_finish_rows_kernel),
                           reinterpret_cast<const void*>(ms::largek_finish_kernel),
                           reinterpret_cast<const void*>(ms::largek_finish_rows_kernel),
+                          reinterpret_cast<const void*>(ms::mixed_finish_kernel),
+                          reinterpret_cast<const void*>(ms::mixed_finish_rows_kernel),
                           reinterpret_cast<const void*>(ms::nucleus_sparse_kernel),
                           reinterpret_cast<const void*>(ms::nucleus_sparse_rows_kernel),
                           reinterpret_cast<const void*>(ms::exact_rows_kernel),

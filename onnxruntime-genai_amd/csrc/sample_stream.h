@@ -282,6 +282,12 @@ __device__ __forceinline__ int row_mode(mi355x_sample_params prm, int vocab, int
   return kModeNucleus;
 }
 
+// The same for a call whose rows are in several modes (see mixed_stream_body).
+__device__ __forceinline__ int row_mode_of_mixed(mi355x_sample_params prm, int vocab, int chunks) {
+  const int mode = row_mode(prm, vocab, chunks);
+  return mode == kModeTopkSmall ? kModeTopkLarge : mode;
+}
+
 // Depth below the row maximum (in score units) past which no element can lie strictly inside the
 // nucleus: once exp((s-max)/T) <= (1-p)/(p*V) -- with a margin of e^2 for fp32 rounding -- the stop
 // test prefix >= p*(prefix + (V-i-1)*e) of FindNucleus is certainly true, because prefix >= 1.
@@ -1654,6 +1660,28 @@ __device__ __forceinline__ void sample_fused_body(const SampleArgs& a) {
   }
 }
 
+// Calls whose rows are in several modes: one launch streams all of them, a row of k <= 64 as a large-k row (its chunks'
+// candidate lists serve any k), and one finish launch ends them.  The modes' own kernels would follow each other on
+// the stream (12 + 42 + 39 us for top-k, nucleus and large-k rows of 64 x 128256), and side by side on streams forked
+// from the caller's the forks and joins cost the host 23 us each, more than the kernels they overlap take.
+template <typename InT, bool INLINE, bool XFORM>
+__device__ __forceinline__ void mixed_stream_body(const SampleArgs& a) {
+  const mi355x_sample_params uniform_prm = args_up_front<XFORM>(a);
+  const int row = blockIdx.y, chunk = blockIdx.x;
+  __shared__ FusedShared sm;
+  const mi355x_sample_params prm = row_params<INLINE>(a, row, uniform_prm);
+  const void* const row0 = row_start<INLINE>(a, row, sizeof(InT));
+  const int mode = row_mode_of_mixed(prm, a.vocab, a.chunks);
+  if (mode == kModeNucleus) {
+    if constexpr (XFORM) {
+      if (a.xf.mask && a.row_done && a.row_done[row] != 0u) return;  // finished by the sparse-mask kernel
+    }
+    stream_row<InT, true, XFORM, false>(a, row, row0, chunk, prm, sm);
+  } else if (mode == kModeTopkLarge) {
+    stream_row<InT, true, XFORM, true>(a, row, row0, chunk, prm, sm);
+  }
+}
+
 // Kernel variants: per-row parameter table in the arguments or not (_rows); nucleus rows, top-k rows with
 // 64 < k <= kLargeKMax (largek) or all other rows; with or without the code of the logits processing (_xf);
 // one set per element type of the logits (SUFFIX: none for fp32, _f16, _bf16), each in a source file of its own.
@@ -1666,9 +1694,17 @@ __device__ __forceinline__ void sample_fused_body(const SampleArgs& a) {
     sample_fused_body<InT, true, NUCLEUS, XFORM, LARGEK>(a);                                                             \
   }
 
-// Defines the streaming kernels of one element type (twelve for sampling, two for argmax) and
+#define MS_MIXED_KERNEL(NAME, SUFFIX, InT, XFORM)                                                                        \
+  __global__ __launch_bounds__(kNucleusBlock) void NAME##SUFFIX##_kernel(const SampleArgs a) {                           \
+    mixed_stream_body<InT, false, XFORM>(a);                                                                             \
+  }                                                                                                                      \
+  __global__ __launch_bounds__(kNucleusBlock) void NAME##SUFFIX##_rows_kernel(const SampleArgs a, const InlineParams) {  \
+    mixed_stream_body<InT, true, XFORM>(a);                                                                              \
+  }
+
+// Defines the streaming kernels of one element type (sixteen for sampling, two for argmax) and
 // ms_launch_stream##SUFFIX, which launches the one a call needs: which = 0 rows of every other mode (argmax
-// calls: the argmax kernels), 1 nucleus rows, 2 rows with 64 < k <= kLargeKMax.
+// calls: the argmax kernels), 1 nucleus rows, 2 rows with 64 < k <= kLargeKMax, 3 a call's rows of all three kinds.
 #define MS_STREAM_KERNELS(SUFFIX, InT)                                                                                   \
   namespace ms {                                                                                                         \
   MS_STREAM_KERNEL(sample_fused, SUFFIX, InT, false, false, false)                                                       \
@@ -1677,6 +1713,8 @@ __device__ __forceinline__ void sample_fused_body(const SampleArgs& a) {
   MS_STREAM_KERNEL(nucleus_stream_xf, SUFFIX, InT, true, true, false)                                                    \
   MS_STREAM_KERNEL(largek_stream, SUFFIX, InT, true, false, true)                                                        \
   MS_STREAM_KERNEL(largek_stream_xf, SUFFIX, InT, true, true, true)                                                      \
+  MS_MIXED_KERNEL(mixed_stream, SUFFIX, InT, false)                                                                      \
+  MS_MIXED_KERNEL(mixed_stream_xf, SUFFIX, InT, true)                                                                    \
   __global__ __launch_bounds__(kTopkBlock) void argmax_stream##SUFFIX##_kernel(const SampleArgs a) {                     \
     sample_fused_body<InT, false, false, false, false, true>(a);                                                         \
   }                                                                                                                      \
@@ -1694,11 +1732,13 @@ __device__ __forceinline__ void sample_fused_body(const SampleArgs& a) {
     } else if (table) {                                                                                                         \
       auto* f = which == 0   ? (xf ? ms::sample_fused_xf##SUFFIX##_rows_kernel : ms::sample_fused##SUFFIX##_rows_kernel) \
                 : which == 1 ? (xf ? ms::nucleus_stream_xf##SUFFIX##_rows_kernel : ms::nucleus_stream##SUFFIX##_rows_kernel) \
+                : which == 3 ? (xf ? ms::mixed_stream_xf##SUFFIX##_rows_kernel : ms::mixed_stream##SUFFIX##_rows_kernel) \
                              : (xf ? ms::largek_stream_xf##SUFFIX##_rows_kernel : ms::largek_stream##SUFFIX##_rows_kernel); \
       hipLaunchKernelGGL(f, grid, block, 0, stream, *a, *table);                                                         \
     } else {                                                                                                             \
       auto* f = which == 0   ? (xf ? ms::sample_fused_xf##SUFFIX##_kernel : ms::sample_fused##SUFFIX##_kernel)           \
                 : which == 1 ? (xf ? ms::nucleus_stream_xf##SUFFIX##_kernel : ms::nucleus_stream##SUFFIX##_kernel)       \
+                : which == 3 ? (xf ? ms::mixed_stream_xf##SUFFIX##_kernel : ms::mixed_stream##SUFFIX##_kernel)           \
                              : (xf ? ms::largek_stream_xf##SUFFIX##_kernel : ms::largek_stream##SUFFIX##_kernel);        \
       hipLaunchKernelGGL(f, grid, block, 0, stream, *a);                                                                 \
     }                                                                                                                    \
