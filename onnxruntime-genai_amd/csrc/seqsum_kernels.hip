@@ -81,18 +81,29 @@ __global__ __launch_bounds__(kSegBlock) void softmax_apply_kernel(float* scores,
   const float max_score = a.out_max[row], sum = a.out_sum[row];
   const float lse = LOG ? em::logf_exact(sum) : 0.0f;
   const float inv_sum = 1.0f / sum;
+  auto finish = [=](float v, int i) {
+    if (LOG) {
+      // x - max is never -0 where it shows (see softmax_kernel): the maximum here lost the sign of its zero
+      const float d = v - max_score;
+      return (d == 0.0f ? 0.0f : d) * a.inv_temp - lse;
+    }
+    const float ex = erow[i];
+    return sum > 0.0f ? ex * inv_sum : ex;
+  };
+  // four elements per load and store (whatever the row's alignment), the loads of a thread under way together
+  float v[kSegPer];
+  seg_load<float>(x, a.vocab, seg, 0.0f, v);
 #pragma unroll
-  for (int j = 0; j < kSegPer; ++j) {
-    const int i = seg * kSegElems + j * kSegBlock + static_cast<int>(threadIdx.x);
-    if (i < a.vocab) {
-      if (LOG) {
-        // x - max is never -0 where it shows (see softmax_kernel): the maximum here lost the sign of its zero
-        const float d = x[i] - max_score;
-        x[i] = (d == 0.0f ? 0.0f : d) * a.inv_temp - lse;
-      } else {
-        const float ex = erow[i];
-        x[i] = sum > 0.0f ? ex * inv_sum : ex;
-      }
+  for (int e0 = 0; e0 < kSegPer; e0 += 4) {
+    const int i = seg_index<float>(seg, e0);
+    if (i + 4 <= a.vocab) {
+      v4f_any q;
+      q.x = finish(v[e0], i), q.y = finish(v[e0 + 1], i + 1), q.z = finish(v[e0 + 2], i + 2), q.w = finish(v[e0 + 3], i + 3);
+      *reinterpret_cast<v4f_any*>(x + i) = q;
+    } else {
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        if (i + c < a.vocab) x[i + c] = finish(v[e0 + c], i + c);
     }
   }
 }
