@@ -13,9 +13,10 @@
  * sequences live in are part of the launch, so a replay would repeat one step; they return
  * MI355X_E_UNSUPPORTED on a capturing stream).  The three calls that take a table from a caller's HOST array
  * (mi355x_sample* with per-row parameters for more than 64 rows, mi355x_logits_handoff with token_index,
- * mi355x_kv_gather) copy it into pinned memory of the context when they are called and record a copy from
- * there, so the caller's array is not read again at a replay; every such call captured takes one of the
- * context's 56 permanent staging slots (MI355X_E_UNSUPPORTED once they are used up).
+ * mi355x_kv_gather) read it when they are called -- the first copies it into pinned memory of the context and records
+ * a copy from there, the others carry it inside the kernel arguments -- so the caller's array is not read again at a
+ * replay; every such call captured takes one of the context's 56 permanent staging slots (MI355X_E_UNSUPPORTED once
+ * they are used up).
  *
  * Versions: MI355X_ABI_VERSION names the layout of the structures below and the set of entry points;
  * mi355x_search_abi_version() returns the value the loaded library was built with, so a caller built
@@ -233,8 +234,8 @@ int mi355x_beam_scorer_create(mi355x_search_ctx* ctx, int batch, int beams, int 
                               int pad_token_id, const int32_t* eos_ids, int n_eos,
                               float length_penalty, int early_stopping, mi355x_beam_scorer** out);
 void mi355x_beam_scorer_destroy(mi355x_beam_scorer* s);
-/* Sets the prompt: tokens HOST [batch, prompt_len], replicated to every beam (BeamSearch_Cpu::AppendTokens,
- * src/search.cpp:326-343). */
+/* Sets the prompt: tokens HOST [batch, prompt_len], read by the call, replicated to every beam
+ * (BeamSearch_Cpu::AppendTokens, src/search.cpp:326-343). */
 int mi355x_beam_scorer_set_prompt(mi355x_beam_scorer* s, void* stream, const int32_t* tokens,
                                   int prompt_len);
 /* One BeamSearchScorer::Process + AppendNextTokensToSequences on the candidates produced by
@@ -265,8 +266,8 @@ int mi355x_beam_scorer_hypothesis(mi355x_beam_scorer* s, void* stream, int batch
 /* KV-cache beam reorder: DefaultKeyValueCache::PickPastState (src/models/kv_cache.cpp:710-740):
  * for every tensor t and row j, past[t][j] = present[t][beam_indices[j]], blocks of block_bytes
  * bytes (any size; blocks and tensors aligned to 16 bytes move with 128-bit accesses, others with the
- * widest access they are aligned to).  present/past: HOST arrays of n_tensors device pointers (copied by the
- * call into pinned staging memory of the context, from where one asynchronous copy takes them to the device);
+ * widest access they are aligned to).  present/past: HOST arrays of n_tensors device pointers (read by the
+ * call: they travel inside the kernel arguments, 64 tensors per launch, at most 2048 in all);
  * beam_indices: device [rows]. */
 int mi355x_kv_gather(mi355x_search_ctx* ctx, void* stream, const void* const* present,
                      void* const* past, int n_tensors, const int32_t* beam_indices, int rows,
@@ -358,8 +359,8 @@ int mi355x_cast(mi355x_search_ctx* ctx, void* stream, const void* in, int in_dty
 /* Logits hand-off before the path: Logits::Get (src/models/logits.cpp:33-82) copies the logits of each
  * row's last real token out of the model's [rows, seq_len, vocab] output and widens fp16/bf16 to fp32;
  * here both happen in one pass.  raw: device, dtype MI355X_F32 / MI355X_F16 / MI355X_BF16;
- * token_index: HOST [rows] positions inside seq_len (copied by the call, through pinned staging memory of the
- * context), or NULL for seq_len - 1;
+ * token_index: HOST [rows] positions inside seq_len (read by the call: they travel inside the kernel
+ * arguments), or NULL for seq_len - 1;
  * out: device [rows] rows of vocab floats, row r at out + r*out_stride. */
 int mi355x_logits_handoff(mi355x_search_ctx* ctx, void* stream, const void* raw, int dtype, int rows,
                           int seq_len, int vocab, const int32_t* token_index, float* out,

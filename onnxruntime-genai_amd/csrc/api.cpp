@@ -9,6 +9,7 @@
 #include <cstdlib>
 #include <new>
 #include <string>
+#include <type_traits>
 #include <vector>
 #include "api_internal.h"
 
@@ -69,8 +70,6 @@ struct mi355x_search_ctx {
   int poll_limit{ms::kDefaultPollLimit};
   uint32_t* ban{};  // [max_rows, mask words]: ids banned by the no-repeat-n-gram rule
   mi355x_sample_params* params_dev{};
-  void** ptr_table{};      // device copy of pointer tables (kv gather)
-  size_t ptr_table_cap{};
   float* beam_row_scores{};
   ms::u64* seg_cand{};  // [max_rows][max_segs][kBeamMaxCand] beam-search candidates per segment
   int max_segs{};
@@ -83,16 +82,19 @@ struct mi355x_search_ctx {
   float* row_sum{};
   ms::WideRow* wide_rows{};
   uint32_t* wide_tile_start{};
-  int32_t* row_index{};  // device copy of per-row host indices (logits hand-off)
   int32_t* beam_row_tokens{};
-  // Pinned host staging for the calls that take a table from a caller's HOST array (per-row parameters of more
-  // than 64 rows, the KV gather's pointer tables, token_index): the call copies the array into a slot here and
-  // records a copy from the slot to the device table.  Slots of the ring are reused once the copy that read them
+  // Pinned host staging for the per-row parameters of more than 64 rows, which come in a caller's HOST array and do
+  // not fit the kernel arguments: the call copies the array into a slot here and records a copy from the slot to the
+  // device table.  Slots of the ring are reused once the copy that read them
   // is done (an event per slot); a call on a capturing stream gets a slot of its own that is never reused, so the
   // copy node of its graph reads the same bytes at every replay.
   static constexpr int kStageRing = 8, kStageCaptured = 56;
   char* stage{};
   size_t stage_slot_bytes{};
+  // The last kReadbackBytes of that pinned memory: where small results and states go between host and device, by
+  // calls that wait for their copy before they return.
+  static constexpr size_t kReadbackBytes = 256 * 1024;
+  char* readback{};
   hipEvent_t stage_event[kStageRing]{};
   bool stage_pending[kStageRing]{};
   int stage_next{}, stage_captured{};
@@ -231,15 +233,13 @@ int mi355x_search_create(int device, int max_rows, int max_vocab, mi355x_search_
   ok(c->Alloc(&c->sub_se, static_cast<size_t>(max_rows) * c->max_segs * ms::kSegSubs, false));
   ok(c->Alloc(&c->row_max, static_cast<size_t>(max_rows), false));
   ok(c->Alloc(&c->row_sum, static_cast<size_t>(max_rows), false));
-  ok(c->Alloc(&c->row_index, static_cast<size_t>(max_rows), false));
-  c->ptr_table_cap = 4096;
-  ok(c->Alloc(&c->ptr_table, c->ptr_table_cap, false));
-  c->stage_slot_bytes = std::max(c->ptr_table_cap * sizeof(void*), static_cast<size_t>(max_rows) * sizeof(mi355x_sample_params));
-  c->stage_slot_bytes = (c->stage_slot_bytes + 255) & ~static_cast<size_t>(255);
+  c->stage_slot_bytes = (static_cast<size_t>(max_rows) * sizeof(mi355x_sample_params) + 255) & ~static_cast<size_t>(255);
   if (e == hipSuccess) {
     void* pinned = nullptr;
-    e = hipHostMalloc(&pinned, c->stage_slot_bytes * (mi355x_search_ctx::kStageRing + mi355x_search_ctx::kStageCaptured), hipHostMallocDefault);
+    const size_t slots = c->stage_slot_bytes * (mi355x_search_ctx::kStageRing + mi355x_search_ctx::kStageCaptured);
+    e = hipHostMalloc(&pinned, slots + mi355x_search_ctx::kReadbackBytes, hipHostMallocDefault);
     c->stage = static_cast<char*>(pinned);
+    c->readback = c->stage + slots;
   }
   for (int i = 0; i < mi355x_search_ctx::kStageRing && e == hipSuccess; ++i)
     e = hipEventCreateWithFlags(&c->stage_event[i], hipEventDisableTiming);
@@ -347,6 +347,16 @@ bool Capturing(hipStream_t s) {
   return hipStreamIsCapturing(s, &status) == hipSuccess && status != hipStreamCaptureStatusNone;
 }
 
+// A captured call that takes a table from a caller's host array counts against the context's bound on such calls,
+// whether its table needs a permanent staging slot or travels inside the kernel arguments.
+int TakeCapturedSlot(mi355x_search_ctx* ctx, int* slot) {
+  if (ctx->stage_captured == mi355x_search_ctx::kStageCaptured)
+    return Fail(MI355X_E_UNSUPPORTED, "this context has staged %d host tables for graph capture, all it provides for",
+                mi355x_search_ctx::kStageCaptured);
+  *slot = mi355x_search_ctx::kStageRing + ctx->stage_captured++;
+  return MI355X_OK;
+}
+
 // Records a copy of `bytes` bytes of the caller's host array `src` to the device table `dst` on stream s, through a
 // pinned staging slot of the context (see mi355x_search_ctx::stage).
 int StageToDevice(mi355x_search_ctx* ctx, hipStream_t s, void* dst, const void* src, size_t bytes) {
@@ -354,10 +364,7 @@ int StageToDevice(mi355x_search_ctx* ctx, hipStream_t s, void* dst, const void* 
   const bool capturing = Capturing(s);
   int slot;
   if (capturing) {
-    if (ctx->stage_captured == mi355x_search_ctx::kStageCaptured)
-      return Fail(MI355X_E_UNSUPPORTED, "this context has staged %d host tables for graph capture, all it provides for",
-                  mi355x_search_ctx::kStageCaptured);
-    slot = mi355x_search_ctx::kStageRing + ctx->stage_captured++;
+    if (int rc = TakeCapturedSlot(ctx, &slot)) return rc;
   } else {
     slot = ctx->stage_next;
     ctx->stage_next = (slot + 1) % mi355x_search_ctx::kStageRing;
@@ -786,17 +793,24 @@ int mi355x_logits_handoff(mi355x_search_ctx* ctx, void* stream, const void* raw,
   if (rows > 65535) return Fail(MI355X_E_CAPACITY, "too many rows (%d)", rows);
   const int kind = dtype == MI355X_F16 ? 0 : dtype == MI355X_BF16 ? 1 : dtype == MI355X_F32 ? 2 : -1;
   if (kind < 0) return Fail(MI355X_E_UNSUPPORTED, "dtype %d not supported", dtype);
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  const int32_t* index_dev = nullptr;
   if (token_index) {
     if (rows > ctx->max_rows) return Fail(MI355X_E_CAPACITY, "rows (%d) exceed the context's %d", rows, ctx->max_rows);
     for (int r = 0; r < rows; ++r)
       if (token_index[r] < 0 || token_index[r] >= seq_len)
         return Fail(MI355X_E_INVALID, "token_index[%d] = %d outside [0, %d)", r, token_index[r], seq_len);
-    if (int rc = StageToDevice(ctx, s, ctx->row_index, token_index, sizeof(int32_t) * rows)) return rc;
-    index_dev = ctx->row_index;
   }
-  HIP_TRY(ms_launch_logits_handoff(raw, kind, rows, seq_len, vocab, index_dev, out, out_stride, s));
+  if (int slot; token_index && Capturing(static_cast<hipStream_t>(stream)))
+    if (int rc = TakeCapturedSlot(ctx, &slot)) return rc;
+  // the positions travel inside the kernel arguments, kTokenIndexRows rows per launch
+  const int per_launch = token_index ? ms::kTokenIndexRows : rows;
+  const size_t row_bytes = static_cast<size_t>(seq_len) * vocab * (kind == 2 ? 4 : 2);
+  for (int r0 = 0; r0 < rows; r0 += per_launch) {
+    const int n = rows - r0 < per_launch ? rows - r0 : per_launch;
+    ms::TokenIndex index;
+    if (token_index) std::copy_n(token_index + r0, n, index.token);
+    HIP_TRY(ms_launch_logits_handoff(&index, token_index ? 1 : 0, static_cast<const char*>(raw) + static_cast<size_t>(r0) * row_bytes, kind, n,
+                                     seq_len, vocab, out + static_cast<size_t>(r0) * out_stride, out_stride, static_cast<hipStream_t>(stream)));
+  }
   return MI355X_OK;
 }
 
@@ -804,7 +818,7 @@ int mi355x_kv_gather(mi355x_search_ctx* ctx, void* stream, const void* const* pr
                      int n_tensors, const int32_t* beam_indices, int rows, size_t block_bytes) {
   if (!ctx || !present || !past || !beam_indices) return Fail(MI355X_E_INVALID, "null argument");
   if (n_tensors <= 0 || rows <= 0 || block_bytes == 0) return Fail(MI355X_E_INVALID, "non-positive size");
-  if (static_cast<size_t>(n_tensors) * 2 > ctx->ptr_table_cap || n_tensors > 65535 || rows > 65535)
+  if (n_tensors > 2048 || rows > 65535)
     return Fail(MI355X_E_CAPACITY, "too many tensors (%d) or rows (%d)", n_tensors, rows);
   // Widest power-of-two access (at most 16 bytes) that every block of every tensor is aligned to.
   uintptr_t align = static_cast<uintptr_t>(block_bytes);
@@ -814,14 +828,16 @@ int mi355x_kv_gather(mi355x_search_ctx* ctx, void* stream, const void* const* pr
   }
   int width = 16;
   while (align & static_cast<uintptr_t>(width - 1)) width >>= 1;
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  {
-    std::vector<const void*> both(static_cast<size_t>(n_tensors) * 2);  // one table: present pointers, then past pointers
-    std::copy_n(present, n_tensors, both.begin());
-    std::copy_n(past, n_tensors, both.begin() + n_tensors);
-    if (int rc = StageToDevice(ctx, s, ctx->ptr_table, both.data(), sizeof(void*) * both.size())) return rc;
+  if (int slot; Capturing(static_cast<hipStream_t>(stream)))
+    if (int rc = TakeCapturedSlot(ctx, &slot)) return rc;
+  // the addresses travel inside the kernel arguments, kKvTensors tensors per launch
+  for (int t0 = 0; t0 < n_tensors; t0 += ms::kKvTensors) {
+    const int n = n_tensors - t0 < ms::kKvTensors ? n_tensors - t0 : ms::kKvTensors;
+    ms::KvTensors tensors;
+    std::copy_n(present + t0, n, tensors.present);
+    std::copy_n(past + t0, n, tensors.past);
+    HIP_TRY(ms_launch_kv_gather(&tensors, n, beam_indices, rows, block_bytes, width, static_cast<hipStream_t>(stream)));
   }
-  HIP_TRY(ms_launch_kv_gather(ctx->ptr_table, ctx->ptr_table + n_tensors, n_tensors, beam_indices, rows, block_bytes, width, s));
   return MI355X_OK;
 }
 
@@ -873,15 +889,19 @@ int mi355x_search_set_poll_limit(mi355x_search_ctx* ctx, int polls) {
 struct mi355x_beam_scorer {
   mi355x_search_ctx* ctx{};
   ms::ScorerState st{};
-  std::vector<void*> allocs;
+  char* memory{};  // everything below, one allocation: creating eighteen of them and clearing each took 0.25 ms
   int32_t* seq[2]{};
   int cur{};
   int length{};
   bool finalized{};
-  float* pow_dev{};
   float* cand_scores{};    // [batch, 2*beams]: the candidates of mi355x_beam_search_step
   int32_t* cand_tokens{};
   int32_t* cand_beams{};
+  // The hypotheses' lists as the device holds them after the finalisation, read back together by the first
+  // mi355x_beam_scorer_hypothesis (and again after a further step): used counts, lengths, slots, scores -- and, where
+  // they fit the readback area next to them, the tokens.
+  size_t lists_bytes{}, tokens_bytes{};
+  std::vector<char> lists;  // empty: not read back
 };
 
 int mi355x_beam_scorer_create(mi355x_search_ctx* ctx, int batch, int beams, int max_length, int pad_token_id,
@@ -896,16 +916,7 @@ int mi355x_beam_scorer_create(mi355x_search_ctx* ctx, int batch, int beams, int 
   auto* s = new (std::nothrow) mi355x_beam_scorer;
   if (!s) return Fail(MI355X_E_INVALID, "out of host memory");
   s->ctx = ctx;
-  const size_t bb = static_cast<size_t>(batch) * beams;
-  hipError_t e = hipSuccess;
-  auto alloc = [&](void** p, size_t bytes) {
-    if (e != hipSuccess) return;
-    e = hipMalloc(p, bytes ? bytes : 16);
-    if (e == hipSuccess) {
-      s->allocs.push_back(*p);
-      e = hipMemset(*p, 0, bytes ? bytes : 16);
-    }
-  };
+  const size_t bb = static_cast<size_t>(batch) * beams, ranks = static_cast<size_t>(batch) * (beams + 1);
   ms::ScorerState& st = s->st;
   st.batch = batch;
   st.beams = beams;
@@ -914,39 +925,59 @@ int mi355x_beam_scorer_create(mi355x_search_ctx* ctx, int batch, int beams, int 
   st.early_stopping = early_stopping != 0;
   st.n_eos = n_eos;
   for (int i = 0; i < n_eos; ++i) st.eos[i] = eos_ids[i];
-  alloc(reinterpret_cast<void**>(&st.next_scores), bb * sizeof(float));
-  alloc(reinterpret_cast<void**>(&st.next_tokens), bb * sizeof(int32_t));
-  alloc(reinterpret_cast<void**>(&st.next_indices), bb * sizeof(int32_t));
-  alloc(reinterpret_cast<void**>(&st.hyp_score), bb * sizeof(float));
-  alloc(reinterpret_cast<void**>(&st.hyp_len), bb * sizeof(int));
-  alloc(reinterpret_cast<void**>(&st.hyp_slot), static_cast<size_t>(batch) * (beams + 1) * sizeof(int));
-  alloc(reinterpret_cast<void**>(&st.hyp_tokens), static_cast<size_t>(batch) * (beams + 1) * max_length * sizeof(int32_t));
-  alloc(reinterpret_cast<void**>(&st.hyp_used), batch * sizeof(int));
-  alloc(reinterpret_cast<void**>(&st.done), batch * sizeof(int));
-  alloc(reinterpret_cast<void**>(&st.not_done), sizeof(int));
-  alloc(reinterpret_cast<void**>(&st.pending), batch * sizeof(int));
-  alloc(reinterpret_cast<void**>(&st.arrive), sizeof(unsigned));
-  alloc(reinterpret_cast<void**>(&s->pow_dev), (static_cast<size_t>(max_length) + 1) * sizeof(float));
-  alloc(reinterpret_cast<void**>(&s->seq[0]), bb * max_length * sizeof(int32_t));
-  alloc(reinterpret_cast<void**>(&s->seq[1]), bb * max_length * sizeof(int32_t));
-  alloc(reinterpret_cast<void**>(&s->cand_scores), 2 * bb * sizeof(float));
-  alloc(reinterpret_cast<void**>(&s->cand_tokens), 2 * bb * sizeof(int32_t));
-  alloc(reinterpret_cast<void**>(&s->cand_beams), 2 * bb * sizeof(int32_t));
+  // Placed twice: to learn the size, and once there is memory.  The small arrays that start with something else than
+  // zeros or are read back together come first.
+  size_t at = 0, head_bytes = 0;
+  float* pow_table = nullptr;
+  auto place = [&](auto** p, size_t count) {
+    at = (at + 255) & ~static_cast<size_t>(255);
+    *p = reinterpret_cast<std::remove_reference_t<decltype(*p)>>(s->memory + at);
+    at += count * sizeof(**p);
+  };
+  auto layout = [&] {
+    at = 0;
+    place(&st.hyp_used, batch);
+    place(&st.hyp_len, bb);
+    place(&st.hyp_slot, ranks);
+    place(&st.hyp_score, bb);
+    s->lists_bytes = at;
+    place(&st.next_scores, bb);
+    place(&st.not_done, 1);
+    place(&pow_table, static_cast<size_t>(max_length) + 1);
+    head_bytes = at;
+    place(&st.hyp_tokens, ranks * max_length);
+    s->tokens_bytes = ranks * max_length * sizeof(int32_t);
+    place(&st.next_tokens, bb);
+    place(&st.next_indices, bb);
+    place(&st.done, batch);
+    place(&st.pending, batch);
+    place(&st.arrive, 1);
+    place(&s->seq[0], bb * max_length);
+    place(&s->seq[1], bb * max_length);
+    place(&s->cand_scores, 2 * bb);
+    place(&s->cand_tokens, 2 * bb);
+    place(&s->cand_beams, 2 * bb);
+  };
+  layout();
+  void* memory = nullptr;
+  hipError_t e = hipMalloc(&memory, at);
   if (e == hipSuccess) {
+    s->memory = static_cast<char*>(memory);
+    layout();
+    st.pow_table = pow_table;
     // initial beam scores 0, -1e9, -1e9, ... per batch entry (src/beam_search_scorer.cpp:76-81); rank -> row
-    // identity; pow(length, length_penalty) from the host libm, the function the reference calls.
-    std::vector<float> init(bb, 0.0f), powt(static_cast<size_t>(max_length) + 1);
-    for (int b = 0; b < batch; ++b)
-      for (int j = 1; j < beams; ++j) init[static_cast<size_t>(b) * beams + j] = -1e9;
-    std::vector<int> slots(static_cast<size_t>(batch) * (beams + 1));
-    for (size_t i = 0; i < slots.size(); ++i) slots[i] = static_cast<int>(i % (beams + 1));
-    for (int l = 0; l <= max_length; ++l) powt[l] = std::pow(static_cast<float>(l), length_penalty);
-    e = hipMemcpy(st.next_scores, init.data(), bb * sizeof(float), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(st.hyp_slot, slots.data(), slots.size() * sizeof(int), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(s->pow_dev, powt.data(), powt.size() * sizeof(float), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(st.not_done, &batch, sizeof(int), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);  // the fills are done before any stream uses the state
-    st.pow_table = s->pow_dev;
+    // identity; pow(length, length_penalty) from the host libm, the function the reference calls (pow(x, 1) is x).
+    std::vector<char> head(head_bytes, 0);
+    auto host = [&](auto* device) { return reinterpret_cast<std::remove_const_t<std::remove_pointer_t<decltype(device)>>*>(head.data() + (reinterpret_cast<const char*>(device) - s->memory)); };
+    for (size_t i = 0; i < bb; ++i) host(st.next_scores)[i] = i % beams ? -1e9f : 0.0f;
+    for (size_t i = 0; i < ranks; ++i) host(st.hyp_slot)[i] = static_cast<int>(i % (beams + 1));
+    for (int l = 0; l <= max_length; ++l) host(pow_table)[l] = length_penalty == 1.0f ? static_cast<float>(l) : std::pow(static_cast<float>(l), length_penalty);
+    *host(st.not_done) = batch;
+    e = hipMemsetAsync(s->memory + head_bytes, 0, at - head_bytes, nullptr);
+    const char* from = head.data();
+    if (head_bytes <= mi355x_search_ctx::kReadbackBytes) from = static_cast<const char*>(std::memcpy(ctx->readback, head.data(), head_bytes));
+    if (e == hipSuccess) e = hipMemcpyAsync(s->memory, from, head_bytes, hipMemcpyHostToDevice, nullptr);
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);  // the state is there before any stream uses it
   }
   if (e != hipSuccess) {
     mi355x_beam_scorer_destroy(s);
@@ -958,7 +989,7 @@ int mi355x_beam_scorer_create(mi355x_search_ctx* ctx, int batch, int beams, int 
 
 void mi355x_beam_scorer_destroy(mi355x_beam_scorer* s) {
   if (!s) return;
-  for (void* p : s->allocs) (void)hipFree(p);
+  if (s->memory) (void)hipFree(s->memory);
   delete s;
 }
 
@@ -966,13 +997,19 @@ int mi355x_beam_scorer_set_prompt(mi355x_beam_scorer* s, void* stream, const int
   if (!s || !tokens) return Fail(MI355X_E_INVALID, "null argument");
   if (prompt_len < 0 || prompt_len > s->st.max_length) return Fail(MI355X_E_INVALID, "User-defined tokens exceed max_length.");
   const int bb = s->st.batch * s->st.beams;
-  std::vector<int32_t> host(static_cast<size_t>(bb) * s->st.max_length, 0);
-  for (int i = 0; i < bb; ++i)
-    std::memcpy(host.data() + static_cast<size_t>(i) * s->st.max_length,
-                tokens + static_cast<size_t>(i / s->st.beams) * prompt_len, sizeof(int32_t) * prompt_len);
   hipStream_t st = static_cast<hipStream_t>(stream);
-  HIP_TRY(hipMemcpyAsync(s->seq[s->cur], host.data(), host.size() * sizeof(int32_t), hipMemcpyHostToDevice, st));
-  HIP_TRY(hipStreamSynchronize(st));  // `host` goes out of scope
+  if (static_cast<size_t>(s->st.batch) * prompt_len <= ms::kPromptTokens) {  // inside the kernel arguments
+    ms::PromptTokens prompt;
+    std::copy_n(tokens, static_cast<size_t>(s->st.batch) * prompt_len, prompt.token);
+    HIP_TRY(ms_launch_scorer_prompt(&prompt, prompt_len, s->st.beams, bb, s->st.max_length, s->seq[s->cur], st));
+  } else {
+    std::vector<int32_t> host(static_cast<size_t>(bb) * s->st.max_length, 0);
+    for (int i = 0; i < bb; ++i)
+      std::memcpy(host.data() + static_cast<size_t>(i) * s->st.max_length,
+                  tokens + static_cast<size_t>(i / s->st.beams) * prompt_len, sizeof(int32_t) * prompt_len);
+    HIP_TRY(hipMemcpyAsync(s->seq[s->cur], host.data(), host.size() * sizeof(int32_t), hipMemcpyHostToDevice, st));
+    HIP_TRY(hipStreamSynchronize(st));  // `host` goes out of scope
+  }
   s->length = prompt_len;
   return MI355X_OK;
 }
@@ -988,6 +1025,7 @@ int mi355x_beam_scorer_step(mi355x_beam_scorer* s, void* stream, const float* ca
                                 cand_beam_indices, st));
   s->cur = 1 - s->cur;
   s->length += 1;
+  s->lists.clear();
   return MI355X_OK;
 }
 
@@ -1005,6 +1043,7 @@ int mi355x_beam_search_step(mi355x_beam_scorer* s, void* stream, const void* log
   if (!fused) return mi355x_beam_scorer_step(s, stream, s->cand_scores, s->cand_tokens, s->cand_beams);
   s->cur = 1 - s->cur;
   s->length += 1;
+  s->lists.clear();
   return MI355X_OK;
 }
 
@@ -1019,11 +1058,12 @@ const int32_t* mi355x_beam_scorer_sequences(const mi355x_beam_scorer* s, int* le
 
 int mi355x_beam_scorer_is_done(mi355x_beam_scorer* s, void* stream, int* done) {
   if (!s || !done) return Fail(MI355X_E_INVALID, "null argument");
-  int nd = 0;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  HIP_TRY(hipMemcpyAsync(&nd, s->st.not_done, sizeof(int), hipMemcpyDeviceToHost, st));
+  // (through pinned memory: a copy into an ordinary variable waits twice, 21 us instead of 12)
+  int* const nd = reinterpret_cast<int*>(s->ctx->readback);
+  HIP_TRY(hipMemcpyAsync(nd, s->st.not_done, sizeof(int), hipMemcpyDeviceToHost, st));
   HIP_TRY(hipStreamSynchronize(st));
-  *done = (nd == 0) || (s->length == s->st.max_length);  // BeamSearch_Cpu::IsDone, src/search.cpp:345-352
+  *done = (*nd == 0) || (s->length == s->st.max_length);  // BeamSearch_Cpu::IsDone, src/search.cpp:345-352
   return MI355X_OK;
 }
 
@@ -1037,20 +1077,30 @@ int mi355x_beam_scorer_hypothesis(mi355x_beam_scorer* s, void* stream, int batch
     s->finalized = true;
   }
   const int nb = s->st.beams;
-  int used = 0;
-  HIP_TRY(hipMemcpyAsync(&used, s->st.hyp_used + batch, sizeof(int), hipMemcpyDeviceToHost, st));
-  HIP_TRY(hipStreamSynchronize(st));
-  if (index < 0 || index >= used) return Fail(MI355X_E_INVALID, "GetHypothesis index out of bounds");
-  int len = 0, slot = 0;
-  float sc = 0.0f;
-  HIP_TRY(hipMemcpy(&len, s->st.hyp_len + batch * nb + index, sizeof(int), hipMemcpyDeviceToHost));
-  HIP_TRY(hipMemcpy(&slot, s->st.hyp_slot + batch * (nb + 1) + index, sizeof(int), hipMemcpyDeviceToHost));
-  HIP_TRY(hipMemcpy(&sc, s->st.hyp_score + batch * nb + index, sizeof(float), hipMemcpyDeviceToHost));
+  const bool tokens_too = s->lists_bytes + s->tokens_bytes <= mi355x_search_ctx::kReadbackBytes;
+  char* const area = s->ctx->readback;
+  if (s->lists.empty()) {
+    const bool fits = s->lists_bytes <= mi355x_search_ctx::kReadbackBytes;
+    std::vector<char> lists(s->lists_bytes + (tokens_too ? s->tokens_bytes : 0));
+    HIP_TRY(hipMemcpyAsync(fits ? area : lists.data(), s->memory, s->lists_bytes, hipMemcpyDeviceToHost, st));
+    if (tokens_too) HIP_TRY(hipMemcpyAsync(area + s->lists_bytes, s->st.hyp_tokens, s->tokens_bytes, hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipStreamSynchronize(st));
+    if (fits) std::memcpy(lists.data(), area, lists.size());
+    s->lists = std::move(lists);
+  }
+  auto host = [&](auto* device) { return reinterpret_cast<decltype(device)>(s->lists.data() + (reinterpret_cast<char*>(device) - s->memory)); };
+  if (index < 0 || index >= host(s->st.hyp_used)[batch]) return Fail(MI355X_E_INVALID, "GetHypothesis index out of bounds");
+  const int len = host(s->st.hyp_len)[batch * nb + index], slot = host(s->st.hyp_slot)[batch * (nb + 1) + index];
   const int n = len < capacity ? len : capacity;
-  HIP_TRY(hipMemcpy(out, s->st.hyp_tokens + (static_cast<size_t>(batch) * (nb + 1) + slot) * s->st.max_length,
-                    sizeof(int32_t) * n, hipMemcpyDeviceToHost));
+  const size_t first = (static_cast<size_t>(batch) * (nb + 1) + slot) * s->st.max_length;
+  if (tokens_too) {
+    std::memcpy(out, s->lists.data() + s->lists_bytes + first * sizeof(int32_t), sizeof(int32_t) * n);
+  } else {
+    HIP_TRY(hipMemcpyAsync(out, s->st.hyp_tokens + first, sizeof(int32_t) * n, hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipStreamSynchronize(st));
+  }
   *length = len;
-  if (score) *score = sc;
+  if (score) *score = host(s->st.hyp_score)[batch * nb + index];
   return MI355X_OK;
 }
 

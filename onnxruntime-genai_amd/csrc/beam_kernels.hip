@@ -366,6 +366,14 @@ __global__ __launch_bounds__(64) void beam_scorer_finalize_kernel(const ScorerSt
   }
 }
 
+// The prompt (inside the kernel arguments, the first one) replicated to every beam's row, zeros behind it.
+__global__ __launch_bounds__(256) void beam_scorer_prompt_kernel(const PromptTokens, int prompt_len, int beams, int max_length,
+                                                                 int32_t* sequences) {
+  typedef __attribute__((address_space(4))) const int32_t* TablePtr;
+  const TablePtr token = (TablePtr)__builtin_amdgcn_kernarg_segment_ptr() + static_cast<int>(blockIdx.x) / beams * prompt_len;
+  int32_t* row = sequences + static_cast<size_t>(blockIdx.x) * max_length;
+  for (int i = threadIdx.x; i < max_length; i += 256) row[i] = i < prompt_len ? token[i] : 0;
+}
 
 // ---- long rows: candidates per segment, scored once the exact sum is known --------------------------------
 //
@@ -699,6 +707,11 @@ extern "C" hipError_t ms_launch_scorer_step(const ms::ScorerState* s, const int3
                                             hipStream_t stream) {
   hipLaunchKernelGGL(ms::beam_scorer_step_kernel, dim3(s->batch), dim3(64), 0, stream, *s, sequences, sequences_next,
                      sequence_length, cs, ct, ci);
+  return hipGetLastError();
+}
+extern "C" hipError_t ms_launch_scorer_prompt(const ms::PromptTokens* prompt, int prompt_len, int beams, int rows, int max_length,
+                                              int32_t* sequences, hipStream_t stream) {
+  hipLaunchKernelGGL(ms::beam_scorer_prompt_kernel, dim3(rows), dim3(256), 0, stream, *prompt, prompt_len, beams, max_length, sequences);
   return hipGetLastError();
 }
 extern "C" hipError_t ms_launch_scorer_finalize(const ms::ScorerState* s, const int32_t* sequences, int sequence_length,

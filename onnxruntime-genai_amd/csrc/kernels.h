@@ -110,6 +110,22 @@ struct WideTable<true> {
   typedef InlineParams type;
 };
 
+// Tables that travel inside the kernel arguments, as the first one.
+constexpr int kKvTensors = 64;
+struct KvTensors {
+  const void* present[kKvTensors];
+  void* past[kKvTensors];
+};
+constexpr int kTokenIndexRows = 256;
+struct TokenIndex {
+  int32_t token[kTokenIndexRows];
+};
+
+constexpr int kPromptTokens = 512;
+struct PromptTokens {
+  int32_t token[kPromptTokens];
+};
+
 struct ArgmaxArgs {
   const void* logits;
   int64_t row_stride;
@@ -235,9 +251,8 @@ hipError_t ms_launch_ngram_ban(const ms::Xform* xf, int rows, int vocab, int ngr
 hipError_t ms_launch_draw_in_order(const int32_t* kept_count, const int32_t* kept_ids, const float* kept_probs, int cap, int rows,
                                     const int32_t* skip, const double* pool, int32_t* out_tokens, int32_t* draws_used,
                                     hipStream_t stream);
-hipError_t ms_launch_kv_gather(const void* const* present_dev, void* const* past_dev, int n_tensors,
-                               const int32_t* beam_indices, int rows, size_t block_bytes, int width,
-                               hipStream_t stream);
+hipError_t ms_launch_kv_gather(const ms::KvTensors* tensors, int n_tensors, const int32_t* beam_indices, int rows, size_t block_bytes,
+                               int width, hipStream_t stream);
 hipError_t ms_launch_spec_verify(const float* p_target, const float* p_draft, const int32_t* draft_tokens,
                                  const float* accept_u, const double* sample_u, int batch, int K, int vocab,
                                  int32_t* accepted_len, int32_t* final_token, hipStream_t stream);
@@ -246,8 +261,8 @@ hipError_t ms_launch_greedy_tail(int32_t* next_tokens, int32_t* eos_seen, int ba
                                  hipStream_t stream);
 hipError_t ms_launch_spec_verify_sparse(const ms::SpecSparseArgs* a, int batch, hipStream_t stream);
 hipError_t ms_launch_cast(const void* in, void* out, size_t count, int kind, hipStream_t stream);
-hipError_t ms_launch_logits_handoff(const void* raw, int kind, int rows, int seq_len, int vocab,
-                                    const int32_t* token_index, float* out, int64_t out_stride, hipStream_t stream);
+hipError_t ms_launch_logits_handoff(const ms::TokenIndex* index, int indexed, const void* raw, int kind, int rows, int seq_len, int vocab,
+                                    float* out, int64_t out_stride, hipStream_t stream);
 hipError_t ms_launch_beam_select(const ms::BeamArgs* a, int dtype, hipStream_t stream);
 hipError_t ms_launch_beam_exp_step(const ms::SeqSumArgs* q, const ms::BeamArgs* a, int dtype, hipStream_t stream);
 // step != null: every batch entry's workgroup goes on with the entry's scorer step (ms_launch_scorer_step's work).
@@ -260,6 +275,8 @@ hipError_t ms_launch_softmax_apply(float* scores, int64_t row_stride, const ms::
 hipError_t ms_launch_scorer_step(const ms::ScorerState* s, const int32_t* sequences, int32_t* sequences_next,
                                  int sequence_length, const float* cs, const int32_t* ct, const int32_t* ci,
                                  hipStream_t stream);
+hipError_t ms_launch_scorer_prompt(const ms::PromptTokens* prompt, int prompt_len, int beams, int rows, int max_length, int32_t* sequences,
+                                   hipStream_t stream);
 hipError_t ms_launch_scorer_finalize(const ms::ScorerState* s, const int32_t* sequences, int sequence_length,
                                      hipStream_t stream);
 }
