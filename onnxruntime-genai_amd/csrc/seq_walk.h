@@ -6,25 +6,77 @@
 
 namespace ms {
 
-// ---- the walk: one wave per row walks, fifteen more prepare its way ------------------------------------
-// Steps compose associatively as long as the sum stays in one binade, so the walking wave does not visit the
-// segments one by one: lane l takes the record of segment seg + l, the compositions over lanes are scanned, and
-// every lane checks whether the sum would still be inside the binade after its segment.  All lanes before the
-// first one that fails are exact; the failing segment is handled through the records of its 64 parts in the same
-// way, a part that fails is added element by element (a chain of lane-shifted float additions), and the wave goes
-// on behind it with the binade the sum then has.
-//
-// Which records compose with which is known before the sum is: a record says for which binade it holds, so the
-// lanes fall into runs of equal binade, and the composition of a run from its first lane up to every lane of it
-// (a scan that starts afresh at every run) does not depend on the sum.  The workgroup's other waves prepare
-// these scans -- one wave for the segments' records, one per segment whose parts are needed -- and fetch the
-// elements of the parts that will most likely be added one by one, all at the same time; the walking wave then
-// only applies a prepared composition to the sum it holds wherever it stands at the first lane of a run in the
-// binade the run expects, and falls back to a scan of its own anywhere else.
+// Steps compose associatively as long as the sum stays in one binade, and where it leaves one is known in advance up
+// to the few parts of 64 elements in which the estimate of the running sum straddles a power of two (kPartMayCross),
+// or nothing is known about it (a negative binade: the row's first part, whose sums change binade every few
+// additions).  These parts are the row's events, ten to thirty of them; everything between two events is one composed
+// step, whatever its length.  So the workgroup prepares, all at the same time,
+//   * for every segment that has part records, the compositions of the parts before, between and behind its events,
+//     and from those and the records of the other segments one composition ahead of every event of the row;
+//   * for every event its 64 elements, the compositions of its first l elements under the lower binade and of its
+//     last l elements under the next one.
+// The first wave then goes from event to event with the sum it holds: one composed step, a compare over the 64
+// prefixes that finds the element at which the binade is left, one real float addition, one composed step for the rest.
+// Every application is checked against the binade the step holds for, which makes the result exact whatever the
+// estimates were.  An event that turns out otherwise is added element by element; where a composition between events
+// holds for another binade than the sum is in, the group of segments is walked by walk_group_checked.
+// (The walk as one wave that scanned part records wherever it stood took 12.7 us of the 18.4 us this launch took at
+// 16 x 151936, most of it chains of 64 additions for the parts that leave a binade.)
 constexpr Step kStepIdentity{0u, 0u};
 constexpr Step kStepLeaves{kStepSat, kStepSat};  // composed with anything, it still says "left the binade"
-constexpr int kWalkSpecials = 16;                 // segments per group of 64 whose part records are cached in LDS
 constexpr int kWalkWaves = 16;
+constexpr int kWalkSpecials = kWalkWaves;  // segments with part records per group of 64 segments, a wave each
+constexpr int kWalkEvents = 40;            // events per group
+constexpr int kWalkPart = 64;              // elements of a part
+static_assert(kSegSubs == 64 && kSegElems == kSegSubs * kWalkPart, "one part per lane");
+
+struct WalkShared {
+  uint2 prefix[kWalkEvents][kWalkPart];  // [l]: the steps of elements 0 .. l under the event's lower binade
+  uint2 suffix[kWalkEvents][kWalkPart];  // [l]: the steps of elements l .. 63 under the next one
+  float x[kWalkEvents][kWalkPart];
+  uint2 before[kWalkEvents];             // everything between the event before and this one
+  int2 event[kWalkEvents];               // lower binade (-1: to be added element by element), binade `before` holds for (-1: any)
+  int first[kWalkEvents], count[kWalkEvents];  // the part's elements
+  float after[kWalkEvents];              // the sum behind the event (ENDS)
+  uint2 tail[kWalkSpecials];             // per segment with part records: everything behind its last event ...
+  int tail_se[kWalkSpecials];            // ... the binade that holds for
+  int events_of[kWalkSpecials];
+};
+
+// A row in segments of equal length (all but the last): segment sg starts at element sg * kSegElems.
+struct EvenSegments {
+  int segs, length;
+  const int4* seg_step;  // this row's records, see SeqSumArgs
+  const int4* sub_step;
+  const int* sub_se;
+  const float* e;
+  __device__ __forceinline__ int first(int sg) const { return sg * kSegElems; }
+  __device__ __forceinline__ int count(int sg) const { return length - sg * kSegElems < kSegElems ? length - sg * kSegElems : kSegElems; }
+  __device__ __forceinline__ float value(int i) const { return e[i]; }
+};
+
+__device__ __forceinline__ Step step_from_below_or(Step none, Step x) {  // wave_shr:1, `none` into lane 0
+  Step y;
+  y.d0 = dpp_from_below_or<0x138, 0xf, uint32_t>(none.d0, x.d0);
+  y.d1 = dpp_from_below_or<0x138, 0xf, uint32_t>(none.d1, x.d1);
+  return y;
+}
+
+// Inclusive scan of compositions in which the lane's own step comes first and the lanes below it follow.
+__device__ __forceinline__ Step wave_scan_steps_backwards(Step x) {
+  x = step_compose(x, step_from_below<0x111, 0xf>(x));  // row_shr:1
+  x = step_compose(x, step_from_below<0x112, 0xf>(x));  // row_shr:2
+  x = step_compose(x, step_from_below<0x114, 0xf>(x));  // row_shr:4
+  x = step_compose(x, step_from_below<0x118, 0xf>(x));  // row_shr:8
+  x = step_compose(x, step_from_below<0x142, 0xa>(x));  // row_bcast:15 into rows 1 and 3
+  x = step_compose(x, step_from_below<0x143, 0xc>(x));  // row_bcast:31 into rows 2 and 3
+  return x;
+}
+
+// The additions of a wave's 64 values to s, one by one.
+__device__ __forceinline__ float wave_add_chain(float s, float x) {
+  return wave_read_lane(wave_serial_prefix(lane_id() == 0 ? s + x : x, 64), 63);
+}
 
 // Applies the steps f (one per lane; identity below `from`, kStepLeaves where no valid record exists) to the sum
 // s in lane order and returns the number of leading lanes from `from` on, below `limit`, whose results are exact;
@@ -40,65 +92,55 @@ __device__ __forceinline__ int wave_apply_steps(float& s, Step f, int from, int 
   return stop;
 }
 
-// A prepared run: `run` composes the steps from lane `head` up to this lane; `se` is the binade they hold for
-// (negative: none).  Applied to the sum s standing at lane `from`: the number of leading lanes from `from` on that
-// are exact (from itself if the run does not start there or expects another binade); s moves behind them.
-// *same_run: the lane it stopped at belongs to the run too, so the sum leaves the binade inside that lane's share.
-__device__ __forceinline__ int wave_apply_run(float& s, uint2 run, int head, int se, int from, int limit, bool* same_run) {
+// One wave walks segments g0 .. g0 + g_n - 1 with scans of its own wherever it stands, and adds element by element what
+// leaves the binade it is in: right for any records (r: the lane's segment record), at about ten times the cost.
+// ends, when not null: the sum behind every segment.
+template <typename Row>
+__device__ __forceinline__ float walk_group_checked(const Row& a, float s, int g0, int g_n, int4 r, float* ends) {
   const int lane = lane_id();
-  const SeqState st = seq_decompose(s);
-  const uint32_t n2 = step_apply(st.n, Step{run.x, run.y});
-  const bool mine = lane >= from && lane < limit && head == from && se == st.se;
-  const unsigned long long in_run = __ballot(mine);
-  const unsigned long long not_good = ~__ballot(mine && n2 < kMantLimit) & (~0ull << from);
-  const int stop = not_good != 0ull ? __ffsll(static_cast<long long>(not_good)) - 1 : 64;
-  if (stop > from) s = seq_recompose(wave_read_lane(n2, stop - 1), st.se);
-  *same_run = stop < 64 && ((in_run >> stop) & 1ull) != 0ull;
-  return stop;
+  int seg = 0;  // inside the group
+  while (seg < g_n) {
+    const int z = wave_read_lane(r.z, seg);
+    if (z != -2) {
+      const int se = seq_decompose(s).se;
+      const Step f = lane < seg ? kStepIdentity : (r.z == se ? Step{static_cast<uint32_t>(r.x), static_cast<uint32_t>(r.y)} : kStepLeaves);
+      const int next = wave_apply_steps(s, f, seg, ends != nullptr ? seg + 1 : g_n);
+      if (next > seg) {
+        if (ends != nullptr && lane == 0) ends[g0 + seg] = s;
+        seg = next;
+        continue;
+      }
+    }
+    const int first = a.first(g0 + seg), n = a.count(g0 + seg);
+    const int n_parts = (n + kWalkPart - 1) / kWalkPart;
+    int4 q = make_int4(0, 0, 0, 0);
+    int pse = -1;
+    if (z == -2) {
+      q = a.sub_step[static_cast<size_t>(g0 + seg) * kSegSubs + lane];
+      pse = a.sub_se[static_cast<size_t>(g0 + seg) * kSegSubs + lane];
+      if (pse >= 0) pse &= kPartMayCross - 1;
+    }
+    int part = 0;
+    while (part < n_parts) {
+      const int pe = seq_decompose(s).se;
+      Step pf = kStepLeaves;
+      if (lane < part) pf = kStepIdentity;
+      else if (pse >= 0 && pse == pe) pf = Step{static_cast<uint32_t>(q.x), static_cast<uint32_t>(q.y)};
+      else if (pse >= 0 && pse + 1 == pe) pf = Step{static_cast<uint32_t>(q.z), static_cast<uint32_t>(q.w)};
+      part = wave_apply_steps(s, pf, part, n_parts);
+      if (part >= n_parts) break;
+      const int np = n - part * kWalkPart < kWalkPart ? n - part * kWalkPart : kWalkPart;
+      s = wave_add_chain(s, lane < np ? a.value(first + part * kWalkPart + lane) : 0.0f);
+      ++part;
+    }
+    if (ends != nullptr && lane == 0) ends[g0 + seg] = s;
+    ++seg;
+  }
+  return s;
 }
-
-// Scan of steps that starts afresh at every lane whose `se` differs from the lane's below (and at every lane
-// without a valid step): the composition from the run's first lane up to each lane, and that first lane.
-__device__ __forceinline__ void wave_prepare_runs(Step st, int se, uint2* run, int* head) {
-  const int lane = lane_id();
-  const int below = dpp_from_below_or<0x138, 0xf, int>(-4, se);  // wave_shr:1; lane 0 sees a value no lane holds
-  int h = (lane == 0 || se < 0 || se != below) ? lane : -1;
-  wave_segscan_steps(st, h);
-  *run = make_uint2(st.d0, st.d1);
-  *head = h;
-}
-
-constexpr int kWalkAhead = 8;  // parts per cached segment whose elements are fetched ahead into LDS
-
-
-constexpr int kWalkPart = 64;  // elements of a part: one round of the addition chain
-static_assert(kSegSubs == 64 && kSegElems == kSegSubs * kWalkPart, "one part per lane");
-
-struct WalkShared {
-  int4 part_rec[kWalkSpecials][kSegSubs];
-  int part_se[kWalkSpecials][kSegSubs];
-  uint2 part_run[kWalkSpecials][kSegSubs];
-  unsigned char part_head[kWalkSpecials][kSegSubs];
-  float ahead[kWalkSpecials][kWalkAhead][kWalkPart];
-  int ahead_part[kWalkSpecials][kWalkAhead];
-  uint2 seg_run[64];
-  int seg_head[64];
-};
-
-// A row in segments of equal length (all but the last): segment sg starts at element sg * kSegElems.
-struct EvenSegments {
-  int segs, length;
-  const int4* seg_step;  // this row's records, see SeqSumArgs
-  const int4* sub_step;
-  const int* sub_se;
-  const float* e;
-  __device__ __forceinline__ int first(int sg) const { return sg * kSegElems; }
-  __device__ __forceinline__ int count(int sg) const { return length - sg * kSegElems < kSegElems ? length - sg * kSegElems : kSegElems; }
-  __device__ __forceinline__ float value(int i) const { return e[i]; }
-};
 
 // The exact sequential sum of a row's elements, by a workgroup of kWalkWaves waves (every thread calls; the result is
-// the first wave's).  ENDS: the walking wave also leaves the sum behind every segment in ends[segment].
+// the first wave's).  ENDS: the sum behind every segment goes to ends[segment].
 template <bool ENDS, typename Row>
 __device__ __forceinline__ float walk_segments(const Row& a, WalkShared& sh, float* ends) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -107,138 +149,178 @@ __device__ __forceinline__ float walk_segments(const Row& a, WalkShared& sh, flo
     const int g_n = a.segs - g0 < 64 ? a.segs - g0 : 64;
     const int4 r = lane < g_n ? a.seg_step[g0 + lane] : make_int4(0, 0, -3, 0);
     const unsigned long long special = __ballot(lane < g_n && r.z == -2);
-    const int n_special = __popcll(special) < kWalkSpecials ? __popcll(special) : kWalkSpecials;
+    const int n_special = __popcll(special);
     __syncthreads();  // the walk through the previous group is over
-    // task 0: the runs of the segments' records; task 1 + slot: the parts of the slot-th segment that has part
-    // records -- its runs and the elements of the parts that will most likely be added one by one (those whose
-    // estimated binade differs from the next part's, and those without an estimate)
-    for (int task = wave; task <= n_special; task += kWalkWaves) {
-      if (task == 0) {
-        uint2 run;
-        int head;
-        wave_prepare_runs(r.z >= 0 ? Step{static_cast<uint32_t>(r.x), static_cast<uint32_t>(r.y)} : kStepLeaves, r.z, &run,
-                          &head);
-        sh.seg_run[lane] = run;
-        sh.seg_head[lane] = head;
-        continue;
-      }
-      const int slot = task - 1;
+    // Wave w takes the w-th segment that has part records, a part per lane.
+    int4 q = make_int4(0, 0, 0, 0);
+    int pse = -1, sg = 0, n_parts = 0;
+    unsigned long long events = 0ull;
+    const bool has_segment = wave < n_special && n_special <= kWalkSpecials;
+    if (has_segment) {
       unsigned long long left = special;
-      for (int i = 0; i < slot; ++i) left &= left - 1ull;
-      const int sg = __ffsll(static_cast<long long>(left)) - 1;
-      const size_t at = static_cast<size_t>(g0 + sg) * kSegSubs;
-      const int sg_first = a.first(g0 + sg), sg_end = sg_first + a.count(g0 + sg);
-      const int4 q = a.sub_step[at + lane];
-      const int pse = a.sub_se[at + lane];
-      sh.part_rec[slot][lane] = q;
-      sh.part_se[slot][lane] = pse;
-      const int next_se = static_cast<int>(__builtin_amdgcn_update_dpp(0u, static_cast<uint32_t>(pse), 0x130, 0xf, 0xf, false));  // wave_shl:1: the lane above
-      unsigned long long want = __ballot(pse < 0 || (lane < 63 && next_se != pse));
-      int pp[kWalkAhead];
-      float val[kWalkAhead];
-#pragma unroll
-      for (int c = 0; c < kWalkAhead; ++c) {
-        pp[c] = -1;
-        val[c] = 0.0f;
-        if (want != 0ull) {
-          pp[c] = __ffsll(static_cast<long long>(want)) - 1;
-          want &= want - 1ull;
-          const int idx = sg_first + pp[c] * kWalkPart + lane;
-          if (idx < sg_end) val[c] = a.value(idx);
-        }
+      for (int i = 0; i < wave; ++i) left &= left - 1ull;
+      sg = g0 + __ffsll(static_cast<long long>(left)) - 1;
+      q = a.sub_step[static_cast<size_t>(sg) * kSegSubs + lane];
+      pse = a.sub_se[static_cast<size_t>(sg) * kSegSubs + lane];
+      n_parts = (a.count(sg) + kWalkPart - 1) / kWalkPart;
+      events = __ballot(lane < n_parts && (pse < 0 || (pse & kPartMayCross)));
+      if (pse >= 0) pse &= kPartMayCross - 1;
+    }
+    if (lane == 0) sh.events_of[wave] = __popcll(events);
+    __syncthreads();
+    const int in_segment = sh.events_of[lane & (kWalkWaves - 1)];
+    const int upto = wave_prefix_sum<int>(lane < kWalkWaves ? in_segment : 0);
+    const int total = wave_read_lane(upto, 63);
+    const bool fits = total <= kWalkEvents && n_special <= kWalkSpecials;
+    if (fits && has_segment) {
+      const int base = wave_read_lane(upto, wave) - wave_read_lane(in_segment, wave);
+      const bool is_event = (events >> lane) & 1ull, real = lane < n_parts;
+      // the compositions of the parts behind an event, up to every lane; a part under another binade than the one
+      // below it in the same run makes the run useless (and the walk finds out)
+      const int se_below = dpp_from_below_or<0x138, 0xf, int>(-1, is_event || !real ? -1 : pse);
+      const bool starts = lane == 0 || ((events >> (lane - 1)) & 1ull) || is_event;
+      Step f = is_event || !real ? kStepIdentity : Step{static_cast<uint32_t>(q.x), static_cast<uint32_t>(q.y)};
+      if (real && !is_event && !starts && se_below != pse) f = kStepLeaves;
+      int h = starts ? lane : -1;
+      wave_segscan_steps(f, h);
+      const Step ahead = step_from_below_or(kStepIdentity, f);
+      if (is_event) {
+        const int e = base + __popcll(events & ((1ull << lane) - 1ull));
+        sh.before[e] = make_uint2(ahead.d0, ahead.d1);
+        sh.event[e] = make_int2(pse, se_below);
+        sh.first[e] = a.first(sg) + lane * kWalkPart;
+        sh.count[e] = a.count(sg) - lane * kWalkPart < kWalkPart ? a.count(sg) - lane * kWalkPart : kWalkPart;
       }
-      uint2 run;
-      int head;
-      wave_prepare_runs(pse >= 0 ? Step{static_cast<uint32_t>(q.x), static_cast<uint32_t>(q.y)} : kStepLeaves, pse, &run, &head);
-      sh.part_run[slot][lane] = run;
-      sh.part_head[slot][lane] = static_cast<unsigned char>(head);
-#pragma unroll
-      for (int c = 0; c < kWalkAhead; ++c) {
-        if (lane == 0) sh.ahead_part[slot][c] = pp[c];
-        if (pp[c] >= 0) sh.ahead[slot][c][lane] = val[c];
+      if (lane == 63) sh.tail[wave] = make_uint2(f.d0, f.d1);
+      // (the last part is an event: nothing is behind it)
+      const int last_se = n_parts > 0 && !((events >> (n_parts - 1)) & 1ull) ? wave_read_lane(pse, n_parts - 1) : -1;
+      if (lane == 0) sh.tail_se[wave] = last_se;
+    }
+    __syncthreads();
+    // Every event's elements and their compositions, an event per wave in turn; the first wave, meanwhile, composes
+    // the segments between the events.
+    Step seg_upto = kStepIdentity;  // wave 0: everything from the last event at or before this lane's segment to its end
+    int seg_upto_se = -1, events_upto = 0;
+    if (fits) {
+      if (wave == 0) {
+        const int slot = __popcll(special & ((1ull << lane) - 1ull));
+        const bool is_special = (special >> lane) & 1ull;
+        const int mine = is_special ? sh.events_of[slot] : 0;
+        Step f = kStepIdentity;
+        int se = -1;
+        if (is_special) {
+          f = Step{sh.tail[slot].x, sh.tail[slot].y};
+          se = sh.tail_se[slot];
+          if (mine == 0 && se < 0) f = kStepLeaves;  // (a segment of no parts: it would hide its neighbours' binades from each other)
+        } else if (r.z >= 0) {
+          f = Step{static_cast<uint32_t>(r.x), static_cast<uint32_t>(r.y)};
+          se = r.z;
+        }
+        const bool starts = lane == 0 || mine > 0;
+        const int se_below = dpp_from_below_or<0x138, 0xf, int>(-1, se);
+        if (!starts && se >= 0 && se_below >= 0 && se != se_below) f = kStepLeaves;
+        int h = starts ? lane : -1;
+        wave_segscan_steps(f, h);
+        const Step ahead = step_from_below_or(kStepIdentity, f);
+        events_upto = wave_prefix_sum<int>(mine);
+        if (mine > 0) {  // the segment's first event: what its own segment has before it, behind all that
+          const int e = events_upto - mine;
+          int2 ev = sh.event[e];
+          Step own{sh.before[e].x, sh.before[e].y};
+          if (ev.y >= 0 && se_below >= 0 && ev.y != se_below) own = kStepLeaves;
+          const Step both = step_compose(ahead, own);
+          sh.before[e] = make_uint2(both.d0, both.d1);
+          if (ev.y < 0) ev.y = se_below;
+          sh.event[e] = ev;
+        }
+        seg_upto = f;
+        seg_upto_se = se;
+      }
+      for (int e = wave; e < total; e += kWalkWaves) {
+        const int first = sh.first[e], n = sh.count[e];
+        const float x = lane < n ? a.value(first + lane) : 0.0f;
+        sh.x[e][lane] = x;
+        // (wave 0 is still to rewrite an event's second word, not its first)
+        const int se = sh.event[e].x;
+        if (se >= 0) {
+          const float back = 63 - lane < n ? a.value(first + 63 - lane) : 0.0f;
+          const Step p = wave_scan_steps(seq_make_step(x, se));
+          sh.prefix[e][lane] = make_uint2(p.d0, p.d1);
+          const Step b = wave_scan_steps_backwards(seq_make_step(back, se + 1));
+          sh.suffix[e][63 - lane] = make_uint2(b.d0, b.d1);
+        }
       }
     }
     __syncthreads();
     if (wave != 0) continue;
-    const uint2 s_run = sh.seg_run[lane];
-    const int s_head = sh.seg_head[lane];
-    int seg = 0;  // inside the group
-    while (seg < g_n) {
-      bool same_run;
-      // the prepared run of whole segments, if one starts here in the binade the sum is in now
-      const SeqState at_seg = seq_decompose(s);
-      const int ahead_seg = wave_apply_run(s, s_run, s_head, r.z, seg, g_n, &same_run);
-      if (ahead_seg > seg) {
-        if (ENDS && lane >= seg && lane < ahead_seg)
-          ends[g0 + lane] = seq_recompose(step_apply(at_seg.n, Step{s_run.x, s_run.y}), at_seg.se);
-        seg = ahead_seg;
-        continue;
+    const float s_start = s;
+    bool good = fits;
+    if (fits) {
+      // what the next event needs is read while the current one is worked on
+      uint2 before = make_uint2(0u, 0u), pre = before, suf = before;
+      int2 ev = make_int2(-1, -1);
+      float x = 0.0f;
+      auto fetch = [&](int e) __attribute__((always_inline)) {
+        before = sh.before[e];
+        ev = sh.event[e];
+        pre = sh.prefix[e][lane];
+        suf = sh.suffix[e][lane];
+        x = sh.x[e][lane];
+      };
+      if (total > 0) fetch(0);
+      for (int e = 0; e < total && good; ++e) {
+        const uint2 c_before = before, c_pre = pre, c_suf = suf;
+        const int c_se = __builtin_amdgcn_readfirstlane(ev.x), c_before_se = __builtin_amdgcn_readfirstlane(ev.y);
+        const float c_x = x;
+        if (e + 1 < total) fetch(e + 1);
+        SeqState st = seq_decompose(s);
+        if (c_before_se >= 0) {
+          st.n = step_apply(st.n, Step{c_before.x, c_before.y});
+          good = c_before_se == st.se && st.n < kMantLimit;
+          if (!good) break;
+        }
+        const float s0 = seq_recompose(st.n, st.se);
+        bool done = false;
+        if (st.se == c_se) {
+          const uint32_t n = step_apply(st.n, Step{c_pre.x, c_pre.y});
+          const unsigned long long gone = __ballot(n >= kMantLimit);
+          if (gone == 0ull) {
+            s = seq_recompose(wave_read_lane(n, 63), st.se);
+            done = true;
+          } else {
+            const int j = __ffsll(static_cast<long long>(gone)) - 1;  // the element that leaves the binade
+            const float sj = (j > 0 ? seq_recompose(wave_read_lane(n, j - 1), st.se) : s0) + wave_read_lane(c_x, j);
+            const SeqState next = seq_decompose(sj);
+            Step rest = kStepIdentity;
+            if (j < 63) rest = Step{wave_read_lane(c_suf.x, j + 1), wave_read_lane(c_suf.y, j + 1)};
+            const uint32_t n2 = step_apply(next.n, rest);
+            done = next.se == c_se + 1 && n2 < kMantLimit;
+            s = seq_recompose(n2, next.se);
+          }
+        } else if (c_se >= 0 && st.se == c_se + 1) {
+          const uint32_t n2 = step_apply(st.n, Step{wave_read_lane(c_suf.x, 0), wave_read_lane(c_suf.y, 0)});
+          done = n2 < kMantLimit;
+          s = seq_recompose(n2, st.se);
+        }
+        if (!done) s = wave_add_chain(s0, c_x);
+        if (ENDS && lane == 0) sh.after[e] = s;
       }
-      const int z = wave_read_lane(r.z, seg);
-      if (z != -2) {
-        // a segment with a record of its own that the prepared runs did not take: the scan from here
-        const int se = seq_decompose(s).se;
-        const Step f = lane < seg ? kStepIdentity : (r.z == se ? Step{static_cast<uint32_t>(r.x), static_cast<uint32_t>(r.y)} : kStepLeaves);
-        // (where every segment's end is asked for, one segment at a time: this case is rare)
-        const int next = wave_apply_steps(s, f, seg, ENDS ? seg + 1 : g_n);
-        if (next > seg) {
-          if (ENDS && lane == 0) ends[g0 + seg] = s;
-          seg = next;
-          continue;
+      if (good) {
+        // the sum behind every segment, from the last event before its end
+        const float from = ENDS ? (events_upto > 0 ? sh.after[events_upto - 1] : s_start) : s;
+        const SeqState st = seq_decompose(from);
+        const uint32_t n = step_apply(st.n, seg_upto);
+        const bool fine = (seg_upto_se < 0 && seg_upto.d0 == 0u && seg_upto.d1 == 0u) || (seg_upto_se == st.se && n < kMantLimit);
+        const bool counts = ENDS ? lane < g_n : lane == g_n - 1;
+        good = __ballot(counts && !fine) == 0ull;
+        const float at_end = seg_upto_se < 0 ? from : seq_recompose(n, st.se);
+        if (good) {
+          if (ENDS && lane < g_n) ends[g0 + lane] = at_end;
+          s = wave_read_lane(at_end, g_n - 1);
         }
       }
-      // segment `seg` part by part
-      const int first = a.first(g0 + seg), n = a.count(g0 + seg);
-      const int n_parts = (n + kWalkPart - 1) / kWalkPart;
-      const int slot = __popcll(special & ((1ull << seg) - 1ull));
-      const bool cached = z == -2 && slot < kWalkSpecials;
-      int4 q = make_int4(0, 0, 0, 0);
-      int pse = -1;
-      uint2 p_run = make_uint2(0u, 0u);
-      int p_head = -1;
-      if (cached) {
-        q = sh.part_rec[slot][lane];
-        pse = sh.part_se[slot][lane];
-        p_run = sh.part_run[slot][lane];
-        p_head = sh.part_head[slot][lane];
-      } else if (z == -2) {
-        q = a.sub_step[static_cast<size_t>(g0 + seg) * kSegSubs + lane];
-        pse = a.sub_se[static_cast<size_t>(g0 + seg) * kSegSubs + lane];
-      }
-      int part = 0;
-      while (part < n_parts) {
-        // the prepared run of parts, if one starts here in the binade the sum is in now; where it ends inside
-        // its own run, the sum leaves the binade in that part
-        const int ahead_part_n = wave_apply_run(s, p_run, p_head, pse, part, n_parts, &same_run);
-        if (ahead_part_n > part) {
-          part = ahead_part_n;
-          if (part >= n_parts) break;
-          if (!same_run) continue;
-        } else {
-          const int pe = seq_decompose(s).se;
-          Step pf = kStepLeaves;
-          if (lane < part) pf = kStepIdentity;
-          else if (pse >= 0 && pse == pe) pf = Step{static_cast<uint32_t>(q.x), static_cast<uint32_t>(q.y)};
-          else if (pse >= 0 && pse + 1 == pe) pf = Step{static_cast<uint32_t>(q.z), static_cast<uint32_t>(q.w)};
-          part = wave_apply_steps(s, pf, part, n_parts);
-          if (part >= n_parts) break;
-        }
-        // this part's elements one by one, from LDS where they were fetched ahead
-        const int np = n - part * kWalkPart < kWalkPart ? n - part * kWalkPart : kWalkPart;
-        const int from = first + part * kWalkPart;
-        int hit = -1;
-        if (cached) {
-#pragma unroll
-          for (int c = 0; c < kWalkAhead; ++c)
-            if (sh.ahead_part[slot][c] == part) hit = c;
-        }
-        const float x = hit >= 0 ? sh.ahead[slot][hit][lane] : (lane < np ? a.value(from + lane) : 0.0f);
-        s = wave_read_lane(wave_serial_prefix(lane == 0 ? s + x : x, 64), 63);
-        ++part;
-      }
-      if (ENDS && lane == 0) ends[g0 + seg] = s;
-      ++seg;
     }
+    if (!good) s = walk_group_checked(a, s_start, g0, g_n, r, ENDS ? ends : nullptr);
   }
   return s;
 }

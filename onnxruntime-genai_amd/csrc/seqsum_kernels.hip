@@ -10,11 +10,9 @@
 //                       knows the binade its running sum will be in -- unless a power of two may fall
 //                       inside it -- and composes the step functions of its elements under that binade
 //                       into one (d0, d1) pair.
-//   3. seqsum_walk:     one wave per row walks the segments in order: composed steps are applied after
+//   3. seqsum_walk:     one wave per row goes through the composed steps (seq_walk.h): each is applied after
 //                       checking that the running sum really is in the assumed binade and stays in it
-//                       (then the composition is exactly the sequential result); a segment that may hold
-//                       a power of two is walked through the composed steps of its 64 parts, and a
-//                       part that fails the check is added element by element.
+//                       (then the composition is exactly the sequential result).
 // The check in step 3 makes the result independent of the estimate in step 2: a wrong guess only
 // costs a scan.
 #include "kernels.h"
@@ -46,7 +44,8 @@ __global__ __launch_bounds__(kSegBlock) void seqsum_max_kernel(const SeqSumArgs 
 }
 
 __global__ __launch_bounds__(64 * kWalkWaves) void seqsum_walk_kernel(const SeqSumArgs a) {
-  __shared__ WalkShared sh;
+  extern __shared__ u64 walk_lds[];
+  WalkShared& sh = *reinterpret_cast<WalkShared*>(walk_lds);
   const int row = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const size_t rbase = static_cast<size_t>(row) * a.segs;
   float max_score = 0.0f;
@@ -119,7 +118,7 @@ extern "C" hipError_t ms_launch_seqsum_max(const ms::SeqSumArgs* a, int dtype, h
 }
 
 extern "C" hipError_t ms_launch_seqsum_walk(const ms::SeqSumArgs* a, hipStream_t stream) {
-  hipLaunchKernelGGL(ms::seqsum_walk_kernel, dim3(a->rows), dim3(64 * ms::kWalkWaves), 0, stream, *a);
+  hipLaunchKernelGGL(ms::seqsum_walk_kernel, dim3(a->rows), dim3(64 * ms::kWalkWaves), sizeof(ms::WalkShared), stream, *a);
   return hipGetLastError();
 }
 

@@ -464,7 +464,8 @@ __global__ __launch_bounds__(kWideRankBlock) void wide_rank_kernel(const SampleA
     const float plo = __double2float_rd(start * (1.0 - seq_drift(p_first)));
     const float phi = __double2float_ru((start + mine) * (1.0 + seq_drift(p_first + kWalkPart)));
     int pse = seq_decompose(plo).se;
-    if (!(plo > 0.0f && phi < 3.0e38f && seq_decompose(phi).se <= pse + 1)) pse = -1;  // the walk adds this part itself
+    const int pse_end = seq_decompose(phi).se;
+    if (!(plo > 0.0f && phi < 3.0e38f && pse_end <= pse + 1)) pse = -1;  // the walk adds this part itself
     Step lo_step{0u, 0u}, hi_step{0u, 0u};
     if (pse >= 0) {
       lo_step = seq_compose_run(ev, kWideRankPer, pse);
@@ -476,7 +477,7 @@ __global__ __launch_bounds__(kWideRankBlock) void wide_rank_kernel(const SampleA
       const size_t at = rec_at * kSegSubs + part_i;
       w.sub_step[at] = make_int4(static_cast<int>(lo_step.d0), static_cast<int>(lo_step.d1), static_cast<int>(hi_step.d0),
                                       static_cast<int>(hi_step.d1));
-      w.sub_se[at] = pse;
+      w.sub_se[at] = pse >= 0 && pse_end != pse ? pse | kPartMayCross : pse;
     }
     if (tid == 0) *rec = make_int4(0, 0, -2, 0);
     return;
