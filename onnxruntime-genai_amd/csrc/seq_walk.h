@@ -13,10 +13,12 @@ namespace ms {
 // step, whatever its length.  So the workgroup prepares, all at the same time,
 //   * for every segment that has part records, the compositions of the parts before, between and behind its events,
 //     and from those and the records of the other segments one composition ahead of every event of the row;
-//   * for every event its 64 elements, the compositions of its first l elements under the lower binade and of its
-//     last l elements under the next one.
-// The first wave then goes from event to event with the sum it holds: one composed step, a compare over the 64
-// prefixes that finds the element at which the binade is left, one real float addition, one composed step for the rest.
+//   * for every event and each of its 64 elements l, the composition of all that lies between the event before and
+//     element l, under the event's lower binade, and of all its elements behind l, under the next one.
+// The first wave then goes from event to event with the sum it holds: every lane takes the sum in front of its element,
+// adds the element for real and goes on to the end of the part as if the binade were left right there; the first lane
+// whose addition does leave it has the sum behind the event.  About thirty instructions an event: the wave is alone on
+// its SIMD by then and issues one every ten cycles.
 // Every application is checked against the binade the step holds for, which makes the result exact whatever the
 // estimates were.  An event that turns out otherwise is added element by element; where a composition between events
 // holds for another binade than the sum is in, the group of segments is walked by walk_group_checked.
@@ -31,12 +33,15 @@ constexpr int kWalkPart = 64;              // elements of a part
 static_assert(kSegSubs == 64 && kSegElems == kSegSubs * kWalkPart, "one part per lane");
 
 struct WalkShared {
-  uint2 prefix[kWalkEvents][kWalkPart];  // [l]: the steps of elements 0 .. l under the event's lower binade
-  uint2 suffix[kWalkEvents][kWalkPart];  // [l]: the steps of elements l .. 63 under the next one
+  uint2 upto[kWalkEvents][kWalkPart];    // [l]: `before` and the steps of elements 0 .. l - 1 under the event's lower binade
+  uint2 behind[kWalkEvents][kWalkPart];  // [l]: the steps of elements l + 1 .. 63 under the next one
   float x[kWalkEvents][kWalkPart];
+  uint2 all[kWalkEvents];                // the steps of all elements under the next binade
   uint2 before[kWalkEvents];             // everything between the event before and this one
   int2 event[kWalkEvents];               // lower binade (-1: to be added element by element), binade `before` holds for (-1: any)
   int first[kWalkEvents], count[kWalkEvents];  // the part's elements
+  int led;                               // events at the row's start that are added up already ...
+  float lead;                            // ... to this
   float after[kWalkEvents];              // the sum behind the event (ENDS)
   uint2 tail[kWalkSpecials];             // per segment with part records: everything behind its last event ...
   int tail_se[kWalkSpecials];            // ... the binade that holds for
@@ -236,19 +241,50 @@ __device__ __forceinline__ float walk_segments(const Row& a, WalkShared& sh, flo
         seg_upto = f;
         seg_upto_se = se;
       }
-      for (int e = wave; e < total; e += kWalkWaves) {
+    }
+    // (an event's second word and what lies before it are still wave 0's to rewrite: they are used behind the barrier)
+    constexpr int kPerWave = (kWalkEvents + kWalkWaves - 1) / kWalkWaves;
+    Step in_front[kPerWave];
+#pragma unroll
+    for (int i = 0; i < kPerWave; ++i) {
+      const int e = wave + i * kWalkWaves;
+      in_front[i] = kStepIdentity;
+      if (fits && e < total) {
         const int first = sh.first[e], n = sh.count[e];
         const float x = lane < n ? a.value(first + lane) : 0.0f;
         sh.x[e][lane] = x;
-        // (wave 0 is still to rewrite an event's second word, not its first)
         const int se = sh.event[e].x;
         if (se >= 0) {
           const float back = 63 - lane < n ? a.value(first + 63 - lane) : 0.0f;
-          const Step p = wave_scan_steps(seq_make_step(x, se));
-          sh.prefix[e][lane] = make_uint2(p.d0, p.d1);
-          const Step b = wave_scan_steps_backwards(seq_make_step(back, se + 1));
-          sh.suffix[e][63 - lane] = make_uint2(b.d0, b.d1);
+          in_front[i] = step_from_below_or(kStepIdentity, wave_scan_steps(seq_make_step(x, se)));
+          const Step b = wave_scan_steps_backwards(seq_make_step(back, se + 1));  // lane l: elements 63 - l .. 63
+          if (lane < 63) sh.behind[e][62 - lane] = make_uint2(b.d0, b.d1);
+          else sh.all[e] = make_uint2(b.d0, b.d1);
+          if (lane == 63) sh.behind[e][63] = make_uint2(0u, 0u);
         }
+      }
+    }
+    // A row starts with parts whose sums change binade every few additions: one wave adds those up meanwhile.
+    if (wave == kWalkWaves - 1 && g0 == 0) {
+      int e = 0;
+      float sum = 0.0f;
+      for (; fits && e < total && sh.event[e].x < 0 && sh.first[e] == e * kWalkPart; ++e) {
+        sum = wave_add_chain(sum, lane < sh.count[e] ? a.value(e * kWalkPart + lane) : 0.0f);
+        if (ENDS && lane == 0) sh.after[e] = sum;
+      }
+      if (lane == 0) {
+        sh.led = e;
+        sh.lead = sum;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kPerWave; ++i) {
+      const int e = wave + i * kWalkWaves;
+      if (fits && e < total) {
+        const int2 ev = sh.event[e];
+        const Step both = ev.y >= 0 && ev.y != ev.x ? kStepLeaves : step_compose(Step{sh.before[e].x, sh.before[e].y}, in_front[i]);
+        sh.upto[e][lane] = make_uint2(both.d0, both.d1);
       }
     }
     __syncthreads();
@@ -257,52 +293,50 @@ __device__ __forceinline__ float walk_segments(const Row& a, WalkShared& sh, flo
     bool good = fits;
     if (fits) {
       // what the next event needs is read while the current one is worked on
-      uint2 before = make_uint2(0u, 0u), pre = before, suf = before;
+      uint2 upto_l = make_uint2(0u, 0u), behind_l = upto_l;
       int2 ev = make_int2(-1, -1);
       float x = 0.0f;
       auto fetch = [&](int e) __attribute__((always_inline)) {
-        before = sh.before[e];
         ev = sh.event[e];
-        pre = sh.prefix[e][lane];
-        suf = sh.suffix[e][lane];
+        upto_l = sh.upto[e][lane];
+        behind_l = sh.behind[e][lane];
         x = sh.x[e][lane];
       };
-      if (total > 0) fetch(0);
-      for (int e = 0; e < total && good; ++e) {
-        const uint2 c_before = before, c_pre = pre, c_suf = suf;
-        const int c_se = __builtin_amdgcn_readfirstlane(ev.x), c_before_se = __builtin_amdgcn_readfirstlane(ev.y);
+      const int e0 = g0 == 0 ? wave_read_lane(sh.led, 0) : 0;
+      if (e0 > 0) s = wave_read_lane(sh.lead, 0);
+      if (e0 < total) fetch(e0);
+      for (int e = e0; e < total; ++e) {
+        const uint2 c_upto = upto_l, c_behind = behind_l;
+        const int2 c_ev = ev;
         const float c_x = x;
-        if (e + 1 < total) fetch(e + 1);
-        SeqState st = seq_decompose(s);
-        if (c_before_se >= 0) {
-          st.n = step_apply(st.n, Step{c_before.x, c_before.y});
-          good = c_before_se == st.se && st.n < kMantLimit;
-          if (!good) break;
-        }
-        const float s0 = seq_recompose(st.n, st.se);
-        bool done = false;
-        if (st.se == c_se) {
-          const uint32_t n = step_apply(st.n, Step{c_pre.x, c_pre.y});
-          const unsigned long long gone = __ballot(n >= kMantLimit);
-          if (gone == 0ull) {
-            s = seq_recompose(wave_read_lane(n, 63), st.se);
-            done = true;
-          } else {
-            const int j = __ffsll(static_cast<long long>(gone)) - 1;  // the element that leaves the binade
-            const float sj = (j > 0 ? seq_recompose(wave_read_lane(n, j - 1), st.se) : s0) + wave_read_lane(c_x, j);
-            const SeqState next = seq_decompose(sj);
-            Step rest = kStepIdentity;
-            if (j < 63) rest = Step{wave_read_lane(c_suf.x, j + 1), wave_read_lane(c_suf.y, j + 1)};
-            const uint32_t n2 = step_apply(next.n, rest);
-            done = next.se == c_se + 1 && n2 < kMantLimit;
-            s = seq_recompose(n2, next.se);
+        fetch(e + 1 < total ? e + 1 : e);
+        // One branch: where the sum is not in the event's lower binade no lane is right, and where no addition leaves
+        // it the last lane has the sum.
+        const SeqState st = seq_decompose(s);
+        const uint32_t n = step_apply(st.n, Step{c_upto.x, c_upto.y});  // in front of the lane's element
+        const float with = seq_recompose(n, c_ev.x) + c_x;
+        const SeqState next = seq_decompose(with);
+        const uint32_t n2 = step_apply(next.n, Step{c_behind.x, c_behind.y});
+        const bool leaves = n >= kMantLimit || next.se != c_ev.x;
+        const bool right = st.se == c_ev.x && n < kMantLimit && (next.se == c_ev.x || (next.se == c_ev.x + 1 && n2 < kMantLimit));
+        const unsigned long long gone = __ballot(leaves), rights = __ballot(right);
+        const int j = gone != 0ull ? __ffsll(static_cast<long long>(gone)) - 1 : 63;
+        if ((rights >> j) & 1ull) {
+          s = wave_read_lane(leaves ? seq_recompose(n2, c_ev.x + 1) : with, j);
+        } else {
+          const int c_se = __builtin_amdgcn_readfirstlane(c_ev.x), c_before_se = __builtin_amdgcn_readfirstlane(c_ev.y);
+          const uint2 before = sh.before[e];
+          uint32_t n = st.n;
+          if (c_before_se >= 0) {
+            n = step_apply(n, Step{before.x, before.y});
+            good = c_before_se == st.se && n < kMantLimit;
+            if (!good) break;
           }
-        } else if (c_se >= 0 && st.se == c_se + 1) {
-          const uint32_t n2 = step_apply(st.n, Step{wave_read_lane(c_suf.x, 0), wave_read_lane(c_suf.y, 0)});
-          done = n2 < kMantLimit;
-          s = seq_recompose(n2, st.se);
+          const uint2 all = sh.all[e];
+          const uint32_t n_all = step_apply(n, Step{all.x, all.y});
+          if (c_se >= 0 && st.se == c_se + 1 && n_all < kMantLimit) s = seq_recompose(n_all, st.se);
+          else s = wave_add_chain(seq_recompose(n, st.se), c_x);
         }
-        if (!done) s = wave_add_chain(s0, c_x);
         if (ENDS && lane == 0) sh.after[e] = s;
       }
       if (good) {
