@@ -27,7 +27,7 @@ extern "C" int ms_sample_padded(mi355x_search_ctx* ctx, void* stream, const void
                                 mi355x_sample_params params, const mi355x_sample_params* per_row_params, const double* uniforms,
                                 int32_t* out_tokens, int32_t* kept_count, int32_t* kept_ids, float* kept_probs,
                                 int kept_capacity);
-extern "C" int ms_copy_on_stream(void* stream, void* dst, const void* src, size_t bytes);
+extern "C" int ms_copy_words_on_stream(void* stream, void* dst, const void* src, size_t words);
 
 namespace {
 
@@ -849,7 +849,7 @@ MS_METHOD(is_done) {
 Tensor CopyOf(const Scorer& s, const void* from, at::IntArrayRef sizes, at::ScalarType type) {
   Require(from != nullptr, "the scorer is closed");
   const Tensor out = Empty(sizes, type, c10::Device(c10::DeviceType::CUDA, s.device));
-  Check(ms_copy_on_stream(CurrentStream(), out.data_ptr(), from, out.nbytes()));
+  Check(ms_copy_words_on_stream(CurrentStream(), out.data_ptr(), from, out.nbytes() / 4));
   return out;
 }
 PyObject* get_next_scores(PyObject* self, void*) {

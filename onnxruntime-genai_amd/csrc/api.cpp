@@ -2,11 +2,14 @@
 // management and kernel launches.  No computation happens here, and there is no CPU fallback: every
 // entry point either launches the HIP kernels or fails.
 #include <hip/hip_runtime.h>
+#include <atomic>
 #include <cstdarg>
 #include <cstdio>
 #include <cmath>
 #include <cstring>
 #include <cstdlib>
+#include <memory>
+#include <mutex>
 #include <new>
 #include <string>
 #include <type_traits>
@@ -49,6 +52,25 @@ int NextPow2(int v) {
 }
 
 }  // namespace
+
+// Pinned host memory with a word per beam scorer of a context, which the step that finishes the last batch entry sets,
+// so that asking whether a search is done takes no copy.  Scorers past kCount at a time have no word.  (Held by the
+// context and by its scorers: a scorer may be destroyed after its context.)
+struct DoneWords {
+  static constexpr int kCount = 64;
+  int* words{};
+  std::atomic<uint64_t> used{};  // bit i: word i is taken
+  ~DoneWords() {
+    if (words) (void)hipHostFree(words);
+  }
+  int Take() {  // -1: none left
+    uint64_t seen = used.load();
+    while (~seen != 0 && !used.compare_exchange_weak(seen, seen | (seen + 1))) {
+    }
+    return ~seen != 0 ? __builtin_ctzll(~seen) : -1;
+  }
+  void GiveBack(int word) { used.fetch_and(~(uint64_t{1} << word)); }
+};
 
 struct mi355x_search_ctx {
   int device{};
@@ -95,6 +117,8 @@ struct mi355x_search_ctx {
   // calls that wait for their copy before they return.
   static constexpr size_t kReadbackBytes = 256 * 1024;
   char* readback{};
+  std::mutex readback_mutex;  // (scorers of one context may belong to different threads)
+  std::shared_ptr<DoneWords> done_words;
   hipEvent_t stage_event[kStageRing]{};
   bool stage_pending[kStageRing]{};
   int stage_next{}, stage_captured{};
@@ -240,6 +264,10 @@ int mi355x_search_create(int device, int max_rows, int max_vocab, mi355x_search_
     e = hipHostMalloc(&pinned, slots + mi355x_search_ctx::kReadbackBytes, hipHostMallocDefault);
     c->stage = static_cast<char*>(pinned);
     c->readback = c->stage + slots;
+  }
+  if (e == hipSuccess) {
+    c->done_words = std::make_shared<DoneWords>();
+    e = hipHostMalloc(reinterpret_cast<void**>(&c->done_words->words), DoneWords::kCount * sizeof(int), hipHostMallocDefault);
   }
   for (int i = 0; i < mi355x_search_ctx::kStageRing && e == hipSuccess; ++i)
     e = hipEventCreateWithFlags(&c->stage_event[i], hipEventDisableTiming);
@@ -547,9 +575,10 @@ int ms_sample_padded(mi355x_search_ctx* ctx, void* stream, const void* logits, c
                     kept_ids, kept_probs, kept_capacity, true);
 }
 
-// Device-to-device copy in stream order.
-int ms_copy_on_stream(void* stream, void* dst, const void* src, size_t bytes) {
-  HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, static_cast<hipStream_t>(stream)));
+// Copies 32-bit words between buffers of one device in stream order.
+int ms_copy_words_on_stream(void* stream, void* dst, const void* src, size_t words) {
+  if (words == 0) return MI355X_OK;
+  HIP_TRY(ms_launch_copy_words(static_cast<const uint32_t*>(src), static_cast<uint32_t*>(dst), words, static_cast<hipStream_t>(stream)));
   return MI355X_OK;
 }
 
@@ -902,6 +931,8 @@ struct mi355x_beam_scorer {
   // they fit the readback area next to them, the tokens.
   size_t lists_bytes{}, tokens_bytes{};
   std::vector<char> lists;  // empty: not read back
+  std::shared_ptr<DoneWords> done_words;
+  int done_word{-1};  // which of them st.all_done is (-1: none, the count is read back)
 };
 
 int mi355x_beam_scorer_create(mi355x_search_ctx* ctx, int batch, int beams, int max_length, int pad_token_id,
@@ -973,6 +1004,13 @@ int mi355x_beam_scorer_create(mi355x_search_ctx* ctx, int batch, int beams, int 
     for (size_t i = 0; i < ranks; ++i) host(st.hyp_slot)[i] = static_cast<int>(i % (beams + 1));
     for (int l = 0; l <= max_length; ++l) host(pow_table)[l] = length_penalty == 1.0f ? static_cast<float>(l) : std::pow(static_cast<float>(l), length_penalty);
     *host(st.not_done) = batch;
+    s->done_words = ctx->done_words;
+    s->done_word = s->done_words->Take();
+    if (s->done_word >= 0) {
+      st.all_done = s->done_words->words + s->done_word;
+      *st.all_done = 0;
+    }
+    std::lock_guard<std::mutex> hold(s->ctx->readback_mutex);
     e = hipMemsetAsync(s->memory + head_bytes, 0, at - head_bytes, nullptr);
     const char* from = head.data();
     if (head_bytes <= mi355x_search_ctx::kReadbackBytes) from = static_cast<const char*>(std::memcpy(ctx->readback, head.data(), head_bytes));
@@ -989,7 +1027,8 @@ int mi355x_beam_scorer_create(mi355x_search_ctx* ctx, int batch, int beams, int 
 
 void mi355x_beam_scorer_destroy(mi355x_beam_scorer* s) {
   if (!s) return;
-  if (s->memory) (void)hipFree(s->memory);
+  if (s->memory) (void)hipFree(s->memory);  // (waits for the steps under way: no launch sets the word after this)
+  if (s->done_word >= 0) s->done_words->GiveBack(s->done_word);
   delete s;
 }
 
@@ -1059,11 +1098,18 @@ const int32_t* mi355x_beam_scorer_sequences(const mi355x_beam_scorer* s, int* le
 int mi355x_beam_scorer_is_done(mi355x_beam_scorer* s, void* stream, int* done) {
   if (!s || !done) return Fail(MI355X_E_INVALID, "null argument");
   hipStream_t st = static_cast<hipStream_t>(stream);
-  // (through pinned memory: a copy into an ordinary variable waits twice, 21 us instead of 12)
-  int* const nd = reinterpret_cast<int*>(s->ctx->readback);
-  HIP_TRY(hipMemcpyAsync(nd, s->st.not_done, sizeof(int), hipMemcpyDeviceToHost, st));
-  HIP_TRY(hipStreamSynchronize(st));
-  *done = (*nd == 0) || (s->length == s->st.max_length);  // BeamSearch_Cpu::IsDone, src/search.cpp:345-352
+  bool all_done = false;
+  if (s->st.all_done) {
+    HIP_TRY(hipStreamSynchronize(st));
+    all_done = *static_cast<volatile int*>(s->st.all_done) != 0;
+  } else {
+    std::lock_guard<std::mutex> hold(s->ctx->readback_mutex);
+    int* const nd = reinterpret_cast<int*>(s->ctx->readback);
+    HIP_TRY(hipMemcpyAsync(nd, s->st.not_done, sizeof(int), hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipStreamSynchronize(st));
+    all_done = *nd == 0;
+  }
+  *done = all_done || (s->length == s->st.max_length);  // BeamSearch_Cpu::IsDone, src/search.cpp:345-352
   return MI355X_OK;
 }
 
@@ -1081,6 +1127,7 @@ int mi355x_beam_scorer_hypothesis(mi355x_beam_scorer* s, void* stream, int batch
   char* const area = s->ctx->readback;
   if (s->lists.empty()) {
     const bool fits = s->lists_bytes <= mi355x_search_ctx::kReadbackBytes;
+    std::lock_guard<std::mutex> hold(s->ctx->readback_mutex);
     std::vector<char> lists(s->lists_bytes + (tokens_too ? s->tokens_bytes : 0));
     HIP_TRY(hipMemcpyAsync(fits ? area : lists.data(), s->memory, s->lists_bytes, hipMemcpyDeviceToHost, st));
     if (tokens_too) HIP_TRY(hipMemcpyAsync(area + s->lists_bytes, s->st.hyp_tokens, s->tokens_bytes, hipMemcpyDeviceToHost, st));

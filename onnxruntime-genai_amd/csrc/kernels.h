@@ -219,6 +219,7 @@ struct ScorerState {
   int* hyp_used;          // [batch]
   int* done;              // [batch]
   int* not_done;          // [1]
+  int* all_done;          // pinned host memory, set once not_done reaches 0 (or null)
   const float* pow_table; // [max_length+1]: powf(length, length_penalty), computed by the host libm
   int* pending;           // [batch]: entries whose "can a later candidate still improve" test waits for all entries' candidates
   unsigned* arrive;       // [1]: workgroups of a fused selection + scorer launch that are through; 0 between launches
@@ -258,6 +259,7 @@ hipError_t ms_launch_kv_gather(const ms::KvTensors* tensors, int n_tensors, cons
 hipError_t ms_launch_spec_verify(const float* p_target, const float* p_draft, const int32_t* draft_tokens,
                                  const float* accept_u, const double* sample_u, int batch, int K, int vocab,
                                  int32_t* accepted_len, int32_t* final_token, hipStream_t stream);
+hipError_t ms_launch_copy_words(const uint32_t* src, uint32_t* dst, size_t words, hipStream_t stream);
 hipError_t ms_launch_greedy_tail(int32_t* next_tokens, int32_t* eos_seen, int batch, const int32_t* eos_ids, int n_eos,
                                  int32_t pad, int32_t* sequences, int max_length, int current_length, int32_t* done,
                                  hipStream_t stream);

@@ -608,3 +608,34 @@ def test_logits_handoff_slices_and_widens(ctx, orc, dtype, kind):
         assert np.array_equal(bits(got), bits(want))
     with pytest.raises(RuntimeError, match="outside"):
         ctx.logits_handoff(raw, [0, 0, 0, 0, 7])
+
+
+def test_each_of_many_scorers_tells_its_own_end():
+    """A scorer's end is told through a word of its context's; the scorers past the 64th have none and read the count
+    back, words of closed scorers are used again, and a scorer may outlive its context."""
+    ctx = pkg().SearchContext(2, 100)
+    dev = torch.device("cuda")
+    scores = torch.tensor([-0.1, -0.2, -0.3, -0.4], device=dev)
+    beams = torch.tensor([0, 1, 0, 1], dtype=torch.int32, device=dev)
+    going_on = torch.tensor([5, 6, 7, 8], dtype=torch.int32, device=dev)
+    ending = torch.tensor([2, 2, 5, 6], dtype=torch.int32, device=dev)
+
+    def scorer():
+        s = pkg().BeamScorer(ctx, 1, 2, 16, 0, [2], 1.0, True)
+        s.set_prompt(np.array([[3]], np.int32))
+        return s
+
+    scorers = [scorer() for _ in range(67)]
+    for end in (lambda i: i % 3 == 0, lambda i: True):
+        for i, s in enumerate(scorers):
+            if not s.is_done():
+                s.step(scores, ending if end(i) else going_on, beams)
+        assert [s.is_done() for s in scorers] == [end(i) for i in range(67)]
+    for s in scorers[::2]:
+        s.close()
+    again = [scorer() for _ in range(40)]
+    assert not any(s.is_done() for s in again) and all(s.is_done() for s in scorers[1::2])
+    assert again[0].next_indices.shape == (2,)
+    ctx.close()
+    for s in scorers[1::2] + again:
+        s.close()
