@@ -657,6 +657,97 @@ struct RowOutputs {
   int pad;  // non-zero: entries from the kept count to the capacity get id -1 and probability 0
 };
 
+// Position, in rank order, of the token a nucleus row draws, without the exact sum of its exponentials: for calls that
+// ask for the token alone.  e(0 .. n) are the row's largest exponentials, best first (e(0) = 1 for finite rows), n at most
+// blockDim * ITEMS.  With S_i the sum of e(0 .. i) -- in double here, a chain of fp32 additions in the reference, which is
+// off by at most i * 2^-24 of it -- and T_i = (V - i - 1) * e(i), FindNucleus stops at the first i with
+// prefix >= p * (prefix + T_i).  Its roundings move both sides by no more than
+//     err_i = S_i (1 - p) (i + 1) 2^-24 + 2^-22 (S_i + T_i)    (a little more here)
+// so it stops nowhere before the first i with S_i (1 - p) - p T_i >= -err_i (`lo`) and at the latest at the first one
+// with a difference above err_i (`hi`).  The draw compares shares S_k / S_stop with u, off by 2^-23 for the rounding of
+// the reference's fp32 weights; when it falls on one and the same position for every stop between lo and hi, that is
+// the token's.  Otherwise (a share closer to u than that, a stop the reference misses at the end of one of its batches,
+// no certain stop among the n, NaNs): -1, and the caller does the exact sums.
+// keep > 0: the stop is known (the exact sums have been done), keep elements are kept; only the draw is decided.
+// (A row of 1700 keys spends 4.9 us in the exact sum and 2.1 in the draw behind it, one of 9400 keys 10 and 4.  Steps of
+// 32 x 151936 bf16, p = 0.9: 44.6 -> 40.2 us.)
+template <int ITEMS, typename Exps>
+__device__ __forceinline__ int block_nucleus_token(int n, Exps exps, int V, float p, double u, SeqShared& sh, int keep) {
+  const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6, nw = static_cast<int>(blockDim.x) >> 6;
+  const int base = tid * ITEMS;
+  float ev[ITEMS];
+  double loc = 0.0;
+#pragma unroll
+  for (int j = 0; j < ITEMS; ++j) {
+    ev[j] = base + j < n ? exps(base + j) : 0.0f;
+    loc += static_cast<double>(ev[j]);
+  }
+  const double inc = wave_scan_add(loc);
+  if (lane == 63) sh.dscan[wave] = inc;
+  __syncthreads();
+  const double ws = row_scan_add(lane < nw ? sh.dscan[lane] : 0.0);
+  const double before = (wave > 0 ? wave_read_lane(ws, wave - 1) : 0.0) + (inc - loc);
+  const double pd = static_cast<double>(p), rest = 1.0 - pd;
+  auto tail = [=](int i, float e) { return static_cast<double>(V - i - 1) * static_cast<double>(e); };
+  auto error = [=](double s, double t, int i) { return s * rest * (static_cast<double>(i + 1) * 6.1e-8) + 2.6e-7 * (s + t); };
+  int lo = keep > 0 ? keep - 1 : kIntMax, hi = lo;
+  if (keep == 0 && base < n) {
+    // (S_i (1 - p) - p T_i never decreases: most threads are settled by the ends of their run)
+    const int last = (base + ITEMS < n ? base + ITEMS : n) - 1;
+    float e_last = ev[0];
+#pragma unroll
+    for (int j = 1; j < ITEMS; ++j) e_last = base + j == last ? ev[j] : e_last;
+    const double s_first = before + static_cast<double>(ev[0]), t_first = tail(base, ev[0]);
+    const double s_end = before + loc;
+    const bool none = s_end * rest - pd * tail(last, e_last) < -error(s_end, t_first, last);
+    const bool first_is_sure = s_first * rest - pd * t_first > error(s_first, t_first, base);
+    if (first_is_sure) {
+      lo = hi = base;
+    } else if (!none) {
+      double s = before;
+#pragma unroll
+      for (int j = 0; j < ITEMS; ++j) {
+        const int i = base + j;
+        s += static_cast<double>(ev[j]);
+        const double t = tail(i, ev[j]), g = s * rest - pd * t, err = error(s, t, i);
+        if (i < n && !(g < -err) && i < lo) lo = i;
+        if (i < n && g > err && i < hi) hi = i;
+      }
+    }
+  }
+  if (keep == 0) {
+    block_min2(lo, hi, sh);
+    if (hi == kIntMax) return -1;  // (the same in all threads, as every return here)
+    // a stop on the last element of one of the reference's batches (16, 64, 256, ... elements) is missed
+    bool batch_end = false;
+    for (int end = 16; end <= hi + 1 && end < V; end *= 4) batch_end = batch_end || end >= lo + 1;
+    if (batch_end) return -1;
+  }
+  auto sum_to = [&](int at) __attribute__((always_inline)) {
+    double s = before;
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) s += base + j <= at ? static_cast<double>(ev[j]) : 0.0;
+    return s;
+  };
+  if (lo >= base && lo < base + ITEMS) sh.dred[0] = sum_to(lo);
+  if (hi >= base && hi < base + ITEMS) sh.dred[1] = sum_to(hi);
+  __syncthreads();
+  const double s_lo = sh.dred[0], s_hi = sh.dred[1];
+  const double maybe = (u - 1.3e-7) * s_lo, sure = (u + 1.3e-7) * s_hi;
+  int first = kIntMax, first_sure = kIntMax;
+  if (base <= hi && before + loc >= maybe && before <= sure) {
+    double s = before;
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) {
+      s += static_cast<double>(ev[j]);
+      if (base + j < n && s >= maybe && base + j < first) first = base + j;
+      if (base + j < n && s >= sure && base + j < first_sure) first_sure = base + j;
+    }
+  }
+  block_min2(first, first_sure, sh);
+  return first == first_sure && first <= lo ? first : -1;
+}
+
 // The reference's ComputeSampledCategorical + SampleCategoricalToken
 // (src/sampling_distribution.h:218-297) on a row whose elements are available in rank order:
 // sorted(i) returns the key64 of the i-th best element for i < n_sorted.  exps(i) must return
@@ -669,8 +760,10 @@ template <int ITEMS, typename Sorted, typename Exps, typename IdAt = IdAsSorted>
 __device__ __forceinline__ bool block_sample_epilogue(Sorted sorted, Exps exps, int n_sorted, int vocab,
                                       mi355x_sample_params prm, double u, const RowOutputs& out,
                                       SeqShared& sh, bool synced = false, IdAt id_at = IdAt{}) {
-  int keep;
-  float scale;     // kept probability j = base_j * scale, base_j = exps(j) or exps(j)/sum
+  const bool token_alone = out.kept_count == nullptr && out.kept_ids == nullptr;
+  int early_pos = -1;  // the token's position, when it is known without the kept set
+  int keep = 0;
+  float scale = 0.0f;  // kept probability j = base_j * scale, base_j = exps(j) or exps(j)/sum
   float sum = 1.0f;
   bool divide_by_sum = false;
   int idx_dummy;
@@ -700,44 +793,59 @@ __device__ __forceinline__ bool block_sample_epilogue(Sorted sorted, Exps exps, 
     const float p = prm.p;
     const int limit = n_sorted < vocab ? n_sorted : vocab;
     const int V = vocab;
-    // The reference sorts in batches that end at 16, 64, 256, ... elements and recognises a stop
-    // only when it lies strictly inside a batch (src/sampling_distribution.h:166-181): a stop
-    // on the last element of a batch smaller than the row is missed and the search goes on in
-    // the next batch with the running sum it has.
-    int base = 0;
-    int cutoff;
-    float prefix = 0.0f;
-    bool prefix_is_keep_sum = true;
-    for (;;) {
-      const int b = base;
-      int si;
-      prefix = block_seq_sum<ITEMS>(prefix, limit - b, [=](int i) { return exps(i + b); }, StopAtNucleus{p, V, b}, &si, sh,
-                                    nullptr, b == 0 ? kEpiHead : 0, synced && b == 0);
-      if (si < 0) {
-        if (limit != vocab) return false;
-        cutoff = vocab;
-        break;
-      }
-      cutoff = b + si + 1;
-      const bool batch_end = cutoff >= 16 && (cutoff & (cutoff - 1)) == 0 && ((__ffs(cutoff) - 1) & 1) == 0;
-      if (!batch_end || cutoff >= vocab) break;
-      if (cutoff >= limit) return false;
-      base = cutoff;
-    }
-    if (vocab <= 64) {  // exact-partition override, src/sampling_distribution.h:186-203
-      if (n_sorted < vocab) return false;
-      const float global = block_seq_sum<ITEMS>(0.0f, vocab, exps, NoStop{}, &idx_dummy, sh, nullptr, kEpiHead);
-      int sj;
-      const float c = block_seq_sum<ITEMS>(0.0f, vocab, exps, StopAtMass{p * global}, &sj, sh, nullptr, kEpiHead);
-      (void)c;
-      if (sj >= 0) {
-        cutoff = sj + 1;
-        prefix_is_keep_sum = false;
+    // Token-only rows try to do without the exact sum where it is likely to work out: nuclei of n elements leave the
+    // stop open by n^2 * 6e-8 elements or so, each (1 - p) / (p V) of the total, and the draw meets one of the n shares
+    // in that range in n^3 * 2e-8 * (1 - p) / (p V) of the rows -- one of which is enough to make the launch longer by
+    // the attempt (2 us; the sum it saves takes 5).
+    if constexpr (ITEMS == 8) {
+      const float len = static_cast<float>(limit), rows = static_cast<float>(gridDim.x);
+      if (token_alone && p > 0.0f && p < 1.0f && vocab > 64 && limit <= static_cast<int>(blockDim.x) * ITEMS &&
+          rows * (len * len * len) * 2e-8f * (1.0f - p) < 0.25f * p * static_cast<float>(vocab)) {
+        if (!synced) __syncthreads();
+        early_pos = block_nucleus_token<ITEMS>(limit, exps, V, p, u, sh, 0);
+        synced = false;
       }
     }
-    if (!prefix_is_keep_sum) prefix = block_seq_sum<ITEMS>(0.0f, cutoff, exps, NoStop{}, &idx_dummy, sh, nullptr, kEpiHead);
-    keep = cutoff;
-    scale = prefix > 0.0f ? 1.0f / prefix : 0.0f;
+    if (early_pos < 0) {
+      // The reference sorts in batches that end at 16, 64, 256, ... elements and recognises a stop
+      // only when it lies strictly inside a batch (src/sampling_distribution.h:166-181): a stop
+      // on the last element of a batch smaller than the row is missed and the search goes on in
+      // the next batch with the running sum it has.
+      int base = 0;
+      int cutoff;
+      float prefix = 0.0f;
+      bool prefix_is_keep_sum = true;
+      for (;;) {
+        const int b = base;
+        int si;
+        prefix = block_seq_sum<ITEMS>(prefix, limit - b, [=](int i) { return exps(i + b); }, StopAtNucleus{p, V, b}, &si, sh,
+                                      nullptr, b == 0 ? kEpiHead : 0, synced && b == 0);
+        if (si < 0) {
+          if (limit != vocab) return false;
+          cutoff = vocab;
+          break;
+        }
+        cutoff = b + si + 1;
+        const bool batch_end = cutoff >= 16 && (cutoff & (cutoff - 1)) == 0 && ((__ffs(cutoff) - 1) & 1) == 0;
+        if (!batch_end || cutoff >= vocab) break;
+        if (cutoff >= limit) return false;
+        base = cutoff;
+      }
+      if (vocab <= 64) {  // exact-partition override, src/sampling_distribution.h:186-203
+        if (n_sorted < vocab) return false;
+        const float global = block_seq_sum<ITEMS>(0.0f, vocab, exps, NoStop{}, &idx_dummy, sh, nullptr, kEpiHead);
+        int sj;
+        const float c = block_seq_sum<ITEMS>(0.0f, vocab, exps, StopAtMass{p * global}, &sj, sh, nullptr, kEpiHead);
+        (void)c;
+        if (sj >= 0) {
+          cutoff = sj + 1;
+          prefix_is_keep_sum = false;
+        }
+      }
+      if (!prefix_is_keep_sum) prefix = block_seq_sum<ITEMS>(0.0f, cutoff, exps, NoStop{}, &idx_dummy, sh, nullptr, kEpiHead);
+      keep = cutoff;
+      scale = prefix > 0.0f ? 1.0f / prefix : 0.0f;
+    }
   }
   const float fsum = sum;
   const bool dv2 = divide_by_sum;
@@ -757,7 +865,17 @@ __device__ __forceinline__ bool block_sample_epilogue(Sorted sorted, Exps exps, 
       if (out.kept_probs) out.kept_probs[i] = in ? q(i) : 0.0f;
     }
   }
-  const int pos = block_discrete_draw<ITEMS>(keep, q, u, sh);
+  int pos = early_pos;
+  if constexpr (ITEMS == 8) {
+    // (a nucleus of more than one window of block_discrete_draw, which sums it first: 6.3 us for 9200 elements, 4.0 this way;
+    // 48 rows x 50257 in several modes: 56.4 -> 53.0 us per step)
+    const int span = static_cast<int>(blockDim.x) * ITEMS;
+    if (pos < 0 && prm.k <= 1 && keep > span && keep <= 2 * span && scale > 0.0f) {
+      __syncthreads();  // (the sums' readers are done)
+      pos = block_nucleus_token<2 * ITEMS>(keep, exps, vocab, prm.p, u, sh, keep);
+    }
+  }
+  if (pos < 0) pos = block_discrete_draw<ITEMS>(keep, q, u, sh);
   uint32_t id;
   if constexpr (std::is_same<IdAt, IdAsSorted>::value) id = key64_index(sorted(pos));
   else id = id_at(pos);

@@ -284,6 +284,44 @@ def test_token_only_calls_on_the_edges_of_their_guard_bands(ctx, orc, vocab, k, 
             assert np.array_equal(tokens_only(ctx, x, u, k, mass, t), orc.sample_batch(x, k, mass, t, u)), (j, mass)
 
 
+@pytest.mark.parametrize("vocab,sigma,p,dtype", [
+    (128256, 5.0, 0.9, np.float32), (50257, 3.0, 0.9, np.float16), (151936, 4.0, 0.95, np.float32), (5000, 1.0, 0.6, np.float32),
+    (65, 2.0, 0.9, np.float32), (64, 2.0, 0.9, np.float32), (20000, 2.0, 0.999999, np.float16), (32064, 0.0, 0.5, np.float32),
+])
+def test_token_only_nucleus_rows_on_the_edges_of_their_guard_bands(ctx, orc, vocab, sigma, p, dtype):
+    """Nucleus rows whose token alone is asked for are drawn from one fp64 prefix sum unless the stop or the draw is too
+    close to call: draws placed on, and within the guard bands beside, the reference's cumulative values (lists of a few
+    tokens, of one window and of two), and masses on both sides of the ones at which the reference's search changes its
+    mind -- also where it misses a stop, at the end of a batch of 16, 64, 256 ... elements."""
+    say("token only nucleus", vocab, sigma, p, dtype)
+    rng = np.random.default_rng(vocab + int(10 * p))
+    base = (rng.standard_normal(vocab) * sigma).astype(dtype)
+    kept = lambda mass: len(orc.sampled_categorical(base.astype(np.float32), 0, mass, 1.0)[0])
+    _, probs = orc.sampled_categorical(base.astype(np.float32), 0, p, 1.0)
+    cp = np.cumsum(np.asarray(probs, np.float64)) / np.sum(np.asarray(probs, np.float64))
+    us = list(rng.random(16)) + [0.0, np.nextafter(1.0, 0.0)]
+    for j in sorted({0, 1, len(cp) // 3, len(cp) // 2, len(cp) - 2} & set(range(len(cp)))):
+        us += [cp[j], np.nextafter(cp[j], 0.0), np.nextafter(cp[j], 1.0), cp[j] - 1e-7, cp[j] + 1e-7, cp[j] - 3e-7, cp[j] + 3e-7]
+    us = np.array([v for v in us if 0.0 <= v < 1.0], np.float64)
+    x = np.tile(base, (len(us), 1))
+    assert np.array_equal(tokens_only(ctx, x, us, 0, p, 1.0), orc.sample_batch(x.astype(np.float32), 0, p, 1.0, us))
+    if vocab > 20000:
+        return
+    u = rng.random(6)
+    x = np.tile(base, (len(u), 1))
+    for count in (1, 15, 16, 63, 64, 256, 1024):
+        low, high = np.float32(0.0), np.float32(1.0)  # the masses between which the search goes past `count` elements
+        for _ in range(40):
+            mid = np.float32((low + high) / 2)
+            if mid in (low, high):
+                break
+            low, high = (mid, high) if kept(float(mid)) <= count else (low, mid)
+        for mass in (low, high):
+            if 0.0 < mass < 1.0:
+                want = orc.sample_batch(x.astype(np.float32), 0, float(mass), 1.0, u)
+                assert np.array_equal(tokens_only(ctx, x, u, 0, float(mass), 1.0), want), (count, mass)
+
+
 def test_results_written_straight_to_pinned_host_memory(ctx, orc):
     """The output pointers may name pinned host memory that the device can address (the reference mirrors its
     results through pinned memory, src/cuda/interface.cpp:51-60): the kernels store the tokens there themselves, no
