@@ -15,7 +15,7 @@
  * (mi355x_sample* with per-row parameters for more than 64 rows, mi355x_logits_handoff with token_index,
  * mi355x_kv_gather) read it when they are called -- the first copies it into pinned memory of the context and records
  * a copy from there, the others carry it inside the kernel arguments -- so the caller's array is not read again at a
- * replay; every such call captured takes one of the context's 56 permanent staging slots (MI355X_E_UNSUPPORTED once
+ * replay; every captured call of the first kind takes one of the context's 56 permanent staging slots (MI355X_E_UNSUPPORTED once
  * they are used up).
  *
  * Versions: MI355X_ABI_VERSION names the layout of the structures below and the set of entry points;
