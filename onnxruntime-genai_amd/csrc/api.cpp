@@ -53,23 +53,37 @@ int NextPow2(int v) {
 
 }  // namespace
 
-// Pinned host memory with a word per beam scorer of a context, which the step that finishes the last batch entry sets,
-// so that asking whether a search is done takes no copy.  Scorers past kCount at a time have no word.  (Held by the
-// context and by its scorers: a scorer may be destroyed after its context.)
-struct DoneWords {
-  static constexpr int kCount = 64;
+// What a context shares with its beam scorers, which may be destroyed after it and may belong to different threads:
+// pinned host memory, held until the last of them is gone.
+//  - A word per scorer, which the step that finishes the last batch entry sets, so that asking whether a search is done
+//    takes no copy.  Scorers past kWords at a time have no word.
+//  - An area where small results and states go between host and device, by calls that hold its mutex and wait for
+//    their copy before they return.
+struct ScorerHost {
+  static constexpr int kWords = 64;
+  static constexpr size_t kReadbackBytes = 256 * 1024;
+  char* readback{};
+  std::mutex readback_mutex;
   int* words{};
   std::atomic<uint64_t> used{};  // bit i: word i is taken
-  ~DoneWords() {
-    if (words) (void)hipHostFree(words);
+  ~ScorerHost() {
+    if (readback) (void)hipHostFree(readback);
   }
-  int Take() {  // -1: none left
+  hipError_t Allocate() {
+    void* pinned = nullptr;
+    const hipError_t e = hipHostMalloc(&pinned, kReadbackBytes + kWords * sizeof(int), hipHostMallocDefault);
+    if (e != hipSuccess) return e;
+    readback = static_cast<char*>(pinned);
+    words = reinterpret_cast<int*>(readback + kReadbackBytes);
+    return hipSuccess;
+  }
+  int TakeWord() {  // -1: none left
     uint64_t seen = used.load();
     while (~seen != 0 && !used.compare_exchange_weak(seen, seen | (seen + 1))) {
     }
     return ~seen != 0 ? __builtin_ctzll(~seen) : -1;
   }
-  void GiveBack(int word) { used.fetch_and(~(uint64_t{1} << word)); }
+  void GiveBackWord(int word) { used.fetch_and(~(uint64_t{1} << word)); }
 };
 
 struct mi355x_search_ctx {
@@ -113,12 +127,7 @@ struct mi355x_search_ctx {
   static constexpr int kStageRing = 8, kStageCaptured = 56;
   char* stage{};
   size_t stage_slot_bytes{};
-  // The last kReadbackBytes of that pinned memory: where small results and states go between host and device, by
-  // calls that wait for their copy before they return.
-  static constexpr size_t kReadbackBytes = 256 * 1024;
-  char* readback{};
-  std::mutex readback_mutex;  // (scorers of one context may belong to different threads)
-  std::shared_ptr<DoneWords> done_words;
+  std::shared_ptr<ScorerHost> scorer_host;
   hipEvent_t stage_event[kStageRing]{};
   bool stage_pending[kStageRing]{};
   int stage_next{}, stage_captured{};
@@ -261,13 +270,12 @@ int mi355x_search_create(int device, int max_rows, int max_vocab, mi355x_search_
   if (e == hipSuccess) {
     void* pinned = nullptr;
     const size_t slots = c->stage_slot_bytes * (mi355x_search_ctx::kStageRing + mi355x_search_ctx::kStageCaptured);
-    e = hipHostMalloc(&pinned, slots + mi355x_search_ctx::kReadbackBytes, hipHostMallocDefault);
+    e = hipHostMalloc(&pinned, slots, hipHostMallocDefault);
     c->stage = static_cast<char*>(pinned);
-    c->readback = c->stage + slots;
   }
   if (e == hipSuccess) {
-    c->done_words = std::make_shared<DoneWords>();
-    e = hipHostMalloc(reinterpret_cast<void**>(&c->done_words->words), DoneWords::kCount * sizeof(int), hipHostMallocDefault);
+    c->scorer_host = std::make_shared<ScorerHost>();
+    e = c->scorer_host->Allocate();
   }
   for (int i = 0; i < mi355x_search_ctx::kStageRing && e == hipSuccess; ++i)
     e = hipEventCreateWithFlags(&c->stage_event[i], hipEventDisableTiming);
@@ -931,8 +939,8 @@ struct mi355x_beam_scorer {
   // they fit the readback area next to them, the tokens.
   size_t lists_bytes{}, tokens_bytes{};
   std::vector<char> lists;  // empty: not read back
-  std::shared_ptr<DoneWords> done_words;
-  int done_word{-1};  // which of them st.all_done is (-1: none, the count is read back)
+  std::shared_ptr<ScorerHost> host;  // (only the search steps use `ctx` itself after the creation: it may be gone before the others)
+  int done_word{-1};  // which of its words st.all_done is (-1: none, the count is read back)
 };
 
 int mi355x_beam_scorer_create(mi355x_search_ctx* ctx, int batch, int beams, int max_length, int pad_token_id,
@@ -1004,16 +1012,16 @@ int mi355x_beam_scorer_create(mi355x_search_ctx* ctx, int batch, int beams, int 
     for (size_t i = 0; i < ranks; ++i) host(st.hyp_slot)[i] = static_cast<int>(i % (beams + 1));
     for (int l = 0; l <= max_length; ++l) host(pow_table)[l] = length_penalty == 1.0f ? static_cast<float>(l) : std::pow(static_cast<float>(l), length_penalty);
     *host(st.not_done) = batch;
-    s->done_words = ctx->done_words;
-    s->done_word = s->done_words->Take();
+    s->host = ctx->scorer_host;
+    s->done_word = s->host->TakeWord();
     if (s->done_word >= 0) {
-      st.all_done = s->done_words->words + s->done_word;
+      st.all_done = s->host->words + s->done_word;
       *st.all_done = 0;
     }
-    std::lock_guard<std::mutex> hold(s->ctx->readback_mutex);
+    std::lock_guard<std::mutex> hold(s->host->readback_mutex);
     e = hipMemsetAsync(s->memory + head_bytes, 0, at - head_bytes, nullptr);
     const char* from = head.data();
-    if (head_bytes <= mi355x_search_ctx::kReadbackBytes) from = static_cast<const char*>(std::memcpy(ctx->readback, head.data(), head_bytes));
+    if (head_bytes <= ScorerHost::kReadbackBytes) from = static_cast<const char*>(std::memcpy(s->host->readback, head.data(), head_bytes));
     if (e == hipSuccess) e = hipMemcpyAsync(s->memory, from, head_bytes, hipMemcpyHostToDevice, nullptr);
     if (e == hipSuccess) e = hipStreamSynchronize(nullptr);  // the state is there before any stream uses it
   }
@@ -1028,7 +1036,7 @@ int mi355x_beam_scorer_create(mi355x_search_ctx* ctx, int batch, int beams, int 
 void mi355x_beam_scorer_destroy(mi355x_beam_scorer* s) {
   if (!s) return;
   if (s->memory) (void)hipFree(s->memory);  // (waits for the steps under way: no launch sets the word after this)
-  if (s->done_word >= 0) s->done_words->GiveBack(s->done_word);
+  if (s->done_word >= 0) s->host->GiveBackWord(s->done_word);
   delete s;
 }
 
@@ -1103,8 +1111,8 @@ int mi355x_beam_scorer_is_done(mi355x_beam_scorer* s, void* stream, int* done) {
     HIP_TRY(hipStreamSynchronize(st));
     all_done = *static_cast<volatile int*>(s->st.all_done) != 0;
   } else {
-    std::lock_guard<std::mutex> hold(s->ctx->readback_mutex);
-    int* const nd = reinterpret_cast<int*>(s->ctx->readback);
+    std::lock_guard<std::mutex> hold(s->host->readback_mutex);
+    int* const nd = reinterpret_cast<int*>(s->host->readback);
     HIP_TRY(hipMemcpyAsync(nd, s->st.not_done, sizeof(int), hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));
     all_done = *nd == 0;
@@ -1123,11 +1131,11 @@ int mi355x_beam_scorer_hypothesis(mi355x_beam_scorer* s, void* stream, int batch
     s->finalized = true;
   }
   const int nb = s->st.beams;
-  const bool tokens_too = s->lists_bytes + s->tokens_bytes <= mi355x_search_ctx::kReadbackBytes;
-  char* const area = s->ctx->readback;
+  const bool tokens_too = s->lists_bytes + s->tokens_bytes <= ScorerHost::kReadbackBytes;
+  char* const area = s->host->readback;
   if (s->lists.empty()) {
-    const bool fits = s->lists_bytes <= mi355x_search_ctx::kReadbackBytes;
-    std::lock_guard<std::mutex> hold(s->ctx->readback_mutex);
+    const bool fits = s->lists_bytes <= ScorerHost::kReadbackBytes;
+    std::lock_guard<std::mutex> hold(s->host->readback_mutex);
     std::vector<char> lists(s->lists_bytes + (tokens_too ? s->tokens_bytes : 0));
     HIP_TRY(hipMemcpyAsync(fits ? area : lists.data(), s->memory, s->lists_bytes, hipMemcpyDeviceToHost, st));
     if (tokens_too) HIP_TRY(hipMemcpyAsync(area + s->lists_bytes, s->st.hyp_tokens, s->tokens_bytes, hipMemcpyDeviceToHost, st));

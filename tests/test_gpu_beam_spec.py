@@ -639,3 +639,36 @@ def test_each_of_many_scorers_tells_its_own_end():
     ctx.close()
     for s in scorers[1::2] + again:
         s.close()
+
+
+def test_scorers_that_outlive_their_context_still_answer():
+    """is_done and the hypotheses of a scorer need its context no longer: neither of a scorer with a word of its own for
+    the search's end nor of one past the 64th, which reads the count back."""
+    say("scorers without their context")
+    dev = torch.device("cuda")
+    scores = torch.tensor([-0.1, -0.2, -0.3, -0.4], device=dev)
+    beams = torch.tensor([0, 1, 0, 1], dtype=torch.int32, device=dev)
+    ending = torch.tensor([2, 2, 5, 6], dtype=torch.int32, device=dev)
+    going_on = torch.tensor([5, 6, 7, 8], dtype=torch.int32, device=dev)
+
+    def scorers_of(ctx):
+        made = []
+        for i in range(66):
+            s = pkg().BeamScorer(ctx, 1, 2, 16, 0, [2], 1.0, True)
+            s.set_prompt(np.array([[3, 4 + i]], np.int32))
+            s.step(scores, going_on if i % 2 else ending, beams)
+            made.append(s)
+        return made
+
+    alive, gone = pkg().SearchContext(2, 100), pkg().SearchContext(2, 100)
+    kept, orphans = scorers_of(alive), scorers_of(gone)
+    gone.close()
+    other = pkg().SearchContext(2, 100)  # (takes what the closed context gave back)
+    for i in (0, 1, 62, 63, 64, 65):
+        assert orphans[i].is_done() == kept[i].is_done() == (i % 2 == 0), i
+        for index in range(2):
+            assert orphans[i].hypothesis(0, index) == kept[i].hypothesis(0, index), (i, index)
+    for s in orphans + kept:
+        s.close()
+    other.close()
+    alive.close()
