@@ -235,7 +235,8 @@ int mi355x_beam_scorer_create(mi355x_search_ctx* ctx, int batch, int beams, int 
                               float length_penalty, int early_stopping, mi355x_beam_scorer** out);
 void mi355x_beam_scorer_destroy(mi355x_beam_scorer* s);
 /* Sets the prompt: tokens HOST [batch, prompt_len], read by the call, replicated to every beam
- * (BeamSearch_Cpu::AppendTokens, src/search.cpp:326-343). */
+ * (BeamSearch_Cpu::AppendTokens, src/search.cpp:326-343).  Synchronous: the prompt is in place on return, for steps and
+ * readers on any stream; MI355X_E_UNSUPPORTED on a capturing stream. */
 int mi355x_beam_scorer_set_prompt(mi355x_beam_scorer* s, void* stream, const int32_t* tokens,
                                   int prompt_len);
 /* One BeamSearchScorer::Process + AppendNextTokensToSequences on the candidates produced by

@@ -1045,6 +1045,8 @@ int mi355x_beam_scorer_set_prompt(mi355x_beam_scorer* s, void* stream, const int
   if (prompt_len < 0 || prompt_len > s->st.max_length) return Fail(MI355X_E_INVALID, "User-defined tokens exceed max_length.");
   const int bb = s->st.batch * s->st.beams;
   hipStream_t st = static_cast<hipStream_t>(stream);
+  if (Capturing(st))
+    return Fail(MI355X_E_UNSUPPORTED, "the prompt is in place on return and sets the scorer's length: a graph replay would do neither");
   if (static_cast<size_t>(s->st.batch) * prompt_len <= ms::kPromptTokens) {  // inside the kernel arguments
     ms::PromptTokens prompt;
     std::copy_n(tokens, static_cast<size_t>(s->st.batch) * prompt_len, prompt.token);
@@ -1057,6 +1059,7 @@ int mi355x_beam_scorer_set_prompt(mi355x_beam_scorer* s, void* stream, const int
     HIP_TRY(hipMemcpyAsync(s->seq[s->cur], host.data(), host.size() * sizeof(int32_t), hipMemcpyHostToDevice, st));
     HIP_TRY(hipStreamSynchronize(st));  // `host` goes out of scope
   }
+  HIP_TRY(hipStreamSynchronize(st));  // steps and readers on any stream find the prompt
   s->length = prompt_len;
   return MI355X_OK;
 }

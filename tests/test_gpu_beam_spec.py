@@ -672,3 +672,38 @@ def test_scorers_that_outlive_their_context_still_answer():
         s.close()
     other.close()
     alive.close()
+
+
+@pytest.mark.parametrize("prompt_len", [3, 300])
+def test_a_prompt_is_in_place_when_the_call_returns(prompt_len):
+    """set_prompt waits, for a prompt of any length (up to 512 tokens travel inside the kernel arguments): a step or a
+    reader on another stream finds it.  A capturing stream is refused, and its capture goes on."""
+    say("set_prompt", prompt_len)
+    ctx = pkg().SearchContext(4, 5000)
+    scorer = pkg().BeamScorer(ctx, 2, 2, 400, 0, [2], 1.0, True)
+    prompt = np.arange(2 * prompt_len, dtype=np.int32).reshape(2, prompt_len) % 4000
+    busy = torch.cuda.Stream()
+    with torch.cuda.stream(busy):
+        torch.cuda._sleep(20_000_000)  # some milliseconds of GPU time in front of the prompt
+        scorer.set_prompt(prompt)
+        assert busy.query()  # nothing of it is left to do
+    seqs, length = scorer.sequences()
+    assert length == prompt_len and np.array_equal(seqs.cpu().numpy(), np.repeat(prompt, 2, axis=0))
+    x = torch.randn(4, 5000, device="cuda")
+    want = ctx.argmax(x).cpu().numpy()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            with pytest.raises(RuntimeError, match="error -4"):
+                scorer.set_prompt(prompt)
+            out = ctx.argmax(x)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(out.cpu().numpy(), want)
+    assert scorer.sequences()[1] == prompt_len
+    scorer.close()
+    ctx.close()
