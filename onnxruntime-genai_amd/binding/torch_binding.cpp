@@ -21,13 +21,13 @@
 #include "mi355x_search.h"
 
 // Entry points of libmi355x_search.so that have no place in the C ABI: mi355x_sample* whose kept sets are padded with
-// (id -1, probability 0) up to their capacity, and a copy of one of a scorer's arrays to `dst` on a stream.
+// (id -1, probability 0) up to their capacity, and a copy of one of a scorer's arrays to `dst` that is done on return.
 extern "C" int ms_sample_padded(mi355x_search_ctx* ctx, void* stream, const void* logits, const void* const* row_ptrs, int dtype,
                                 int64_t row_stride, int rows, int vocab, const mi355x_logits_xform* xf,
                                 mi355x_sample_params params, const mi355x_sample_params* per_row_params, const double* uniforms,
                                 int32_t* out_tokens, int32_t* kept_count, int32_t* kept_ids, float* kept_probs,
                                 int kept_capacity);
-extern "C" int ms_copy_words_on_stream(void* stream, void* dst, const void* src, size_t words);
+extern "C" int ms_copy_words_and_wait(void* stream, void* dst, const void* src, size_t words);
 
 namespace {
 
@@ -845,11 +845,18 @@ MS_METHOD(is_done) {
   });
 }
 
-// A copy of one of the scorer's arrays, made on the current stream (later steps on it overwrite the scorer's own).
+// A copy of one of the scorer's arrays as the work of the current stream leaves it (later steps overwrite the scorer's
+// own).  It is complete when the caller has it, whichever stream goes on with it.
 Tensor CopyOf(const Scorer& s, const void* from, at::IntArrayRef sizes, at::ScalarType type) {
   Require(from != nullptr, "the scorer is closed");
   const Tensor out = Empty(sizes, type, c10::Device(c10::DeviceType::CUDA, s.device));
-  Check(ms_copy_words_on_stream(CurrentStream(), out.data_ptr(), from, out.nbytes() / 4));
+  void* const stream = CurrentStream();
+  int rc;
+  {
+    Unlocked u;
+    rc = ms_copy_words_and_wait(stream, out.data_ptr(), from, out.nbytes() / 4);
+  }
+  Check(rc);
   return out;
 }
 PyObject* get_next_scores(PyObject* self, void*) {

@@ -583,10 +583,14 @@ int ms_sample_padded(mi355x_search_ctx* ctx, void* stream, const void* logits, c
                     kept_ids, kept_probs, kept_capacity, true);
 }
 
-// Copies 32-bit words between buffers of one device in stream order.
-int ms_copy_words_on_stream(void* stream, void* dst, const void* src, size_t words) {
-  if (words == 0) return MI355X_OK;
-  HIP_TRY(ms_launch_copy_words(static_cast<const uint32_t*>(src), static_cast<uint32_t*>(dst), words, static_cast<hipStream_t>(stream)));
+// Copies 32-bit words between buffers of one device, behind the work of `stream`, and waits for it: what the Python
+// binding hands out as the scorer's state is complete when the caller has it, on any stream.
+int ms_copy_words_and_wait(void* stream, void* dst, const void* src, size_t words) {
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (Capturing(s))
+    return Fail(MI355X_E_UNSUPPORTED, "a copy of a scorer's state is complete on return: it cannot be recorded into a graph");
+  if (words != 0) HIP_TRY(ms_launch_copy_words(static_cast<const uint32_t*>(src), static_cast<uint32_t*>(dst), words, s));
+  HIP_TRY(hipStreamSynchronize(s));
   return MI355X_OK;
 }
 

@@ -707,3 +707,41 @@ def test_a_prompt_is_in_place_when_the_call_returns(prompt_len):
     assert scorer.sequences()[1] == prompt_len
     scorer.close()
     ctx.close()
+
+
+def test_copies_of_a_scorers_state_are_complete_when_they_are_handed_out():
+    """next_scores, next_tokens, next_indices and sequences() wait for the work of the current stream: their tensors
+    can be read on any stream.  A capturing stream is refused, and its capture goes on."""
+    say("scorer views")
+    ctx = pkg().SearchContext(4, 5000)
+    scorer = pkg().BeamScorer(ctx, 2, 2, 16, 0, [2], 1.0, True)
+    scorer.set_prompt(np.array([[5, 6], [7, 8]], np.int32))
+    x = torch.randn(4, 5000, device="cuda")
+    torch.cuda.synchronize()
+    views = {"next_scores": lambda: scorer.next_scores, "next_tokens": lambda: scorer.next_tokens,
+             "next_indices": lambda: scorer.next_indices, "sequences": lambda: scorer.sequences()[0]}
+    busy = torch.cuda.Stream()
+    with torch.cuda.stream(busy):
+        for name, view in views.items():
+            torch.cuda._sleep(20_000_000)
+            scorer.search_step(x)
+            got = view()
+            assert busy.query(), name
+    assert got.shape == (4, 2 + len(views))
+    want = ctx.argmax(x).cpu().numpy()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            for view in views.values():
+                with pytest.raises(RuntimeError, match="error -4"):
+                    view()
+            out = ctx.argmax(x)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(out.cpu().numpy(), want)
+    scorer.close()
+    ctx.close()
