@@ -322,3 +322,50 @@ def test_draws_that_fall_into_runs_of_ties(ctx, orc, dtype, k, p, temp):
         u = rng.random(rows)
         got = ctx.sample(x16, torch.from_numpy(u).cuda(), k=k, p=p, temperature=temp).cpu().numpy()
         assert np.array_equal(got, orc.sample_batch(wide, k, p, temp, u)), rep
+
+
+def rows_with_one_run(rng, rows, vocab, run, dtype):
+    """`run` ids of every row share the best score, the first and the last id among them; the rest lies far below."""
+    x = (rng.standard_normal((rows, vocab)) - 25.0).astype(np.float32)
+    for r in range(rows):
+        ids = rng.permutation(vocab - 2)[: run - 2] + 1
+        x[r, ids] = x[r, 0] = x[r, vocab - 1] = 5.0
+    return torch.from_numpy(x).cuda().to(dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("vocab,run", [(40001, 2), (40001, 64), (128256, 65), (128256, 1025), (70001, 5000), (524288, 9000), (128256, 16000)])
+def test_the_token_of_a_run_of_ties(orc, vocab, run, dtype):
+    """A nucleus whose entries share one score, token only: the run is not ordered before the draw, the id of the drawn
+    rank is found among its ids afterwards -- pair by pair for short runs, by a selection for long ones."""
+    say("run of ties", vocab, run, dtype)
+    rng = np.random.default_rng(run)
+    rows = 6
+    c = pkg().SearchContext(rows, vocab)
+    x = rows_with_one_run(rng, rows, vocab, run, dtype)
+    u = np.array([0.0, 1.0 - 2.0 ** -53, 0.5 / run, 0.5, 0.25, 0.999])
+    got = c.sample(x, torch.from_numpy(u).cuda(), k=0, p=0.9, temperature=1.0).cpu().numpy()
+    assert np.array_equal(got, orc.sample_batch(x.float().cpu().numpy(), 0, 0.9, 1.0, u))
+    c.close()
+
+
+def test_long_runs_of_ties_take_linear_time():
+    """A run of 16000 ties costs a step no more than a few times what the sort of as many distinct entries does (fp32
+    rows); a compare per pair of ties made it sixty times as much."""
+    say("time of a run of ties")
+    rng = np.random.default_rng(1)
+    c = pkg().SearchContext(8, 128256)
+    u = torch.from_numpy(rng.random(8)).cuda()
+    best = {}
+    for dtype in (torch.float32, torch.float16):
+        x = rows_with_one_run(rng, 8, 128256, 16000, dtype)
+        for _ in range(6):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            for _ in range(4):
+                c.sample(x, u, k=0, p=0.9, temperature=1.0)
+            end.record()
+            end.synchronize()
+            best[dtype] = min(best.get(dtype, 1e9), start.elapsed_time(end))
+    assert best[torch.float16] < 5 * best[torch.float32], best
+    c.close()
