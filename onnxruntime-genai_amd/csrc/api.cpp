@@ -118,6 +118,7 @@ struct mi355x_search_ctx {
   float* row_sum{};
   ms::WideRow* wide_rows{};
   uint32_t* wide_tile_start{};
+  uint2* wide_cut_bucket{};
   int32_t* beam_row_tokens{};
   // Pinned host staging for the per-row parameters of more than 64 rows, which come in a caller's HOST array and do
   // not fit the kernel arguments: the call copies the array into a slot here and records a copy from the slot to the
@@ -256,6 +257,7 @@ int mi355x_search_create(int device, int max_rows, int max_vocab, mi355x_search_
   static_assert(ms::kWideTile <= ms::kSegElems, "room for either");
   ok(c->Alloc(&c->wide_rows, static_cast<size_t>(max_rows), false));
   ok(c->Alloc(&c->wide_tile_start, static_cast<size_t>(max_rows) * (c->max_segs + 1), false));
+  ok(c->Alloc(&c->wide_cut_bucket, static_cast<size_t>(max_rows) * (c->max_segs + 1), false));
   ok(c->Alloc(&c->seg_max, static_cast<size_t>(max_rows) * c->max_segs, false));
   ok(c->Alloc(&c->seg_sum, static_cast<size_t>(max_rows) * c->max_segs, false));
   // "not written yet" everywhere (all bits set): the state the exact-sum kernels expect and leave behind
@@ -488,7 +490,7 @@ int SampleImpl(mi355x_search_ctx* ctx, hipStream_t s, const void* logits, const 
   a.poll_limit = ctx->poll_limit;
   a.row_done = ctx->row_done;
   a.exact_kernel = (any_exact ? ms::kExactRows : 0) | (any_wide ? ms::kWideRows : 0);
-  const ms::WideArgs wide{(vocab + ms::kWideChunk - 1) / ms::kWideChunk, tiles, ctx->wide_rows, ctx->wide_tile_start, ctx->seg_sum,
+  const ms::WideArgs wide{(vocab + ms::kWideChunk - 1) / ms::kWideChunk, tiles, ctx->wide_rows, ctx->wide_tile_start, ctx->wide_cut_bucket, ctx->seg_sum,
                           ctx->seg_step, ctx->sub_step, ctx->sub_se, ctx->chunk_next};
   // a caller that bounds the number of allowed ids per row lets the sparse-mask kernel work alone
   if (xf && xf->mask && xf->mask_allowed_max > 0) {

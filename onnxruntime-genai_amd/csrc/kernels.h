@@ -83,7 +83,7 @@ struct SampleArgs {
 constexpr int kWideChunk = 8192;      // logits per workgroup of the passes over the row
 constexpr int kWideBuckets = 2048;    // buckets of the row's histogram
 constexpr int kWideTile = 3072;       // keys after which a new tile begins, with the next bucket
-constexpr int kWideBucketMax = 1024;  // keys of a bucket
+constexpr int kWideBucketMax = 1024;  // keys of a bucket that a tile takes whole
 constexpr int kWideMaxTiles = 192;    // tiles of the longest row (589824 logits)
 constexpr int kWideMinVocab = 4096;   // shorter rows are a single workgroup's work anyway
 struct WideRow {
@@ -94,6 +94,7 @@ struct WideArgs {
   int chunks, max_tiles;
   WideRow* rows;         // [rows]
   uint32_t* tile_start;  // [rows][max_tiles + 1]
+  uint2* cut_bucket;     // [rows][max_tiles + 1]: first and end place of the bucket a tile's start lies inside; zeros: of none
   double* tile_sum;      // [rows][max_tiles]
   int4* tile_step;       // [rows][max_tiles]: see SeqSumArgs::seg_step, and sub_step / sub_se
   int4* sub_step;

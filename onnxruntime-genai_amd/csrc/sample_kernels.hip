@@ -391,10 +391,6 @@ struct EmitTopk {
 // presorted: lds_keys[0 .. n_c) are sorted and hold their exponentials already (sort_gathered), only the epilogue is left.
 // TIES: ties_row0, when not null, says that entries of one score are in no particular order and where the row's logits
 // (of type ties_dtype) start: the run of entries that share the drawn one's exponential is ordered before its id is taken.
-// Runs of up to kTiePairs entries are ordered by comparing them pair by pair, in longer ones the id is selected
-// (block_tie_id): steps of 16 x 128256 fp16 take 28.6 us by pairs and 28.7 by the selection for a run of 64, 30.3 and
-// 29.1 for one of 128, 34.0 and 29.2 for one of 256.
-constexpr int kTiePairs = 64;
 template <bool TIES = false>
 __device__ __forceinline__ bool finish_candidates(u64* lds_keys, uint32_t* bucket_start, uint32_t n_c, u64 best_below,
                                                   uint32_t rmax, uint32_t thr, bool cut_at_best_below,

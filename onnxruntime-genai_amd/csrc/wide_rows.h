@@ -21,11 +21,13 @@
 //                    seqsum_exp_step).
 //   5. wide_finish:  a workgroup per row walks the records (the exact sum behind every tile), searches the one tile
 //                    in which the stop of FindNucleus can lie, and draws from the double sums of the tiles.
-// Elements of equal score need not be told apart before the draw: a run of ties weighs the same in any order.  Large
-// runs of ties (bf16 logits have hundreds per value) stay in arrival order, and the one run the draw falls into is
-// ordered by id then.  A call that asks for the kept ids has its ties ordered by wide_rank.
-// A row this does not fit (a bucket of more than kWideBucketMax keys, a maximum that is not finite, a stop beyond the
-// listed elements) is finished by the exact path inside wide_finish.
+// Elements of equal score need not be told apart before the draw: a run of ties weighs the same in any order.  Runs
+// of ties (bf16 logits have hundreds to thousands per value, the more the further their bulk lies from zero) stay in
+// arrival order, also across the tiles they are cut into, and the id of the drawn rank is taken from the run the draw
+// falls into.  A call that asks for the kept ids has its ties ordered by wide_rank.  A bucket of several scores too
+// large for a tile (a flat row, or one whose bulk is narrow) is cut between ranks its tiles select (wide_gather_cut).
+// A row this does not fit (a maximum that is not finite, a stop beyond the listed elements) is finished by the exact
+// path inside wide_finish.
 #pragma once
 #include "sample_stream.h"
 #include "seqsum_exp_step.h"
@@ -171,7 +173,7 @@ template <typename InT, bool INLINE>
 __global__ __launch_bounds__(kWideBlock) void wide_scatter_kernel(const SampleArgs a, const typename WideTable<INLINE>::type, const WideArgs w) {
   extern __shared__ u64 lds_keys[];
   WideScatterShared& sh = *reinterpret_cast<WideScatterShared*>(lds_keys);
-  __shared__ uint32_t wave_sums[16], wave_own[16], red[16];
+  __shared__ uint32_t wave_sums[16], wave_own[16];
   __shared__ u64 red64[16];
   const WideShare mine = wide_share(w.chunks);
   const int chunk = mine.item, row = mine.row, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -210,15 +212,11 @@ __global__ __launch_bounds__(kWideBlock) void wide_scatter_kernel(const SampleAr
     wave_sums[wave] = inc;
     wave_own[wave] = own_inc;
   }
-  const uint32_t widest = block_max<uint32_t>(all0 > all1 ? all0 : all1, red, false);  // (its barrier publishes the waves' sums)
+  __syncthreads();
   const uint32_t ws = wave_prefix_sum<uint32_t>(lane < 16 ? wave_sums[lane] : 0u), wo = wave_prefix_sum<uint32_t>(lane < 16 ? wave_own[lane] : 0u);
   const uint32_t n = wave_read_lane(ws, 15), n_own = wave_read_lane(wo, 15);
   const uint32_t start0 = (wave > 0 ? wave_read_lane(ws, wave - 1) : 0u) + inc - (all0 + all1), start1 = start0 + all0;
   const uint32_t here0 = (wave > 0 ? wave_read_lane(wo, wave - 1) : 0u) + own_inc - (own0 + own1), here1 = here0 + own0;
-  if (widest > static_cast<uint32_t>(kWideBucketMax)) {
-    if (chunk == 0 && tid == 0) *info = WideRow{0u, 0u, 1u, 0.0f};
-    return;
-  }
   sh.place[2 * tid] = here0;
   sh.place[2 * tid + 1] = here1;
   sh.shift[2 * tid] = start0 + before0 - here0;
@@ -226,17 +224,29 @@ __global__ __launch_bounds__(kWideBlock) void wide_scatter_kernel(const SampleAr
   if (chunk == 0) {
     // Tile t begins with the first bucket that starts at or after t * kWideTile: a bucket's start and the one before
     // it enclose the multiples it is the first after.  (The first bucket starts tile 0; an empty tile begins where
-    // the next one does.)
+    // the next one does.)  A bucket of more than kWideBucketMax keys is cut at the multiples themselves, and the cut
+    // remembers the bucket.
     uint32_t* const tile = w.tile_start + static_cast<size_t>(row) * (w.max_tiles + 1);
+    uint2* const cut = w.cut_bucket + static_cast<size_t>(row) * (w.max_tiles + 1);
     auto enclose = [&](uint32_t prev, uint32_t at) {
-      for (uint32_t t = prev / kWideTile + 1u; t <= at / kWideTile; ++t) tile[t] = at;
+      for (uint32_t t = prev / kWideTile + 1u; t <= at / kWideTile; ++t) {
+        const bool inside = at - prev > static_cast<uint32_t>(kWideBucketMax) && t * kWideTile < at;
+        tile[t] = inside ? t * kWideTile : at;
+        cut[t] = inside ? make_uint2(prev, at) : make_uint2(0u, 0u);
+      }
     };
-    if (tid == 0) tile[0] = 0u;
+    if (tid == 0) {
+      tile[0] = 0u;
+      cut[0] = make_uint2(0u, 0u);
+    }
     enclose(start0, start1);  // (the start after the last bucket's is n)
     enclose(start1, start1 + all1);
     const uint32_t tiles = (n + kWideTile - 1u) / kWideTile;
     if (tid == 0) {
-      if (n % kWideTile != 0u) tile[tiles] = n;  // (where n is a multiple itself, it is enclosed above)
+      if (n % kWideTile != 0u) {  // (where n is a multiple itself, it is enclosed above)
+        tile[tiles] = n;
+        cut[tiles] = make_uint2(0u, 0u);
+      }
       *info = WideRow{n, tiles, 0u, key_to_float(rmax)};
     }
   }
@@ -276,7 +286,117 @@ struct WideRankShared {  // 50 KB: three workgroups a CU
   uint32_t red[8], red2[8];
   double dred[8];
   Step wave_tot[8];
+  u64 low[8], high[8];     // a cut bucket's extremes
+  uint32_t pick[2], fill;  // the selection's digit and the rank inside it; the next free place in keys
 };
+
+// The key of rank r (from 0, best first) among the m distinct keys at src, whose lowest and highest are given: a
+// selection by twelve bits at a time below the bits all keys share.  (Two or three passes over the bucket: its keys
+// differ in the lower bits of their scores, or in their ids alone.)  Ends with a barrier.
+__device__ __forceinline__ u64 wide_select_key(const u64* src, uint32_t m, uint32_t r, u64 lowest, u64 highest, WideRankShared& sh) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr int kDigitBits = 12, kPer = (1 << kDigitBits) / kWideRankBlock;
+  static_assert(1 << kDigitBits == kWideSubBuckets, "the counts take the sub-buckets' place");
+  int open = 64 - __clzll(static_cast<long long>(lowest ^ highest));  // bits still to be decided
+  u64 prefix = open < 64 ? highest >> open : 0;
+  while (open > 0) {
+    const int take = open < kDigitBits ? open : kDigitBits, above = open;
+    open -= take;
+    for (int d = tid; d < kWideSubBuckets; d += kWideRankBlock) sh.start[d] = 0u;
+    __syncthreads();
+#pragma unroll 4
+    for (uint32_t i = tid; i < m; i += kWideRankBlock) {
+      const u64 k = src[i];
+      if ((above < 64 ? k >> above : 0) == prefix) atomicAdd(&sh.start[(k >> open) & ((1u << take) - 1u)], 1u);
+    }
+    __syncthreads();
+    uint32_t cnt[kPer], local = 0u;  // the highest digits belong to the first thread
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      cnt[j] = sh.start[kWideSubBuckets - 1 - (tid * kPer + j)];
+      local += cnt[j];
+    }
+    const uint32_t inc = wave_prefix_sum<uint32_t>(local);
+    if (lane == 63) sh.red[wave] = inc;
+    __syncthreads();
+    const uint32_t ws = wave_prefix_sum<uint32_t>(lane < kWideRankBlock / 64 ? sh.red[lane] : 0u);
+    uint32_t before = (wave > 0 ? wave_read_lane(ws, wave - 1) : 0u) + inc - local;
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      if (r >= before && r < before + cnt[j]) {
+        sh.pick[0] = static_cast<uint32_t>(kWideSubBuckets - 1 - (tid * kPer + j));
+        sh.pick[1] = r - before;
+      }
+      before += cnt[j];
+    }
+    __syncthreads();
+    prefix = (prefix << take) | sh.pick[0];
+    r = sh.pick[1];
+  }
+  return prefix;
+}
+
+// The keys of tile [first, first + n) of the row's list, in any order, in sh.keys, where one of its ends cuts a bucket
+// (head / tail: the buckets its two ends lie inside, or zeros).  The keys of a cut bucket lie in the list in the order
+// of arrival.  Where they all have one score, and nobody asks for the order of ties, any share of them will do: the one
+// at the tile's own places.  Otherwise the tile takes the keys whose ranks are its places, between two keys that it
+// selects from the bucket: every tile of the bucket reads all of it.
+__device__ __forceinline__ void wide_gather_cut(const u64* list, uint32_t first, uint32_t n, uint2 head, uint2 tail, bool order_ties,
+                                                WideRankShared& sh) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const uint32_t end = first + n;
+  auto copy = [&](uint32_t from, uint32_t to) {
+    for (uint32_t i = from + tid; i < to; i += kWideRankBlock) sh.keys[i - first] = list[i];
+  };
+  auto share = [&](uint2 bucket, uint32_t from, uint32_t to) {  // places from .. to of the list lie in the bucket
+    const u64* const src = list + bucket.x;
+    const uint32_t m = bucket.y - bucket.x;
+    u64 highest = 0, below = 0;  // (below: complement of the lowest)
+#pragma unroll 4
+    for (uint32_t i = tid; i < m; i += kWideRankBlock) {
+      const u64 k = src[i];
+      highest = k > highest ? k : highest;
+      below = ~k > below ? ~k : below;
+    }
+    highest = wave_max<u64>(highest);
+    below = wave_max<u64>(below);
+    if (lane == 0) {
+      sh.high[wave] = highest;
+      sh.low[wave] = below;
+    }
+    if (tid == 0) sh.fill = from - first;
+    __syncthreads();
+    highest = row16_max<u64>(lane < kWideRankBlock / 64 ? sh.high[lane] : 0);
+    const u64 lowest = ~row16_max<u64>(lane < kWideRankBlock / 64 ? sh.low[lane] : 0);
+    if (!order_ties && key64_okey(lowest) == key64_okey(highest)) {
+      copy(from, to);
+    } else {
+      const u64 best = from > bucket.x ? wide_select_key(src, m, from - bucket.x, lowest, highest, sh) : highest;
+      const u64 last = to < bucket.y ? wide_select_key(src, m, to - 1u - bucket.x, lowest, highest, sh) : lowest;
+      for (uint32_t i = tid; i < m; i += kWideRankBlock) {
+        const u64 k = src[i];
+        if (k <= best && k >= last) sh.keys[atomicAdd(&sh.fill, 1u)] = k;
+      }
+    }
+    __syncthreads();
+  };
+  uint32_t mid = first, mid_end = end;
+  if (head.y != 0u) {
+    mid = head.y < end ? head.y : end;
+    share(head, first, mid);
+  }
+  if (tail.y != 0u && tail.x >= mid) {  // (a tile inside one bucket has its only share already)
+    mid_end = tail.x;
+    share(tail, mid_end, end);
+  }
+  if (mid < mid_end) copy(mid, mid_end);
+  __syncthreads();
+}
+
+// Sub-buckets that have to be ranked are, by comparing the keys of each, unless one holds more than this: then the tile
+// is sorted by a network.  (Kept sets of 16 x 128256 bf16 rows, in order: by the network from 129 keys on and by pairs
+// 190 and 188 us a step for runs of up to 270 ties, 195 and 202 for runs of up to 400, 208 and 594 for runs of 1600.)
+constexpr uint32_t kWideRankCap = 256;
 
 template <bool INLINE>
 __global__ __launch_bounds__(kWideRankBlock) void wide_rank_kernel(const SampleArgs a, const typename WideTable<INLINE>::type, const WideArgs w) {
@@ -290,7 +410,11 @@ __global__ __launch_bounds__(kWideRankBlock) void wide_rank_kernel(const SampleA
   if (info.declined != 0u || static_cast<uint32_t>(t) >= info.tiles) return;
   const uint32_t* const tile = w.tile_start + static_cast<size_t>(row) * (w.max_tiles + 1) + t;
   const uint32_t first = tile[0], n = tile[1] - first;
-  const u64* const src = a.big2 + static_cast<size_t>(row) * a.big_stride + first;
+  const u64* const keys = a.big2 + static_cast<size_t>(row) * a.big_stride;
+  const uint2* const cut = w.cut_bucket + static_cast<size_t>(row) * (w.max_tiles + 1) + t;
+  const uint2 head = cut[0], tail = cut[1];
+  const bool order_ties = a.kept_ids != nullptr;
+  const u64* const src = keys + first;
   u64 k[kWideRankPer];
 #pragma unroll
   for (int r = 0; r < kWideRankPer; ++r) {
@@ -300,6 +424,16 @@ __global__ __launch_bounds__(kWideRankBlock) void wide_rank_kernel(const SampleA
   for (int b = tid; b <= kWideSubBuckets; b += kWideRankBlock) sh.start[b] = 0u;
   if (tid < kWideSubBuckets / 32) sh.mixed[tid] = 0u;
   if (tid >= 64 && tid < 96) sh.exp_tab[tid - 64] = em::exp2_tab(static_cast<uint32_t>(tid - 64));
+  if ((head.y | tail.y) != 0u) {
+    __syncthreads();  // (the gather uses the table as well)
+    wide_gather_cut(keys, first, n, head, tail, order_ties, sh);
+#pragma unroll
+    for (int r = 0; r < kWideRankPer; ++r) {
+      const uint32_t i = static_cast<uint32_t>(r * kWideRankBlock + tid);
+      k[r] = i < n ? sh.keys[i] : 0;
+    }
+    for (int b = tid; b <= kWideSubBuckets; b += kWideRankBlock) sh.start[b] = 0u;
+  }
   uint32_t hi = 0u, lo = 0xffffffffu;
 #pragma unroll
   for (int r = 0; r < kWideRankPer; ++r) {
@@ -340,18 +474,24 @@ __global__ __launch_bounds__(kWideRankBlock) void wide_rank_kernel(const SampleA
       if (sh.first_key[b] != key64_okey(k[r])) atomicOr(&sh.mixed[b >> 5], 1u << (b & 31u));
     }
   }
+  bool crowded;  // some bucket holds more than kWideRankCap keys
   {  // the buckets' first places: eight consecutive buckets per thread
     constexpr int kPer = kWideSubBuckets / kWideRankBlock;
-    uint32_t cnt[kPer], local = 0u;
+    constexpr uint32_t kCrowded = 1u << 31;
+    uint32_t cnt[kPer], local = 0u, most = 0u;
 #pragma unroll
     for (int i = 0; i < kPer; ++i) {
       cnt[i] = sh.start[tid * kPer + i];
       local += cnt[i];
+      most = cnt[i] > most ? cnt[i] : most;
     }
     const uint32_t inc = wave_prefix_sum<uint32_t>(local);
-    if (lane == 63) sh.red[wave] = inc;
+    const bool crowded_wave = __ballot(most > kWideRankCap) != 0;
+    if (lane == 63) sh.red[wave] = inc | (crowded_wave ? kCrowded : 0u);
     __syncthreads();
-    const uint32_t ws = wave_prefix_sum<uint32_t>(lane < kWideRankBlock / 64 ? sh.red[lane] : 0u);
+    const uint32_t of_wave = lane < kWideRankBlock / 64 ? sh.red[lane] : 0u;
+    crowded = __ballot((of_wave & kCrowded) != 0u) != 0;
+    const uint32_t ws = wave_prefix_sum<uint32_t>(of_wave & ~kCrowded);
     uint32_t c = (wave > 0 ? wave_read_lane(ws, wave - 1) : 0u) + inc - local;
 #pragma unroll
     for (int i = 0; i < kPer; ++i) {
@@ -367,7 +507,23 @@ __global__ __launch_bounds__(kWideRankBlock) void wide_rank_kernel(const SampleA
   __syncthreads();
   // Ranks, place by place (the lanes of a wave then look at the same few buckets).  A bucket of one score is in order
   // as it lies unless the ids are asked for; so are its exponentials.
-  const bool order_ties = a.kept_ids != nullptr;
+  auto must_rank = [&](uint32_t b) { return order_ties || ((sh.mixed[b >> 5] >> (b & 31u)) & 1u); };
+  bool by_network = false;
+  if (crowded) {
+    int too_full = 0;
+#pragma unroll
+    for (int r = 0; r < kWideRankPer; ++r) {
+      const uint32_t p = static_cast<uint32_t>(r * kWideRankBlock + tid);
+      if (p < n) {
+        const uint32_t b = bucket_of(sh.keys[p]);
+        if (sh.start[b + 1u] - sh.start[b] > kWideRankCap && must_rank(b)) too_full = 1;
+      } else {
+        sh.keys[p] = 0;
+      }
+    }
+    by_network = __syncthreads_or(too_full) != 0;
+    if (by_network) block_sort_desc(sh.keys, kSegElems);
+  }
   uint32_t fin[kWideRankPer];
 #pragma unroll
   for (int r = 0; r < kWideRankPer; ++r) {
@@ -378,7 +534,7 @@ __global__ __launch_bounds__(kWideRankBlock) void wide_rank_kernel(const SampleA
       k[r] = sh.keys[p];
       const uint32_t b = bucket_of(k[r]);
       const uint32_t s0 = sh.start[b], s1 = sh.start[b + 1u];
-      if (s1 - s0 > 1u && (order_ties || ((sh.mixed[b >> 5] >> (b & 31u)) & 1u))) {
+      if (s1 - s0 > 1u && !by_network && must_rank(b)) {
         uint32_t rank = 0u;
         for (uint32_t j = s0; j < s1; ++j) rank += sh.keys[j] > k[r] ? 1u : 0u;
         fin[r] = s0 + rank;
@@ -508,10 +664,12 @@ struct WideSegments {
 struct WideFinishShared {
   WalkShared walk;
   uint32_t tile_start[kWideMaxTiles + 1];
+  uint2 cut_bucket[kWideMaxTiles + 1];
   float ends[kWideMaxTiles];       // the exact sequential sum behind every tile
   double weight[kWideMaxTiles];    // a tile's share of the kept weight ...
   double upto[kWideMaxTiles];      // ... and the shares of all tiles up to it
-  u64 ties[kSegElems];
+  u64 ties[kTiePairs];
+  uint32_t tie_table[kTieTable];
 };
 static_assert(sizeof(WideFinishShared) <= kFinishLds, "the finish runs in the finish kernels' LDS");
 
@@ -575,6 +733,17 @@ __device__ __forceinline__ int wide_draw(W w, int keep, int used, double u, doub
   return calm == 0 || found == kIntMax ? -1 : found;
 }
 
+// Id of the element of rank `pos`, one of the entries run_lo .. run_lo + run of the list.  (A call of its own: inlined
+// into the finish, which seldom needs it, it made every row's 1 us longer.)
+__device__ __noinline__ uint32_t wide_tie_id(const u64* list, int run_lo, int run, int pos, const void* row0, int dtype, uint32_t* table) {
+  const RowPtr<AnyDtype> lrow(row0, dtype);
+  auto whole_key = [=](int i) {
+    const uint32_t id = key64_index(list[i]);
+    return make_key64(order_key(lrow[id]), id);
+  };
+  return block_tie_id(run, pos - run_lo, key64_okey(whole_key(pos)), [=](int i) { return whole_key(run_lo + i); }, table);
+}
+
 // Runs by the whole workgroup; false: the row needs the exact path.
 template <bool INLINE>
 __device__ __forceinline__ bool wide_finish_row(const SampleArgs& a, const WideArgs& w, int row, mi355x_sample_params prm, WideFinishShared& sh, SeqShared& seqsh) {
@@ -583,7 +752,10 @@ __device__ __forceinline__ bool wide_finish_row(const SampleArgs& a, const WideA
   if (info.declined != 0u || info.n == 0u) return false;
   const int n = static_cast<int>(info.n), tiles = static_cast<int>(info.tiles);
   const size_t rbase = static_cast<size_t>(row) * w.max_tiles;
-  for (int t = tid; t <= tiles; t += kFinishBlock) sh.tile_start[t] = w.tile_start[static_cast<size_t>(row) * (w.max_tiles + 1) + t];
+  for (int t = tid; t <= tiles; t += kFinishBlock) {
+    sh.tile_start[t] = w.tile_start[static_cast<size_t>(row) * (w.max_tiles + 1) + t];
+    sh.cut_bucket[t] = w.cut_bucket[static_cast<size_t>(row) * (w.max_tiles + 1) + t];
+  }
   for (int t = tid; t < tiles; t += kFinishBlock) sh.weight[t] = w.tile_sum[rbase + t];
   const u64 below = w.best_below[row];  // the best element past the list; it follows the list's last
   const u64* const list = a.big + static_cast<size_t>(row) * a.big_stride;
@@ -684,36 +856,58 @@ __device__ __forceinline__ bool wide_finish_row(const SampleArgs& a, const WideA
     if (tid == 0) *out.token = static_cast<int32_t>(key64_index(below));
     return true;
   }
-  // entries of one exponential may be ties in arrival order: the run the draw fell into is ordered by whole keys
-  const uint32_t mine = static_cast<uint32_t>(list[pos] >> 32);
+  // Unless the order of ties was asked for, entries of one exponential may be ties in the order of arrival, within a tile
+  // and, in a bucket that is cut, over all of its tiles: the id of the drawn rank is taken from all of these.
+  if (out.kept_ids) {
+    if (tid == 0) *out.token = static_cast<int32_t>(key64_index(list[pos]));
+    return true;
+  }
   int lo = 0, hi = tiles - 1;
   while (lo < hi) {
     const int mid = (lo + hi) >> 1;
     if (static_cast<int>(sh.tile_start[mid + 1]) > pos) hi = mid;
     else lo = mid + 1;
   }
-  const int t0 = static_cast<int>(sh.tile_start[lo]), t1 = static_cast<int>(sh.tile_start[lo + 1]);
-  int run_lo = kIntMax, run_hi = kIntMax;  // first entry of the run, and minus its last
-  for (int i = t0 + tid; i < t1; i += kFinishBlock) {
-    if (static_cast<uint32_t>(list[i] >> 32) == mine) {
-      run_lo = i < run_lo ? i : run_lo;
-      run_hi = -i < run_hi ? -i : run_hi;
+  const uint2 head = sh.cut_bucket[lo], tail = sh.cut_bucket[lo + 1];
+  int run_lo, run;  // the entries to choose from: as many before the first of them as elements rank before them all
+  if (static_cast<int>(head.y) > pos) {
+    run_lo = static_cast<int>(head.x);
+    run = static_cast<int>(head.y - head.x);
+  } else if (tail.y != 0u && static_cast<int>(tail.x) <= pos) {
+    run_lo = static_cast<int>(tail.x);
+    run = static_cast<int>(tail.y - tail.x);
+  } else {
+    const uint32_t mine = static_cast<uint32_t>(list[pos] >> 32);
+    const int t0 = static_cast<int>(sh.tile_start[lo]), t1 = static_cast<int>(sh.tile_start[lo + 1]);
+    int run_hi = kIntMax;  // minus the run's last entry
+    run_lo = kIntMax;
+    for (int i = t0 + tid; i < t1; i += kFinishBlock) {
+      if (static_cast<uint32_t>(list[i] >> 32) == mine) {
+        run_lo = i < run_lo ? i : run_lo;
+        run_hi = -i < run_hi ? -i : run_hi;
+      }
     }
+    block_min2(run_lo, run_hi, seqsh);
+    run = -run_hi - run_lo + 1;
   }
-  block_min2(run_lo, run_hi, seqsh);
-  const int run = -run_hi - run_lo + 1;
   if (run == 1) {
     if (tid == 0) *out.token = static_cast<int32_t>(key64_index(list[pos]));
     return true;
   }
-  const RowPtr<AnyDtype> lrow(row_start<INLINE>(a, row, dtype_bytes(a.dtype)), a.dtype);
-  for (int i = tid; i < run; i += kFinishBlock) {
-    const uint32_t id = key64_index(list[run_lo + i]);
-    sh.ties[i] = make_key64(order_key(lrow[id]), id);
+  const void* const row0 = row_start<INLINE>(a, row, dtype_bytes(a.dtype));
+  if (run > kTiePairs) {
+    const uint32_t id = wide_tie_id(list, run_lo, run, pos, row0, a.dtype, sh.tie_table);
+    if (tid == 0) *out.token = static_cast<int32_t>(id);
+    return true;
+  }
+  const RowPtr<AnyDtype> lrow(row0, a.dtype);
+  if (tid < run) {
+    const uint32_t id = key64_index(list[run_lo + tid]);
+    sh.ties[tid] = make_key64(order_key(lrow[id]), id);
   }
   __syncthreads();
-  for (int i = tid; i < run; i += kFinishBlock) {
-    const u64 k = sh.ties[i];
+  if (tid < run) {
+    const u64 k = sh.ties[tid];
     int rank = 0;
     for (int j = 0; j < run; ++j) rank += sh.ties[j] > k ? 1 : 0;
     if (rank == pos - run_lo) *out.token = static_cast<int32_t>(key64_index(k));

@@ -1450,3 +1450,75 @@ def test_whole_vocabulary_rows_spread_over_the_gpu(ctx, orc, vocab, dtype):
     params = [[(0, 1.0, 0.8), (20, 0.9, 1.0), (0, 0.7, 1.0)][r % 3] for r in range(rows)]
     got = ctx.sample([row.clone() for row in xd], ud, per_row=params).cpu().numpy()
     assert np.array_equal(got, [orc.sample_row(xw[r], *params[r], u[r]) for r in range(rows)])
+
+
+def crowded_rows(name, rng, rows, vocab):
+    """Rows of which many ids share a score, or lie so close together that a bucket of the row's histogram (a 2048th of
+    about thirty temperatures) holds more of them than a tile takes whole: (logits, element type, temperatures)."""
+    x = rng.standard_normal((rows, vocab)).astype(np.float32)
+    if name == "far_from_zero":  # bf16 has a value per 0.0625 around 12
+        return 2.0 * x + 12.0, torch.bfloat16, (1.0, 0.4)
+    if name == "far_below_zero":  # and one per 0.25 around -33, as GPT-2's logits lie
+        return 2.0 * x - 33.0, torch.bfloat16, (1.0, 2.5)
+    if name == "narrow":
+        return 0.02 * x, torch.float16, (1.0, 5.0)
+    if name == "flat":  # temperatures past the spread of the scores
+        return x, torch.float32, (1.0, 6.0, 40.0)
+    if name == "narrow_below_a_peak":
+        x[:, 17] = 250.0
+        x[:, vocab - 1] = -300.0
+        return x, torch.float32, (20.0,)
+    if name == "one_score":
+        return np.full_like(x, -0.0), torch.float32, (1.0,)
+    if name == "two_scores":
+        return np.where(x > 0.3, np.float32(1.0), np.float32(1.001)), torch.float32, (1.0,)
+    if name == "neighbouring_scores":  # a few hundred scores an ulp apart, in one bucket with everything else
+        return np.nextafter(np.float32(1.0), np.float32(2.0)) + (rng.integers(0, 300, (rows, vocab)) * 2.0 ** -23).astype(np.float32), torch.float32, (1.0,)
+    raise KeyError(name)
+
+
+@pytest.mark.parametrize("vocab", [4099, 50257, 128256])
+@pytest.mark.parametrize("name", ["far_from_zero", "far_below_zero", "narrow", "flat", "narrow_below_a_peak", "one_score", "two_scores",
+                                  "neighbouring_scores"])
+def test_whole_vocabulary_rows_with_crowded_buckets(ctx, orc, name, vocab):
+    """Temperature-only sampling of rows whose histogram has buckets larger than a tile: tokens without the order of
+    ties, and kept sets in their order."""
+    say("crowded buckets", name, vocab)
+    rng = np.random.default_rng(vocab)
+    rows = 5
+    x, dtype, temperatures = crowded_rows(name, rng, rows, vocab)
+    xd = torch.from_numpy(np.ascontiguousarray(x)).cuda().to(dtype)
+    xw = xd.float().cpu().numpy()
+    u = rng.random(rows)
+    u[0], u[1] = 0.0, 0.999999
+    ud = torch.from_numpy(u).cuda()
+    for t in temperatures:
+        want = orc.sample_batch(xw, 0, 1.0, t, u)
+        assert np.array_equal(ctx.sample(xd, ud, k=0, p=1.0, temperature=t).cpu().numpy(), want), t
+        tok, kc, ki, kp = [v.cpu().numpy() for v in ctx.sample(xd[:2], ud, k=0, p=1.0, temperature=t, kept_capacity=vocab)]
+        assert np.array_equal(tok, want[:2]), t
+        for r in range(2):
+            idx, probs = orc.sampled_categorical(xw[r], 0, 1.0, t)
+            n = len(idx)
+            assert kc[r] == n and np.array_equal(ki[r, :n], idx) and np.array_equal(bits(kp[r, :n]), bits(probs)), (t, r)
+
+
+@pytest.mark.parametrize("vocab,shift", [(128256, 12.0), (50257, -33.0)])
+def test_rows_far_from_zero_are_spread_over_the_gpu_too(ctx, vocab, shift):
+    """bf16 rows whose bulk lies where the type has few values cost a temperature-only step about what rows around zero
+    do (one workgroup per row took 17 to 30 times as much)."""
+    say("time of rows far from zero", vocab, shift)
+    g = torch.Generator(device="cuda").manual_seed(vocab)
+    u = torch.rand(8, generator=g, device="cuda", dtype=torch.float64)
+    best = {}
+    for mean in (0.0, shift):
+        x = (torch.randn(8, vocab, generator=g, device="cuda") * 2 + mean).to(torch.bfloat16)
+        for _ in range(6):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            for _ in range(8):
+                ctx.sample(x, u, k=0, p=1.0, temperature=1.0)
+            end.record()
+            end.synchronize()
+            best[mean] = min(best.get(mean, 1e9), start.elapsed_time(end))
+    assert best[shift] < 3 * best[0.0], best
