@@ -144,7 +144,7 @@ __global__ __launch_bounds__(1024) void argmax_row_kernel(const ArgmaxArgs a) {
 }
 
 // mask -> min-length -> repetition penalty, written back in place
-// (LaunchAddLogitsMask / ApplyMinLength / ApplyRepetitionPenalty).
+// (LaunchAddLogitsMask / ApplyMinLength / ApplyRepetitionPenalty); rows without a mask go to process_ids_kernel.
 __global__ __launch_bounds__(kBlock) void process_logits_kernel(float* logits, int64_t row_stride, int vocab, const Xform xf) {
   const int row = blockIdx.y, chunk = blockIdx.x;
   __shared__ uint32_t hist_bits[kChunk / 32];
@@ -153,7 +153,7 @@ __global__ __launch_bounds__(kBlock) void process_logits_kernel(float* logits, i
   float v[kElems];
   Loader<float>::load(lrow, vocab, chunk, v);
   if (xf.use_penalty()) build_history_bitmap(xf, row, chunk * kChunk, hist_bits);
-  xform_chunk<float>(xf, row, vocab, chunk, hist_bits, v);
+  xform_chunk<float, true>(xf, row, vocab, chunk, hist_bits, v);
 #pragma unroll
   for (int j = 0; j < Loader<float>::NV; ++j) {
     const int i0 = Loader<float>::index_of(chunk, j, 0);
@@ -226,11 +226,11 @@ extern "C" hipError_t ms_launch_argmax(const ms::ArgmaxArgs* a, int dtype, hipSt
 
 extern "C" hipError_t ms_launch_process_logits(float* logits, int64_t row_stride, int rows, int vocab,
                                                const ms::Xform* xf, hipStream_t stream) {
-  dim3 grid((vocab + ms::kChunk - 1) / ms::kChunk, rows);
   if (!xf->mask) {
     hipLaunchKernelGGL(ms::process_ids_kernel, dim3(rows), dim3(512), 0, stream, logits, row_stride, vocab, *xf);
     return hipGetLastError();
   }
+  dim3 grid((vocab + ms::kChunk - 1) / ms::kChunk, rows);
   hipLaunchKernelGGL(ms::process_logits_kernel, grid, dim3(ms::kBlock), 0, stream, logits, row_stride, vocab, *xf);
   return hipGetLastError();
 }

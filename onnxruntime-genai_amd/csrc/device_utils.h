@@ -422,12 +422,12 @@ struct Loader<uint16_t> : Loader16<uint16_t> {};
 template <>
 struct Loader<bf16_t> : Loader16<bf16_t> {};
 
-// Applies the logits processing to the registers loaded by Loader<InT>::load.
-template <typename InT>
+// Applies the logits processing to the registers loaded by Loader<InT>::load.  MASKED: the caller knows of a mask.
+template <typename InT, bool MASKED = false>
 __device__ __forceinline__ void xform_chunk(const Xform& xf, int row, int vocab, int chunk,
                                             const uint32_t* hist_bits, float (&v)[kElems]) {
   using L = Loader<InT>;
-  const bool has_mask = xf.mask != nullptr;
+  const bool has_mask = MASKED || xf.mask != nullptr;
   const bool pen = xf.use_penalty();
   const uint32_t* mrow = has_mask ? xf.mask + static_cast<size_t>(row) * ((vocab - 1) / 32 + 1) : nullptr;
   const int n_eos = xf.eos_count(row);
