@@ -9,14 +9,16 @@
  *
  * Graph capture: every entry point only launches kernels on `stream`, with workspace from the context, and can be
  * captured into a HIP graph -- except the synchronous ones (create / destroy, *_is_done, *_hypothesis,
- * *_fallback_rows, *_wait_gave_up, beam_scorer_set_prompt) and the two that advance a scorer's host-side state (mi355x_beam_scorer_step, mi355x_beam_search_step: the sequence length and the buffer the
- * sequences live in are part of the launch, so a replay would repeat one step; they return
- * MI355X_E_UNSUPPORTED on a capturing stream).  The three calls that take a table from a caller's HOST array
+ * *_fallback_rows, *_wait_gave_up, *_sum_waits_gave_up, beam_scorer_set_prompt) and the two that advance a scorer's
+ * host-side state (mi355x_beam_scorer_step, mi355x_beam_search_step: the sequence length and the buffer the
+ * sequences live in are part of the launch, so a replay would repeat one step).  These two and
+ * beam_scorer_set_prompt return MI355X_E_UNSUPPORTED on a capturing stream.  The three calls that take a table from a caller's HOST array
  * (mi355x_sample* with per-row parameters for more than 64 rows, mi355x_logits_handoff with token_index,
  * mi355x_kv_gather) read it when they are called -- the first copies it into pinned memory of the context and records
  * a copy from there, the others carry it inside the kernel arguments -- so the caller's array is not read again at a
- * replay; every captured call of the first kind takes one of the context's 56 permanent staging slots (MI355X_E_UNSUPPORTED once
- * they are used up).
+ * replay.  Every captured call of these three counts against the 56 that a context provides for, and one beyond them is
+ * refused with MI355X_E_UNSUPPORTED.  (The first kind needs a permanent staging slot each; the others need none any
+ * more, and are counted because callers may rely on the bound.)
  *
  * Versions: MI355X_ABI_VERSION names the layout of the structures below and the set of entry points;
  * mi355x_search_abi_version() returns the value the loaded library was built with, so a caller built
@@ -368,7 +370,10 @@ int mi355x_logits_handoff(mi355x_search_ctx* ctx, void* stream, const void* raw,
                           int64_t out_stride);
 
 /* Diagnostics: number of rows, since the context was created, that the single-pass fast paths
- * declined and the exact general path finished (synchronises `stream`). */
+ * declined and the exact general path finished (synchronises `stream`).  Rows that sample from the whole vocabulary
+ * (k <= 1, p >= 1) count, whether they are spread over the GPU (tens of microseconds a step) or finished by one
+ * workgroup each (from 4096 logits on only those whose maximum is not finite, or that are processed on the way in:
+ * half a millisecond and up). */
 int mi355x_search_fallback_rows(mi355x_search_ctx* ctx, void* stream, unsigned* rows);
 
 /* Failure handling of the top-k path (no counterpart in the reference).  The workgroup that finishes

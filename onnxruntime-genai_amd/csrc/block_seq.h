@@ -725,7 +725,8 @@ struct RowOutputs {
 // no certain stop among the n, NaNs): -1, and the caller does the exact sums.
 // keep > 0: the stop is known (the exact sums have been done), keep elements are kept; only the draw is decided.
 // (A row of 1700 keys spends 4.9 us in the exact sum and 2.1 in the draw behind it, one of 9400 keys 10 and 4.  Steps of
-// 32 x 151936 bf16, p = 0.9: 44.6 -> 40.2 us.)
+// 32 x 151936 bf16, p = 0.9: 44.6 -> 40.2 us.  Counted over batches of the sizes and parameters that decoding meets, 0 to
+// 1.4 % of the rows that try it are turned down, 6 of 3072 at 32 x 151936.)
 template <int ITEMS, typename Exps>
 __device__ __forceinline__ int block_nucleus_token(int n, Exps exps, int V, float p, double u, SeqShared& sh, int keep) {
   const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6, nw = static_cast<int>(blockDim.x) >> 6;

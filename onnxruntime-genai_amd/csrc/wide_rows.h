@@ -5,10 +5,10 @@
 // The reference sorts such a row, adds the exponentials of all of it one after the other and draws from the result.
 // One workgroup per row (exact_rows_kernel) spends 0.55 ms on that however few rows there are: its sort moves every
 // key three times at the memory rate of a single CU, and its sums run over 128 K exponentials in one workgroup.  Here
-// every step but the last is spread over the GPU, in five launches (16 x 128256 fp16: 557 -> 59 us per step:
-// 4.7 + 4.7 + 12 + 21 + 21 us by a trace; every one of them is a chain of dependent phases of a few barriers each, no
-// launch moves more than 33 MB):
-//   1. wide_max:     the maximum of every 16384-logit chunk.
+// every step but the last is spread over the GPU, in five launches (16 x 128256 fp16: 557 -> 59 us per
+// step on the same rows again and 66 on rows that come from memory: 4.7 + 4.7 + 11.5 + 21.6 + 20 us by a trace; every
+// one of them is a chain of dependent phases of a few barriers each, no launch moves more than 33 MB):
+//   1. wide_max:     the maximum of every chunk of kWideChunk logits.
 //   2. wide_count:   a histogram per chunk over kWideBuckets buckets, linear in the score below the row's maximum down
 //                    to the depth past which no element can lie inside the kept set.
 //   3. wide_scatter: every workgroup scans the row's histograms, gives its chunk's keys their places, bucket by
@@ -63,7 +63,7 @@ __device__ __forceinline__ WideShare wide_share(int per_row) {
   return WideShare{xcd + 8 * (slot / per_row), slot % per_row};
 }
 
-// The 16 logits of thread t in a chunk, in loads of 16 bytes; ids past the vocabulary are NaN.
+// The kWidePer logits of thread t in a chunk, in loads of 16 bytes; ids past the vocabulary are NaN.
 template <typename InT>
 __device__ __forceinline__ void wide_load(const InT* row, int V, int chunk, float (&v)[kWidePer]) {
   constexpr int VEC = 16 / static_cast<int>(sizeof(InT));
@@ -155,8 +155,8 @@ __global__ __launch_bounds__(kWideBlock) void wide_count_kernel(const SampleArgs
     if (b < static_cast<uint32_t>(kWideBuckets)) atomicAdd(&hist[b], 1u);
   }
   __syncthreads();
-  // two buckets a thread, packed: a chunk holds at most 16384 keys
-  static_assert(kWideBuckets == 2 * kWideBlock, "a pair of buckets per thread");
+  // two buckets a thread, packed: a chunk holds at most kWideChunk keys
+  static_assert(kWideBuckets == 2 * kWideBlock && kWideChunk < 1 << 16, "a pair of buckets per thread, of 16 bits each");
   uint32_t* out = reinterpret_cast<uint32_t*>(a.big + static_cast<size_t>(row) * a.big_stride) + static_cast<size_t>(chunk) * kWideBlock;
   out[tid] = hist[2 * tid] | (hist[2 * tid + 1] << 16);
 }

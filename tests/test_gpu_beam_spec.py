@@ -612,7 +612,7 @@ def test_logits_handoff_slices_and_widens(ctx, orc, dtype, kind):
 
 def test_each_of_many_scorers_tells_its_own_end():
     """A scorer's end is told through a word of its context's; the scorers past the 64th have none and read the count
-    back, words of closed scorers are used again, and a scorer may outlive its context."""
+    back, words of closed scorers are used again, and a scorer may be closed after its context."""
     ctx = pkg().SearchContext(2, 100)
     dev = torch.device("cuda")
     scores = torch.tensor([-0.1, -0.2, -0.3, -0.4], device=dev)

@@ -1419,8 +1419,8 @@ def test_draw_in_order_follows_one_engine(ctx, orc, rows, cap):
 def test_whole_vocabulary_rows_spread_over_the_gpu(ctx, orc, vocab, dtype):
     """Temperature-only sampling (k = 0, p >= 1): token-only calls, whose ties stay unordered until the draw, on rows
     that end on and beside the edges of chunks and tiles; kept sets of a few entries; a batch of scattered rows of
-    which only some sample from the whole vocabulary; rows the spread path declines (one score for all, a maximum of
-    -1e38, a bucket too full) among the others."""
+    which only some sample from the whole vocabulary; rows the spread path declines (a maximum of -1e38 or infinity)
+    and rows whose buckets it cuts (one score for all, runs of ties) among the others."""
     say("whole vocabulary", vocab, dtype)
     rng = np.random.default_rng(vocab)
     rows = 11
