@@ -372,8 +372,8 @@ int mi355x_logits_handoff(mi355x_search_ctx* ctx, void* stream, const void* raw,
 /* Diagnostics: number of rows, since the context was created, that the single-pass fast paths
  * declined and the exact general path finished (synchronises `stream`).  Rows that sample from the whole vocabulary
  * (k <= 1, p >= 1) count, whether they are spread over the GPU (tens of microseconds a step) or finished by one
- * workgroup each (from 4096 logits on only those whose maximum is not finite, or that are processed on the way in:
- * half a millisecond and up). */
+ * workgroup each, half a millisecond and up (from 4096 logits on only those whose maximum is not finite, that are
+ * processed on the way in, or that have more than 32768 scores within about 0.015 temperatures). */
 int mi355x_search_fallback_rows(mi355x_search_ctx* ctx, void* stream, unsigned* rows);
 
 /* Failure handling of the top-k path (no counterpart in the reference).  The workgroup that finishes

@@ -86,9 +86,12 @@ constexpr int kWideTile = 3072;       // keys after which a new tile begins, wit
 constexpr int kWideBucketMax = 1024;  // keys of a bucket that a tile takes whole
 constexpr int kWideMaxTiles = 192;    // tiles of the longest row (589824 logits)
 constexpr int kWideMinVocab = 4096;   // shorter rows are a single workgroup's work anyway
+constexpr uint32_t kWideDeclined = 1, kWideGivenBack = 2;
 struct WideRow {
-  uint32_t n, tiles, declined;  // listed keys, their tiles; declined: the row is not one for this path
-  float top;                    // the row's maximum
+  uint32_t n, tiles;  // listed keys, their tiles
+  uint32_t declined;  // kWideDeclined: the row is not one for this path; kWideGivenBack: a tile of it found so (other tiles
+                      // of that launch go on: one that returned would leave those behind it waiting for its sum)
+  float top;          // the row's maximum
 };
 struct WideArgs {
   int chunks, max_tiles;

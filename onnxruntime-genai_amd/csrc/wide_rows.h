@@ -26,8 +26,8 @@
 // arrival order, also across the tiles they are cut into, and the id of the drawn rank is taken from the run the draw
 // falls into.  A call that asks for the kept ids has its ties ordered by wide_rank.  A bucket of several scores too
 // large for a tile (a flat row, or one whose bulk is narrow) is cut between ranks its tiles select (wide_gather_cut).
-// A row this does not fit (a maximum that is not finite, a stop beyond the listed elements) is finished by the exact
-// path inside wide_finish.
+// A row this does not fit (a maximum that is not finite, a stop beyond the listed elements, more than kWideSelectMax keys
+// of several scores in one bucket) is finished by the exact path inside wide_finish.
 #pragma once
 #include "sample_stream.h"
 #include "seqsum_exp_step.h"
@@ -183,7 +183,7 @@ __global__ __launch_bounds__(kWideBlock) void wide_scatter_kernel(const SampleAr
   WideRow* const info = w.rows + row;
   const uint32_t rmax = wide_row_max(a, w, row);
   if (rmax == 0xffffffffu) {
-    if (chunk == 0 && tid == 0) *info = WideRow{0u, 0u, 1u, 0.0f};
+    if (chunk == 0 && tid == 0) *info = WideRow{0u, 0u, kWideDeclined, 0.0f};
     return;
   }
   float v[kWidePer];
@@ -340,17 +340,37 @@ __device__ __forceinline__ u64 wide_select_key(const u64* src, uint32_t m, uint3
 // (head / tail: the buckets its two ends lie inside, or zeros).  The keys of a cut bucket lie in the list in the order
 // of arrival.  Where they all have one score, and nobody asks for the order of ties, any share of them will do: the one
 // at the tile's own places.  Otherwise the tile takes the keys whose ranks are its places, between two keys that it
-// selects from the bucket: every tile of the bucket reads all of it.
-__device__ __forceinline__ void wide_gather_cut(const u64* list, uint32_t first, uint32_t n, uint2 head, uint2 tail, bool order_ties,
+// selects from the bucket: every tile of the bucket reads all of it, 5.5 us per 1000 keys.  False, for one tile of the
+// bucket at least, where that would be more than kWideSelectMax keys (a bulk of nearly one score far from outliers, a
+// temperature of 40 spreads, kept ids of as many ties): the row is given back.  (Largest bucket 29 K keys: 64 x 201088
+// fp32 rows of sigma 1 at T = 25 take 1014 us a step against 1154 on the exact path, 24 x 128256 at T = 40 368 against
+// 602, one 208 against 537; with all of a row in one or two buckets 24 x 128256 took 1400 to 1800 against 620 to 930.)
+constexpr uint32_t kWideSelectMax = 32768;
+__device__ __forceinline__ bool wide_gather_cut(const u64* list, uint32_t first, uint32_t n, uint2 head, uint2 tail, bool order_ties,
                                                 WideRankShared& sh) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const uint32_t end = first + n;
-  auto copy = [&](uint32_t from, uint32_t to) {
-    for (uint32_t i = from + tid; i < to; i += kWideRankBlock) sh.keys[i - first] = list[i];
-  };
-  auto share = [&](uint2 bucket, uint32_t from, uint32_t to) {  // places from .. to of the list lie in the bucket
+  uint32_t done = first;  // the tile's places up to here have their keys
+#pragma unroll 1
+  for (int side = 0; side < 2; ++side) {  // (loops, so that the passes over a bucket are compiled once)
+    const uint2 bucket = side == 0 ? head : tail;
+    if (bucket.y == 0u || (side == 1 && bucket.x < done)) continue;  // (a tile inside one bucket has its only share already)
+    const uint32_t from = side == 0 ? first : bucket.x, to = bucket.y < end ? bucket.y : end;
+    for (uint32_t i = done + tid; i < from; i += kWideRankBlock) sh.keys[i - first] = list[i];  // the buckets between the two
+    done = to;
     const u64* const src = list + bucket.x;
     const uint32_t m = bucket.y - bucket.x;
+    if (m > kWideSelectMax) {  // (all of its tiles together see whether it has one score)
+      int differs = order_ties ? 1 : 0;
+      const uint32_t score = key64_okey(src[0]);
+      for (uint32_t i = from + tid; i < to && !order_ties; i += kWideRankBlock) {
+        const u64 k = list[i];
+        sh.keys[i - first] = k;
+        differs |= key64_okey(k) != score ? 1 : 0;
+      }
+      if (__syncthreads_or(differs)) return false;
+      continue;
+    }
     u64 highest = 0, below = 0;  // (below: complement of the lowest)
 #pragma unroll 4
     for (uint32_t i = tid; i < m; i += kWideRankBlock) {
@@ -369,28 +389,26 @@ __device__ __forceinline__ void wide_gather_cut(const u64* list, uint32_t first,
     highest = row16_max<u64>(lane < kWideRankBlock / 64 ? sh.high[lane] : 0);
     const u64 lowest = ~row16_max<u64>(lane < kWideRankBlock / 64 ? sh.low[lane] : 0);
     if (!order_ties && key64_okey(lowest) == key64_okey(highest)) {
-      copy(from, to);
+      for (uint32_t i = from + tid; i < to; i += kWideRankBlock) sh.keys[i - first] = list[i];
     } else {
-      const u64 best = from > bucket.x ? wide_select_key(src, m, from - bucket.x, lowest, highest, sh) : highest;
-      const u64 last = to < bucket.y ? wide_select_key(src, m, to - 1u - bucket.x, lowest, highest, sh) : lowest;
+      u64 best = highest, last = lowest;
+#pragma unroll 1
+      for (int e = 0; e < 2; ++e) {
+        if (e == 0 ? from == bucket.x : to == bucket.y) continue;
+        const u64 key = wide_select_key(src, m, (e == 0 ? from : to - 1u) - bucket.x, lowest, highest, sh);
+        if (e == 0) best = key;
+        else last = key;
+      }
       for (uint32_t i = tid; i < m; i += kWideRankBlock) {
         const u64 k = src[i];
         if (k <= best && k >= last) sh.keys[atomicAdd(&sh.fill, 1u)] = k;
       }
     }
     __syncthreads();
-  };
-  uint32_t mid = first, mid_end = end;
-  if (head.y != 0u) {
-    mid = head.y < end ? head.y : end;
-    share(head, first, mid);
   }
-  if (tail.y != 0u && tail.x >= mid) {  // (a tile inside one bucket has its only share already)
-    mid_end = tail.x;
-    share(tail, mid_end, end);
-  }
-  if (mid < mid_end) copy(mid, mid_end);
+  for (uint32_t i = done + tid; i < end; i += kWideRankBlock) sh.keys[i - first] = list[i];
   __syncthreads();
+  return true;
 }
 
 // Sub-buckets that have to be ranked are, by comparing the keys of each, unless one holds more than this: then the tile
@@ -407,7 +425,7 @@ __global__ __launch_bounds__(kWideRankBlock) void wide_rank_kernel(const SampleA
   const mi355x_sample_params prm = row_params<INLINE>(a, row);
   if (!wide_row(prm)) return;
   const WideRow info = w.rows[row];
-  if (info.declined != 0u || static_cast<uint32_t>(t) >= info.tiles) return;
+  if (info.declined == kWideDeclined || static_cast<uint32_t>(t) >= info.tiles) return;
   const uint32_t* const tile = w.tile_start + static_cast<size_t>(row) * (w.max_tiles + 1) + t;
   const uint32_t first = tile[0], n = tile[1] - first;
   const u64* const keys = a.big2 + static_cast<size_t>(row) * a.big_stride;
@@ -426,7 +444,13 @@ __global__ __launch_bounds__(kWideRankBlock) void wide_rank_kernel(const SampleA
   if (tid >= 64 && tid < 96) sh.exp_tab[tid - 64] = em::exp2_tab(static_cast<uint32_t>(tid - 64));
   if ((head.y | tail.y) != 0u) {
     __syncthreads();  // (the gather uses the table as well)
-    wide_gather_cut(keys, first, n, head, tail, order_ties, sh);
+    if (!wide_gather_cut(keys, first, n, head, tail, order_ties, sh)) {
+      if (tid == 0) {
+        w.rows[row].declined = kWideGivenBack;
+        store_sum_bits(w.tile_sum + static_cast<size_t>(row) * w.max_tiles + t, 0ull);  // (other tiles of the row wait for one)
+      }
+      return;
+    }
 #pragma unroll
     for (int r = 0; r < kWideRankPer; ++r) {
       const uint32_t i = static_cast<uint32_t>(r * kWideRankBlock + tid);
