@@ -709,7 +709,8 @@ struct RowOutputs {
   int32_t* kept_ids;
   float* kept_probs;
   int kept_capacity;
-  int pad;  // non-zero: entries from the kept count to the capacity get id -1 and probability 0
+  int pad;   // non-zero: entries from the kept count to the capacity get id -1 and probability 0
+  int rows;  // of the call
 };
 
 // Position, in rank order, of the token a nucleus row draws, without the exact sum of its exponentials: for calls that
@@ -811,8 +812,10 @@ __device__ __forceinline__ int block_nucleus_token(int n, Exps exps, int V, floa
 // writing outputs -- when the nucleus does not end inside the n_sorted available elements.  synced: every thread
 // has passed a barrier since `sh` was last used, so the first sum need not begin with one.  id_at(i), when given: the
 // id of the i-th best element, called by the whole block for the drawn position (the id in sorted(i) otherwise).
+// NUCLEUS: the row is known to be one of k <= 1 over more than 64 logits, and the kernel keeps what is not its straight way
+// behind the rest.
 struct IdAsSorted {};
-template <int ITEMS, typename Sorted, typename Exps, typename IdAt = IdAsSorted>
+template <int ITEMS, bool NUCLEUS = false, typename Sorted, typename Exps, typename IdAt = IdAsSorted>
 __device__ __forceinline__ bool block_sample_epilogue(Sorted sorted, Exps exps, int n_sorted, int vocab,
                                       mi355x_sample_params prm, double u, const RowOutputs& out,
                                       SeqShared& sh, bool synced = false, IdAt id_at = IdAt{}) {
@@ -823,7 +826,7 @@ __device__ __forceinline__ bool block_sample_epilogue(Sorted sorted, Exps exps, 
   float sum = 1.0f;
   bool divide_by_sum = false;
   int idx_dummy;
-  if (prm.k > 1) {
+  if (!NUCLEUS && prm.k > 1) {
     const int m = prm.k < vocab ? prm.k : vocab;
     if (m > n_sorted) return false;
     sum = block_seq_sum<ITEMS>(0.0f, m, exps, NoStop{}, &idx_dummy, sh, nullptr, kEpiHead, synced);
@@ -854,9 +857,10 @@ __device__ __forceinline__ bool block_sample_epilogue(Sorted sorted, Exps exps, 
     // in that range in n^3 * 2e-8 * (1 - p) / (p V) of the rows -- one of which is enough to make the launch longer by
     // the attempt (2 us; the sum it saves takes 5).
     if constexpr (ITEMS == 8) {
-      const float len = static_cast<float>(limit), rows = static_cast<float>(gridDim.x);
-      if (token_alone && p > 0.0f && p < 1.0f && vocab > 64 && limit <= static_cast<int>(blockDim.x) * ITEMS &&
-          rows * (len * len * len) * 2e-8f * (1.0f - p) < 0.25f * p * static_cast<float>(vocab)) {
+      const float len = static_cast<float>(limit), rows = static_cast<float>(out.rows);
+      const bool attempt = token_alone && p > 0.0f && p < 1.0f && vocab > 64 && limit <= static_cast<int>(blockDim.x) * ITEMS &&
+                           rows * (len * len * len) * 2e-8f * (1.0f - p) < 0.25f * p * static_cast<float>(vocab);
+      if (NUCLEUS ? __builtin_expect(attempt, 0) != 0 : attempt) {
         if (!synced) __syncthreads();
         early_pos = block_nucleus_token<ITEMS>(limit, exps, V, p, u, sh, 0);
         synced = false;
@@ -887,7 +891,7 @@ __device__ __forceinline__ bool block_sample_epilogue(Sorted sorted, Exps exps, 
         if (cutoff >= limit) return false;
         base = cutoff;
       }
-      if (vocab <= 64) {  // exact-partition override, src/sampling_distribution.h:186-203
+      if (!NUCLEUS && vocab <= 64) {  // exact-partition override, src/sampling_distribution.h:186-203
         if (n_sorted < vocab) return false;
         const float global = block_seq_sum<ITEMS>(0.0f, vocab, exps, NoStop{}, &idx_dummy, sh, nullptr, kEpiHead);
         int sj;
@@ -926,7 +930,8 @@ __device__ __forceinline__ bool block_sample_epilogue(Sorted sorted, Exps exps, 
     // (a nucleus of more than one window of block_discrete_draw, which sums it first: 6.3 us for 9200 elements, 4.0 this way;
     // 48 rows x 50257 in several modes: 56.4 -> 53.0 us per step)
     const int span = static_cast<int>(blockDim.x) * ITEMS;
-    if (pos < 0 && prm.k <= 1 && keep > span && keep <= 2 * span && scale > 0.0f) {
+    const bool two_windows = pos < 0 && prm.k <= 1 && keep > span && keep <= 2 * span && scale > 0.0f;
+    if (NUCLEUS ? __builtin_expect(two_windows, 0) != 0 : two_windows) {
       __syncthreads();  // (the sums' readers are done)
       pos = block_nucleus_token<2 * ITEMS>(keep, exps, vocab, prm.p, u, sh, keep);
     }

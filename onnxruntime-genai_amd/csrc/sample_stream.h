@@ -66,7 +66,7 @@ __device__ __forceinline__ RowOutputs row_outputs(const SampleArgs& a, int row) 
   return RowOutputs{a.out_tokens + row, a.kept_count ? a.kept_count + row : nullptr,
                     a.kept_ids ? a.kept_ids + static_cast<size_t>(row) * a.kept_capacity : nullptr,
                     a.kept_probs ? a.kept_probs + static_cast<size_t>(row) * a.kept_capacity : nullptr,
-                    a.kept_capacity, a.kept_pad};
+                    a.kept_capacity, a.kept_pad, a.rows};
 }
 
 // A row of the logits as fp32 values, whatever it is stored as: InT float, uint16_t (fp16 bits) or bf16_t,
