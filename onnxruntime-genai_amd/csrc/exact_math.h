@@ -76,12 +76,11 @@ EM_HD uint64_t exp2_tab(uint32_t i) {
   return tab[i];
 }
 
-// expf(x), bit-identical to glibc's.  `tab(i)` must return exp2_tab(i); callers that already hold the
+// The arithmetic of expf(x), bit-identical to glibc's where no special case applies: for -103.97 <= x < 88.72.  (Further
+// down, to -600 and beyond, the result is a zero as well.)  `tab(i)` must return exp2_tab(i); callers that already hold the
 // table in registers or LDS pass their own accessor.
 template <typename Tab>
-EM_HD float expf_core(float x, Tab tab) {
-  const uint32_t ix = as_u32(x);
-  const uint32_t abstop = (ix >> 20) & 0x7ff;
+EM_HD float expf_in_range(float x, Tab tab) {
   const double N = 32.0;
   const double inv_ln2_n = 0x1.71547652b82fep+0 * N;
   const double shift = 0x1.8p+52;
@@ -106,7 +105,15 @@ EM_HD float expf_core(float x, Tab tab) {
   double y = mad(c2, r, 1.0);
   y = mad(z, r2, y);
   y = y * s;
-  float res = (float)y;
+  return (float)y;
+}
+
+// expf(x), bit-identical to glibc's.
+template <typename Tab>
+EM_HD float expf_core(float x, Tab tab) {
+  const uint32_t ix = as_u32(x);
+  const uint32_t abstop = (ix >> 20) & 0x7ff;
+  float res = expf_in_range(x, tab);
   if (abstop >= 0x42b) {  // |x| >= 88 or NaN/Inf
     if (ix == 0xff800000u) res = 0.0f;
     else if (abstop >= 0x7f8) res = x + x;

@@ -2,6 +2,7 @@
 // mi355x_sample (the streaming kernels of fp16 and bf16 rows are instantiated in sample_kernels_f16.hip and
 // sample_kernels_bf16.hip from the same templates).
 #include "sample_stream.h"
+#include "token_pick.h"
 
 extern "C" {
 hipError_t ms_launch_stream(const ms::SampleArgs* a, const ms::InlineParams* table, int which, hipStream_t stream);
@@ -883,12 +884,26 @@ __device__ __forceinline__ void nucleus_finish_body(const SampleArgs& a) {
     const int c = q >> head_shift, u = q & ((1 << head_shift) - 1);
     pre[q] = (a.chunks <= kAheadChunks && c < a.chunks) ? big_row[static_cast<size_t>(c) * kSChunk + u * kFinishBlock + tid] : 0;
   }
-  for (int b = tid; b <= kSortBuckets; b += kFinishBlock) bucket_start[b] = 0u;  // the sort's table, while the loads are on their way
   // Rows of sixteen-bit logits whose token alone is asked for keep ties as they come (see rank_and_cache_exps); the
   // run of ties the draw falls into is ordered then.  (fp32 rows have few; rows whose logits are processed on the way
   // in would need that processing there.)
   const bool free_ties = a.dtype != MI355X_F32 && a.kept_ids == nullptr && a.emit_topk == 0 && !a.xf.active();
   if (tid < kSortBuckets / 32) mixed_buckets[tid] = 0u;
+  // A nucleus row whose token alone is asked for is not sorted at all unless that leaves its token open (token_pick.h;
+  // what it works on lies where the sort's table and keys would).
+  __shared__ uint64_t exp_tab[32];
+  PickShared& pick_sh = *reinterpret_cast<PickShared*>(bucket_start);
+  static_assert(sizeof(PickShared) <= kSortBuckets * sizeof(uint32_t) && kPickBlock == kFinishBlock && kPickRoom <= kNucleusCap, "the pick fits the sort's room");
+  const bool try_pick = kMayBeNucleus && !large_k && a.kept_ids == nullptr && a.kept_count == nullptr && prm.p > 0.0f && prm.p < 1.0f && V > 64;
+  auto clear_buckets = [&]() __attribute__((always_inline)) {
+    for (int b = tid; b <= kSortBuckets; b += kFinishBlock) bucket_start[b] = 0u;
+  };
+  if (try_pick) {  // (while the loads are on their way)
+    TokenPick::clear(pick_sh);
+    if (tid < 32) exp_tab[tid] = em::exp2_tab(static_cast<uint32_t>(tid));
+  } else {
+    clear_buckets();
+  }
   // Lane c of every wave reads what chunk c left behind (at most 16 chunks), so the row's maximum and threshold
   // are reductions inside the wave, with no exchange between the waves; wave 0 publishes the counts and where
   // every list's rows begin, behind the one barrier that follows.
@@ -1009,6 +1024,95 @@ __device__ __forceinline__ void nucleus_finish_body(const SampleArgs& a) {
     }
     flat_batches(fn);
   };
+  if (try_pick) {
+    if (sh_all != 0u && TokenPick::worth_it(a.rows, sh_all) && rmax < order_key(1e30f) && thr > order_key(-1e30f)) {
+      TokenPick pick(pick_sh, lds_keys, exp_tab, rmax, thr, prm, V, a.uniforms[row], sh_all);
+      const float thr_score = key_to_float(thr);
+      float below = best_below != 0 ? key_to_float(key64_okey(best_below)) : -__builtin_inff();
+      auto score_of = [](u64 raw) { return __uint_as_float(static_cast<uint32_t>(raw >> 32)); };
+      // Half of what the heads hold lies below the row's threshold (a chunk knows its own only): every wave moves its
+      // candidates together first, so that the two looks at them take that many fewer instructions.
+      constexpr int kWaveKeys = kHeadSlots * 64;
+      u64* const mine = lds_keys + (tid >> 6) * kWaveKeys;
+      int n_mine = 0;
+#pragma unroll
+      for (int q = 0; q < kHeadSlots; ++q) {
+        const int c = q >> head_shift;
+        const uint32_t first = static_cast<uint32_t>(q & ((1 << head_shift) - 1)) * kFinishBlock;
+        const uint32_t listed = head != 0u && c < a.chunks ? wave_read_lane(cnt, c) : 0u;
+        if (first < listed) {
+          const float score = first + tid < listed ? score_of(pre[q]) : -__builtin_inff();
+          const u64 hits = __ballot(score >= thr_score);  // (false for NaN)
+          if (score >= thr_score) mine[__builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(hits >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(hits), n_mine))] = pre[q];
+          below = fmaxf(below, score >= thr_score ? below : score);
+          n_mine += static_cast<int>(__popcll(hits));
+        }
+      }
+      constexpr int kAtOnce = 4;  // exponentials side by side
+      float e[kHeadSlots];
+#pragma unroll
+      for (int q0 = 0; q0 < kHeadSlots; q0 += kAtOnce) {
+        if (q0 * 64 < n_mine) {
+#pragma unroll
+          for (int q = q0; q < q0 + kAtOnce; ++q) pre[q] = mine[q * 64 + lane];
+#pragma unroll
+          for (int q = q0; q < q0 + kAtOnce; ++q) e[q] = pick.exp_of(score_of(pre[q]));
+#pragma unroll
+          for (int q = q0; q < q0 + kAtOnce; ++q)
+            if (q * 64 + lane < n_mine) pick.count(score_of(pre[q]), e[q]);
+        }
+      }
+      flat_batches([&](const u64 (&raw)[kGather], const bool (&valid)[kGather], uint32_t) {
+#pragma unroll
+        for (int u = 0; u < kGather; ++u) {
+          const float score = valid[u] ? score_of(raw[u]) : -__builtin_inff();
+          if (score >= thr_score) pick.count(score, pick.exp_of(score));
+          else below = fmaxf(below, score);
+        }
+      });
+      if (pick.find(below)) {
+#pragma unroll
+        for (int q0 = 0; q0 < kHeadSlots; q0 += kAtOnce) {
+          if (q0 * 64 < n_mine) {
+            bool have[kAtOnce];
+            u64 raw[kAtOnce];
+            float ex[kAtOnce];
+#pragma unroll
+            for (int i = 0; i < kAtOnce; ++i) {
+              have[i] = (q0 + i) * 64 + lane < n_mine;
+              raw[i] = pre[q0 + i];
+              ex[i] = e[q0 + i];
+            }
+            pick.gather(have, raw, ex);
+          }
+        }
+        flat_batches([&](const u64 (&raw)[kGather], const bool (&valid)[kGather], uint32_t) {
+          bool have[kGather];
+          float ex[kGather];
+#pragma unroll
+          for (int u = 0; u < kGather; ++u) {
+            have[u] = valid[u] && score_of(raw[u]) >= thr_score;
+            ex[u] = pick.exp_of(score_of(raw[u]));
+          }
+          pick.gather(have, raw, ex);
+        });
+        const uint32_t id = pick.resolve();
+        if (id != kNoPick) {
+          if (tid == 0) *row_outputs(a, row).token = static_cast<int32_t>(id);
+          return;
+        }
+      }
+      __syncthreads();
+      // (the heads, moved together above, are read again)
+#pragma unroll
+      for (int q = 0; q < kHeadSlots; ++q) {
+        const int c = q >> head_shift, u = q & ((1 << head_shift) - 1);
+        pre[q] = (a.chunks <= kAheadChunks && c < a.chunks) ? big_row[static_cast<size_t>(c) * kSChunk + u * kFinishBlock + tid] : 0;
+      }
+    }
+    clear_buckets();
+    __syncthreads();
+  }
   // A nucleus row's usual way: a counting sort over the lists where they lie.  A first pass over them counts the
   // candidates (at or above the row's threshold) into the sort's buckets; the histogram tells how many buckets the
   // nucleus can reach at all (and how many fit the sort); a second pass gives every key of those buckets a place in
@@ -1374,6 +1478,10 @@ __device__ __forceinline__ bool sparse_slot_used(int u, uint32_t n_gathered, uin
   return u < kSparseIds ? static_cast<uint32_t>(u * kFinishBlock) < n_gathered
                         : static_cast<uint32_t>((u - kSparseIds) * kFinishBlock) < n_extra;
 }
+// Lists of the token alone are picked from (token_pick.h) beyond this, and where the network would have to sort them: in
+// between the counting sort and the exact sums take less (64 x 128256 with 2 % allowed: 20.6 us a step sorted, 22.4 picked;
+// 128 x 32064 with 6 %: 18.0 and 20.2; 256 x 201088 with 5 %, 10000 ids: 59.2 and 50.1).
+constexpr uint32_t kSparsePickMin = 4608;
 constexpr uint32_t kSparseDirectMin = 2 * kFinishBlock;  // shorter lists take the general tail (a sorting network)
 
 // The bucket sort of a row whose elements the block's threads hold in registers (ids[u] with the order key ok[u] of
@@ -1435,7 +1543,8 @@ __device__ __forceinline__ uint32_t sort_counted(u64* keys, uint32_t* start, con
 }
 
 // Returns 1 when the row is finished, 0 when it is not, -1 when it is not a nucleus row.
-template <bool INLINE>
+// PICK: the token alone is asked for.
+template <bool INLINE, bool PICK>
 __device__ __forceinline__ int nucleus_sparse_body(const SampleArgs& a) {
   extern __shared__ u64 lds_keys[];
   uint32_t* const bucket_start = reinterpret_cast<uint32_t*>(lds_keys + kNucleusCap);
@@ -1449,7 +1558,9 @@ __device__ __forceinline__ int nucleus_sparse_body(const SampleArgs& a) {
   __shared__ uint32_t red32[16], red32_rest[16];  // (two: the reductions below follow each other without a barrier between)
   __shared__ u64 red64[16];
   __shared__ uint32_t sh_extra, sh_count;
+  __shared__ uint64_t exp_tab[32];
   const int row = blockIdx.x, tid = threadIdx.x, lane = lane_id(), wave = tid >> 6;
+  if (PICK && tid < 32) exp_tab[tid] = em::exp2_tab(static_cast<uint32_t>(tid));  // (barriers follow before it is used)
   const int V = a.vocab;
   const mi355x_sample_params prm = row_params<INLINE>(a, row);
   if (row_mode(prm, V, a.chunks) != kModeNucleus) return -1;
@@ -1616,14 +1727,87 @@ __device__ __forceinline__ int nucleus_sparse_body(const SampleArgs& a) {
   for (int u = 0; u < kSparseExtraRegs; ++u) {
     const uint32_t i = static_cast<uint32_t>(tid + u * kFinishBlock);
     ids[kSparseIds + u] = i < n_extra ? extra_idx[i] : 0xffffffffu;
-    ok[kSparseIds + u] = i < n_extra ? order_key(extra_val[i]) : 0u;
+    ok[kSparseIds + u] = i < n_extra ? __float_as_uint(extra_val[i]) : 0u;
   }
   first_masked = ~block_max<uint32_t>(~first_masked, red32);  // (its barriers: every thread has read its extras)
   const bool direct = n_allowed + n_extra > kSparseDirectMin;
-  if (direct)
+  const bool try_pick = PICK && prm.p > 0.0f && prm.p < 1.0f &&
+                        (!direct || n_allowed + n_extra > kSparsePickMin) && TokenPick::worth_it(a.rows, n_allowed + n_extra);
+  PickShared& pick_sh = *reinterpret_cast<PickShared*>(bucket_start);  // (as in the finish kernel)
+  if (try_pick) TokenPick::clear(pick_sh);
+  else if (direct)
     for (int b = tid; b <= kSortBuckets; b += kFinishBlock) bucket_start[b] = 0u;  // while the gather is in flight
   asm volatile("" ::: "memory");
   gather_slots(std::integral_constant<int, kFirstLoads>{}, std::integral_constant<int, kSparseIds>{});
+  bool widened = false;  // ok[] holds the gathered logits as fp32 bits
+  if (try_pick) {
+    // The token alone is asked for: it is picked, not sorted for (token_pick.h).  (Every exponential needs the row's
+    // maximum, so nothing is counted before the last load is there.)
+    float best = -__builtin_inff();
+#pragma unroll
+    for (int u = 0; u < kSparseRegs; ++u) {
+      if (sparse_slot_used(u, n_allowed, n_extra)) {
+        if (u < kSparseIds) ok[u] = __float_as_uint(logit_of_bits(ok[u], a.dtype));
+        best = fmaxf(best, ids[u] != 0xffffffffu ? __uint_as_float(ok[u]) : -__builtin_inff());
+      }
+    }
+    widened = true;
+    const uint32_t rmax = block_max<uint32_t>(order_key(best), red32, false);
+    const uint32_t thr = order_key(key_to_float(rmax) - nucleus_depth(prm, V));
+    if (thr > order_key(-1e30f) && rmax < order_key(1e30f)) {
+      TokenPick pick(pick_sh, lds_keys, exp_tab, rmax, thr, prm, V, a.uniforms[row], n_allowed + n_extra);
+      const float thr_score = key_to_float(thr);
+      constexpr int kAtOnce = 6;
+      static_assert(kSparseRegs % kAtOnce == 0, "whole groups");
+      float below = -__builtin_inff(), e[kSparseRegs];
+      auto score_of = [&](int u) { return ids[u] != 0xffffffffu ? __uint_as_float(ok[u]) : -__builtin_inff(); };
+      auto group_used = [&](int u0) {  // (some slot of the group holds elements)
+        return sparse_slot_used(u0, n_allowed, n_extra) || (u0 + kAtOnce > kSparseIds && n_extra != 0u);
+      };
+#pragma unroll
+      for (int u0 = 0; u0 < kSparseRegs; u0 += kAtOnce) {
+        if (group_used(u0)) {
+#pragma unroll
+          for (int u = u0; u < u0 + kAtOnce; ++u) e[u] = pick.exp_of(__uint_as_float(ok[u]));
+#pragma unroll
+          for (int u = u0; u < u0 + kAtOnce; ++u) {
+            if (sparse_slot_used(u, n_allowed, n_extra)) {
+              const float score = score_of(u);
+              if (score >= thr_score) pick.count(score, e[u]);
+              else below = fmaxf(below, score);
+            }
+          }
+        }
+      }
+      if (pick.find(below, first_masked != 0xffffffffu)) {
+#pragma unroll
+        for (int u0 = 0; u0 < kSparseRegs; u0 += kAtOnce) {
+          if (group_used(u0)) {
+            bool have[kAtOnce];
+            u64 raw[kAtOnce];
+            float ex[kAtOnce];
+#pragma unroll
+            for (int i = 0; i < kAtOnce; ++i) {
+              const int u = u0 + i;
+              have[i] = sparse_slot_used(u, n_allowed, n_extra) && score_of(u) >= thr_score;
+              raw[i] = (static_cast<u64>(ok[u]) << 32) | static_cast<uint32_t>(~ids[u]);
+              ex[i] = e[u];
+            }
+            pick.gather(have, raw, ex);
+          }
+        }
+        const uint32_t id = pick.resolve();
+        if (id != kNoPick) {
+          if (tid == 0) *row_outputs(a, row).token = static_cast<int32_t>(id);
+          return leave(true);
+        }
+      }
+    }
+    __syncthreads();
+    if (direct)
+      for (int b = tid; b <= kSortBuckets; b += kFinishBlock) bucket_start[b] = 0u;
+    __syncthreads();
+  }
   // The slots of the first loads and the processed history ids are there before the rest: their maximum stands in
   // for the row's where only a reference point is needed (the threshold below it, the buckets of the sort), so that
   // they are counted into their buckets while the other loads are still on their way.
@@ -1634,7 +1818,7 @@ __device__ __forceinline__ int nucleus_sparse_body(const SampleArgs& a) {
       const uint32_t bits = ok[u];
       ok[u] = 0u;
       if (sparse_slot_used(u, n_allowed, n_extra)) {
-        ok[u] = ids[u] != 0xffffffffu ? order_key(logit_of_bits(bits, a.dtype)) : 0u;
+        ok[u] = ids[u] != 0xffffffffu ? order_key(widened ? __uint_as_float(bits) : logit_of_bits(bits, a.dtype)) : 0u;
         kmax = ok[u] > kmax ? ok[u] : kmax;
       }
     }
@@ -1642,7 +1826,10 @@ __device__ __forceinline__ int nucleus_sparse_body(const SampleArgs& a) {
   };
   uint32_t kmax = keys_of_slots(std::integral_constant<int, 0>{}, std::integral_constant<int, kFirstLoads>{});
 #pragma unroll
-  for (int u = kSparseIds; u < kSparseRegs; ++u) kmax = ok[u] > kmax ? ok[u] : kmax;
+  for (int u = kSparseIds; u < kSparseRegs; ++u) {
+    ok[u] = ids[u] != 0xffffffffu ? order_key(__uint_as_float(ok[u])) : 0u;
+    kmax = ok[u] > kmax ? ok[u] : kmax;
+  }
   const uint32_t rtop = block_max<uint32_t>(kmax, red32, false);  // (red32 is next written behind a later barrier)
   if (rtop == 0u) return leave(false);
   const uint32_t thr = order_key(key_to_float(rtop) - nucleus_depth(prm, V));
@@ -1747,9 +1934,9 @@ __device__ __forceinline__ int nucleus_sparse_body(const SampleArgs& a) {
                                  row_outputs(a, row), seqsh, red32, EmitTopk{}, presorted, presorted ? 0 : second_below));
 }
 
-template <bool INLINE>
+template <bool INLINE, bool PICK>
 __device__ __forceinline__ void nucleus_sparse_entry(const SampleArgs& a) {
-  int done = nucleus_sparse_body<INLINE>(a);
+  int done = nucleus_sparse_body<INLINE, PICK>(a);
   if (done < 0) return;
   const int row = blockIdx.x;
   if (done == 0 && a.sparse_only) {  // no dense kernels follow: the exact path, here
@@ -1767,9 +1954,11 @@ __device__ __forceinline__ void nucleus_sparse_entry(const SampleArgs& a) {
   if (threadIdx.x == 0) a.row_done[row] = static_cast<uint32_t>(done);
 }
 
-__global__ __launch_bounds__(kFinishBlock) void nucleus_sparse_kernel(const SampleArgs a) { nucleus_sparse_entry<false>(a); }
+template <bool PICK>
+__global__ __launch_bounds__(kFinishBlock) void nucleus_sparse_kernel(const SampleArgs a) { nucleus_sparse_entry<false, PICK>(a); }
+template <bool PICK>
 __global__ __launch_bounds__(kFinishBlock) void nucleus_sparse_rows_kernel(const SampleArgs a, const InlineParams) {
-  nucleus_sparse_entry<true>(a);
+  nucleus_sparse_entry<true, PICK>(a);
 }
 
 // Rows whose parameters alone put them on the exact path (k above kLargeKMax, more chunks than a finishing
@@ -1814,8 +2003,14 @@ extern "C" hipError_t ms_launch_sample(const ms::SampleArgs* a, const ms::Inline
   hipError_t e = hipSuccess;
   const bool sparse = any_nucleus && a->xf.mask && a->row_done;
   if (sparse) {  // nucleus rows under a sparse grammar mask are finished here; the kernels after it skip them
-    if (table) hipLaunchKernelGGL(ms::nucleus_sparse_rows_kernel, fgrid, fblock, ms::kFinishLds, stream, *a, *table);
-    else hipLaunchKernelGGL(ms::nucleus_sparse_kernel, fgrid, fblock, ms::kFinishLds, stream, *a);
+    // (Picking is code of its own: where no row's list is of a length it takes, jumping over it costs 2 % of the step.)
+    const int listed = a->sparse_only;
+    const bool pick = a->kept_ids == nullptr && a->kept_count == nullptr &&
+                      (listed <= static_cast<int>(ms::kSparseDirectMin) || listed > static_cast<int>(ms::kSparsePickMin));
+    auto* plain_rows = pick ? ms::nucleus_sparse_rows_kernel<true> : ms::nucleus_sparse_rows_kernel<false>;
+    auto* plain = pick ? ms::nucleus_sparse_kernel<true> : ms::nucleus_sparse_kernel<false>;
+    if (table) hipLaunchKernelGGL(plain_rows, fgrid, fblock, ms::kFinishLds, stream, *a, *table);
+    else hipLaunchKernelGGL(plain, fgrid, fblock, ms::kFinishLds, stream, *a);
     e = hipGetLastError();
     if (a->sparse_only) any_nucleus = false;  // (and no kernel after it has any to do)
   }
@@ -1852,8 +2047,10 @@ extern "C" hipError_t ms_sample_init() {
                           reinterpret_cast<const void*>(ms::largek_finish_rows_kernel),
                           reinterpret_cast<const void*>(ms::mixed_finish_kernel),
                           reinterpret_cast<const void*>(ms::mixed_finish_rows_kernel),
-                          reinterpret_cast<const void*>(ms::nucleus_sparse_kernel),
-                          reinterpret_cast<const void*>(ms::nucleus_sparse_rows_kernel),
+                          reinterpret_cast<const void*>(ms::nucleus_sparse_kernel<false>),
+                          reinterpret_cast<const void*>(ms::nucleus_sparse_kernel<true>),
+                          reinterpret_cast<const void*>(ms::nucleus_sparse_rows_kernel<false>),
+                          reinterpret_cast<const void*>(ms::nucleus_sparse_rows_kernel<true>),
                           reinterpret_cast<const void*>(ms::exact_rows_kernel),
                           reinterpret_cast<const void*>(ms::exact_rows_rows_kernel),
                           reinterpret_cast<const void*>(ms::wide_finish_kernel<false>),

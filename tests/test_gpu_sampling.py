@@ -322,6 +322,48 @@ def test_token_only_nucleus_rows_on_the_edges_of_their_guard_bands(ctx, orc, voc
                 assert np.array_equal(tokens_only(ctx, x, u, 0, float(mass), 1.0), want), (count, mass)
 
 
+@pytest.mark.parametrize("kind,vocab,p,t", [
+    ("flat", 128256, 0.9, 1.0), ("flat", 40000, 0.97, 1.5), ("ties", 128256, 0.9, 1.0), ("ties", 50257, 0.6, 0.7), ("crowd", 128256, 0.5, 1.0),
+    ("peaks", 151936, 0.9, 1.0), ("peaks", 4099, 0.95, 0.5), ("deep", 32064, 0.9995, 1.0), ("one", 151936, 0.3, 1.0), ("penalty", 50257, 0.9, 1.0),
+])
+def test_token_only_nucleus_rows_that_are_picked_instead_of_sorted(ctx, orc, kind, vocab, p, t):
+    """Token-only nucleus rows whose token is picked from two buckets of a histogram: more candidates than a thread keeps in
+    registers, ties by the dozen and by the ten thousand in the buckets of the stop and of the draw, nuclei that end with the
+    first element below the candidates or after one element, exponentials down to nothing, processed logits."""
+    say("picked", kind, vocab, p, t)
+    rng = np.random.default_rng(vocab + int(100 * p))
+    rows = 12
+    x = rng.standard_normal((rows, vocab)).astype(np.float32)
+    dtype, xf = torch.float32, {}
+    if kind == "flat":
+        x *= np.linspace(0.5, 2.5, rows, dtype=np.float32)[:, None]
+    elif kind == "ties":
+        x, dtype = 2.0 * x + 12.0, torch.bfloat16
+    elif kind == "crowd":
+        x = np.round(x)
+    elif kind == "peaks":
+        x[:, :20] += np.linspace(6.0, 30.0, rows, dtype=np.float32)[:, None]
+    elif kind == "deep":
+        x *= 6.0
+    elif kind == "one":
+        x[:, 77] += 40.0
+    else:
+        x *= 3.0
+        xf = dict(history=rng.integers(0, vocab, (rows, 200)).astype(np.int32), penalty=1.2)
+    xd = torch.from_numpy(np.ascontiguousarray(x, np.float32)).cuda().to(dtype)
+    xw = xd.float().cpu().numpy()
+    form = pkg().LogitsXform(history=torch.from_numpy(xf["history"]).cuda(), repetition_penalty=xf["penalty"]) if xf else None
+    if xf:
+        y = xd.clone()
+        ctx.process_logits(y, form)
+        xw = y.cpu().numpy()
+    for rep in range(3):
+        u = rng.random(rows)
+        u[0], u[1] = 0.0, np.nextafter(1.0, 0.0)
+        got = ctx.sample(xd, torch.from_numpy(u).cuda(), k=0, p=p, temperature=t, xf=form).cpu().numpy()
+        assert np.array_equal(got, orc.sample_batch(xw, 0, p, t, u)), rep
+
+
 def test_results_written_straight_to_pinned_host_memory(ctx, orc):
     """The output pointers may name pinned host memory that the device can address (the reference mirrors its
     results through pinned memory, src/cuda/interface.cpp:51-60): the kernels store the tokens there themselves, no
