@@ -491,7 +491,7 @@ int SampleImpl(mi355x_search_ctx* ctx, hipStream_t s, const void* logits, const 
   a.row_done = ctx->row_done;
   a.exact_kernel = (any_exact ? ms::kExactRows : 0) | (any_wide ? ms::kWideRows : 0);
   const ms::WideArgs wide{(vocab + ms::kWideChunk - 1) / ms::kWideChunk, tiles, ctx->wide_rows, ctx->wide_tile_start, ctx->wide_cut_bucket, ctx->seg_sum,
-                          ctx->seg_step, ctx->sub_step, ctx->sub_se, ctx->chunk_next};
+                          ctx->seg_step, ctx->sub_step, ctx->sub_se, ctx->chunk_next, kept_ids == nullptr && kept_count == nullptr};
   // a caller that bounds the number of allowed ids per row lets the sparse-mask kernel work alone
   if (xf && xf->mask && xf->mask_allowed_max > 0) {
     const int hist = a.xf.history_lens ? a.xf.history_stride : a.xf.history_len;

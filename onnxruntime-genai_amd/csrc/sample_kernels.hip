@@ -2055,6 +2055,12 @@ extern "C" hipError_t ms_sample_init() {
                           reinterpret_cast<const void*>(ms::exact_rows_rows_kernel),
                           reinterpret_cast<const void*>(ms::wide_finish_kernel<false>),
                           reinterpret_cast<const void*>(ms::wide_finish_kernel<true>),
+                          reinterpret_cast<const void*>(ms::wide_pick_kernel<float, false>),
+                          reinterpret_cast<const void*>(ms::wide_pick_kernel<float, true>),
+                          reinterpret_cast<const void*>(ms::wide_pick_kernel<uint16_t, false>),
+                          reinterpret_cast<const void*>(ms::wide_pick_kernel<uint16_t, true>),
+                          reinterpret_cast<const void*>(ms::wide_pick_kernel<ms::bf16_t, false>),
+                          reinterpret_cast<const void*>(ms::wide_pick_kernel<ms::bf16_t, true>),
                           reinterpret_cast<const void*>(ms::wide_scatter_kernel<float, false>),
                           reinterpret_cast<const void*>(ms::wide_scatter_kernel<float, true>),
                           reinterpret_cast<const void*>(ms::wide_scatter_kernel<uint16_t, false>),

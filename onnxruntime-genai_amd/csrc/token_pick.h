@@ -92,7 +92,8 @@ struct TokenPick {
   const mi355x_sample_params prm;
   const int V;
   const double u;
-  const float top, scale;  // bucket = (top - score) * scale, within 0 .. kPickBuckets - 1
+  const float top;
+  float scale;  // bucket = (top - score) * scale, within 0 .. kPickBuckets - 1
   const float inv_temp;
   const int shift;  // of the counts in a word; the mass below them has `frac` fractional bits
   const int frac;
@@ -105,6 +106,7 @@ struct TokenPick {
   float e_end, e_end_low;  // its exponential at most and at least
   bool ends_in_zero = false;  // it is the first one of no weight
   float sub_from[2], sub_scale[2];
+  double base = 0.0;  // mass in front of what the words count
   // the thread's share
   float rounding = 0.0f, slack = 0.0f;
   int n_hits = 0;  // the wave's
@@ -162,7 +164,7 @@ struct TokenPick {
     return (1.0 - static_cast<double>(prm.p)) * (eps + quant) + 6.03e-8 * static_cast<double>(prm.p) * (2.0 * s + 3.0 * t);
   }
   __device__ __forceinline__ double draw_guard(double kept, double n) const {
-    return kept * (u * (1.0 - u) * 1.21e-7 + 16.0 * 1.2e-16 * n + 1e-12) + 2.0 * quant;
+    return kept * (u * (1.0 - u) * 1.21e-7 + 16.0 * 1.2e-16 * n + 1e-11) + 2.0 * quant;
   }
   // Half the unit of a running sum of c elements near s.
   __device__ __forceinline__ float half_unit(double s, int c) const {
@@ -431,12 +433,12 @@ struct TokenPick {
     const int lo = sh.stop_lo, hi = sh.stop_hi;
     if (hi == kIntMax) return;
     // A stop on the last element of one of the reference's batches (16, 64, 256, ... elements) is missed
-    // (src/sampling_distribution.h:166-181).
+    // (src/sampling_distribution.h:166-181).  (For p = 1 the element it then goes on to has next to no weight.)
     bool batch_end = false;
-    for (int end = 16; end <= hi + 1 && end < V; end *= 4) batch_end = batch_end || end >= lo + 1;
+    for (int end = 16; end <= hi + 1 && end < V && prm.p < 1.0f; end *= 4) batch_end = batch_end || end >= lo + 1;
     const double kept_hi = sh.kept_hi, guard = draw_guard(kept_hi, static_cast<double>(hi) + 1.0);
     const double t_lo = u * sh.kept_lo - guard, t_hi = u * kept_hi + guard;
-    const u64 w_lo = word_mass(t_lo), w_hi = word_mass(t_hi) + 1, mask = (1ull << shift) - 1ull;
+    const u64 w_lo = word_mass(t_lo - base), w_hi = word_mass(t_hi - base) + 1, mask = (1ull << shift) - 1ull;
     // the finer bucket the target falls into
     int b_lo = kIntMax, b_hi = kIntMax;
     u64 front = 0;
@@ -454,7 +456,7 @@ struct TokenPick {
     if (batch_end || sub != sub_sure || sub == kIntMax) return;  // (a boundary between two elements lies in reach)
     front = wave_read_lane(front, first_lane(__ballot(b_lo == sub)));
     const int n = count_of(sh.sub[1].sum[sub]), at = count_of(front);
-    const double s = mass_of(front);
+    const double s = base + mass_of(front);
     const uint32_t okey = sh.sub[1].tag_min[sub];
     if (n > 64) {
       // If they are ties, which of them it is comes from their ids.
@@ -506,6 +508,10 @@ struct TokenPick {
     if (wave == 1) run = scan_subs(1, draw_before, sum);
     __syncthreads();
     if (wave == 1) resolve_draw(sum, run, n_list);
+    return resolved(n_list);
+  }
+  // What resolve_draw has left behind.
+  __device__ __forceinline__ uint32_t resolved(int n_list) const {
     __syncthreads();
     if (sh.tie_rank >= 0) {
       const u64* const keys = list;

@@ -7,7 +7,9 @@
 // key three times at the memory rate of a single CU, and its sums run over 128 K exponentials in one workgroup.  Here
 // every step but the last is spread over the GPU, in five launches (16 x 128256 fp16: 557 -> 59 us per
 // step on the same rows again and 66 on rows that come from memory: 4.7 + 4.7 + 11.5 + 21.6 + 20 us by a trace; every
-// one of them is a chain of dependent phases of a few barriers each, no launch moves more than 33 MB):
+// one of them is a chain of dependent phases of a few barriers each, no launch moves more than 33 MB).  Rows whose token
+// alone is asked for need no order: for p = 1 a launch between 2 and 3 picks it from the histogram (wide_pick_kernel), and
+// the launches behind it find nothing to do for 99.7 % of such rows.
 //   1. wide_max:     the maximum of every chunk of kWideChunk logits.
 //   2. wide_count:   a histogram per chunk over kWideBuckets buckets, linear in the score below the row's maximum down
 //                    to the depth past which no element can lie inside the kept set.
@@ -31,6 +33,7 @@
 #pragma once
 #include "sample_stream.h"
 #include "seqsum_exp_step.h"
+#include "token_pick.h"
 #include "seq_walk.h"
 
 namespace ms {
@@ -85,6 +88,52 @@ __device__ __forceinline__ void wide_load(const InT* row, int V, int chunk, floa
     }
   }
 }
+// The same loads, not widened yet (a chunk past the last one: the last one's).
+template <typename InT>
+struct WideRaw {
+  static constexpr int kVec = 16 / static_cast<int>(sizeof(InT)), kLoads = kWidePer / kVec;
+  v4u q[kLoads];
+  __device__ __forceinline__ void load(const InT* row, int V, int chunks, int chunk) {
+    const int c = chunk < chunks ? chunk : chunks - 1;
+#pragma unroll
+    for (int j = 0; j < kLoads; ++j) {
+      const int i0 = c * kWideChunk + (j * kWideBlock + static_cast<int>(threadIdx.x)) * kVec;
+      q[j] = *reinterpret_cast<const v4u_any*>(row + (i0 + kVec <= V ? i0 : V - kVec));  // (the row's end: shifted below)
+    }
+  }
+  // Value e of the chunk, NaN past the end of the row.
+  __device__ __forceinline__ void widen(int V, int chunk, float (&v)[kWidePer]) const {
+#pragma unroll
+    for (int j = 0; j < kLoads; ++j) {
+      if constexpr (kVec == 4) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) v[j * 4 + c] = __uint_as_float(q[j][c]);
+      } else if constexpr (__is_same(InT, uint16_t)) {
+        widen_half8(q[j], &v[j * 8]);
+      } else {
+        widen_bf16x8(q[j], &v[j * 8]);
+      }
+    }
+    if ((chunk + 1) * kWideChunk > V) {  // (the row's last chunk: a group that crosses the end holds the row's last values)
+#pragma unroll
+      for (int j = 0; j < kLoads; ++j) {
+        const int i0 = chunk * kWideChunk + (j * kWideBlock + static_cast<int>(threadIdx.x)) * kVec;
+        if (i0 + kVec > V) {
+          const int past = i0 + kVec - V;  // value c of the group came as value c + past
+          float w[kVec];
+#pragma unroll
+          for (int c = 0; c < kVec; ++c) {
+            w[c] = __uint_as_float(0x7fc00000u);
+#pragma unroll
+            for (int d = 0; d < kVec; ++d) w[c] = d == c + past ? v[j * kVec + d] : w[c];
+          }
+#pragma unroll
+          for (int c = 0; c < kVec; ++c) v[j * kVec + c] = w[c];
+        }
+      }
+    }
+  }
+};
 template <typename InT>
 __device__ __forceinline__ int wide_index(int chunk, int e) {
   constexpr int VEC = 16 / static_cast<int>(sizeof(InT));
@@ -134,9 +183,17 @@ struct WideBuckets {
   }
 };
 
+// The masses of a row's buckets lie behind the counts, chunk by chunk; the first one of a chunk that has a NaN is negative.
+__device__ __forceinline__ double2* wide_masses(const SampleArgs& a, const WideArgs& w, int row) {
+  return reinterpret_cast<double2*>(a.big + static_cast<size_t>(row) * a.big_stride + static_cast<size_t>(w.chunks) * (kWideBlock / 2));
+}
+
 template <typename InT, bool INLINE>
 __global__ __launch_bounds__(kWideBlock) void wide_count_kernel(const SampleArgs a, const typename WideTable<INLINE>::type, const WideArgs w) {
   __shared__ uint32_t hist[kWideBuckets + 1];
+  __shared__ double mass[kWideBuckets];
+  __shared__ uint64_t exp_tab[32];
+  __shared__ int has_nan;
   const WideShare mine = wide_share(w.chunks);
   const int chunk = mine.item, row = mine.row, tid = threadIdx.x;
   if (row >= a.rows) return;
@@ -147,18 +204,211 @@ __global__ __launch_bounds__(kWideBlock) void wide_count_kernel(const SampleArgs
   float v[kWidePer];
   wide_load<InT>(static_cast<const InT*>(row_start<INLINE>(a, row, sizeof(InT))), a.vocab, chunk, v);
   for (int b = tid; b <= kWideBuckets; b += kWideBlock) hist[b] = 0u;
+  const bool pick = w.pick != 0 && prm.p == 1.0f;
+  if (pick) {
+    mass[tid] = mass[tid + kWideBlock] = 0.0;
+    if (tid < 32) exp_tab[tid] = em::exp2_tab(static_cast<uint32_t>(tid));
+    if (tid == 0) has_nan = 0;
+  }
   __syncthreads();
   const WideBuckets bucket_of(key_to_float(rmax), wide_depth(prm, a.vocab));
+  if (pick) {
+    const float top = key_to_float(rmax), inv_temp = 1.0f / prm.temperature;
+    const uint64_t* const tab = exp_tab;
+    float ex[kWidePer];
 #pragma unroll
-  for (int e = 0; e < kWidePer; ++e) {
-    const uint32_t b = bucket_of(v[e]);
-    if (b < static_cast<uint32_t>(kWideBuckets)) atomicAdd(&hist[b], 1u);
+    for (int e = 0; e < kWidePer; ++e) ex[e] = em::expf_in_range((v[e] - top) * inv_temp, [=](uint32_t i) { return tab[i]; });
+#pragma unroll
+    for (int e = 0; e < kWidePer; ++e) {
+      const uint32_t b = bucket_of(v[e]);
+      if (b < static_cast<uint32_t>(kWideBuckets)) {
+        atomicAdd(&hist[b], 1u);
+        __hip_atomic_fetch_add(&mass[b], static_cast<double>(ex[e]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      } else if (v[e] != v[e] && wide_index<InT>(chunk, e) < a.vocab) {
+        has_nan = 1;
+      }
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < kWidePer; ++e) {
+      const uint32_t b = bucket_of(v[e]);
+      if (b < static_cast<uint32_t>(kWideBuckets)) atomicAdd(&hist[b], 1u);
+    }
   }
   __syncthreads();
   // two buckets a thread, packed: a chunk holds at most kWideChunk keys
   static_assert(kWideBuckets == 2 * kWideBlock && kWideChunk < 1 << 16, "a pair of buckets per thread, of 16 bits each");
   uint32_t* out = reinterpret_cast<uint32_t*>(a.big + static_cast<size_t>(row) * a.big_stride) + static_cast<size_t>(chunk) * kWideBlock;
   out[tid] = hist[2 * tid] | (hist[2 * tid + 1] << 16);
+  if (pick) {
+    double2* const masses = wide_masses(a, w, row) + static_cast<size_t>(chunk) * kWideBlock;
+    masses[tid] = make_double2(tid == 0 && has_nan ? -mass[0] : mass[2 * tid], mass[2 * tid + 1]);
+  }
+}
+
+// The token of a row of p = 1 whose kept set nobody asks for, without ordering the row (see token_pick.h).  The search
+// stops where (V - i - 1) e_i is half a unit of the running sum or less, so whatever it keeps past there weighs less than
+// 2^-24 of the sum, and the draw is decided by the histogram of masses and the keys of the bucket it points into -- unless
+// a share lies closer to u than what the reference's roundings may move it by (u (1 - u) 2^-23) and that rest: 0.1 to 0.3 %
+// of rows of 128256 and 201088 logits, which go the long way behind this.  (Masses as whole numbers of 2^-43, whose rounding
+// such rows of a few heavy tokens notice: twice as many.)  One workgroup per row: it adds the chunks' histograms up,
+// finds the bucket and looks the row through once more for its keys.  A trace of 16 x 128256 fp16: 3.2 (maximum) + 7.1
+// (counts and masses, 4.8 without these) + 20.4 + 10.5 us, the last for the three launches that find nothing to do; steps
+// 62.9 -> 35.3 us, 64 x 128256 fp16 142 -> 58, 1 x 128256 fp32 50 -> 29, 24 x 201088 bf16 129 -> 51.  A compare of every logit with the two
+// buckets and a load of four chunks at a time instead of eight ahead: 23.0 us for this launch.
+template <typename InT, bool INLINE>
+__global__ __launch_bounds__(kWideBlock) void wide_pick_kernel(const SampleArgs a, const typename WideTable<INLINE>::type, const WideArgs w) {
+  extern __shared__ u64 lds_keys[];
+  PickShared& sh = *reinterpret_cast<PickShared*>(lds_keys + kPickRoom);
+  __shared__ uint64_t exp_tab[32];
+  __shared__ uint32_t wave_counts[16];
+  static_assert(kPickBlock == kWideBlock && kPickRoom * sizeof(u64) + sizeof(PickShared) <= kFinishLds, "the pick's room");
+  const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, V = a.vocab;
+  const mi355x_sample_params prm = row_params<INLINE>(a, row);
+  if (!wide_row(prm)) return;
+  const uint32_t rmax = wide_row_max(a, w, row);
+  if (rmax == 0xffffffffu || !(prm.p == 1.0f)) {
+    if (tid == 0) w.rows[row].declined = 0u;
+    return;
+  }
+  // The first of the row's chunks are requested now: they are looked through last.
+  constexpr int kAhead = WideRaw<InT>::kLoads == 1 ? 8 : 4;
+  const InT* const x = static_cast<const InT*>(row_start<INLINE>(a, row, sizeof(InT)));
+  WideRaw<InT> raw[kAhead];
+#pragma unroll
+  for (int c = 0; c < kAhead; ++c) raw[c].load(x, V, w.chunks, c);
+  // the thread's two buckets in the whole row
+  double m0 = 0.0, m1 = 0.0;
+  uint32_t n_own = 0u, n_first = 0u;
+  bool nan = false;
+  const double2* const masses = wide_masses(a, w, row) + tid;
+  const uint32_t* const counts = reinterpret_cast<const uint32_t*>(a.big + static_cast<size_t>(row) * a.big_stride) + tid;
+  for (int c0 = 0; c0 < w.chunks; c0 += 8) {
+    double2 m[8];
+    uint32_t n[8];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      m[c] = c0 + c < w.chunks ? masses[static_cast<size_t>(c0 + c) * kWideBlock] : make_double2(0.0, 0.0);
+      n[c] = c0 + c < w.chunks ? counts[static_cast<size_t>(c0 + c) * kWideBlock] : 0u;
+    }
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      nan |= signbit(m[c].x);
+      m0 += fabs(m[c].x);
+      m1 += m[c].y;
+      n_first += n[c] & 0xffffu;
+      n_own += (n[c] & 0xffffu) + (n[c] >> 16);
+    }
+  }
+  TokenPick::clear(sh);
+  if (tid < 32) exp_tab[tid] = em::exp2_tab(static_cast<uint32_t>(tid));
+  const double inc = wave_prefix_sum<double>(m0 + m1);
+  const uint32_t n_inc = wave_prefix_sum<uint32_t>(n_own);
+  if (lane == 63) {
+    sh.sums[wave] = em::as_u64(inc);
+    wave_counts[wave] = n_inc;
+  }
+  if (__syncthreads_or(nan)) {  // (one that is kept makes all weights NaN: the long way)
+    if (tid == 0) w.rows[row].declined = 0u;
+    return;
+  }
+  const double ws = wave_prefix_sum<double>(lane < 16 ? em::as_double(sh.sums[lane]) : 0.0);
+  const uint32_t wn = wave_prefix_sum<uint32_t>(lane < 16 ? wave_counts[lane] : 0u);
+  const double before = (wave > 0 ? wave_read_lane(ws, wave - 1) : 0.0) + (inc - (m0 + m1)), total = wave_read_lane(ws, 15);
+  const uint32_t n_before = (wave > 0 ? wave_read_lane(wn, wave - 1) : 0u) + n_inc - n_own;
+  const double u = a.uniforms[row];
+  // the first bucket in which the search may stop: up to it, (V - i - 1) e_i exceeds half a unit of any running sum
+  const WideBuckets bucket_of(key_to_float(rmax), wide_depth(prm, V));
+  const float step = 1.0f / (prm.temperature * bucket_of.scale);
+  const float rest = static_cast<float>(total) * 5.97e-8f * (1.02f + static_cast<float>(V) * 6.1e-8f);
+  auto may_stop = [&](uint32_t n, int bucket_end) { return !(static_cast<float>(V - static_cast<int>(n)) * __expf(-step * static_cast<float>(bucket_end)) > rest); };
+  const bool stop0 = may_stop(n_before + n_first, 2 * tid + 1), stop1 = may_stop(n_before + n_own, 2 * tid + 2);
+  u64 kept_bits = em::as_u64(stop0 ? before : before + m0), stop_bucket = static_cast<u64>(stop0 ? 2 * tid : 2 * tid + 1);
+  int at, at_again;
+  block_firsts(stop0 || stop1, kept_bits, at, stop0 || stop1, stop_bucket, at_again, sh.firsts[0]);
+  const double kept_lo = at == kIntMax ? total : em::as_double(kept_bits);
+  if (at == kIntMax) stop_bucket = kWideBuckets;
+  // (what follows the listed elements: two of them at most, each under e^-18 / V)
+  const double kept_hi = total + 4e-8 / static_cast<double>(V);
+  const double guard = kept_hi * (u * (1.0 - u) * 1.21e-7 + 16.0 * 1.2e-16 * static_cast<double>(V) + 1e-11);
+  const double t_lo = u * kept_lo - guard, t_hi = u * kept_hi + guard;
+  // the buckets the draw may fall into
+  const double mid = before + m0, upto = mid + m1;
+  const bool lo_first = m0 != 0.0 && mid >= t_lo, hi_first = m0 != 0.0 && mid >= t_hi;
+  // (which of the two it is takes the lowest bit of the mass in front of it)
+  u64 front = (em::as_u64(lo_first ? before : mid) & ~1ull) | (lo_first ? 0u : 1u), hi_second = hi_first ? 0u : 1u;
+  int d_lo, d_hi;
+  block_firsts(m0 + m1 != 0.0 && upto >= t_lo, front, d_lo, m0 + m1 != 0.0 && upto >= t_hi, hi_second, d_hi, sh.firsts[1]);
+  const uint32_t bucket_lo = 2u * static_cast<uint32_t>(d_lo) + static_cast<uint32_t>(front & 1u);
+  const uint32_t bucket_hi = 2u * static_cast<uint32_t>(d_hi) + static_cast<uint32_t>(hi_second);
+  bool ok = d_lo != kIntMax && d_hi != kIntMax && bucket_hi < stop_bucket;
+  uint32_t id = kNoPick;
+  if (ok) {
+    // their keys
+    u64* const list = lds_keys + kPickHits * (kPickBlock / 64);
+    // (A score of these buckets lies within `reach` of their middle; one in a few thousand that does is not of them.)
+    const float middle = key_to_float(rmax) - 0.5f * static_cast<float>(bucket_lo + bucket_hi + 1u) / bucket_of.scale;
+    const float reach = 0.505f * static_cast<float>(bucket_hi - bucket_lo + 1u) / bucket_of.scale + 1e-5f * (fabsf(middle) + fabsf(key_to_float(rmax)));
+    for (int c0 = 0; c0 < w.chunks; c0 += kAhead) {
+#pragma unroll
+      for (int c = 0; c < kAhead; ++c) {
+        if (c0 + c < w.chunks) {
+          float v[kWidePer];
+          raw[c].widen(V, c0 + c, v);
+          bool near = false;
+#pragma unroll
+          for (int e = 0; e < kWidePer; ++e) near |= fabsf(v[e] - middle) <= reach;
+          if (near) {
+#pragma unroll
+            for (int e = 0; e < kWidePer; ++e) {
+              if (bucket_of(v[e]) - bucket_lo <= bucket_hi - bucket_lo) {
+                const uint32_t i = atomicAdd(&sh.n_list, 1u);
+                if (i < static_cast<uint32_t>(kPickList)) list[i] = make_key64(order_key(v[e]), static_cast<uint32_t>(wide_index<InT>(c0 + c, e)));
+              }
+            }
+          }
+        }
+        raw[c].load(x, V, w.chunks, c0 + c + kAhead);
+      }
+    }
+    if (tid == 0) {
+      sh.token = kNoPick;
+      sh.tie_rank = -1;
+      sh.stop_lo = sh.stop_hi = V - 1;  // (all of the buckets' elements are kept)
+      sh.kept_lo = kept_lo;
+      sh.kept_hi = kept_hi;
+    }
+    __syncthreads();
+    const int n_list = static_cast<int>(sh.n_list);
+    ok = n_list > 0 && n_list <= kPickList;
+    if (ok) {
+      TokenPick pick(sh, lds_keys, exp_tab, rmax, 0u, prm, V, u, static_cast<uint32_t>(n_list));
+      pick.scale = bucket_of.scale;
+      pick.sub_from[1] = static_cast<float>(bucket_lo);
+      pick.sub_scale[1] = static_cast<float>(kPickSubs - 1) / static_cast<float>(bucket_hi - bucket_lo + 1u);
+      pick.base = em::as_double(front);
+      pick.draw_before = 0;
+      for (int i = tid; i < n_list; i += kWideBlock) {
+        const uint32_t okey = key64_okey(list[i]);
+        const float score = key_to_float(okey);
+        pick.refine(1, pick.sub_of(1, score), pick.exp_of(score), okey);
+      }
+      __syncthreads();
+      if (wave == 0) {
+        u64 sum[TokenPick::kSubPer];
+        const u64 run = pick.scan_subs(1, 0, sum);
+        pick.resolve_draw(sum, run, n_list);
+      }
+      id = pick.resolved(n_list);
+    }
+  }
+  if (tid == 0) {
+    w.rows[row].declined = id != kNoPick ? kWidePicked : 0u;
+    if (id != kNoPick) {
+      *row_outputs(a, row).token = static_cast<int32_t>(id);
+      atomicAdd(a.fallback_rows, 1u);  // (a row of the exact path, spread over the GPU)
+    }
+  }
 }
 
 // The keys go to LDS in bucket order first and from there to memory, so that neighbouring lanes write neighbouring
@@ -181,6 +431,7 @@ __global__ __launch_bounds__(kWideBlock) void wide_scatter_kernel(const SampleAr
   const mi355x_sample_params prm = row_params<INLINE>(a, row);
   if (!wide_row(prm)) return;
   WideRow* const info = w.rows + row;
+  if (w.pick != 0 && info->declined == kWidePicked) return;
   const uint32_t rmax = wide_row_max(a, w, row);
   if (rmax == 0xffffffffu) {
     if (chunk == 0 && tid == 0) *info = WideRow{0u, 0u, kWideDeclined, 0.0f};
@@ -425,7 +676,7 @@ __global__ __launch_bounds__(kWideRankBlock) void wide_rank_kernel(const SampleA
   const mi355x_sample_params prm = row_params<INLINE>(a, row);
   if (!wide_row(prm)) return;
   const WideRow info = w.rows[row];
-  if (info.declined == kWideDeclined || static_cast<uint32_t>(t) >= info.tiles) return;
+  if (info.declined == kWideDeclined || info.declined == kWidePicked || static_cast<uint32_t>(t) >= info.tiles) return;
   const uint32_t* const tile = w.tile_start + static_cast<size_t>(row) * (w.max_tiles + 1) + t;
   const uint32_t first = tile[0], n = tile[1] - first;
   const u64* const keys = a.big2 + static_cast<size_t>(row) * a.big_stride;
@@ -947,7 +1198,7 @@ __global__ __launch_bounds__(kFinishBlock) void wide_finish_kernel(const SampleA
   __shared__ u64 red64[16];
   const int row = blockIdx.x;
   const mi355x_sample_params prm = row_params<INLINE>(a, row);
-  if (!wide_row(prm)) return;
+  if (!wide_row(prm) || w.rows[row].declined == kWidePicked) return;
   if (wide_finish_row<INLINE>(a, w, row, prm, *reinterpret_cast<WideFinishShared*>(lds_keys), seqsh)) {
     if (threadIdx.x == 0) atomicAdd(a.fallback_rows, 1u);  // (a row of the exact path, spread over the GPU)
     return;
@@ -965,6 +1216,7 @@ hipError_t launch_wide(const SampleArgs& a, const typename WideTable<INLINE>::ty
     typedef decltype(elt) InT;
     hipLaunchKernelGGL((wide_max_kernel<InT, INLINE>), grid, block, 0, stream, a, table, w);
     hipLaunchKernelGGL((wide_count_kernel<InT, INLINE>), grid, block, 0, stream, a, table, w);
+    if (w.pick != 0) hipLaunchKernelGGL((wide_pick_kernel<InT, INLINE>), dim3(a.rows), block, kFinishLds, stream, a, table, w);
     hipLaunchKernelGGL((wide_scatter_kernel<InT, INLINE>), grid, block, sizeof(WideScatterShared), stream, a, table, w);
   };
   if (a.dtype == MI355X_F16) passes(uint16_t{});

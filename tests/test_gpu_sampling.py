@@ -1494,6 +1494,26 @@ def test_whole_vocabulary_rows_spread_over_the_gpu(ctx, orc, vocab, dtype):
     assert np.array_equal(got, [orc.sample_row(xw[r], *params[r], u[r]) for r in range(rows)])
 
 
+@pytest.mark.parametrize("vocab,sigma,t,dtype", [
+    (9001, 3.0, 1.0, np.float32), (50257, 2.0, 1.0, np.float16), (128256, 5.0, 0.7, np.float32), (40960, 0.5, 2.0, np.float32), (8192, 12.0, 0.5, np.float16),
+])
+def test_whole_vocabulary_draws_on_the_edges_of_their_guard_bands(ctx, orc, vocab, sigma, t, dtype):
+    """Temperature-only rows whose token alone is asked for are picked from the masses of a histogram's buckets unless a
+    cumulative value lies too close to the draw: draws placed on the reference's cumulative values and within and beyond the
+    band beside them, at the first and the last elements that have any weight, and on both ends."""
+    say("whole vocabulary edges", vocab, sigma, t, dtype)
+    rng = np.random.default_rng(vocab)
+    base = (rng.standard_normal(vocab) * sigma).astype(dtype)
+    _, probs = orc.sampled_categorical(base.astype(np.float32), 0, 1.0, t)
+    cp = np.cumsum(np.asarray(probs, np.float64)) / np.sum(np.asarray(probs, np.float64))
+    us = list(rng.random(12)) + [0.0, 1e-300, np.nextafter(1.0, 0.0), 1.0 - 1e-9]
+    for j in sorted({0, 1, len(cp) // 50, len(cp) // 5, len(cp) // 2, len(cp) - 2}):
+        us += [cp[j], np.nextafter(cp[j], 0.0), np.nextafter(cp[j], 1.0), cp[j] - 1e-8, cp[j] + 1e-8, cp[j] - 2e-7, cp[j] + 2e-7]
+    us = np.array([v for v in us if 0.0 <= v < 1.0], np.float64)
+    x = np.tile(base, (len(us), 1))
+    assert np.array_equal(tokens_only(ctx, x, us, 0, 1.0, t), orc.sample_batch(x.astype(np.float32), 0, 1.0, t, us))
+
+
 def crowded_rows(name, rng, rows, vocab):
     """Rows of which many ids share a score, or lie so close together that a bucket of the row's histogram (a 2048th of
     about thirty temperatures) holds more of them than a tile takes whole: (logits, element type, temperatures)."""
