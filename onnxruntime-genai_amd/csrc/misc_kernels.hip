@@ -433,7 +433,7 @@ __global__ __launch_bounds__(256) void greedy_tail_kernel(int32_t* next_tokens, 
 }
 
 // ---- speculative verification on sparse selections ----------------------------------------------------
-// One 256-thread block per sequence.  Target rows 0..K (row i judges proposal token i, row K is the
+// One workgroup per sequence.  Target rows 0..K (row i judges proposal token i, row K is the
 // bonus row) and draft rows 0..K-1 are kept sets: count, ids, probabilities, padded to a capacity.
 //   mode 0  the accept loop of SpeculativeDecodingStrategy::RunRound
 //           (src/speculative_decoding_strategy.cpp:718-762): GetSparseTokenProbability,
@@ -458,19 +458,89 @@ __device__ __forceinline__ float wave_sparse_prob(const int32_t* ids, const floa
   return 0.0f;
 }
 
-__global__ __launch_bounds__(256) void spec_verify_sparse_kernel(const SpecSparseArgs a) {
+// Position std::discrete_distribution returns for the n weights w of the lanes (n <= 64) and canonical draw u: see
+// block_discrete_draw.
+__device__ __forceinline__ int wave_discrete_draw(int n, float w, double u) {
+  if (n < 2) return 0;
+  const int lane = lane_id();
+  const double wd = lane < n ? static_cast<double>(w) : 0.0;
+  const double upto = wave_scan_add(wd), total = wave_read_lane(upto, n - 1), target = u * total;
+  if (total != total) return 0;  // NaN weights
+  const double guard = 16.0 * static_cast<double>(n) * 1.1102230246251565e-16 * total;
+  if (__ballot(lane < n - 1 && fabs(upto - target) <= guard) == 0) return first_lane(__ballot(lane < n && (lane == n - 1 || upto >= target)));
+  const double share = wd / wave_read_lane(wave_serial_prefix(wd, n), n - 1), cp = wave_serial_prefix(share, n);
+  return first_lane(__ballot(lane < n && (lane == n - 1 || cp >= u)));
+}
+
+constexpr int kSpecWaves = 16;  // positions the accept loop's short way judges, a wave each
+
+__global__ __launch_bounds__(64 * kSpecWaves) void spec_verify_sparse_kernel(const SpecSparseArgs a) {
   __shared__ SeqShared sh;
   __shared__ float s_pt[kSpecMaxK], s_pd[kSpecMaxK];
   __shared__ int s_n, s_bad;
+  __shared__ int s_verdict[kSpecWaves], s_token[kSpecWaves], s_count[kSpecWaves];
   const int b = blockIdx.x, tid = threadIdx.x, lane = lane_id(), wave = tid >> 6;
   const int K = a.K;
   const int32_t* tc = a.t_count + static_cast<size_t>(b) * (K + 1);
   const int32_t* prop = a.proposal + static_cast<size_t>(b) * K;
   auto t_ids = [&](int r) { return a.t_ids + (static_cast<size_t>(b) * (K + 1) + r) * a.t_cap; };
   auto t_probs = [&](int r) { return a.t_probs + (static_cast<size_t>(b) * (K + 1) + r) * a.t_cap; };
+  // The accept loop over kept sets of up to 64 entries, the usual case: every position has a wave of its own, which
+  // requests all it may need at once, judges its proposal and draws the token a stop there would end the round with.  Only
+  // which of them it is has to wait for the others.  (With the look-ups, the loop, the residual's look-ups in memory and
+  // its draw one after the other, five barriers between them, 8 sequences of 5 took 11.2 us by a trace; 5.4 this way, the
+  // speculative step 23.6 -> 18.1.)
+  if (a.mode == 0 && K < static_cast<int>(blockDim.x) / 64) {
+    constexpr int kBad = 1, kLong = 2, kAccepts = 4;
+    const int i = wave;
+    const bool judged = i < K;  // (position K is the bonus row)
+    const size_t trow = static_cast<size_t>(b) * (K + 1) + (i < K ? i : K), drow = static_cast<size_t>(b) * K + (judged ? i : 0);
+    const int nt = a.t_count[trow], nd = judged ? a.d_count[drow] : 0;
+    const int32_t proposed = judged ? a.proposal[drow] : -1;
+    const float accept = judged ? a.accept_u[drow] : 0.0f;
+    const double u = a.sample_u[static_cast<size_t>(b) * (K + 1) + (judged ? i + 1 : K)];
+    const bool in_t = lane < a.t_cap, in_d = judged && lane < a.d_cap;
+    const int32_t id = in_t ? a.t_ids[trow * a.t_cap + lane] : -1, d_id = in_d ? a.d_ids[drow * a.d_cap + lane] : -1;
+    const float pr = in_t ? a.t_probs[trow * a.t_cap + lane] : 0.0f, d_pr = in_d ? a.d_probs[drow * a.d_cap + lane] : 0.0f;
+    int verdict = (nt > a.t_cap || nt < 1 || (judged && nd > a.d_cap) ? kBad : 0) | (nt > 64 || nd > 64 ? kLong : 0);
+    if (i <= K && verdict == 0) {
+      float w = pr;
+      if (judged) {
+        const int ft = first_lane(__ballot(lane < nt && id == proposed)), fd = first_lane(__ballot(lane < nd && d_id == proposed));
+        const float pt = ft >= 0 ? wave_read_lane(pr, ft) : 0.0f, pd = fd >= 0 ? wave_read_lane(d_pr, fd) : 0.0f;
+        const float acc = pd <= 0.0f ? 1.0f : fminf(1.0f, pt / pd);  // ComputeAcceptProb
+        if (accept < acc) verdict |= kAccepts;
+        float q = 0.0f;  // the draft's probability of this lane's id: of several entries the first one's
+#pragma unroll 4
+        for (int m = nd - 1; m >= 0; --m) q = id == wave_read_lane(d_id, m) ? wave_read_lane(d_pr, m) : q;
+        const float d = pr - q, r = d > 0.0f ? d : 0.0f;
+        // the reference's sequential fp32 sum of non-negative terms is positive iff one of them is
+        if (__ballot(lane < nt && r > 0.0f) != 0) w = r;
+      }
+      const int32_t token = wave_read_lane(id, wave_discrete_draw(nt, w, u));
+      if (lane == 0) s_token[i] = token;
+    }
+    if (lane == 0) {
+      s_verdict[i] = i <= K ? verdict : 0;
+      s_count[i] = nt;
+    }
+    __syncthreads();
+    const int of_wave = lane <= K ? s_verdict[lane] : 0;
+    const bool any_bad = __ballot(of_wave & kBad) != 0;
+    const int stop = first_lane(__ballot(lane < K && (of_wave & kAccepts) == 0)), n = stop >= 0 ? stop : K;
+    if (any_bad || __ballot(of_wave & kLong) == 0) {
+      if (tid == 0) {
+        const int evaluated = n < K ? n + 1 : K;
+        a.accepted_len[b] = any_bad ? -1 : n;
+        a.final_token[b] = any_bad ? -1 : s_token[n];
+        a.engine_draws[b] = any_bad ? 0 : evaluated + (s_count[n] >= 2 ? 2 : 0);
+      }
+      return;
+    }
+  }
   if (tid == 0) s_bad = 0;
   __syncthreads();
-  for (int r = tid; r <= K; r += 256) {
+  for (int r = tid; r <= K; r += blockDim.x) {
     bool bad = tc[r] > a.t_cap || tc[r] < 1;
     if (a.mode == 0 && r < K) bad = bad || a.d_count[static_cast<size_t>(b) * K + r] > a.d_cap;
     if (bad) s_bad = 1;
@@ -516,7 +586,7 @@ __global__ __launch_bounds__(256) void spec_verify_sparse_kernel(const SpecSpars
   }
   // mode 0: every position's two look-ups at once, a wave per position
   const int32_t* dc = a.d_count + static_cast<size_t>(b) * K;
-  for (int i = wave; i < K; i += 4) {
+  for (int i = wave; i < K; i += static_cast<int>(blockDim.x) / 64) {
     const float pt = wave_sparse_prob(t_ids(i), t_probs(i), tc[i], prop[i]);
     const float pd = wave_sparse_prob(a.d_ids + (static_cast<size_t>(b) * K + i) * a.d_cap,
                                       a.d_probs + (static_cast<size_t>(b) * K + i) * a.d_cap, dc[i], prop[i]);
@@ -547,7 +617,7 @@ __global__ __launch_bounds__(256) void spec_verify_sparse_kernel(const SpecSpars
     const float* dp = a.d_probs + (static_cast<size_t>(b) * K + n) * a.d_cap;
     const int nd = dc[n];
     int any = 0;
-    for (int j = tid; j < nt; j += 256) {
+    for (int j = tid; j < nt; j += blockDim.x) {
       const int32_t id = ids[j];
       float q = 0.0f;
       for (int m = 0; m < nd; ++m)
@@ -728,7 +798,8 @@ extern "C" hipError_t ms_launch_greedy_tail(int32_t* next_tokens, int32_t* eos_s
 }
 
 extern "C" hipError_t ms_launch_spec_verify_sparse(const ms::SpecSparseArgs* a, int batch, hipStream_t stream) {
-  hipLaunchKernelGGL(ms::spec_verify_sparse_kernel, dim3(batch), dim3(256), 0, stream, *a);
+  const int waves = a->mode == 0 && a->K < ms::kSpecWaves && a->K >= 4 ? a->K + 1 : 4;
+  hipLaunchKernelGGL(ms::spec_verify_sparse_kernel, dim3(batch), dim3(64 * waves), 0, stream, *a);
   return hipGetLastError();
 }
 

@@ -282,6 +282,44 @@ def test_spec_verify_sparse_randomised(ctx, orc, seed):
         assert (acc[s].item(), tok[s].item(), used[s].item()) == (n, int(t[n][0][0]), 0), s
 
 
+@pytest.mark.parametrize("K,nt,nd", [(1, 1, 1), (3, 64, 64), (4, 63, 64), (5, 64, 65), (5, 65, 20), (14, 2, 64), (15, 64, 40), (16, 64, 64), (20, 30, 30)])
+def test_spec_verify_sparse_at_the_edges_of_a_wave_per_position(ctx, orc, K, nt, nd):
+    """The accept loop with kept sets just below, at and above the 64 entries a position's wave holds and as many positions
+    as a workgroup has waves, one more and one less; a draft that lists an id twice, one that equals the target (its
+    residual is empty) and draws on and beside the cumulative values of the target row."""
+    say("spec_verify_sparse edges", K, nt, nd)
+    rng = np.random.default_rng(K * 10007 + nt * 101 + nd)
+    batch = 6
+
+    def row(n, pool):
+        ids = rng.permutation(pool)[:n].astype(np.int32)
+        w = rng.random(n).astype(np.float32) + np.float32(1e-3)
+        return ids, (w / w.sum()).astype(np.float32)
+
+    rounds = []
+    for s in range(batch):
+        pool = np.arange(max(nt, nd) + (5 if s % 2 else 400))
+        target, draft = [row(nt, pool) for _ in range(K + 1)], [row(nd, pool) for _ in range(K)]
+        for i in range(K):
+            if s == 1 and nt == nd:
+                draft[i] = target[i]
+            if s == 2 and nd > 1:
+                draft[i][0][nd - 1] = draft[i][0][0]
+        rounds.append((np.array([d[0][0] if s != 3 else t[0][-1] for d, t in zip(draft, target)], np.int32), target, draft))
+    au, su = rng.random((batch, K)).astype(np.float32), rng.random((batch, K + 1))
+    au[4:] = 0.0  # (a proposal the target row holds is taken)
+    for s in range(batch):
+        for i in range(K + 1):
+            cp = np.cumsum(rounds[s][1][i][1].astype(np.float64))
+            v = cp[rng.integers(0, nt)] / cp[-1]
+            su[s, i] = min(max(rng.choice([v, np.nextafter(v, 0.0), np.nextafter(v, 1.0), su[s, i]]), 0.0), np.nextafter(1.0, 0.0))
+    acc, tok, used = ctx.spec_verify_sparse(pack_rows([t for _, t, _ in rounds], nt + 3), pack_rows([d for _, _, d in rounds], nd),
+                                            torch.from_numpy(np.stack([p for p, _, _ in rounds])).cuda(), torch.from_numpy(au).cuda(),
+                                            torch.from_numpy(su).cuda(), mode=0)
+    for s, (prop, t, d) in enumerate(rounds):
+        assert (acc[s].item(), tok[s].item(), used[s].item()) == orc.spec_verify_sparse(prop, t, d, au[s], su[s]), s
+
+
 def test_spec_verify_sparse_end_to_end_with_sampler_outputs(ctx, orc):
     """The verify rows' kept sets come straight from mi355x_sample (device buffers, no host round trip) and
     the proposal is built so that the first positions are accepted; a truncated kept set is reported as -1."""
