@@ -932,11 +932,13 @@ __device__ __forceinline__ void nucleus_finish_body(const SampleArgs& a) {
   // or above it is in its chunk's list.
   uint32_t thr = wave_max<uint32_t>(cthr);
   if (rmax == 0u) thr = 0u;  // (no number in the row)
-  if (tid < 64) {
+  // (wave 0; picks: the heads serve a row that is picked from however long its lists are, the sort's only where all fit its room)
+  auto lay_out = [&](bool picks) __attribute__((always_inline)) {
     const uint32_t listed = gave_up ? 0u : cnt;
     const uint32_t all = wave_sum<uint32_t>(listed);
-    const uint32_t head =
-        (a.chunks <= kAheadChunks && all < static_cast<uint32_t>(kNucleusCap)) ? static_cast<uint32_t>(kFinishBlock) << head_shift : 0u;
+    const uint32_t head = (a.chunks <= kAheadChunks && (all < static_cast<uint32_t>(kNucleusCap) || (picks && TokenPick::worth_it(a.rows, all))))
+                              ? static_cast<uint32_t>(kFinishBlock) << head_shift
+                              : 0u;
     // (in rows of kFinishBlock entries: a row lies in one chunk's list, so its chunk is found once for all threads)
     const uint32_t rows = listed <= head ? 0u : (listed - head + kFinishBlock - 1u) / kFinishBlock;
     const uint32_t before = wave_prefix_sum<uint32_t>(rows) - rows;
@@ -945,12 +947,13 @@ __device__ __forceinline__ void nucleus_finish_body(const SampleArgs& a) {
       sh_head = head;
       sh_all = all;
     }
-  }
+  };
+  if (tid < 64) lay_out(try_pick);
   __syncthreads();
   // The chunks' lists past their heads, as a sequence of rows of kFinishBlock entries (sh_first[c] = rows of the
   // chunks before c; a list's last row may be short).  A cursor walks the rows in order; which chunk a row lies in
   // is the same for every thread, so finding it costs the threads nothing.
-  const uint32_t head = sh_head;
+  uint32_t head = sh_head;
   struct ListCursor {
     int chunk = -1;
     uint32_t next_first = 0u, base = 0u, cnt = 0u;  // rows before the next chunk / before this one, entries of this one's list
@@ -1112,6 +1115,11 @@ __device__ __forceinline__ void nucleus_finish_body(const SampleArgs& a) {
     }
     clear_buckets();
     __syncthreads();
+    if (head != 0u && sh_all >= static_cast<uint32_t>(kNucleusCap)) {
+      if (tid < 64) lay_out(false);
+      __syncthreads();
+      head = sh_head;
+    }
   }
   // A nucleus row's usual way: a counting sort over the lists where they lie.  A first pass over them counts the
   // candidates (at or above the row's threshold) into the sort's buckets; the histogram tells how many buckets the

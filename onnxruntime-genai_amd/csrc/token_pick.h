@@ -113,8 +113,10 @@ struct TokenPick {
 
   // Whether picking is worth a try for one of `rows` rows of n candidates each: what it leaves open grows with the nucleus
   // twice, in the shares a draw may meet and in the roundings of a bucket in which the running sum changes its binade, and
-  // one row that has to be sorted after all makes the launch longer.  (Given back: 0.02 to 0.1 % of rows of 3000 to 10000
-  // candidates, 34 % of those of 110000: 64 x 128256 fp32 rows N(0, 2^2), p = 0.9, took 374 us a step instead of 291.)
+  // one row that has to be sorted after all makes the launch longer by the sort.  Given back: 0.02 to 0.1 % of rows of 3000
+  // to 13000 candidates, 1 to 3 % of flatter ones (16 x 128256 fp32 N(0, 3^2), T = 0.8, p = 0.9: 1.0 %, 48 us picked and 63
+  // sorted; N(0, 4^2), p = 0.95: 1.7 %, 48 and 87), 6 % of N(0, 3^2), T = 1 (68 and 135: the line), 37 % of the 110000
+  // candidates of N(0, 2^2) (105 and 252).
   __device__ static __forceinline__ bool worth_it(int rows, uint32_t n) {
     return static_cast<float>(rows) * static_cast<float>(n) * static_cast<float>(n) < 4e10f;
   }
