@@ -1456,6 +1456,13 @@ def test_draw_in_order_follows_one_engine(ctx, orc, rows, cap):
     assert used.item() == -1
 
 
+@pytest.mark.parametrize("rows,cap", [(1, 1), (2, 2), (63, 63), (64, 64), (65, 64), (130, 64), (200, 3), (70, 65)])
+def test_draw_in_order_at_the_edges_of_a_wave_per_row(ctx, orc, rows, cap):
+    """Lists of up to 64 entries are drawn from by a wave per row, batches around a wave's lanes and beyond; one entry more
+    takes a workgroup per row."""
+    test_draw_in_order_follows_one_engine(ctx, orc, rows, cap)
+
+
 @pytest.mark.parametrize("vocab", [4095, 4096, 8191, 8193, 12289, 50257, 128256])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 def test_whole_vocabulary_rows_spread_over_the_gpu(ctx, orc, vocab, dtype):
