@@ -253,8 +253,8 @@ __global__ __launch_bounds__(kWideBlock) void wide_count_kernel(const SampleArgs
 // of rows of 128256 and 201088 logits, which go the long way behind this.  (Masses as whole numbers of 2^-43, whose rounding
 // such rows of a few heavy tokens notice: twice as many.)  One workgroup per row: it adds the chunks' histograms up,
 // finds the bucket and looks the row through once more for its keys.  A trace of 16 x 128256 fp16: 3.2 (maximum) + 7.1
-// (counts and masses, 4.8 without these) + 20.4 + 10.5 us, the last for the three launches that find nothing to do; steps
-// 62.9 -> 35.3 us, 64 x 128256 fp16 142 -> 58, 1 x 128256 fp32 50 -> 29, 24 x 201088 bf16 129 -> 51.  A compare of every logit with the two
+// (counts and masses, 4.8 without these) + 19.2 + 10.5 us, the last for the three launches that find nothing to do; steps
+// 62.9 -> 35.1 us, 64 x 128256 fp16 142 -> 58, 1 x 128256 fp32 50 -> 29, 24 x 201088 bf16 129 -> 51.  A compare of every logit with the two
 // buckets and a load of four chunks at a time instead of eight ahead: 23.0 us for this launch.
 template <typename InT, bool INLINE>
 __global__ __launch_bounds__(kWideBlock) void wide_pick_kernel(const SampleArgs a, const typename WideTable<INLINE>::type, const WideArgs w) {
@@ -361,7 +361,7 @@ __global__ __launch_bounds__(kWideBlock) void wide_pick_kernel(const SampleArgs 
           if (near) {
 #pragma unroll
             for (int e = 0; e < kWidePer; ++e) {
-              if (bucket_of(v[e]) - bucket_lo <= bucket_hi - bucket_lo) {
+              if (fabsf(v[e] - middle) <= reach && bucket_of(v[e]) - bucket_lo <= bucket_hi - bucket_lo) {
                 const uint32_t i = atomicAdd(&sh.n_list, 1u);
                 if (i < static_cast<uint32_t>(kPickList)) list[i] = make_key64(order_key(v[e]), static_cast<uint32_t>(wide_index<InT>(c0 + c, e)));
               }
