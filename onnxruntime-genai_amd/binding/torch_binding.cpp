@@ -27,7 +27,8 @@ extern "C" int ms_sample_padded(mi355x_search_ctx* ctx, void* stream, const void
                                 mi355x_sample_params params, const mi355x_sample_params* per_row_params, const double* uniforms,
                                 int32_t* out_tokens, int32_t* kept_count, int32_t* kept_ids, float* kept_probs,
                                 int kept_capacity);
-extern "C" int ms_copy_words_and_wait(void* stream, void* dst, const void* src, size_t words);
+extern "C" int ms_scorer_copy_words(mi355x_beam_scorer* s, void* stream, void* dst, const void* src, size_t words);
+extern "C" int ms_scorer_is_done(mi355x_beam_scorer* s, void* stream, int* done);
 
 namespace {
 
@@ -838,7 +839,7 @@ MS_METHOD(is_done) {
     int rc, done = 0;
     {
       Unlocked u;
-      rc = mi355x_beam_scorer_is_done(Scr(self)->handle, s, &done);
+      rc = ms_scorer_is_done(Scr(self)->handle, s, &done);
     }
     Check(rc);
     return PyBool_FromLong(done);
@@ -854,7 +855,7 @@ Tensor CopyOf(const Scorer& s, const void* from, at::IntArrayRef sizes, at::Scal
   int rc;
   {
     Unlocked u;
-    rc = ms_copy_words_and_wait(stream, out.data_ptr(), from, out.nbytes() / 4);
+    rc = ms_scorer_copy_words(s.handle, stream, out.data_ptr(), from, out.nbytes() / 4);
   }
   Check(rc);
   return out;

@@ -585,17 +585,6 @@ int ms_sample_padded(mi355x_search_ctx* ctx, void* stream, const void* logits, c
                     kept_ids, kept_probs, kept_capacity, true);
 }
 
-// Copies 32-bit words between buffers of one device, behind the work of `stream`, and waits for it: what the Python
-// binding hands out as the scorer's state is complete when the caller has it, on any stream.
-int ms_copy_words_and_wait(void* stream, void* dst, const void* src, size_t words) {
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  if (Capturing(s))
-    return Fail(MI355X_E_UNSUPPORTED, "a copy of a scorer's state is complete on return: it cannot be recorded into a graph");
-  if (words != 0) HIP_TRY(ms_launch_copy_words(static_cast<const uint32_t*>(src), static_cast<uint32_t*>(dst), words, s));
-  HIP_TRY(hipStreamSynchronize(s));
-  return MI355X_OK;
-}
-
 int mi355x_topk_scores(mi355x_search_ctx* ctx, void* stream, const void* logits, int dtype, int64_t row_stride,
                        int rows, int vocab, int k, int32_t* out_tokens, float* out_scores) {
   if (int r = CheckRows(ctx, rows, vocab)) return r;
@@ -947,6 +936,16 @@ struct mi355x_beam_scorer {
   std::vector<char> lists;  // empty: not read back
   std::shared_ptr<ScorerHost> host;  // (only the search steps use `ctx` itself after the creation: it may be gone before the others)
   int done_word{-1};  // which of its words st.all_done is (-1: none, the count is read back)
+  // The last step has been waited for: a copy that was made behind it, on the stream it was issued on, is complete.
+  hipStream_t step_stream{};
+  std::atomic<bool> awaited{false};
+  void Stepped(hipStream_t stream) {
+    cur = 1 - cur;
+    length += 1;
+    lists.clear();
+    step_stream = stream;
+    awaited = false;
+  }
 };
 
 int mi355x_beam_scorer_create(mi355x_search_ctx* ctx, int batch, int beams, int max_length, int pad_token_id,
@@ -1079,9 +1078,7 @@ int mi355x_beam_scorer_step(mi355x_beam_scorer* s, void* stream, const float* ca
     return Fail(MI355X_E_UNSUPPORTED, "a scorer step carries the sequence length and buffer of this very step: a graph replay would repeat it");
   HIP_TRY(ms_launch_scorer_step(&s->st, s->seq[s->cur], s->seq[1 - s->cur], s->length, cand_scores, cand_tokens,
                                 cand_beam_indices, st));
-  s->cur = 1 - s->cur;
-  s->length += 1;
-  s->lists.clear();
+  s->Stepped(st);
   return MI355X_OK;
 }
 
@@ -1097,9 +1094,7 @@ int mi355x_beam_search_step(mi355x_beam_scorer* s, void* stream, const void* log
                              s->cand_scores, s->cand_tokens, s->cand_beams, &step, &fused))
     return r;
   if (!fused) return mi355x_beam_scorer_step(s, stream, s->cand_scores, s->cand_tokens, s->cand_beams);
-  s->cur = 1 - s->cur;
-  s->length += 1;
-  s->lists.clear();
+  s->Stepped(static_cast<hipStream_t>(stream));
   return MI355X_OK;
 }
 
@@ -1127,6 +1122,29 @@ int mi355x_beam_scorer_is_done(mi355x_beam_scorer* s, void* stream, int* done) {
     all_done = *nd == 0;
   }
   *done = all_done || (s->length == s->st.max_length);  // BeamSearch_Cpu::IsDone, src/search.cpp:345-352
+  return MI355X_OK;
+}
+
+// Copies words of a scorer's state to a buffer of the same device, behind the work of `stream`, and waits for it: what the
+// Python binding hands out as the scorer's state is complete when the caller has it, on any stream.
+int ms_scorer_copy_words(mi355x_beam_scorer* s, void* stream, void* dst, const void* src, size_t words) {
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (Capturing(st))
+    return Fail(MI355X_E_UNSUPPORTED, "a copy of a scorer's state is complete on return: it cannot be recorded into a graph");
+  if (words != 0) HIP_TRY(ms_launch_copy_words(static_cast<const uint32_t*>(src), static_cast<uint32_t*>(dst), words, st));
+  HIP_TRY(hipStreamSynchronize(st));
+  if (st == s->step_stream) s->awaited = true;
+  return MI355X_OK;
+}
+
+// mi355x_beam_scorer_is_done for the Python binding: where a copy of the state has waited for the last step already, it does
+// not wait for what the stream does besides: the reorder of the caches, usually, behind which the next step can be launched
+// then (2 x 4 x 51865 fp16, 12 steps: 872 -> 735 us a search).
+int ms_scorer_is_done(mi355x_beam_scorer* s, void* stream, int* done) {
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (!s || !done || !s->st.all_done || !s->awaited || st != s->step_stream || Capturing(st))  // (a capturing stream is refused there)
+    return mi355x_beam_scorer_is_done(s, stream, done);
+  *done = *static_cast<volatile int*>(s->st.all_done) != 0 || s->length == s->st.max_length;
   return MI355X_OK;
 }
 

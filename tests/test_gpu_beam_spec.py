@@ -709,6 +709,48 @@ def test_a_prompt_is_in_place_when_the_call_returns(prompt_len):
     ctx.close()
 
 
+@pytest.mark.parametrize("boost", [0.0, 9.0])
+def test_is_done_after_a_copy_of_the_state_does_not_wait_for_later_work(boost):
+    """is_done() behind next_indices knows the step's outcome: it does not wait for work queued since, and says what a
+    scorer that is asked without a copy in between says, step by step, with the steps on one stream and on two."""
+    say("is_done behind a copy", boost)
+    ctx = pkg().SearchContext(4, 20000)
+    scorers = [pkg().BeamScorer(ctx, 2, 2, 12, 0, [2], 1.0, True) for _ in range(3)]
+    for s in scorers:
+        s.set_prompt(np.array([[5, 6], [7, 8]], np.int32))
+    g = torch.Generator(device="cuda").manual_seed(5)
+    stream, other = torch.cuda.Stream(), torch.cuda.Stream()
+    told = []
+    for step in range(10):
+        x = torch.randn(4, 20000, generator=g, device="cuda")
+        x[:, 2] += boost
+        torch.cuda.synchronize()
+        with torch.cuda.stream(stream):
+            scorers[0].search_step(x)
+            scorers[0].next_indices
+            torch.cuda._sleep(4_000_000)
+            copied = scorers[0].is_done()
+            assert not stream.query()
+            plain = (scorers[1].search_step(x), scorers[1].is_done())[1]
+        stream.synchronize()
+        with torch.cuda.stream(other):  # a step here, the copy there: the copy has not waited for this stream
+            scorers[2].search_step(x)
+        with torch.cuda.stream(stream):
+            scorers[2].next_indices
+        with torch.cuda.stream(other):
+            torch.cuda._sleep(1_000_000)
+            apart = scorers[2].is_done()
+            assert other.query()
+        assert copied == plain == apart, step
+        told.append(copied)
+        if copied:
+            break
+    assert told[-1] and len(told) == (10 if boost == 0.0 else len(told))
+    for s in scorers:
+        s.close()
+    ctx.close()
+
+
 def test_copies_of_a_scorers_state_are_complete_when_they_are_handed_out():
     """next_scores, next_tokens, next_indices and sequences() wait for the work of the current stream: their tensors
     can be read on any stream.  A capturing stream is refused, and its capture goes on."""
