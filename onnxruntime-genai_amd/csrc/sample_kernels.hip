@@ -1027,7 +1027,7 @@ __device__ __forceinline__ void nucleus_finish_body(const SampleArgs& a) {
     }
     flat_batches(fn);
   };
-  if (try_pick) {
+  if (MODE == kFinishMixed ? __builtin_expect(try_pick, 0) != 0 : try_pick) {  // (behind the rest where rows of large k pass by)
     if (sh_all != 0u && TokenPick::worth_it(a.rows, sh_all) && rmax < order_key(1e30f) && thr > order_key(-1e30f)) {
       TokenPick pick(pick_sh, lds_keys, exp_tab, rmax, thr, prm, V, a.uniforms[row], sh_all);
       const float thr_score = key_to_float(thr);
