@@ -221,8 +221,11 @@ struct TokenPick {
     float e_below = 0.0f;
     if (stop_hi == kIntMax) {  // the candidates may end before the nucleus does
       const uint32_t okey = row16_max<uint32_t>(lane < 16 ? sh.below[lane] : 0u);
-      if (okey > order_key(-1e30f)) e_below = exp_of(key_to_float(okey));
-      else if (zero_below) ends_in_zero = true;  // (there at the latest: nothing of weight follows)
+      if (okey > order_key(-1e30f)) {
+        // (Nothing says how far below it lies, exp_of is for what a candidate can be: from -104 on a zero, which leaves the stop open.)
+        const float score = key_to_float(okey);
+        e_below = (score - top) * inv_temp > -103.9f ? exp_of(score) : 0.0f;
+      } else if (zero_below) ends_in_zero = true;  // (there at the latest: nothing of weight follows)
       else if (count_of(all) != V) return false;
       e_end = e_below;
       e_end_low = 0.0f;

@@ -364,6 +364,34 @@ def test_token_only_nucleus_rows_that_are_picked_instead_of_sorted(ctx, orc, kin
         assert np.array_equal(got, orc.sample_batch(xw, 0, p, t, u)), rep
 
 
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("dtype,shift,depth", [("f16", -33.0, None), ("f32", 0.0, 1419.6), ("f32", 0.0, 4258.7), ("f32", 3.0, 2839.1), ("f32", 3.0, 104.0)])
+def test_picked_rows_whose_nucleus_ends_in_an_element_far_below(ctx, orc, dtype, shift, depth, masked):
+    """Every third logit lies so far below the others that it weighs nothing, and the search goes on to the first of these:
+    its exponential is a zero however far down it is (None: -inf; 1419.6 = 2048 ln 2 and 4258.7
+    = 6144 ln 2, where an exponent that runs over into the sign gives about minus one, 2839.1 = 4096 ln 2, where it gives one)."""
+    say("far below", dtype, shift, depth, masked)
+    rng = np.random.default_rng(2839)
+    rows, vocab, t, p = 128, 107, 0.4012862343238633, 0.99
+    x = (rng.standard_normal((rows, vocab)) * 0.2 + shift).astype(np.float32)
+    x[:, :4] = x.max(axis=1, keepdims=True)
+    far = -np.inf if depth is None else x.max(axis=1, keepdims=True) - t * (depth + np.linspace(-12.0, 2.0, rows, dtype=np.float32)[:, None])
+    x[:, 4::3] = far
+    xd = torch.from_numpy(x).cuda().to({"f16": torch.float16, "f32": torch.float32}[dtype])
+    xw, form = xd.float().cpu().numpy(), None
+    if masked:
+        words = np.zeros((rows, (vocab + 31) // 32), np.uint32)
+        for i in range(vocab - 7):
+            words[:, i >> 5] |= np.uint32(1 << (i & 31))
+        form = pkg().LogitsXform(mask=torch.from_numpy(words.view(np.int32)).cuda(), mask_allowed_max=vocab - 7)
+        xw[:, vocab - 7:] = np.finfo(np.float32).min
+    for rep in range(3):
+        u = rng.random(rows)
+        u[: rows // 2] *= 0.12  # (among the ties at the top)
+        got = ctx.sample(xd, torch.from_numpy(u).cuda(), k=0, p=p, temperature=t, xf=form).cpu().numpy()
+        assert np.array_equal(got, orc.sample_batch(xw, 0, p, t, u)), rep
+
+
 def test_results_written_straight_to_pinned_host_memory(ctx, orc):
     """The output pointers may name pinned host memory that the device can address (the reference mirrors its
     results through pinned memory, src/cuda/interface.cpp:51-60): the kernels store the tokens there themselves, no
