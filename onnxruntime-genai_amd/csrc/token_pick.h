@@ -122,12 +122,12 @@ struct TokenPick {
   }
 
   // rtop, thr: order keys of the row's maximum and of the lowest candidate; n: at least the number of candidates,
-  // 1 <= n < 2^20 (they take b bits, the mass at most b before its point)
+  // 1 <= n < 2^20 (they and the element below them take b bits, the mass at most b before its point)
   __device__ __forceinline__ TokenPick(PickShared& sh_, u64* room, const uint64_t* exp_tab_, uint32_t rtop, uint32_t thr, mi355x_sample_params prm_, int V_,
                                        double u_, uint32_t n)
       : sh(sh_), hits(room + (threadIdx.x >> 6) * kPickHits), list(room + kPickHits * (kPickBlock / 64)), exp_tab(exp_tab_), prm(prm_), V(V_), u(u_), top(key_to_float(rtop)),
         scale(rtop > thr ? static_cast<float>(kPickBuckets) / (key_to_float(rtop) - key_to_float(thr)) : 0.0f), inv_temp(1.0f / prm_.temperature),
-        shift(__clz(static_cast<int>(n)) + 32), frac(2 * __clz(static_cast<int>(n)) < 44 ? 2 * __clz(static_cast<int>(n)) : 44),
+        shift(__clz(static_cast<int>(n + 1u)) + 32), frac(2 * __clz(static_cast<int>(n + 1u)) < 44 ? 2 * __clz(static_cast<int>(n + 1u)) : 44),
         quant(static_cast<double>(n) * ldexp(0.5, -frac)) {}
 
   __device__ static __forceinline__ void clear(PickShared& sh) {

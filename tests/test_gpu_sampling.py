@@ -392,6 +392,24 @@ def test_picked_rows_whose_nucleus_ends_in_an_element_far_below(ctx, orc, dtype,
         assert np.array_equal(got, orc.sample_batch(xw, 0, p, t, u)), rep
 
 
+@pytest.mark.parametrize("n", [62, 63, 64, 127, 255, 1023, 4095])
+def test_picked_rows_of_nearly_a_power_of_two_candidates(ctx, orc, n):
+    """n candidates and, as the last element kept, the best one below them: one more than n in the counts."""
+    say("power of two", n)
+    rng = np.random.default_rng(n)
+    rows, vocab = 64, n + 700
+    for low in (-30.0, -9.0, -7.0):
+        x = (rng.random((rows, vocab)) * 2.0 + low).astype(np.float32)
+        for r in range(rows):
+            x[r, rng.permutation(vocab)[:n]] = rng.random(n).astype(np.float32)
+        xd = torch.from_numpy(x).cuda()
+        for p in (0.9, 0.95, 0.99):
+            u = rng.random(rows)
+            u[0], u[1] = np.nextafter(1.0, 0.0), 1.0 - 1e-4
+            got = ctx.sample(xd, torch.from_numpy(u).cuda(), k=0, p=p, temperature=1.0).cpu().numpy()
+            assert np.array_equal(got, orc.sample_batch(x, 0, p, 1.0, u)), (low, p)
+
+
 def test_results_written_straight_to_pinned_host_memory(ctx, orc):
     """The output pointers may name pinned host memory that the device can address (the reference mirrors its
     results through pinned memory, src/cuda/interface.cpp:51-60): the kernels store the tokens there themselves, no
