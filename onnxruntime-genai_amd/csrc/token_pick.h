@@ -21,7 +21,7 @@
 // One workgroup per row is bound by vector issue and by the phases between its barriers.  Sorting 7000 candidates took three
 // passes over them, an exponential each, and two exact sums; picking takes two looks and eight barriers.  Finish kernels:
 // 32 x 151936 bf16, p = 0.9: 27.3 -> 22.6 us (2.9 until the lists are there, 1.3 to move candidates together, 2.6 to count
-// them, 4.4 for find(), 3 for the second look, 5 for resolve()), 48 x 50257 fp16 in several modes: 42.5 -> 29.9;
+// them, 4.4 for find(), 3 for the second look, 5 for resolve()), 48 x 50257 fp16 in several modes: 42.5 -> 26.6;
 // 256 x 201088 fp32 under a mask of 5 %: 59.2 -> 50.5 a step, of which the gather is 35.  64 x 128256 fp32 N(0, 5^2): 40.0 ->
 // 33.5 a step; 8 x 201088 bf16, T = 0.7, whose ties the sort gave to the exact path: 1530 -> 60.
 #pragma once
