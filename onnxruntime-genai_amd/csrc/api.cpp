@@ -86,12 +86,15 @@ struct ScorerHost {
   void GiveBackWord(int word) { used.fetch_and(~(uint64_t{1} << word)); }
 };
 
+constexpr int kPlanBlocks = 256;  // a workgroup per CU
+
 struct mi355x_search_ctx {
   int device{};
   int max_rows{}, max_vocab{}, max_chunks{};
   size_t bytes{};
   std::vector<void*> allocs;
   ms::u64* cand_small{};
+  size_t cand_lists{};  // lists of kSmallCap slots
   uint32_t* chunk_cnt{};
   uint32_t* chunk_max{};
   uint32_t* chunk_thr{};
@@ -206,6 +209,47 @@ int ms_make_xform(mi355x_search_ctx* ctx, const mi355x_logits_xform* in, int row
   return MI355X_OK;
 }
 
+// How the rows of a call are cut into chunks, a workgroup each.  small_k: every row is one of top-k (k <= 64) or argmax.
+//
+// A workgroup spends some ten vector instructions on every logit it has room for and a fixed time on selecting and
+// handing over, so chunks are short while the GPU has a CU for each of them (8192, then 16384 logits) and long beyond:
+// twice the workgroups select twice as often.  us, chunks of 32768 -> as chosen, 1 / 8 / 32 rows: argmax of 128256 fp32
+// logits 5.2 -> 4.0, 5.5 -> 4.3, 6.3 -> 5.6, with a penalty over 256 ids 7.5 -> 5.4, 7.7 -> 5.7, 8.2 -> 7.2; top-k of 32064 with the
+// penalty 11.1 -> 8.3, 11.2 -> 8.7, 11.7 -> 9.0; of 151936 fp16 9.1 -> 8.3, 9.7 -> 8.7, 10.2 (as before).  The lines:
+//  * Top-k lists are merged four at a time by a wave, more through LDS: 7 of 8192 instead of 4 of 16384 logits, 1 x 50257 fp32 7.1 -> 7.7.
+//  * More workgroups than CUs, sixteen-bit top-k rows: 16384, whose kernel takes half the registers, so that two fit a CU
+//    (256 x 201088 55.2 -> 42.4, 64 x 151936 16.6 -> 14.6), but 32768 while that is a workgroup per CU (64 x 128256 10.3 against 11.3).
+//  * Argmax of more workgroups than CUs: 16384 up to two per CU (64 x 50257 fp16 7.2 -> 5.3) and where those of 32768 do not all run at
+//    once either (256 x 201088 fp16 23.7 -> 21.8, fp32 34.0 -> 33.0); in between some shapes gain and others lose (64 x 151936 fp16 0.91,
+//    128 x 128256 fp16 1.13).  Sixteen-bit rows with logits processing lose (256 x 128256 22.5 -> 25.9).
+//  * Numbered row by row, rows of an even number of chunks have their finishing workgroups on every other XCD, those of eight on one:
+//    many workgroups are numbered chunk by chunk (256 x 128256 fp16 36.1 -> 28.4, fp32 27.7 -> 26.8); few start and end in order with their
+//    rows side by side (64 x 128256 fp32 11.5, against 12.1).
+//  * A last chunk of few logits has them in few lanes, whose maxima bound nothing: rows are cut evenly then (64 x 50257 fp16 in chunks
+//    of 16384 24.2 -> 9.0, 64 x 33000 in chunks of 32768 23.5 -> 9.5).
+void PlanStream(const mi355x_search_ctx* ctx, ms::SampleArgs* a, bool small_k) {
+  const long long rows = a->rows;
+  const bool argmax = a->emit_topk == ms::kEmitArgmax, wide = a->dtype == MI355X_F32 || a->dtype == 0;
+  auto chunks_of = [&](int room) { return (a->vocab + room - 1) / room; };
+  const int quarters = chunks_of(ms::kSChunk / 4), halves = chunks_of(ms::kSChunk / 2), wholes = chunks_of(ms::kSChunk);
+  const int most = argmax ? 64 : ms::kStreamMaxChunks;  // lists a finishing workgroup takes
+  int room = ms::kSChunk;
+  if (small_k) {
+    if (quarters == 1 || (quarters <= most && (argmax || quarters <= 4 || halves > 4) && rows * quarters <= kPlanBlocks)) room = ms::kSChunk / 4;
+    else if (halves == 1 || (halves <= most && rows * halves <= kPlanBlocks)) room = ms::kSChunk / 2;
+    else if (argmax ? (wide || !a->xf.active()) && ((rows * halves <= 2 * kPlanBlocks && wholes > 1) || rows * wholes > 2 * kPlanBlocks)
+                    : !wide && rows * wholes > kPlanBlocks) room = halves <= most ? ms::kSChunk / 2 : ms::kSChunk;
+    if (static_cast<size_t>(rows) * chunks_of(room) > ctx->cand_lists) room = ms::kSChunk;
+  }
+  a->chunk_room = a->chunk_elems = room;
+  a->chunks = chunks_of(room);
+  if (!small_k) return;
+  const long long many = argmax ? (room < ms::kSChunk ? kPlanBlocks : 2 * kPlanBlocks) : 4 * kPlanBlocks - 1;
+  a->rows_first = rows * a->chunks > many ? 1 : 0;
+  const int last = a->vocab - (a->chunks - 1) * room;
+  if (last < room / 4) a->chunk_elems = ((a->vocab + a->chunks - 1) / a->chunks + 63) & ~63;
+}
+
 extern "C" {
 
 const char* mi355x_search_last_error(void) { return g_error.c_str(); }
@@ -236,7 +280,9 @@ int mi355x_search_create(int device, int max_rows, int max_vocab, mi355x_search_
   auto ok = [&](hipError_t r) {
     if (e == hipSuccess) e = r;
   };
-  const size_t sc = static_cast<size_t>(max_rows) * ((max_vocab + ms::kSChunk - 1) / ms::kSChunk);
+  size_t sc = static_cast<size_t>(max_rows) * ((max_vocab + ms::kSChunk / 2 - 1) / (ms::kSChunk / 2));
+  if (sc < static_cast<size_t>(kPlanBlocks)) sc = kPlanBlocks;  // (what PlanStream asks for at most)
+  c->cand_lists = sc;
   ok(c->Alloc(&c->cand_small, sc * ms::kSmallCap, true));  // all-zero between launches
   ok(c->Alloc(&c->chunk_cnt, rc, true));
   ok(c->Alloc(&c->chunk_max, rc, true));
@@ -327,8 +373,7 @@ int mi355x_argmax(mi355x_search_ctx* ctx, void* stream, const void* logits, int 
     return Fail(MI355X_E_UNSUPPORTED, "dtype %d not supported", dtype);
   if (row_stride < vocab) return Fail(MI355X_E_INVALID, "row_stride smaller than vocab");
   // rows of more than 64 logits go through the fused selection kernel (k = 1, ids only), whatever their type
-  const int fused_chunks = (vocab + ms::kSChunk - 1) / ms::kSChunk;
-  const bool fused = vocab > 64 && fused_chunks * ms::kSmallCap <= ms::kAllCap && rows * fused_chunks >= ms::kArgmaxFusedMinBlocks;
+  const bool fused = vocab > 64 && vocab <= ms::kStreamMaxVocab;
   if (fused) {
     hipStream_t s = static_cast<hipStream_t>(stream);
     ms::SampleArgs f{};
@@ -338,10 +383,10 @@ int mi355x_argmax(mi355x_search_ctx* ctx, void* stream, const void* logits, int 
     f.row_stride = row_stride;
     f.rows = rows;
     f.vocab = vocab;
-    f.chunks = fused_chunks;
     f.uniform = mi355x_sample_params{1, 0.0f, 1.0f};
     f.out_tokens = out_tokens;
     f.emit_topk = ms::kEmitArgmax;
+    PlanStream(ctx, &f, true);
     f.cand_small = ctx->cand_small;
     f.chunk_cnt = ctx->chunk_cnt;
     f.chunk_max = ctx->chunk_max;
@@ -427,18 +472,17 @@ int SampleImpl(mi355x_search_ctx* ctx, hipStream_t s, const void* logits, const 
   ms::SampleArgs a{};
   if (int r = MakeXform(ctx, xf, rows, vocab, s, &a.xf)) return r;
   bool any_nucleus = false, any_other = false, any_large_k = false, any_exact = false, any_wide = false;
-  const int chunks = (vocab + ms::kSChunk - 1) / ms::kSChunk;
   ms::InlineParams table{};
   bool use_table = false;
   // Sampling from the whole vocabulary is spread over the GPU wherever its kernels can take the row as it lies: no
   // logits processing, a row long enough to cut up, no more tiles than the finishing workgroup holds.
   const int tiles = (vocab + ms::kWideTile - 1) / ms::kWideTile;
-  const bool wide_fits = vocab >= ms::kWideMinVocab && tiles <= ms::kWideMaxTiles && chunks * ms::kSmallCap <= ms::kAllCap && !a.xf.active();
+  const bool wide_fits = vocab >= ms::kWideMinVocab && tiles <= ms::kWideMaxTiles && vocab <= ms::kStreamMaxVocab && !a.xf.active();
   auto check = [&](const mi355x_sample_params& p) -> int {
     if (!(p.temperature > 0.0f)) return Fail(MI355X_E_INVALID, "temperature must be positive (got %g)", p.temperature);
     // the kernels' own rule (row_mode) decides; these flags only have to cover it
     const int kk = p.k < vocab ? p.k : vocab;
-    const bool fits = vocab > 64 && chunks * ms::kSmallCap <= ms::kAllCap;
+    const bool fits = vocab > 64 && vocab <= ms::kStreamMaxVocab;
     const bool whole = p.k <= 1 && !(p.p < 1.0f);  // no top-k and no nucleus: the whole vocabulary
     const bool nucleus = p.k <= 1 && !whole, large_k = p.k > 1 && kk > 64 && kk <= ms::kLargeKMax;
     if (nucleus && vocab > 64) any_nucleus = true;
@@ -469,7 +513,6 @@ int SampleImpl(mi355x_search_ctx* ctx, hipStream_t s, const void* logits, const 
   a.row_stride = row_stride;
   a.rows = rows;
   a.vocab = vocab;
-  a.chunks = chunks;
   a.uniform = params;
   a.uniforms = uniforms;
   a.out_tokens = out_tokens;
@@ -489,6 +532,7 @@ int SampleImpl(mi355x_search_ctx* ctx, hipStream_t s, const void* logits, const 
   a.fallback_rows = ctx->fallback_rows;
   a.poll_limit = ctx->poll_limit;
   a.row_done = ctx->row_done;
+  PlanStream(ctx, &a, !any_nucleus && !any_large_k);
   a.exact_kernel = (any_exact ? ms::kExactRows : 0) | (any_wide ? ms::kWideRows : 0);
   const ms::WideArgs wide{(vocab + ms::kWideChunk - 1) / ms::kWideChunk, tiles, ctx->wide_rows, ctx->wide_tile_start, ctx->wide_cut_bucket, ctx->seg_sum,
                           ctx->seg_step, ctx->sub_step, ctx->sub_se, ctx->chunk_next, kept_ids == nullptr && kept_count == nullptr};
@@ -614,7 +658,6 @@ int mi355x_topk_scores(mi355x_search_ctx* ctx, void* stream, const void* logits,
   a.row_stride = row_stride;
   a.rows = rows;
   a.vocab = vocab;
-  a.chunks = (vocab + ms::kSChunk - 1) / ms::kSChunk;
   a.uniform = mi355x_sample_params{k, 0.0f, 1.0f};
   a.out_tokens = out_tokens;
   a.out_scores = out_scores;
@@ -632,10 +675,11 @@ int mi355x_topk_scores(mi355x_search_ctx* ctx, void* stream, const void* logits,
   // up to 64: the fused kernel's sorted candidate lists; up to kLargeKMax: the candidate lists of the large-k
   // sampling route with an epilogue that emits instead of drawing; beyond (and for rows of more chunks than a
   // finishing workgroup ranks): the exact path's whole-row sort.  The kernels' own rule (row_mode) decides.
-  const bool fits = vocab > 64 && a.chunks * ms::kSmallCap <= ms::kAllCap;
+  const bool fits = vocab > 64 && vocab <= ms::kStreamMaxVocab;
   const bool large_k = fits && k > 64 && k <= ms::kLargeKMax;
   const bool exact = vocab > 64 && (!fits || k > ms::kLargeKMax);
   a.exact_kernel = exact ? ms::kExactRows : 0;
+  PlanStream(ctx, &a, !large_k);
   HIP_TRY(ms_launch_sample(&a, nullptr, !large_k && !exact, false, large_k, s, nullptr));
   return MI355X_OK;
 }

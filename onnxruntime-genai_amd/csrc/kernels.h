@@ -5,11 +5,12 @@
 
 namespace ms {
 
-// Shape of the fused sampling kernel: 512 threads x 16 float4 = one 32K-logit chunk per workgroup.
+// Shape of the fused sampling kernel: 512 threads x 16 float4 = one 32K-logit chunk per workgroup, or 8 or 4 float4
+// where the GPU has a CU for more workgroups than that makes (PlanStream has the rule and the figures).
 // Many logits per lane keep the per-wave selection overhead small against the streaming work, few
 // chunks per row keep the finishing merge shallow (a 128K vocabulary is four sorted lists, two merge
 // levels), and thread t's float4s (t, t+512, t+1024, ...) make every wave an even sample of the chunk.
-constexpr int kSChunk = 32768;        // logits per workgroup of the streaming kernels
+constexpr int kSChunk = 32768;        // logits per workgroup of the streaming kernels; those of top-k and argmax rows also come for 16384 and 8192
 constexpr int kTopkBlock = 512;       // threads of a workgroup that streams a top-k row (16 128-bit loads each) ...
 constexpr int kNucleusBlock = 1024;   // ... and a nucleus row (8 each: lighter threads, twice the waves in flight)
 constexpr int kSMaxWaves = 16;
@@ -18,12 +19,12 @@ constexpr int kSMaxWaves = 16;
 constexpr int kDefaultPollLimit = 1 << 21;
 constexpr int kSmallCap = 64;        // sorted candidates a chunk publishes on the k<=64 path
 constexpr int kListCap = 128;        // candidates a chunk can hold before its sort
-constexpr int kAllCap = 1024;        // slots a finishing workgroup ranks (16 chunks x kSmallCap)
+constexpr int kStreamMaxChunks = 16;  // whose lists a finishing workgroup merges
+constexpr int kStreamMaxVocab = kStreamMaxChunks * kSChunk;  // longer rows take the exact path
 constexpr int kNucleusCap = 16384;   // sorted nucleus candidates held in LDS by the finish kernel
 constexpr int kFinishBlock = 1024;
 
 constexpr int kEmitArgmax = 2;
-constexpr int kArgmaxFusedMinBlocks = 1;  // rows x 32768-id chunks from which mi355x_argmax uses the fused kernel
 constexpr int kExactRows = 1, kWideRows = 2;  // SampleArgs::exact_kernel: the one-workgroup kernel / the kernels of wide_rows.h
 constexpr int kModeTopkSmall = 0;
 constexpr int kModeNucleus = 1;
@@ -48,6 +49,8 @@ struct SampleArgs {
   const void* logits;   // rows of fp32, fp16 or bf16 values (dtype), row_stride elements apart
   int64_t row_stride;
   int rows, vocab, chunks;
+  int chunk_room, chunk_elems;  // top-k and argmax rows: logits a workgroup of the kernel has room for, and those of a chunk (a multiple of 64)
+  int rows_first;       // ... not 0: workgroups are numbered chunk by chunk, the rows of one chunk side by side
   int dtype;            // MI355X_F32 / MI355X_F16 / MI355X_BF16 (0 counts as fp32)
   Xform xf;
   mi355x_sample_params uniform;

@@ -861,7 +861,7 @@ __device__ __forceinline__ void nucleus_finish_body(const SampleArgs& a) {
   const int V = a.vocab;
   const int tid = threadIdx.x;
   const mi355x_sample_params prm = row_params<INLINE>(a, row);
-  const int mode = MODE == kFinishMixed ? row_mode_of_mixed(prm, V, a.chunks) : row_mode(prm, V, a.chunks, a.emit_topk);
+  const int mode = MODE == kFinishMixed ? row_mode_of_mixed(prm, V) : row_mode(prm, V, a.emit_topk);
   if (MODE == kFinishMixed ? mode != kModeTopkLarge && mode != kModeNucleus : mode != (MODE == kFinishLargeK ? kModeTopkLarge : kModeNucleus)) return;
   // a large-k row: then every listed element is a candidate and no element after them is needed
   const bool large_k = MODE == kFinishMixed ? mode == kModeTopkLarge : MODE == kFinishLargeK;
@@ -908,11 +908,11 @@ __device__ __forceinline__ void nucleus_finish_body(const SampleArgs& a) {
   // Lane c of every wave reads what chunk c left behind (at most 16 chunks), so the row's maximum and threshold
   // are reductions inside the wave, with no exchange between the waves; wave 0 publishes the counts and where
   // every list's rows begin, behind the one barrier that follows.
-  __shared__ uint32_t sh_cnt[kAllCap / kSmallCap];       // candidates per chunk
-  __shared__ uint32_t sh_first[kAllCap / kSmallCap + 1];  // rows of kFinishBlock entries the lists past their heads take, prefix sums
+  __shared__ uint32_t sh_cnt[kStreamMaxChunks];       // candidates per chunk
+  __shared__ uint32_t sh_first[kStreamMaxChunks + 1];  // rows of kFinishBlock entries the lists past their heads take, prefix sums
   __shared__ int sh_trim;
   __shared__ uint32_t sh_head, sh_all;
-  static_assert(kAllCap / kSmallCap < 64, "a lane per chunk, and one more");
+  static_assert(kStreamMaxChunks < 64, "a lane per chunk, and one more");
   const int lane = lane_id();
   uint32_t cnt = 0u, m = 0u, cthr = 0u;
   u64 best_below = 0;
@@ -1573,7 +1573,7 @@ __device__ __forceinline__ int nucleus_sparse_body(const SampleArgs& a) {
   if (PICK && tid < 32) exp_tab[tid] = em::exp2_tab(static_cast<uint32_t>(tid));  // (barriers follow before it is used)
   const int V = a.vocab;
   const mi355x_sample_params prm = row_params<INLINE>(a, row);
-  if (row_mode(prm, V, a.chunks) != kModeNucleus) return -1;
+  if (row_mode(prm, V) != kModeNucleus) return -1;
   const int words = (V - 1) / 32 + 1;
   const void* const row0 = row_start<INLINE>(a, row, dtype_bytes(a.dtype));
   // A row this kernel cannot finish is left to the dense kernels launched after it -- or, when the caller's
@@ -1983,7 +1983,7 @@ __device__ __forceinline__ void exact_rows_body(const SampleArgs& a) {
   __shared__ u64 red64[16];
   const int row = blockIdx.x;
   const mi355x_sample_params prm = row_params<INLINE>(a, row);
-  if (row_mode(prm, a.vocab, a.chunks, a.emit_topk) != kModeGeneral) return;
+  if (row_mode(prm, a.vocab, a.emit_topk) != kModeGeneral) return;
   if ((a.exact_kernel & kWideRows) && wide_row(prm)) return;
   general_row<AnyDtype, SortWithTile, 8>(a, row, row_start<INLINE>(a, row, dtype_bytes(a.dtype)), prm, a.big + static_cast<size_t>(row) * a.big_stride,
                         seqsh,

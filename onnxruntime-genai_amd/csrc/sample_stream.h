@@ -1,7 +1,7 @@
 // Streaming kernels of the sampling path (templates; a source file per element type instantiates them).
 //
-// sample_fused_kernel (top-k rows, k <= 64; one launch per step): every workgroup (512 threads x 64
-// logits) streams one 32K-logit chunk of one row with 128-bit non-temporal loads, logits processing
+// sample_fused_kernel (top-k rows, k <= 64; one launch per step): every workgroup (512 threads x 16, 32 or 64
+// logits, see StreamPlan) streams one chunk of one row with 128-bit non-temporal loads, logits processing
 // fused, keeps the chunk's best 64 candidates and publishes them sorted; the workgroup of a row's last
 // chunk polls for the other chunks' lists, merges them four at a time (bitonic merges in registers)
 // and runs the reference's scalar epilogue (softmax over the k, nucleus cut, categorical draw) in rank
@@ -271,8 +271,8 @@ __device__ __forceinline__ void general_row(const SampleArgs& a, int row, const 
   if (threadIdx.x == 0) atomicAdd(a.fallback_rows, 1u);
 }
 
-__device__ __forceinline__ int row_mode(mi355x_sample_params prm, int vocab, int chunks, int emit_topk = 0) {
-  if (vocab <= 64 || chunks * kSmallCap > kAllCap) return kModeGeneral;
+__device__ __forceinline__ int row_mode(mi355x_sample_params prm, int vocab, int emit_topk = 0) {
+  if (vocab <= 64 || vocab > kStreamMaxVocab) return kModeGeneral;
   if (emit_topk == kEmitArgmax) return kModeTopkSmall;
   if (prm.k > 1 || emit_topk) {
     const int kk = prm.k < vocab ? prm.k : vocab;
@@ -283,8 +283,8 @@ __device__ __forceinline__ int row_mode(mi355x_sample_params prm, int vocab, int
 }
 
 // The same for a call whose rows are in several modes (see mixed_stream_body).
-__device__ __forceinline__ int row_mode_of_mixed(mi355x_sample_params prm, int vocab, int chunks) {
-  const int mode = row_mode(prm, vocab, chunks);
+__device__ __forceinline__ int row_mode_of_mixed(mi355x_sample_params prm, int vocab) {
+  const int mode = row_mode(prm, vocab);
   return mode == kModeTopkSmall ? kModeTopkLarge : mode;
 }
 
@@ -326,7 +326,7 @@ struct FusedShared {
   u64 wave_list[kSMaxWaves * kWaveListCap];  // each wave's hits of this chunk, before the sort
   u64 list_hi[64];          // second half of a long list, sorted ascending
   u64 own[64];              // the finishing workgroup's own list
-  u64 lists[kAllCap / 4];   // first-level results of the finishing workgroup's merge (rows of > 4 chunks)
+  u64 lists[kStreamMaxChunks * kSmallCap / 4];   // first-level results of the finishing workgroup's merge (rows of > 4 chunks)
   uint32_t pool[64];
   uint32_t poisoned;              // the workgroup's copy of the flag that sends every row to the exact path
   uint32_t n_hits;                // hits of the chunk on the ranking route of the top-k rows
@@ -347,10 +347,10 @@ template <int BLOCK, int VEC>
 __device__ __forceinline__ constexpr int elem_offset(int e) {
   return (e / VEC) * BLOCK * VEC + e % VEC;
 }
-// Vocabulary id of element c of the thread's quad q (registers 4q .. 4q+3).
+// Vocabulary id of element c of the thread's quad q (registers 4q .. 4q+3) of a chunk that begins with id `base`.
 template <int BLOCK, int VEC>
-__device__ __forceinline__ int elem_index(int chunk, int q, int c) {
-  return chunk * kSChunk + static_cast<int>(threadIdx.x) * VEC + elem_offset<BLOCK, VEC>(q * 4 + c);
+__device__ __forceinline__ int elem_index(int base, int q, int c) {
+  return base + static_cast<int>(threadIdx.x) * VEC + elem_offset<BLOCK, VEC>(q * 4 + c);
 }
 
 // The 32-entry table of expf_core, one entry per lane (lane & 31), fetched by lane shuffle.
@@ -587,10 +587,10 @@ __device__ __forceinline__ uint32_t block_kth_largest(const uint32_t (&offer)[N]
 // Applies the two LDS bitmaps of a chunk to the registers of a thread: an id whose bit in `allowed` is
 // clear becomes kLowest, an id whose bit in `history` is set becomes NaN (its processed value lives in
 // the extras list).  Branch-free: the bit, spread over a word, selects between the two bit patterns.
-template <int kSBlock, int VEC, bool ALLOWED, bool HISTORY>
-__device__ __forceinline__ void mask_registers(float (&v)[kSChunk / kSBlock], const uint32_t* allowed,
+template <int CHUNK, int kSBlock, int VEC, bool ALLOWED, bool HISTORY>
+__device__ __forceinline__ void mask_registers(float (&v)[CHUNK / kSBlock], const uint32_t* allowed,
                                                const uint32_t* history, int tid) {
-  constexpr int kSVec = kSChunk / (kSBlock * 4);
+  constexpr int kSVec = CHUNK / (kSBlock * 4);
 #pragma unroll
   for (int j = 0; j < kSVec; ++j) {
     const int rel0 = tid * VEC + elem_offset<kSBlock, VEC>(j * 4);
@@ -616,16 +616,19 @@ __device__ __forceinline__ void mask_registers(float (&v)[kSChunk / kSBlock], co
 
 // Streaming pass of one (row, chunk) of a top-k<=64 or nucleus row.  Returns true when this workgroup
 // must run the general path for the row (it was the last to arrive and the fast path declined).
-template <typename InT, bool NUCLEUS, bool XFORM, bool LARGEK = false, bool ARGMAX = false>
+// CHUNK: the logits the workgroup has room for.  A nucleus row's chunks have that many each, the others' chunk_elems.
+template <typename InT, int CHUNK, bool NUCLEUS, bool XFORM, bool LARGEK = false, bool ARGMAX = false>
 __device__ __forceinline__ bool stream_row(const SampleArgs& a, int row, const void* row0, int chunk,
                                            mi355x_sample_params prm, FusedShared& sm) {
   constexpr int kSBlock = NUCLEUS ? kNucleusBlock : kTopkBlock;  // threads of this workgroup
   constexpr int kSWaves = kSBlock / 64;
-  constexpr int kSVec = kSChunk / (kSBlock * 4);  // quads of logits per thread (fp32 rows: its 128-bit loads)
+  constexpr int kSVec = CHUNK / (kSBlock * 4);  // quads of logits per thread (fp32 rows: its 128-bit loads)
   constexpr int kSElems = kSVec * 4;              // logits held in registers per thread
   constexpr int VEC = 16 / static_cast<int>(sizeof(InT));  // logits per 128-bit load
   constexpr int kSLoads = kSElems / VEC;                   // 128-bit loads per thread
   const int V = a.vocab;
+  const int base = chunk * (NUCLEUS ? CHUNK : a.chunk_elems);  // the chunk's first id
+  const int end = NUCLEUS ? V : (V - base < a.chunk_elems ? V : base + a.chunk_elems);  // (no id from there on is the chunk's)
   const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6;
   u64* big_row = a.big + static_cast<size_t>(row) * a.big_stride;
   const InT* lrow = static_cast<const InT*>(row0);
@@ -637,8 +640,8 @@ __device__ __forceinline__ bool stream_row(const SampleArgs& a, int row, const v
   // The bitmap words and the first history ids of this thread are requested before the logits: loads come back in
   // the order they were asked for, and the history has a chain of its own to start (mark the ids, read their logits
   // again, penalise them) that should run while the logits arrive, not after them.
-  constexpr int kWordsPerThread = kSChunk / 32 / kSBlock;  // bitmap words a thread stages
-  static_assert(kWordsPerThread >= 1 && kSChunk / 32 == kWordsPerThread * kSBlock, "whole bitmap words per thread");
+  constexpr int kWordsPerThread = (CHUNK / 32 + kSBlock - 1) / kSBlock;  // bitmap words a thread stages (some past a short chunk's, which nobody reads)
+  static_assert(kWordsPerThread * kSBlock <= kSChunk / 32, "the bitmaps have room for every thread's words");
   const bool active = XFORM && a.xf.active();  // kernels without logits processing carry none of its code
   const bool pen = active && a.xf.use_penalty();
   const bool has_mask = active && a.xf.mask != nullptr;
@@ -674,7 +677,7 @@ __device__ __forceinline__ bool stream_row(const SampleArgs& a, int row, const v
   for (int q = 0; q < kWordsPerThread; ++q) {
     mask_pre[q] = ~0u;
     if (has_mask) {
-      const int w = chunk * (kSChunk / 32) + tid + q * kSBlock;
+      const int w = base / 32 + tid + q * kSBlock;
       mask_pre[q] = w < words ? mrow[w] : 0u;
     }
   }
@@ -710,11 +713,11 @@ __device__ __forceinline__ bool stream_row(const SampleArgs& a, int row, const v
 #pragma unroll
     for (int q = 0; q < kWordsPerThread; ++q) {
       const int i = tid + q * kSBlock;
-      const int w = chunk * (kSChunk / 32) + i;
+      const int w = base / 32 + i;
       uint32_t word = mask_pre[q];
       for (int e = 0; e < n_eos; ++e)
         if ((a.xf.eos[e] >> 5) == w) word &= ~(1u << (a.xf.eos[e] & 31));
-      const int n_real = V - w * 32;  // ids of this word inside the vocabulary
+      const int n_real = end - w * 32;  // ids of this word inside the chunk
       if (n_real < 32) word |= n_real <= 0 ? ~0u : (~0u << n_real);
       sm.mask_bits[i] = word;
       sm.hist_bits[i] = 0u;
@@ -726,8 +729,8 @@ __device__ __forceinline__ bool stream_row(const SampleArgs& a, int row, const v
       const uint32_t* ban_row = a.xf.ban_row(row, V);
       // the thread that is first to mark an id computes its processed value
       auto visit = [&](int id) {
-        const int rel = id - chunk * kSChunk;
-        if (rel >= 0 && rel < kSChunk && id < V) {
+        const int rel = id - base;
+        if (rel >= 0 && (!NUCLEUS || rel < CHUNK) && id < end) {
           const uint32_t bit = 1u << (rel & 31);
           if (!(atomicOr(&sm.hist_bits[rel >> 5], bit) & bit)) {
             const uint32_t slot = atomicAdd(&sm.n_extra, 1u);
@@ -755,7 +758,7 @@ __device__ __forceinline__ bool stream_row(const SampleArgs& a, int row, const v
     }
   };
   // a chunk that lies inside its row requests its loads without a test between them
-  const bool whole_chunk = (chunk + 1) * kSChunk <= V;
+  const bool whole_chunk = base + CHUNK <= end;
   if constexpr (kOneRun) {
     // Kernels with logits processing request the loads of a chunk in one straight run, whatever the row's end and
     // wherever the row starts: 128-bit loads that only need their elements' alignment (the hardware reads from any
@@ -768,8 +771,8 @@ __device__ __forceinline__ bool stream_row(const SampleArgs& a, int row, const v
     // waits for everything -- so that the preparations would start when the logits are there.
 #pragma unroll
     for (int j = 0; j < kSLoads; ++j) {
-      const int i0 = elem_index<kSBlock, VEC>(chunk, j, 0);
-      const int from = i0 + 4 <= V ? i0 : (i0 < V ? V - 4 : 0);
+      const int i0 = elem_index<kSBlock, VEC>(base, j, 0);
+      const int from = i0 + 4 <= end ? i0 : (i0 < end ? end - 4 : 0);
       const v4f_any q = __builtin_nontemporal_load(reinterpret_cast<const v4f_any*>(lrow + from));
       v[j * 4 + 0] = q.x;
       v[j * 4 + 1] = q.y;
@@ -779,7 +782,7 @@ __device__ __forceinline__ bool stream_row(const SampleArgs& a, int row, const v
     xform_prep();
   } else if constexpr (VEC == 4) {
     if (whole_chunk) {
-      const v4f_any* src = reinterpret_cast<const v4f_any*>(lrow + static_cast<size_t>(chunk) * kSChunk) + tid;
+      const v4f_any* src = reinterpret_cast<const v4f_any*>(lrow + base) + tid;
 #pragma unroll
       for (int j = 0; j < kSLoads; ++j) {
         const v4f_any q = __builtin_nontemporal_load(src + j * kSBlock);
@@ -797,8 +800,8 @@ __device__ __forceinline__ bool stream_row(const SampleArgs& a, int row, const v
       for (int e = 0; e < kSElems; ++e) asm volatile("v_mov_b32 %0, 0x7fc00000" : "=v"(v[e]));
 #pragma unroll
       for (int j = 0; j < kSLoads; ++j) {
-        const int i0 = elem_index<kSBlock, VEC>(chunk, j, 0);
-        if (i0 + 4 <= V) {
+        const int i0 = elem_index<kSBlock, VEC>(base, j, 0);
+        if (i0 + 4 <= end) {
           const v4f_any q = __builtin_nontemporal_load(reinterpret_cast<const v4f_any*>(lrow + i0));
           v[j * 4 + 0] = q.x;
           v[j * 4 + 1] = q.y;
@@ -806,14 +809,14 @@ __device__ __forceinline__ bool stream_row(const SampleArgs& a, int row, const v
           v[j * 4 + 3] = q.w;
         }
       }
-      if ((V & 3) != 0) {
+      if ((end & 3) != 0) {
 #pragma unroll
         for (int j = 0; j < kSLoads; ++j) {
-          const int i0 = elem_index<kSBlock, VEC>(chunk, j, 0);
-          if (i0 < V && i0 + 4 > V) {
+          const int i0 = elem_index<kSBlock, VEC>(base, j, 0);
+          if (i0 < end && i0 + 4 > end) {
 #pragma unroll
             for (int c = 0; c < 3; ++c)
-              if (i0 + c < V) v[j * 4 + c] = load_one<InT>(lrow, i0 + c);
+              if (i0 + c < end) v[j * 4 + c] = load_one<InT>(lrow, i0 + c);
           }
         }
       }
@@ -830,14 +833,14 @@ __device__ __forceinline__ bool stream_row(const SampleArgs& a, int row, const v
       if (!whole_chunk) {  // (ahead of the run, which so is the same number of requests for every chunk)
 #pragma unroll
         for (int c = 0; c < VEC - 1; ++c) {
-          const int i = (V & ~(VEC - 1)) + c;
-          row_end[c] = load_one<InT>(lrow, i < V ? i : 0);
+          const int i = (end & ~(VEC - 1)) + c;
+          row_end[c] = load_one<InT>(lrow, i < end ? i : 0);
         }
       }
 #pragma unroll
       for (int j = 0; j < kSLoads; ++j) {
-        const int i0 = elem_index<kSBlock, VEC>(chunk, 2 * j, 0);
-        raw[j] = __builtin_nontemporal_load(reinterpret_cast<const v4u_any*>(lrow + (i0 + VEC <= V ? i0 : 0)));
+        const int i0 = elem_index<kSBlock, VEC>(base, 2 * j, 0);
+        raw[j] = __builtin_nontemporal_load(reinterpret_cast<const v4u_any*>(lrow + (i0 + VEC <= end ? i0 : 0)));
       }
       xform_prep();
 #pragma unroll
@@ -846,12 +849,12 @@ __device__ __forceinline__ bool stream_row(const SampleArgs& a, int row, const v
         else widen_bf16x8(raw[j], &v[j * VEC]);
       }
       if (!whole_chunk) {
-        const int r = V & (VEC - 1);  // elements of the straddling group that lie inside the row
+        const int r = end & (VEC - 1);  // elements of the straddling group that lie inside the row
 #pragma unroll
         for (int j = 0; j < kSLoads; ++j) {
-          const int i0 = elem_index<kSBlock, VEC>(chunk, 2 * j, 0);
-          if (i0 + VEC > V) {
-            const bool straddles = i0 < V;
+          const int i0 = elem_index<kSBlock, VEC>(base, 2 * j, 0);
+          if (i0 + VEC > end) {
+            const bool straddles = i0 < end;
 #pragma unroll
             for (int c = 0; c < VEC; ++c) v[j * VEC + c] = (straddles && c < r) ? row_end[c < VEC - 1 ? c : 0] : kNaN;
           }
@@ -862,21 +865,21 @@ __device__ __forceinline__ bool stream_row(const SampleArgs& a, int row, const v
       uint32_t whole = 0u;  // bit j: load j lies inside the row
 #pragma unroll
       for (int j = 0; j < kSLoads; ++j) {
-        const int i0 = elem_index<kSBlock, VEC>(chunk, 2 * j, 0);
-        if (i0 + VEC <= V) {
+        const int i0 = elem_index<kSBlock, VEC>(base, 2 * j, 0);
+        if (i0 + VEC <= end) {
           raw[j] = __builtin_nontemporal_load(reinterpret_cast<const v4u_any*>(lrow + i0));
           whole |= 1u << j;
         }
       }
 #pragma unroll
       for (int j = 0; j < kSLoads; ++j) {
-        const int i0 = elem_index<kSBlock, VEC>(chunk, 2 * j, 0);
+        const int i0 = elem_index<kSBlock, VEC>(base, 2 * j, 0);
         if ((whole >> j) & 1u) {
           if constexpr (sizeof(InT) == 2 && !__is_same(InT, bf16_t)) widen_half8(raw[j], &v[j * VEC]);
           else widen_bf16x8(raw[j], &v[j * VEC]);
         } else {
 #pragma unroll
-          for (int c = 0; c < VEC; ++c) v[j * VEC + c] = (i0 + c < V) ? load_one<InT>(lrow, i0 + c) : kNaN;
+          for (int c = 0; c < VEC; ++c) v[j * VEC + c] = (i0 + c < end) ? load_one<InT>(lrow, i0 + c) : kNaN;
         }
       }
     }
@@ -903,9 +906,9 @@ __device__ __forceinline__ bool stream_row(const SampleArgs& a, int row, const v
       if (!whole_chunk) {
 #pragma unroll
         for (int j = 0; j < kSLoads; ++j) {
-          const int i0 = elem_index<kSBlock, VEC>(chunk, j, 0);
-          if (i0 + 4 > V) {  // elements V-4 .. V-1 in the registers where i0 .. V-1 belong, or nothing of the row
-            const int r = i0 < V ? V - i0 : 0;  // elements of the quad that lie inside the row
+          const int i0 = elem_index<kSBlock, VEC>(base, j, 0);
+          if (i0 + 4 > end) {  // elements end-4 .. end-1 in the registers where i0 .. end-1 belong, or nothing of the chunk
+            const int r = i0 < end ? end - i0 : 0;  // elements of the quad that lie inside the chunk
             const float q1 = v[j * 4 + 1], q2 = v[j * 4 + 2], q3 = v[j * 4 + 3];
             v[j * 4 + 0] = r == 0 ? kNaN : (r == 1 ? q3 : (r == 2 ? q2 : q1));
             v[j * 4 + 1] = r < 2 ? kNaN : (r == 2 ? q3 : q2);
@@ -917,8 +920,8 @@ __device__ __forceinline__ bool stream_row(const SampleArgs& a, int row, const v
     }
     if (active) {
       // without a grammar mask and without EOS masking every id is allowed (ids past the vocabulary are NaN already)
-      if (has_mask || n_eos_row > 0) mask_registers<kSBlock, VEC, true, true>(v, sm.mask_bits, sm.hist_bits, tid);
-      else mask_registers<kSBlock, VEC, false, true>(v, sm.mask_bits, sm.hist_bits, tid);
+      if (has_mask || n_eos_row > 0) mask_registers<CHUNK, kSBlock, VEC, true, true>(v, sm.mask_bits, sm.hist_bits, tid);
+      else mask_registers<CHUNK, kSBlock, VEC, false, true>(v, sm.mask_bits, sm.hist_bits, tid);
     }
   }
   // per-thread maximum in the float domain (fmaxf skips NaN), keeping the maximum of every float4
@@ -931,7 +934,7 @@ __device__ __forceinline__ bool stream_row(const SampleArgs& a, int row, const v
   }
   for (uint32_t i = tid; i < n_extra; i += kSBlock) fm = fmaxf(fm, sm.extra_val[i]);
   // 0: the thread holds no element
-  const uint32_t lmax = (elem_index<kSBlock, VEC>(chunk, 0, 0) < V || static_cast<uint32_t>(tid) < n_extra) ? order_key(fm) : 0u;
+  const uint32_t lmax = (elem_index<kSBlock, VEC>(base, 0, 0) < end || static_cast<uint32_t>(tid) < n_extra) ? order_key(fm) : 0u;
   if (tid == 0) {
     sm.count = 0u;
     if constexpr (!NUCLEUS) {
@@ -951,7 +954,7 @@ __device__ __forceinline__ bool stream_row(const SampleArgs& a, int row, const v
     // Rows with 64 < k <= kLargeKMax come here too: their candidates are the elements that reach the
     // k-th best of the chunk's per-thread maxima (or, for larger k, of the maxima of the quarters of every thread's
     // elements: at least k elements do; with fewer than k numbers, all), which contain the chunk's k best.
-    static_assert(kLargeKOneOffer <= kSBlock && 4 * kLargeKOneOffer <= 4 * kSBlock && kLargeKMax <= kSChunk && kSElems % 4 == 0,
+    static_assert(kLargeKOneOffer <= kSBlock && 4 * kLargeKOneOffer <= 4 * kSBlock && kLargeKMax <= CHUNK && kSElems % 4 == 0,
                   "one offer per thread, four, or every element");
     static_assert(sizeof(sm.wave_list) >= kKthBinWords * sizeof(uint32_t) && kSBlock >= 256, "the selection's bins lie in the hit lists' LDS");
     constexpr bool large_k = LARGEK;
@@ -1044,10 +1047,10 @@ __device__ __forceinline__ bool stream_row(const SampleArgs& a, int row, const v
     // into order keys.  The compares are made afresh against a copy of the threshold the compiler
     // cannot identify with the first one, so that the 64 lane masks of the first pass need not stay
     // alive.  Nothing below waits for the stores.
-    char* const dst = reinterpret_cast<char*>(big_row + static_cast<size_t>(chunk) * kSChunk);
+    char* const dst = reinterpret_cast<char*>(big_row + static_cast<size_t>(chunk) * CHUNK);
     float thr2 = thr;
     asm volatile("" : "+v"(thr2));
-    const uint32_t nid0 = ~static_cast<uint32_t>(elem_index<kSBlock, VEC>(chunk, 0, 0));  // ~(id0 + d) = ~id0 - d
+    const uint32_t nid0 = ~static_cast<uint32_t>(elem_index<kSBlock, VEC>(base, 0, 0));  // ~(id0 + d) = ~id0 - d
 #pragma unroll
     for (int e = 0; e < kSElems; ++e) {
       const bool cand = v[e] >= thr2;
@@ -1103,7 +1106,7 @@ __device__ __forceinline__ bool stream_row(const SampleArgs& a, int row, const v
 #pragma unroll
           for (int e = kSElems - 1; e >= 0; --e)
             if (v[e] == bbf) fe = e;
-          const u64 key = make_key64(wbk, static_cast<uint32_t>(elem_index<kSBlock, VEC>(chunk, fe >> 2, fe & 3)));
+          const u64 key = make_key64(wbk, static_cast<uint32_t>(elem_index<kSBlock, VEC>(base, fe >> 2, fe & 3)));
           best_below = key > best_below ? key : best_below;
         }
       }
@@ -1146,7 +1149,7 @@ __device__ __forceinline__ bool stream_row(const SampleArgs& a, int row, const v
     if (cmax != 0u) {
       const float cf = key_to_float(cmax);
       if (__ballot(fm == cf) != 0ull) {
-        const uint32_t wave_id0 = static_cast<uint32_t>(chunk) * kSChunk +
+        const uint32_t wave_id0 = static_cast<uint32_t>(base) +
                                   static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(wave)) * 64u * VEC;
         u64 qe[kSVec];
 #pragma unroll
@@ -1223,8 +1226,7 @@ __device__ __forceinline__ bool stream_row(const SampleArgs& a, int row, const v
   }
   // ---- top-k, k <= 64 ---------------------------------------------------------------------------
   const int kk = prm.k < V ? prm.k : V;
-  int n_valid = V - chunk * kSChunk;
-  if (n_valid > kSChunk) n_valid = kSChunk;
+  const int n_valid = end - base;
   int n_lanes = n_valid >= VEC * kSBlock ? kSBlock : (n_valid + VEC - 1) / VEC;  // threads that hold elements
   if (static_cast<uint32_t>(n_lanes) < n_extra) n_lanes = n_extra < static_cast<uint32_t>(kSBlock) ? static_cast<int>(n_extra) : kSBlock;
   const size_t ci = static_cast<size_t>(row) * n_chunks + chunk;
@@ -1274,7 +1276,7 @@ __device__ __forceinline__ bool stream_row(const SampleArgs& a, int row, const v
             // listed with the raw float bits; the few entries that survive get their order keys later
             if (pos < kWaveListCap)
               sm.wave_list[wave * kWaveListCap + pos] =
-                  make_key64(__float_as_uint(v[j * 4 + c]), static_cast<uint32_t>(elem_index<kSBlock, VEC>(chunk, j, c)));
+                  make_key64(__float_as_uint(v[j * 4 + c]), static_cast<uint32_t>(elem_index<kSBlock, VEC>(base, j, c)));
           }
           woff += static_cast<uint32_t>(__popcll(b));
         }
@@ -1375,7 +1377,7 @@ __device__ __forceinline__ bool stream_row(const SampleArgs& a, int row, const v
       }
     };
     static_assert(VEC == 4 || VEC == 8, "a lane's run of ids is a shift of its number");
-    const uint32_t wave_id0 = static_cast<uint32_t>(chunk) * kSChunk +
+    const uint32_t wave_id0 = static_cast<uint32_t>(base) +
                               static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(wave)) * 64u * VEC;
 #pragma unroll
     for (int j = 0; j < kSVec; ++j) {
@@ -1628,26 +1630,26 @@ __device__ __forceinline__ mi355x_sample_params args_up_front(const SampleArgs& 
   return q;
 }
 
-template <typename InT, bool INLINE, bool NUCLEUS, bool XFORM, bool LARGEK = false, bool ARGMAX = false>
+template <typename InT, int CHUNK, bool INLINE, bool NUCLEUS, bool XFORM, bool LARGEK = false, bool ARGMAX = false>
 __device__ __forceinline__ void sample_fused_body(const SampleArgs& a) {
   const mi355x_sample_params uniform_prm = args_up_front<XFORM>(a);
-  const int row = blockIdx.y, chunk = blockIdx.x;
+  const int row = !NUCLEUS && a.rows_first ? blockIdx.x : blockIdx.y, chunk = !NUCLEUS && a.rows_first ? blockIdx.y : blockIdx.x;
   __shared__ FusedShared sm;
   const mi355x_sample_params prm = row_params<INLINE>(a, row, uniform_prm);
   const void* const row0 = row_start<INLINE>(a, row, sizeof(InT));
-  const int mode = row_mode(prm, a.vocab, a.chunks, a.emit_topk);
+  const int mode = row_mode(prm, a.vocab, a.emit_topk);
   if constexpr (NUCLEUS) {
     if (mode == (LARGEK ? kModeTopkLarge : kModeNucleus)) {
       if constexpr (XFORM && !LARGEK) {
         if (a.xf.mask && a.row_done && a.row_done[row] != 0u) return;  // finished by the sparse-mask kernel
       }
-      stream_row<InT, true, XFORM, LARGEK>(a, row, row0, chunk, prm, sm);
+      stream_row<InT, CHUNK, true, XFORM, LARGEK>(a, row, row0, chunk, prm, sm);
     }
   } else {
     if (mode == kModeNucleus || mode == kModeTopkLarge) return;
     if (mode == kModeGeneral) {
       if (chunk != 0 || a.exact_kernel) return;  // exact_kernel: the exact-rows kernel sorts such rows much faster
-    } else if (!stream_row<InT, false, XFORM, false, ARGMAX>(a, row, row0, chunk, prm, sm)) {
+    } else if (!stream_row<InT, CHUNK, false, XFORM, false, ARGMAX>(a, row, row0, chunk, prm, sm)) {
       return;
     }
     // Rows the fast paths decline end here, in the exact general path (a single inlined call site keeps
@@ -1671,27 +1673,28 @@ __device__ __forceinline__ void mixed_stream_body(const SampleArgs& a) {
   __shared__ FusedShared sm;
   const mi355x_sample_params prm = row_params<INLINE>(a, row, uniform_prm);
   const void* const row0 = row_start<INLINE>(a, row, sizeof(InT));
-  const int mode = row_mode_of_mixed(prm, a.vocab, a.chunks);
+  const int mode = row_mode_of_mixed(prm, a.vocab);
   if (mode == kModeNucleus) {
     if constexpr (XFORM) {
       if (a.xf.mask && a.row_done && a.row_done[row] != 0u) return;  // finished by the sparse-mask kernel
     }
-    stream_row<InT, true, XFORM, false>(a, row, row0, chunk, prm, sm);
+    stream_row<InT, kSChunk, true, XFORM, false>(a, row, row0, chunk, prm, sm);
   } else if (mode == kModeTopkLarge) {
-    stream_row<InT, true, XFORM, true>(a, row, row0, chunk, prm, sm);
+    stream_row<InT, kSChunk, true, XFORM, true>(a, row, row0, chunk, prm, sm);
   }
 }
 
 // Kernel variants: per-row parameter table in the arguments or not (_rows); nucleus rows, top-k rows with
 // 64 < k <= kLargeKMax (largek) or all other rows; with or without the code of the logits processing (_xf);
 // one set per element type of the logits (SUFFIX: none for fp32, _f16, _bf16), each in a source file of its own.
-#define MS_STREAM_KERNEL(NAME, SUFFIX, InT, NUCLEUS, XFORM, LARGEK)                                                      \
+// The kernels of all other rows and of argmax also exist for chunks of half and a quarter of kSChunk (_half, _quarter).
+#define MS_STREAM_KERNEL(NAME, SUFFIX, InT, CHUNK, NUCLEUS, XFORM, LARGEK)                                               \
   __global__ __launch_bounds__(NUCLEUS ? kNucleusBlock : kTopkBlock) void NAME##SUFFIX##_kernel(const SampleArgs a) {   \
-    sample_fused_body<InT, false, NUCLEUS, XFORM, LARGEK>(a);                                                            \
+    sample_fused_body<InT, CHUNK, false, NUCLEUS, XFORM, LARGEK>(a);                                                     \
   }                                                                                                                      \
   __global__ __launch_bounds__(NUCLEUS ? kNucleusBlock : kTopkBlock) void NAME##SUFFIX##_rows_kernel(                    \
       const SampleArgs a, const InlineParams) {                                                                          \
-    sample_fused_body<InT, true, NUCLEUS, XFORM, LARGEK>(a);                                                             \
+    sample_fused_body<InT, CHUNK, true, NUCLEUS, XFORM, LARGEK>(a);                                                      \
   }
 
 #define MS_MIXED_KERNEL(NAME, SUFFIX, InT, XFORM)                                                                        \
@@ -1702,47 +1705,64 @@ __device__ __forceinline__ void mixed_stream_body(const SampleArgs& a) {
     mixed_stream_body<InT, true, XFORM>(a);                                                                              \
   }
 
-// Defines the streaming kernels of one element type (sixteen for sampling, two for argmax) and
-// ms_launch_stream##SUFFIX, which launches the one a call needs: which = 0 rows of every other mode (argmax
-// calls: the argmax kernels), 1 nucleus rows, 2 rows with 64 < k <= kLargeKMax, 3 a call's rows of all three kinds.
-#define MS_STREAM_KERNELS(SUFFIX, InT)                                                                                   \
-  namespace ms {                                                                                                         \
-  MS_STREAM_KERNEL(sample_fused, SUFFIX, InT, false, false, false)                                                       \
-  MS_STREAM_KERNEL(sample_fused_xf, SUFFIX, InT, false, true, false)                                                     \
-  MS_STREAM_KERNEL(nucleus_stream, SUFFIX, InT, true, false, false)                                                      \
-  MS_STREAM_KERNEL(nucleus_stream_xf, SUFFIX, InT, true, true, false)                                                    \
-  MS_STREAM_KERNEL(largek_stream, SUFFIX, InT, true, false, true)                                                        \
-  MS_STREAM_KERNEL(largek_stream_xf, SUFFIX, InT, true, true, true)                                                      \
-  MS_MIXED_KERNEL(mixed_stream, SUFFIX, InT, false)                                                                      \
-  MS_MIXED_KERNEL(mixed_stream_xf, SUFFIX, InT, true)                                                                    \
+#define MS_SMALL_K_KERNELS(SUFFIX, InT, CHUNK)                                                                           \
+  MS_STREAM_KERNEL(sample_fused, SUFFIX, InT, CHUNK, false, false, false)                                                \
+  MS_STREAM_KERNEL(sample_fused_xf, SUFFIX, InT, CHUNK, false, true, false)                                              \
   __global__ __launch_bounds__(kTopkBlock) void argmax_stream##SUFFIX##_kernel(const SampleArgs a) {                     \
-    sample_fused_body<InT, false, false, false, false, true>(a);                                                         \
+    sample_fused_body<InT, CHUNK, false, false, false, false, true>(a);                                                  \
   }                                                                                                                      \
   __global__ __launch_bounds__(kTopkBlock) void argmax_stream_xf##SUFFIX##_kernel(const SampleArgs a) {                  \
-    sample_fused_body<InT, false, false, true, false, true>(a);                                                          \
+    sample_fused_body<InT, CHUNK, false, false, true, false, true>(a);                                                   \
+  }
+
+// The kernel of a chunk size by its name.
+#define MS_OF_CHUNK(NAME, SUFFIX, KIND, a)                                                                               \
+  ((a)->chunk_room == kSChunk / 4   ? NAME##SUFFIX##_quarter##KIND                                                       \
+   : (a)->chunk_room == kSChunk / 2 ? NAME##SUFFIX##_half##KIND                                                          \
+                                    : NAME##SUFFIX##KIND)
+
+// Defines the streaming kernels of one element type and ms_launch_stream##SUFFIX, which launches the one a call needs:
+// which = 0 rows of every other mode (argmax calls: the argmax kernels), 1 nucleus rows, 2 rows with
+// 64 < k <= kLargeKMax, 3 a call's rows of all three kinds (1 to 3: chunks of kSChunk).
+#define MS_STREAM_KERNELS(SUFFIX, InT)                                                                                   \
+  namespace ms {                                                                                                         \
+  MS_SMALL_K_KERNELS(SUFFIX, InT, kSChunk)                                                                               \
+  MS_SMALL_K_KERNELS(SUFFIX##_half, InT, kSChunk / 2)                                                                    \
+  MS_SMALL_K_KERNELS(SUFFIX##_quarter, InT, kSChunk / 4)                                                                 \
+  MS_STREAM_KERNEL(nucleus_stream, SUFFIX, InT, kSChunk, true, false, false)                                             \
+  MS_STREAM_KERNEL(nucleus_stream_xf, SUFFIX, InT, kSChunk, true, true, false)                                           \
+  MS_STREAM_KERNEL(largek_stream, SUFFIX, InT, kSChunk, true, false, true)                                               \
+  MS_STREAM_KERNEL(largek_stream_xf, SUFFIX, InT, kSChunk, true, true, true)                                             \
+  MS_MIXED_KERNEL(mixed_stream, SUFFIX, InT, false)                                                                      \
+  MS_MIXED_KERNEL(mixed_stream_xf, SUFFIX, InT, true)                                                                    \
+  static hipError_t launch_stream##SUFFIX(const SampleArgs* a, const InlineParams* table, int which, hipStream_t stream) { \
+    const dim3 block(which == 0 ? kTopkBlock : kNucleusBlock);                                                           \
+    const dim3 grid = which == 0 && a->rows_first ? dim3(a->rows, a->chunks) : dim3(a->chunks, a->rows);                 \
+    const bool xf = a->xf.active();                                                                                      \
+    if (which == 0 && a->emit_topk == kEmitArgmax && !table) {                                                           \
+      auto* f = xf ? MS_OF_CHUNK(argmax_stream_xf, SUFFIX, _kernel, a) : MS_OF_CHUNK(argmax_stream, SUFFIX, _kernel, a); \
+      hipLaunchKernelGGL(f, grid, block, 0, stream, *a);                                                                 \
+    } else if (table) {                                                                                                  \
+      auto* f = which == 0   ? (xf ? MS_OF_CHUNK(sample_fused_xf, SUFFIX, _rows_kernel, a)                               \
+                                   : MS_OF_CHUNK(sample_fused, SUFFIX, _rows_kernel, a))                                 \
+                : which == 1 ? (xf ? nucleus_stream_xf##SUFFIX##_rows_kernel : nucleus_stream##SUFFIX##_rows_kernel)     \
+                : which == 3 ? (xf ? mixed_stream_xf##SUFFIX##_rows_kernel : mixed_stream##SUFFIX##_rows_kernel)         \
+                             : (xf ? largek_stream_xf##SUFFIX##_rows_kernel : largek_stream##SUFFIX##_rows_kernel);      \
+      hipLaunchKernelGGL(f, grid, block, 0, stream, *a, *table);                                                         \
+    } else {                                                                                                             \
+      auto* f = which == 0   ? (xf ? MS_OF_CHUNK(sample_fused_xf, SUFFIX, _kernel, a)                                    \
+                                   : MS_OF_CHUNK(sample_fused, SUFFIX, _kernel, a))                                      \
+                : which == 1 ? (xf ? nucleus_stream_xf##SUFFIX##_kernel : nucleus_stream##SUFFIX##_kernel)               \
+                : which == 3 ? (xf ? mixed_stream_xf##SUFFIX##_kernel : mixed_stream##SUFFIX##_kernel)                   \
+                             : (xf ? largek_stream_xf##SUFFIX##_kernel : largek_stream##SUFFIX##_kernel);                \
+      hipLaunchKernelGGL(f, grid, block, 0, stream, *a);                                                                 \
+    }                                                                                                                    \
+    return hipGetLastError();                                                                                            \
   }                                                                                                                      \
   }                                                                                                                      \
   extern "C" hipError_t ms_launch_stream##SUFFIX(const ms::SampleArgs* a, const ms::InlineParams* table, int which,      \
                                                  hipStream_t stream) {                                                   \
-    const dim3 grid(a->chunks, a->rows), block(which == 0 ? ms::kTopkBlock : ms::kNucleusBlock);                         \
-    const bool xf = a->xf.active();                                                                                      \
-    if (which == 0 && a->emit_topk == ms::kEmitArgmax && !table) {                                                       \
-      hipLaunchKernelGGL(xf ? ms::argmax_stream_xf##SUFFIX##_kernel : ms::argmax_stream##SUFFIX##_kernel, grid, block, 0, \
-                         stream, *a);                                                                                    \
-    } else if (table) {                                                                                                         \
-      auto* f = which == 0   ? (xf ? ms::sample_fused_xf##SUFFIX##_rows_kernel : ms::sample_fused##SUFFIX##_rows_kernel) \
-                : which == 1 ? (xf ? ms::nucleus_stream_xf##SUFFIX##_rows_kernel : ms::nucleus_stream##SUFFIX##_rows_kernel) \
-                : which == 3 ? (xf ? ms::mixed_stream_xf##SUFFIX##_rows_kernel : ms::mixed_stream##SUFFIX##_rows_kernel) \
-                             : (xf ? ms::largek_stream_xf##SUFFIX##_rows_kernel : ms::largek_stream##SUFFIX##_rows_kernel); \
-      hipLaunchKernelGGL(f, grid, block, 0, stream, *a, *table);                                                         \
-    } else {                                                                                                             \
-      auto* f = which == 0   ? (xf ? ms::sample_fused_xf##SUFFIX##_kernel : ms::sample_fused##SUFFIX##_kernel)           \
-                : which == 1 ? (xf ? ms::nucleus_stream_xf##SUFFIX##_kernel : ms::nucleus_stream##SUFFIX##_kernel)       \
-                : which == 3 ? (xf ? ms::mixed_stream_xf##SUFFIX##_kernel : ms::mixed_stream##SUFFIX##_kernel)           \
-                             : (xf ? ms::largek_stream_xf##SUFFIX##_kernel : ms::largek_stream##SUFFIX##_kernel);        \
-      hipLaunchKernelGGL(f, grid, block, 0, stream, *a);                                                                 \
-    }                                                                                                                    \
-    return hipGetLastError();                                                                                            \
+    return ms::launch_stream##SUFFIX(a, table, which, stream);                                                           \
   }
 
 }  // namespace ms

@@ -1099,6 +1099,50 @@ def test_logits_processing_on_rows_of_any_alignment_and_end(ctx, orc, vocab):
             assert tok[r] == idx[orc.discrete_draw(probs, u[r])], (k, r)
 
 
+@pytest.mark.parametrize("rows,vocab", [(1, 8191), (300, 8193), (3, 16383), (5, 16385), (2, 32770), (40, 33000), (9, 49161), (130, 50257),
+                                        (16, 131072), (4, 131073), (90, 98400), (1, 262144), (2, 262145), (1, 524288)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_chunks_of_every_size(orc, rows, vocab, dtype):
+    """Rows of top-k and argmax calls are cut into chunks of 8192, 16384 or 32768 logits, or evenly where the last one would be short, by
+    the number of workgroups: vocabularies on both sides of every chunk size and of the most lists a row's finishing workgroup merges,
+    batches on both sides of a workgroup per CU; a row's best on a chunk's first and last ids, masked ids and history ids among them."""
+    say("chunks", rows, vocab, dtype)
+    rng = np.random.default_rng(vocab * 7 + rows)
+    checked = sorted({0, 1 % rows, rows // 2, rows - 1})
+    c = pkg().SearchContext(rows, vocab)
+    try:
+        x = (torch.randn(rows, vocab, generator=torch.Generator().manual_seed(vocab)) * 3).to(dtype)
+        for r in checked:
+            for e in rng.choice([8191, 8192, 16383, 16384, 32767, 32768, vocab - 1, vocab - 2, (vocab - 1) // 64 * 64], 4):
+                x[r, min(int(e), vocab - 1)] = 14.0 + float(rng.integers(0, 3))
+        xd, u = x.cuda(), rng.random(rows)
+        ud = torch.from_numpy(u).cuda()
+        hist = rng.integers(0, vocab, (rows, 70)).astype(np.int32)
+        hist[:, 0], hist[:, 1] = vocab - 1, min(8192, vocab - 2)
+        mask = make_mask(rng, rows, vocab, 0.7)
+        xf = pkg().LogitsXform(mask=torch.from_numpy(mask.view(np.int32)).cuda(), history=torch.from_numpy(hist).cuda(), repetition_penalty=1.3)
+        for processed in (False, True):
+            want = {r: x[r].float().numpy() for r in checked}
+            if processed:
+                want = {r: orc.apply_repetition_penalty(orc.apply_mask(want[r][None], mask[r:r + 1])[0], hist[r], 1.3) for r in checked}
+            got = c.argmax(xd, xf=xf if processed else None).cpu().numpy()
+            for r in checked:
+                assert got[r] == orc.argmax(want[r]), (processed, r)
+            for k in (2, 50, 64):
+                tok, kc, ki, kp = c.sample(xd, ud, k=k, p=0.9, temperature=0.8, xf=xf if processed else None, kept_capacity=64)
+                tok, kc, ki, kp = tok.cpu().numpy(), kc.cpu().numpy(), ki.cpu().numpy(), kp.cpu().numpy()
+                for r in checked:
+                    idx, probs = orc.sampled_categorical(want[r], k, 0.9, 0.8)
+                    n = len(idx)
+                    assert kc[r] == n and np.array_equal(ki[r, :n], idx), (processed, k, r)
+                    assert np.array_equal(bits(kp[r, :n]), bits(probs)), (processed, k, r)
+                    assert tok[r] == idx[orc.discrete_draw(probs, u[r])], (processed, k, r)
+        if vocab > 8192:
+            assert c.fallback_rows() == 0  # no chunk is too short for its bound
+    finally:
+        c.close()
+
+
 @pytest.mark.parametrize("hist_len", [1500, 2500, 3400, 5000])
 def test_sparse_mask_rows_with_thousands_of_distinct_history_ids(orc, hist_len):
     """Nucleus rows under a sparse grammar mask whose history holds more distinct ids than the sparse-mask kernel's
