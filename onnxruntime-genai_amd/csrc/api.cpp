@@ -685,8 +685,7 @@ int mi355x_topk_scores(mi355x_search_ctx* ctx, void* stream, const void* logits,
 }
 
 // Fills the argument block of the multi-workgroup sequential sum when the shape calls for it and the
-// context's workspace covers it (the exponentials go to the key buffer of the sampling paths, which
-// never run at the same time on one context).
+// context's workspace covers it.
 static bool FillSeqSum(mi355x_search_ctx* ctx, const void* x, int64_t row_stride, int rows, int vocab, float inv_temp,
                        ms::SeqSumArgs* q) {
   const int segs = (vocab + ms::kSegElems - 1) / ms::kSegElems;
@@ -702,8 +701,6 @@ static bool FillSeqSum(mi355x_search_ctx* ctx, const void* x, int64_t row_stride
   q->seg_step = ctx->seg_step;
   q->sub_step = ctx->sub_step;
   q->sub_se = ctx->sub_se;
-  q->e = reinterpret_cast<float*>(ctx->big);
-  q->e_stride = ctx->big_stride * 2;
   q->out_max = ctx->row_max;
   q->out_sum = ctx->row_sum;
   q->poll_limit = ctx->poll_limit;
@@ -765,14 +762,14 @@ int BeamSelectImpl(mi355x_search_ctx* ctx, void* stream, const void* logits, int
     a.row_max = q.out_max;
     a.row_sum = q.out_sum;
     if (static_cast<long long>(beams) * q.segs * 2 * beams <= ms::kBeamFinCap) {
-      // long rows: the segments list their best logits inside the launch that writes their exponentials, the
+      // long rows: the segments list their best logits inside the launch that sums their exponentials, the
       // exact sums follow, and one workgroup per batch entry scores the listed candidates
       a.seg_cand = ctx->seg_cand;
       a.seg_max = q.seg_max;
       a.segs = q.segs;
       HIP_TRY(ms_launch_seqsum_max(&q, dtype, static_cast<hipStream_t>(stream)));
       HIP_TRY(ms_launch_beam_exp_step(&q, &a, dtype, static_cast<hipStream_t>(stream)));
-      HIP_TRY(ms_launch_seqsum_walk(&q, static_cast<hipStream_t>(stream)));
+      HIP_TRY(ms_launch_seqsum_walk(&q, dtype, static_cast<hipStream_t>(stream)));
       HIP_TRY(ms_launch_beam_finish(&a, dtype, step, static_cast<hipStream_t>(stream)));
       if (fused) *fused = step != nullptr;
       return MI355X_OK;

@@ -396,7 +396,7 @@ __global__ __launch_bounds__(256) void beam_scorer_prompt_kernel(const PromptTok
 constexpr int kSegCandCap = 512;        // candidates a segment may list before it reports an overflow
 constexpr u64 kSegOverflow = ~0ull;     // first entry of a segment that listed more than kSegCandCap
 
-// Runs inside the launch that writes the exponentials, while a segment's workgroup waits for the sums of the
+// Runs inside the launch that sums the exponentials, while a segment's workgroup waits for the sums of the
 // segments before it: v are the segment's logits as that launch loaded them (zeros past the end of the row).
 template <typename InT>
 struct SegmentLists {
@@ -416,8 +416,8 @@ struct SegmentLists {
     float fm = -__builtin_inff();
 #pragma unroll
     for (int e = 0; e < kSegPer; ++e)
-      if (FULL || seg_index<InT>(seg, e) < V) fm = fmaxf(fm, v[e]);
-    const uint32_t offer = (FULL || seg_index<InT>(seg, 0) < V) ? order_key(fm) : 0u;  // threads past the end of the row offer nothing
+      if (FULL || seg_run_index(seg, e) < V) fm = fmaxf(fm, v[e]);
+    const uint32_t offer = (FULL || seg_run_index(seg, 0) < V) ? order_key(fm) : 0u;  // threads past the end of the row offer nothing
     // A wave's m-th best thread maximum (0 with fewer than m offers) has m of the wave's elements at or above it;
     // so has the largest of the four, and with it everything that can be among the segment's m best.
     const uint32_t mth = wave_read_lane(wave_sort_desc_fast<uint32_t>(offer), m - 1);
@@ -431,7 +431,7 @@ struct SegmentLists {
     uint32_t mine = 0u;
 #pragma unroll
     for (int e = 0; e < kSegPer; ++e) {
-      const bool cand = (FULL || seg_index<InT>(seg, e) < V) && (tau == 0u || order_key(v[e]) >= tau);  // tau == 0: fewer than m offers, list everything
+      const bool cand = (FULL || seg_run_index(seg, e) < V) && (tau == 0u || order_key(v[e]) >= tau);  // tau == 0: fewer than m offers, list everything
       mine |= cand ? 1u << e : 0u;
     }
     const uint32_t n_mine = static_cast<uint32_t>(__popc(mine));
@@ -445,7 +445,7 @@ struct SegmentLists {
 #pragma unroll
     for (int e = 0; e < kSegPer; ++e) {
       if ((mine >> e) & 1u) {
-        if (pos < kSegCandCap) list[pos] = make_key64(order_key(v[e]), static_cast<uint32_t>(seg_index<InT>(seg, e)));
+        if (pos < kSegCandCap) list[pos] = make_key64(order_key(v[e]), static_cast<uint32_t>(seg_run_index(seg, e)));
         ++pos;
       }
     }

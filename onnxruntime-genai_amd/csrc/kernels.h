@@ -166,8 +166,6 @@ struct SeqSumArgs {
   int4* sub_step;     // [rows][segs][kSegSubs]: (d0, d1) of a 64-element part under the binade in sub_se, then under the next
   int* sub_se;        // [rows][segs][kSegSubs]: that binade, with kPartMayCross where the sum may be in the next one by
                       // the end of the part; -1: the walk adds the part element by element
-  float* e;           // [rows][e_stride] exponentials
-  size_t e_stride;
   float* out_max;     // [rows]
   float* out_sum;     // [rows]
   int poll_limit;     // polls a segment's workgroup spends on an earlier segment's sum before it gives up
@@ -282,7 +280,7 @@ hipError_t ms_launch_beam_exp_step(const ms::SeqSumArgs* q, const ms::BeamArgs* 
 hipError_t ms_launch_beam_finish(const ms::BeamArgs* a, int dtype, const ms::ScorerStep* step, hipStream_t stream);
 hipError_t ms_launch_seqsum(const ms::SeqSumArgs* a, int dtype, hipStream_t stream);  // its three launches
 hipError_t ms_launch_seqsum_max(const ms::SeqSumArgs* a, int dtype, hipStream_t stream);
-hipError_t ms_launch_seqsum_walk(const ms::SeqSumArgs* a, hipStream_t stream);
+hipError_t ms_launch_seqsum_walk(const ms::SeqSumArgs* a, int dtype, hipStream_t stream);
 hipError_t ms_launch_softmax_apply(float* scores, int64_t row_stride, const ms::SeqSumArgs* a, int log_softmax,
                                    hipStream_t stream);
 hipError_t ms_launch_scorer_step(const ms::ScorerState* s, const int32_t* sequences, int32_t* sequences_next,

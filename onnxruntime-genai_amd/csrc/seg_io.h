@@ -12,15 +12,19 @@ typedef uint32_t v4u __attribute__((ext_vector_type(4)));
 constexpr int kSegBlock = 256;
 constexpr int kSegPer = kSegElems / kSegBlock;  // 16 elements per thread
 
-// Loads the 16 elements of thread t in segment `seg`: for j, the VEC consecutive ids starting at
-// seg*kSegElems + (j*256 + t)*VEC (VEC = 4 for fp32, 8 for fp16 and bf16).  Ids >= vocab yield `fill`.
-template <typename InT>
-__device__ __forceinline__ void seg_load(const InT* row, int vocab, int seg, float fill, float (&v)[kSegPer]) {
+// Sixteen-byte groups of a segment: load j of thread t brings the VEC (4 fp32, 8 fp16 or bf16) consecutive ids from
+// seg * kSegElems + group * VEC on; ids >= vocab yield `fill`.  Two ways to share them out:
+// seg_load: group j * 256 + t, so that a wave's load is one run of memory;
+// seg_load_run: group t * (16 / VEC) + j, the thread's sixteen ids in a row, for what needs them in order (a wave's loads
+// then touch all the lines of its share, each load again, from the cache).
+template <typename InT, bool RUN>
+__device__ __forceinline__ void seg_load_groups(const InT* row, int vocab, int seg, float fill, float (&v)[kSegPer]) {
   constexpr int VEC = sizeof(InT) == 4 ? 4 : 8;
   constexpr int NV = kSegPer / VEC;
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
-    const int i0 = seg * kSegElems + (j * kSegBlock + static_cast<int>(threadIdx.x)) * VEC;
+    const int t = static_cast<int>(threadIdx.x);
+    const int i0 = seg * kSegElems + (RUN ? t * NV + j : j * kSegBlock + t) * VEC;
     if (i0 + VEC <= vocab) {
       if constexpr (VEC == 4) {
         const v4f_any q = *reinterpret_cast<const v4f_any*>(row + i0);
@@ -44,11 +48,20 @@ __device__ __forceinline__ void seg_load(const InT* row, int vocab, int seg, flo
     }
   }
 }
+template <typename InT>
+__device__ __forceinline__ void seg_load(const InT* row, int vocab, int seg, float fill, float (&v)[kSegPer]) {
+  seg_load_groups<InT, false>(row, vocab, seg, fill, v);
+}
+template <typename InT>
+__device__ __forceinline__ void seg_load_run(const InT* row, int vocab, int seg, float fill, float (&v)[kSegPer]) {
+  seg_load_groups<InT, true>(row, vocab, seg, fill, v);
+}
 
 template <typename InT>
 __device__ __forceinline__ int seg_index(int seg, int e) {
   constexpr int VEC = sizeof(InT) == 4 ? 4 : 8;
   return seg * kSegElems + ((e / VEC) * kSegBlock + static_cast<int>(threadIdx.x)) * VEC + e % VEC;
 }
+__device__ __forceinline__ int seg_run_index(int seg, int e) { return seg * kSegElems + static_cast<int>(threadIdx.x) * kSegPer + e; }
 
 }  // namespace ms

@@ -48,16 +48,26 @@ struct WalkShared {
   int events_of[kWalkSpecials];
 };
 
-// A row in segments of equal length (all but the last): segment sg starts at element sg * kSegElems.
+// A row in segments of equal length (all but the last): segment sg starts at element sg * kSegElems.  Its elements are the
+// exponentials of x, computed once more for the few parts that the walk looks into: written out by the launch
+// that sums them they were as many bytes as the row, for one part in fifty.
+template <typename InT>
 struct EvenSegments {
   int segs, length;
   const int4* seg_step;  // this row's records, see SeqSumArgs
   const int4* sub_step;
   const int* sub_se;
-  const float* e;
+  const InT* x;
+  float max_score, inv_temp;
+  const uint64_t* exp_tab;  // LDS
   __device__ __forceinline__ int first(int sg) const { return sg * kSegElems; }
   __device__ __forceinline__ int count(int sg) const { return length - sg * kSegElems < kSegElems ? length - sg * kSegElems : kSegElems; }
-  __device__ __forceinline__ float value(int i) const { return e[i]; }
+  __device__ __forceinline__ float load(int i) const { return load_one<InT>(x, i); }
+  __device__ __forceinline__ float value_of(float loaded) const {
+    const uint64_t* const tab = exp_tab;
+    return em::expf_core((loaded - max_score) * inv_temp, [=](uint32_t k) { return tab[k]; });
+  }
+  __device__ __forceinline__ float value(int i) const { return value_of(load(i)); }
 };
 
 __device__ __forceinline__ Step step_from_below_or(Step none, Step x) {  // wave_shr:1, `none` into lane 0
@@ -245,17 +255,23 @@ __device__ __forceinline__ float walk_segments(const Row& a, WalkShared& sh, flo
     // (an event's second word and what lies before it are still wave 0's to rewrite: they are used behind the barrier)
     constexpr int kPerWave = (kWalkEvents + kWalkWaves - 1) / kWalkWaves;
     Step in_front[kPerWave];
+    float loaded[kPerWave];  // (all of the wave's loads before the first is used)
+#pragma unroll
+    for (int i = 0; i < kPerWave; ++i) {
+      const int e = wave + i * kWalkWaves;
+      loaded[i] = 0.0f;
+      if (fits && e < total && lane < sh.count[e]) loaded[i] = a.load(sh.first[e] + lane);
+    }
 #pragma unroll
     for (int i = 0; i < kPerWave; ++i) {
       const int e = wave + i * kWalkWaves;
       in_front[i] = kStepIdentity;
       if (fits && e < total) {
-        const int first = sh.first[e], n = sh.count[e];
-        const float x = lane < n ? a.value(first + lane) : 0.0f;
+        const float x = lane < sh.count[e] ? a.value_of(loaded[i]) : 0.0f;
         sh.x[e][lane] = x;
         const int se = sh.event[e].x;
         if (se >= 0) {
-          const float back = 63 - lane < n ? a.value(first + 63 - lane) : 0.0f;
+          const float back = __shfl(x, 63 - lane, 64);
           in_front[i] = step_from_below_or(kStepIdentity, wave_scan_steps(seq_make_step(x, se)));
           const Step b = wave_scan_steps_backwards(seq_make_step(back, se + 1));  // lane l: elements 63 - l .. 63
           if (lane < 63) sh.behind[e][62 - lane] = make_uint2(b.d0, b.d1);
@@ -268,8 +284,13 @@ __device__ __forceinline__ float walk_segments(const Row& a, WalkShared& sh, flo
     if (wave == kWalkWaves - 1 && g0 == 0) {
       int e = 0;
       float sum = 0.0f;
-      for (; fits && e < total && sh.event[e].x < 0 && sh.first[e] == e * kWalkPart; ++e) {
-        sum = wave_add_chain(sum, lane < sh.count[e] ? a.value(e * kWalkPart + lane) : 0.0f);
+      auto leads = [&](int e) { return fits && e < total && sh.event[e].x < 0 && sh.first[e] == e * kWalkPart; };
+      auto load_part = [&](int e) { return leads(e) && lane < sh.count[e] ? a.load(e * kWalkPart + lane) : 0.0f; };
+      float next = load_part(0);
+      for (; leads(e); ++e) {
+        const float mine = next;
+        next = load_part(e + 1);  // (on its way while these are added)
+        sum = wave_add_chain(sum, lane < sh.count[e] ? a.value_of(mine) : 0.0f);
         if (ENDS && lane == 0) sh.after[e] = sum;
       }
       if (lane == 0) {

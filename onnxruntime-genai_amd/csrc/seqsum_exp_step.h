@@ -1,4 +1,4 @@
-// The launch that writes a segment's exponentials and its step record (see seqsum_kernels.hip), as a template so
+// The launch that sums a segment's exponentials and composes its step record (see seqsum_kernels.hip), as a template so
 // that a caller can give the workgroups something to do while they wait for the earlier segments' sums.
 #pragma once
 #include "kernels.h"
@@ -8,13 +8,32 @@
 
 namespace ms {
 
-__device__ __forceinline__ float row_max_of_segments(const SeqSumArgs& a, int row, uint32_t* red) {
+// Every wave for itself: the maxima are few and in the cache, a reduction over the block would be two barriers.
+__device__ __forceinline__ float row_max_of_segments(const SeqSumArgs& a, int row) {
   uint32_t m = 0u;
-  for (int s = threadIdx.x; s < a.segs; s += blockDim.x) {
+  for (int s = lane_id(); s < a.segs; s += 64) {
     const uint32_t k = a.seg_max[static_cast<size_t>(row) * a.segs + s];
     m = k > m ? k : m;
   }
-  return key_to_float(block_max<uint32_t>(m, red));
+  return key_to_float(wave_max<uint32_t>(m));
+}
+
+// expf of N arguments a lane, none of them above 88 (or else its result is not used); reached by whole waves.  Below
+// -103.98 the results are zeros, as expf_in_range's are from there down to -600, so a NaN is all that needs expf's special
+// cases, and the wave looks for one once: N chains of a dozen double-precision operations and a look-up then run side by
+// side, where a branch per argument kept them one behind the other.
+template <int N, typename Tab>
+__device__ __forceinline__ void wave_expf(const float (&x)[N], Tab tab, float (&out)[N]) {
+  bool nan = false;
+#pragma unroll
+  for (int e = 0; e < N; ++e) nan |= x[e] != x[e];
+  if (__builtin_expect(__ballot(nan) == 0ull, 1)) {
+#pragma unroll
+    for (int e = 0; e < N; ++e) out[e] = em::expf_in_range(fmaxf(x[e], -600.0f), tab);
+  } else {
+#pragma unroll 1
+    for (int e = 0; e < N; ++e) out[e] = em::expf_core(x[e], tab);
+  }
 }
 
 // A segment sum that has not been written yet: all bits set, a NaN no sum can be (sums of exponentials are
@@ -37,7 +56,7 @@ __device__ __forceinline__ double seq_drift(int count) {
   return (8.0 * sqrt(static_cast<double>(count)) + 8.0) * 6.0e-8;
 }
 
-// Steps 2 and 3 in one launch.  A segment's workgroup writes its exponentials and publishes their double sum;
+// Steps 2 and 3 in one launch.  A segment's workgroup computes its exponentials and publishes their double sum;
 // then it waits for the sums of the row's earlier segments, which earlier workgroups of the same launch publish
 // (workgroups start in index order and a row's segments are consecutive indices, so whatever a workgroup waits for
 // is running or done), and goes on with its step record from the exponentials it still holds.  A wait that gives
@@ -46,6 +65,12 @@ __device__ __forceinline__ double seq_drift(int count) {
 // `between(v, seg, row)` runs, in all threads, after the sum is out and before the earlier sums are needed: work
 // on the segment's elements v (as loaded: zeros past the end of the row) that would otherwise wait for a launch of
 // its own.
+// Bound by the chain from the loads over the exponentials, the exchange of the sums and the composition to the record, with a
+// third of the time spent issuing vector instructions: exponentials side by side (wave_expf) and a thread's sixteen elements in a row, so that
+// neither a transposition through LDS nor a copy of the exponentials in memory is needed (the walk computes the few it
+// looks at once more, and takes 1 us longer), took the launch from 12.3 to 8.7 us at 16 x 151936 fp32 (9.7 MB, in the cache by
+// then), with the lists of the beam search from 20.4 to 17.1 at 32 x 151936 fp16 and from 11.4 to 8.9 at 8 x 51865.
+//
 // FULL: the segment lies inside the row (all but a row's last segment do), so nothing has to ask where the row ends.
 // `Shared` is what it needs of LDS (declared once, by the kernel, for both forms of the body).
 struct NothingBetween {
@@ -55,10 +80,9 @@ struct NothingBetween {
 };
 
 struct ExpStepShared {
-  uint32_t red[4];
   double dred[4];
+  unsigned long long before;  // the sum of the segments before this one; kSumNotReady: the wait for one gave up
   uint64_t exp_tab[32];  // the table of expf in LDS: a lookup per element from constant memory is a gather
-  __align__(16) float stage[kSegElems];  // the segment's exponentials in element order
   Step wave_tot[4];
   double wave_parts[4];
 };
@@ -66,69 +90,63 @@ struct ExpStepShared {
 template <typename InT, typename Between, bool FULL>
 __device__ __forceinline__ void seqsum_exp_step_body(const SeqSumArgs& a, const Between& between, ExpStepShared& sh,
                                                      typename Between::Shared& between_sh) {
-  uint32_t* const red = sh.red;
   double* const dred = sh.dred;
   uint64_t* const exp_tab = sh.exp_tab;
-  float* const stage = sh.stage;
   Step* const wave_tot = sh.wave_tot;
   double* const wave_parts = sh.wave_parts;
   const int seg = blockIdx.x, row = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const InT* x = static_cast<const InT*>(a.x) + static_cast<size_t>(row) * a.row_stride;
+  // (a thread has sixteen elements in a row: the composition below takes them in order)
   float v[kSegPer];
-  seg_load<InT>(x, FULL ? (seg + 1) * kSegElems : a.vocab, seg, 0.0f, v);
+  seg_load_run<InT>(x, FULL ? (seg + 1) * kSegElems : a.vocab, seg, 0.0f, v);
   if (tid < 32) exp_tab[tid] = em::exp2_tab(static_cast<uint32_t>(tid));
-  const float max_score = row_max_of_segments(a, row, red);  // its barriers also publish the table
+  const float max_score = row_max_of_segments(a, row);
+  if (seg == 0 && tid == 0) a.out_max[row] = max_score;
+  __syncthreads();  // (the table)
   const uint64_t* const tab = exp_tab;
   auto lds_tab = [=](uint32_t i) { return tab[i]; };
-  float* erow = a.e + static_cast<size_t>(row) * a.e_stride;
   const int first = seg * kSegElems;
-  double part = 0.0;
-  // four consecutive exponentials per store (the row of exponentials starts 16-byte aligned and a thread's ids come
-  // in aligned groups of four); a group that crosses the end of the row is stored element by element
+  float ev[kSegPer];  // zeros past the end of the row
+  {
+    float arg[kSegPer];
 #pragma unroll
-  for (int e0 = 0; e0 < kSegPer; e0 += 4) {
-    const int idx = seg_index<InT>(seg, e0);
-    float ex[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      ex[c] = (FULL || idx + c < a.vocab) ? em::expf_core((v[e0 + c] - max_score) * a.inv_temp, lds_tab) : 0.0f;
-      part += static_cast<double>(ex[c]);
-    }
-    v4f q;
-    q.x = ex[0], q.y = ex[1], q.z = ex[2], q.w = ex[3];
-    *reinterpret_cast<v4f*>(stage + (idx - first)) = q;
-    if (FULL || idx + 4 <= a.vocab) {
-      *reinterpret_cast<v4f*>(erow + idx) = q;
-    } else {
-#pragma unroll
-      for (int c = 0; c < 4; ++c)
-        if (idx + c < a.vocab) erow[idx + c] = ex[c];
-    }
+    for (int e = 0; e < kSegPer; ++e) arg[e] = (v[e] - max_score) * a.inv_temp;
+    wave_expf(arg, lds_tab, ev);
   }
+  double part = 0.0;
+#pragma unroll
+  for (int e = 0; e < kSegPer; ++e) {
+    if (!FULL && seg_run_index(seg, e) >= a.vocab) ev[e] = 0.0f;
+    part += static_cast<double>(ev[e]);
+  }
+  const double own_part = part;
   part = wave_sum<double>(part);
   if (lane == 0) dred[wave] = part;
-  __syncthreads();  // (the staged exponentials are complete, too)
+  __syncthreads();
   const double own = (dred[0] + dred[1]) + (dred[2] + dred[3]);
   double* sums = a.seg_sum + static_cast<size_t>(row) * a.segs;
   if (tid == 0) store_sum_bits(sums + seg, static_cast<unsigned long long>(__double_as_longlong(own)));
   between.template run<FULL>(between_sh, v, seg, row);
-  // the sums of the segments before this one
-  double before = 0.0;
-  bool gave_up = false;
-  for (int sg = tid; sg < seg; sg += kSegBlock) {
-    unsigned long long bits = load_sum_bits(sums + sg);
-    for (int spins = 0; bits == kSumNotReady && spins < a.poll_limit; ++spins) {
-      __builtin_amdgcn_s_sleep(1);
-      bits = load_sum_bits(sums + sg);
+  // the sums of the segments before this one: the first wave's to wait for
+  if (wave == 0) {
+    double upto = 0.0;
+    bool gave_up = false;
+    for (int sg = lane; sg < seg; sg += 64) {
+      unsigned long long bits = load_sum_bits(sums + sg);
+      for (int spins = 0; bits == kSumNotReady && spins < a.poll_limit; ++spins) {
+        __builtin_amdgcn_s_sleep(1);
+        bits = load_sum_bits(sums + sg);
+      }
+      if (bits == kSumNotReady) gave_up = true;
+      else upto += __longlong_as_double(static_cast<long long>(bits));
     }
-    if (bits == kSumNotReady) gave_up = true;
-    else before += __longlong_as_double(static_cast<long long>(bits));
+    upto = wave_sum<double>(upto);
+    gave_up = __ballot(gave_up) != 0ull;
+    if (lane == 0) sh.before = gave_up ? kSumNotReady : static_cast<unsigned long long>(__double_as_longlong(upto));
   }
-  gave_up = __syncthreads_or(gave_up ? 1 : 0) != 0;  // (also: every thread has read dred)
-  before = wave_sum<double>(before);
-  if (lane == 0) dred[wave] = before;
   __syncthreads();
-  before = (dred[0] + dred[1]) + (dred[2] + dred[3]);
+  const double before = __longlong_as_double(static_cast<long long>(sh.before));
+  const bool gave_up = sh.before == kSumNotReady;
   const int n = FULL ? kSegElems : a.vocab - first;
   int4* rec = a.seg_step + static_cast<size_t>(row) * a.segs + seg;
   if (gave_up) {
@@ -144,13 +162,6 @@ __device__ __forceinline__ void seqsum_exp_step_body(const SeqSumArgs& a, const 
   const float lo_f = __double2float_rd(lo), hi_f = __double2float_ru(hi);
   const int se = seq_decompose(lo_f).se;
   const bool known = lo_f > 0.0f && hi_f < 3.0e38f && seq_decompose(hi_f).se == se;
-  // thread t continues with elements 16 t .. 16 t + 15 of the segment (zeros past the end of the row)
-  float ev[kSegPer];
-#pragma unroll
-  for (int j = 0; j < kSegPer; j += 4) {
-    const float4 q = *reinterpret_cast<const float4*>(stage + tid * kSegPer + j);
-    ev[j] = q.x, ev[j + 1] = q.y, ev[j + 2] = q.z, ev[j + 3] = q.w;
-  }
   if (!known) {
     // Powers of two may fall inside the segment.  Each of its 64-element parts (four lanes of sixteen elements)
     // estimates the binade the sum has where the part begins, from the double sums of the parts before it, and
@@ -159,9 +170,7 @@ __device__ __forceinline__ void seqsum_exp_step_body(const SeqSumArgs& a, const 
     // estimate was wrong.
     constexpr int kPart = kSegElems / kSegSubs;
     static_assert(kPart == 4 * kSegPer && kSegBlock == kSegSubs * 4, "a part is four lanes");
-    double mine = 0.0;
-#pragma unroll
-    for (int j = 0; j < kSegPer; ++j) mine += static_cast<double>(ev[j]);
+    double mine = own_part;
     mine += __longlong_as_double(static_cast<long long>(lane_xor64<1>(static_cast<u64>(__double_as_longlong(mine)))));
     mine += __longlong_as_double(static_cast<long long>(lane_xor64<2>(static_cast<u64>(__double_as_longlong(mine)))));
     // (all four lanes of a part hold its sum)

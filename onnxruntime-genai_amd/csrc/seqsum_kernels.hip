@@ -5,7 +5,7 @@
 // per row leaves most of the chip idle when there are few, long rows (beam search: 32 rows of 152K).
 // Here a row is cut into segments of kSegElems elements and three launches share the work:
 //   1. seqsum_max:      segment maxima.
-//   2. seqsum_exp_step: e_i = expf((x_i - rowmax) * inv_T) (exact), stored as fp32, plus the segment's
+//   2. seqsum_exp_step: e_i = expf((x_i - rowmax) * inv_T) (exact) and the segment's
 //                       sum in double; then, from the double sums of the segments before it, a segment
 //                       knows the binade its running sum will be in -- unless a power of two may fall
 //                       inside it -- and composes the step functions of its elements under that binade
@@ -43,66 +43,66 @@ __global__ __launch_bounds__(kSegBlock) void seqsum_max_kernel(const SeqSumArgs 
   }
 }
 
+template <typename InT>
 __global__ __launch_bounds__(64 * kWalkWaves) void seqsum_walk_kernel(const SeqSumArgs a) {
   extern __shared__ u64 walk_lds[];
+  __shared__ uint64_t exp_tab[32];
   WalkShared& sh = *reinterpret_cast<WalkShared*>(walk_lds);
   const int row = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const size_t rbase = static_cast<size_t>(row) * a.segs;
-  float max_score = 0.0f;
-  if (wave == 0) {
-    uint32_t m = 0u;
-    for (int sg = lane; sg < a.segs; sg += 64) {
-      const uint32_t k = a.seg_max[rbase + sg];
-      m = k > m ? k : m;
-    }
-    max_score = key_to_float(wave_max<uint32_t>(m));
-  }
+  if (threadIdx.x < 32) exp_tab[threadIdx.x] = em::exp2_tab(threadIdx.x);  // (barriers follow before it is used)
+  const float max_score = a.out_max[row];  // (of the launch before this one)
   // (the row's segment sums have served: back to "not written" for the next launch)
   for (int sg = static_cast<int>(threadIdx.x) - 64; sg >= 0 && sg < a.segs; sg += 64 * (kWalkWaves - 1))
     store_sum_bits(a.seg_sum + rbase + sg, kSumNotReady);
-  const EvenSegments segments{a.segs, a.vocab, a.seg_step + rbase, a.sub_step + rbase * kSegSubs, a.sub_se + rbase * kSegSubs,
-                              a.e + static_cast<size_t>(row) * a.e_stride};
+  const EvenSegments<InT> segments{a.segs, a.vocab, a.seg_step + rbase, a.sub_step + rbase * kSegSubs, a.sub_se + rbase * kSegSubs,
+                                   static_cast<const InT*>(a.x) + static_cast<size_t>(row) * a.row_stride, max_score, a.inv_temp, exp_tab};
   const float s = walk_segments<false>(segments, sh, nullptr);
-  if (wave == 0 && lane == 0) {
-    a.out_sum[row] = s;
-    a.out_max[row] = max_score;
-  }
+  if (wave == 0 && lane == 0) a.out_sum[row] = s;
 }
 
 // Element-wise finish of Softmax / LogSoftMax (src/softmax.h:26-47) once a row's maximum and sum
 // are known: log-softmax writes (x - max) * inv_T - log(sum); softmax writes e * (1 / sum), with e the
-// stored exponential (left as is when the sum is zero).
+// exponential (left as is when the sum is zero).
 template <bool LOG>
 __global__ __launch_bounds__(kSegBlock) void softmax_apply_kernel(float* scores, int64_t row_stride, const SeqSumArgs a) {
   const int seg = blockIdx.x, row = blockIdx.y;
   float* x = scores + static_cast<size_t>(row) * row_stride;
-  const float* erow = a.e + static_cast<size_t>(row) * a.e_stride;
   const float max_score = a.out_max[row], sum = a.out_sum[row];
   const float lse = LOG ? em::logf_exact(sum) : 0.0f;
   const float inv_sum = 1.0f / sum;
-  auto finish = [=](float v, int i) {
-    if (LOG) {
-      // x - max is never -0 where it shows (see softmax_kernel): the maximum here lost the sign of its zero
-      const float d = v - max_score;
-      return (d == 0.0f ? 0.0f : d) * a.inv_temp - lse;
-    }
-    const float ex = erow[i];
-    return sum > 0.0f ? ex * inv_sum : ex;
-  };
   // four elements per load and store (whatever the row's alignment), the loads of a thread under way together
-  float v[kSegPer];
+  float v[kSegPer], r[kSegPer];
   seg_load<float>(x, a.vocab, seg, 0.0f, v);
+  if constexpr (LOG) {
+    // x - max is never -0 where it shows (see softmax_kernel): the maximum here lost the sign of its zero
+#pragma unroll
+    for (int e = 0; e < kSegPer; ++e) {
+      const float d = v[e] - max_score;
+      r[e] = (d == 0.0f ? 0.0f : d) * a.inv_temp - lse;
+    }
+  } else {
+    __shared__ uint64_t exp_tab[32];
+    if (threadIdx.x < 32) exp_tab[threadIdx.x] = em::exp2_tab(threadIdx.x);
+    __syncthreads();
+    const uint64_t* const tab = exp_tab;
+#pragma unroll
+    for (int e = 0; e < kSegPer; ++e) v[e] = (v[e] - max_score) * a.inv_temp;
+    wave_expf(v, [=](uint32_t i) { return tab[i]; }, r);
+#pragma unroll
+    for (int e = 0; e < kSegPer; ++e) r[e] = sum > 0.0f ? r[e] * inv_sum : r[e];
+  }
 #pragma unroll
   for (int e0 = 0; e0 < kSegPer; e0 += 4) {
     const int i = seg_index<float>(seg, e0);
     if (i + 4 <= a.vocab) {
       v4f_any q;
-      q.x = finish(v[e0], i), q.y = finish(v[e0 + 1], i + 1), q.z = finish(v[e0 + 2], i + 2), q.w = finish(v[e0 + 3], i + 3);
+      q.x = r[e0], q.y = r[e0 + 1], q.z = r[e0 + 2], q.w = r[e0 + 3];
       *reinterpret_cast<v4f_any*>(x + i) = q;
     } else {
 #pragma unroll
       for (int c = 0; c < 4; ++c)
-        if (i + c < a.vocab) x[i + c] = finish(v[e0 + c], i + c);
+        if (i + c < a.vocab) x[i + c] = r[e0 + c];
     }
   }
 }
@@ -117,8 +117,9 @@ extern "C" hipError_t ms_launch_seqsum_max(const ms::SeqSumArgs* a, int dtype, h
   return hipGetLastError();
 }
 
-extern "C" hipError_t ms_launch_seqsum_walk(const ms::SeqSumArgs* a, hipStream_t stream) {
-  hipLaunchKernelGGL(ms::seqsum_walk_kernel, dim3(a->rows), dim3(64 * ms::kWalkWaves), sizeof(ms::WalkShared), stream, *a);
+extern "C" hipError_t ms_launch_seqsum_walk(const ms::SeqSumArgs* a, int dtype, hipStream_t stream) {
+  auto* f = dtype == MI355X_F16 ? ms::seqsum_walk_kernel<uint16_t> : dtype == MI355X_BF16 ? ms::seqsum_walk_kernel<ms::bf16_t> : ms::seqsum_walk_kernel<float>;
+  hipLaunchKernelGGL(f, dim3(a->rows), dim3(64 * ms::kWalkWaves), sizeof(ms::WalkShared), stream, *a);
   return hipGetLastError();
 }
 
@@ -133,7 +134,7 @@ extern "C" hipError_t ms_launch_seqsum(const ms::SeqSumArgs* a, int dtype, hipSt
     hipLaunchKernelGGL((ms::seqsum_exp_step_kernel<ms::bf16_t, ms::NothingBetween>), grid, block, 0, stream, *a, nothing);
   else
     hipLaunchKernelGGL((ms::seqsum_exp_step_kernel<float, ms::NothingBetween>), grid, block, 0, stream, *a, nothing);
-  return ms_launch_seqsum_walk(a, stream);
+  return ms_launch_seqsum_walk(a, dtype, stream);
 }
 
 extern "C" hipError_t ms_launch_softmax_apply(float* scores, int64_t row_stride, const ms::SeqSumArgs* a,

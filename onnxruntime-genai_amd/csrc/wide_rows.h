@@ -937,6 +937,8 @@ struct WideSegments {
   __device__ __forceinline__ int first(int sg) const { return static_cast<int>(tile_start[sg]); }
   __device__ __forceinline__ int count(int sg) const { return static_cast<int>(tile_start[sg + 1] - tile_start[sg]); }
   __device__ __forceinline__ float value(int i) const { return __uint_as_float(static_cast<uint32_t>(list[i] >> 32)); }
+  __device__ __forceinline__ float load(int i) const { return value(i); }
+  __device__ __forceinline__ float value_of(float loaded) const { return loaded; }
 };
 
 struct WideFinishShared {

@@ -90,6 +90,29 @@ def test_softmax_bit_exact(ctx, orc, rows, vocab, t):
         assert np.array_equal(bits(lsm[r]), bits(orc.log_softmax(x[r], t)))
 
 
+@pytest.mark.parametrize("vocab", [16384, 16385, 20479, 20481, 40963])
+@pytest.mark.parametrize("t", [1.0, 0.3])
+def test_softmax_of_long_rows_with_masked_infinite_and_nan_logits(ctx, orc, vocab, t):
+    """A wave takes its exponentials side by side unless one of its arguments is a NaN: rows with logits of lowest() and -inf (exponents far
+    below what the arithmetic is for), with a NaN, of one value, and next to a segment's and a wave's ends."""
+    say("softmax of special rows", vocab, t)
+    rng = np.random.default_rng(vocab)
+    x = (rng.standard_normal((6, vocab)) * 3).astype(np.float32)
+    x[0, rng.random(vocab) < 0.6] = np.finfo(np.float32).min
+    x[1, rng.random(vocab) < 0.3] = -np.inf
+    x[2] = -7.25
+    x[3, vocab - 1] = 30.0
+    x[4, [1023, 4095, 4096, vocab - 2]] = np.nan
+    x[5] = rng.uniform(-700.0, 0.0, vocab)
+    sm = ctx.softmax(torch.from_numpy(x.copy()).cuda(), t, log=False).cpu().numpy()
+    lsm = ctx.softmax(torch.from_numpy(x.copy()).cuda(), t, log=True).cpu().numpy()
+    for r in range(6):
+        for got, want in ((sm[r], orc.softmax(x[r], t)), (lsm[r], orc.log_softmax(x[r], t))):
+            number = ~np.isnan(want)
+            assert np.array_equal(np.isnan(got), ~number), r
+            assert np.array_equal(bits(got[number]), bits(want[number])), r
+
+
 def test_log_softmax_extreme_rows(ctx, orc):
     """Sums that start subnormal, cross many binades, or hit exact ties in the running sum."""
     say("softmax extreme")
