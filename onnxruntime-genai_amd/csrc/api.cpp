@@ -86,7 +86,7 @@ struct ScorerHost {
   void GiveBackWord(int word) { used.fetch_and(~(uint64_t{1} << word)); }
 };
 
-constexpr int kPlanBlocks = 256;  // a workgroup per CU
+constexpr int kPlanBlocks = ms::kCus;  // a workgroup per CU
 
 struct mi355x_search_ctx {
   int device{};

@@ -10,6 +10,7 @@ namespace ms {
 // Many logits per lane keep the per-wave selection overhead small against the streaming work, few
 // chunks per row keep the finishing merge shallow (a 128K vocabulary is four sorted lists, two merge
 // levels), and thread t's float4s (t, t+512, t+1024, ...) make every wave an even sample of the chunk.
+constexpr int kCus = 256;             // of the GPU
 constexpr int kSChunk = 32768;        // logits per workgroup of the streaming kernels; those of top-k and argmax rows also come for 16384 and 8192
 constexpr int kTopkBlock = 512;       // threads of a workgroup that streams a top-k row (16 128-bit loads each) ...
 constexpr int kNucleusBlock = 1024;   // ... and a nucleus row (8 each: lighter threads, twice the waves in flight)

@@ -1687,12 +1687,16 @@ __device__ __forceinline__ void mixed_stream_body(const SampleArgs& a) {
 // Kernel variants: per-row parameter table in the arguments or not (_rows); nucleus rows, top-k rows with
 // 64 < k <= kLargeKMax (largek) or all other rows; with or without the code of the logits processing (_xf);
 // one set per element type of the logits (SUFFIX: none for fp32, _f16, _bf16), each in a source file of its own.
-// The kernels of all other rows and of argmax also exist for chunks of half and a quarter of kSChunk (_half, _quarter).
-#define MS_STREAM_KERNEL(NAME, SUFFIX, InT, CHUNK, NUCLEUS, XFORM, LARGEK)                                               \
-  __global__ __launch_bounds__(NUCLEUS ? kNucleusBlock : kTopkBlock) void NAME##SUFFIX##_kernel(const SampleArgs a) {   \
+// The kernels of all other rows and of argmax also exist for chunks of half and a quarter of kSChunk (_half, _quarter),
+// those of nucleus rows for more workgroups than CUs (_many): two of their workgroups fit a CU, for which a wave may have
+// 64 vector registers and 80 scalar ones (800 a SIMD, and the hardware's trap handler takes 16 of every wave's).  256 x 201088 fp32
+// N(0, 5^2), both launches: 123.3 -> 106.3 us, 128 x 128256 fp16 50.5 -> 46.3, with a penalty 64 x 201088 fp16 63.7 -> 58.6; where every workgroup has
+// a CU to itself the other kernels, of up to 104 scalar registers, are 0.2 to 0.4 us faster (16 x 128256 fp16 31.1 against 31.5).
+#define MS_STREAM_KERNEL(NAME, SUFFIX, InT, CHUNK, NUCLEUS, XFORM, LARGEK, WAVES)                                        \
+  __global__ __launch_bounds__(NUCLEUS ? kNucleusBlock : kTopkBlock, WAVES) void NAME##SUFFIX##_kernel(const SampleArgs a) { \
     sample_fused_body<InT, CHUNK, false, NUCLEUS, XFORM, LARGEK>(a);                                                     \
   }                                                                                                                      \
-  __global__ __launch_bounds__(NUCLEUS ? kNucleusBlock : kTopkBlock) void NAME##SUFFIX##_rows_kernel(                    \
+  __global__ __launch_bounds__(NUCLEUS ? kNucleusBlock : kTopkBlock, WAVES) void NAME##SUFFIX##_rows_kernel(             \
       const SampleArgs a, const InlineParams) {                                                                          \
     sample_fused_body<InT, CHUNK, true, NUCLEUS, XFORM, LARGEK>(a);                                                      \
   }
@@ -1706,8 +1710,8 @@ __device__ __forceinline__ void mixed_stream_body(const SampleArgs& a) {
   }
 
 #define MS_SMALL_K_KERNELS(SUFFIX, InT, CHUNK)                                                                           \
-  MS_STREAM_KERNEL(sample_fused, SUFFIX, InT, CHUNK, false, false, false)                                                \
-  MS_STREAM_KERNEL(sample_fused_xf, SUFFIX, InT, CHUNK, false, true, false)                                              \
+  MS_STREAM_KERNEL(sample_fused, SUFFIX, InT, CHUNK, false, false, false, 1)                                                \
+  MS_STREAM_KERNEL(sample_fused_xf, SUFFIX, InT, CHUNK, false, true, false, 1)                                              \
   __global__ __launch_bounds__(kTopkBlock) void argmax_stream##SUFFIX##_kernel(const SampleArgs a) {                     \
     sample_fused_body<InT, CHUNK, false, false, false, false, true>(a);                                                  \
   }                                                                                                                      \
@@ -1729,30 +1733,34 @@ __device__ __forceinline__ void mixed_stream_body(const SampleArgs& a) {
   MS_SMALL_K_KERNELS(SUFFIX, InT, kSChunk)                                                                               \
   MS_SMALL_K_KERNELS(SUFFIX##_half, InT, kSChunk / 2)                                                                    \
   MS_SMALL_K_KERNELS(SUFFIX##_quarter, InT, kSChunk / 4)                                                                 \
-  MS_STREAM_KERNEL(nucleus_stream, SUFFIX, InT, kSChunk, true, false, false)                                             \
-  MS_STREAM_KERNEL(nucleus_stream_xf, SUFFIX, InT, kSChunk, true, true, false)                                           \
-  MS_STREAM_KERNEL(largek_stream, SUFFIX, InT, kSChunk, true, false, true)                                               \
-  MS_STREAM_KERNEL(largek_stream_xf, SUFFIX, InT, kSChunk, true, true, true)                                             \
+  MS_STREAM_KERNEL(nucleus_stream, SUFFIX, InT, kSChunk, true, false, false, 1)                                          \
+  MS_STREAM_KERNEL(nucleus_stream_xf, SUFFIX, InT, kSChunk, true, true, false, 1)                                        \
+  MS_STREAM_KERNEL(nucleus_stream_many, SUFFIX, InT, kSChunk, true, false, false, 8)                                     \
+  MS_STREAM_KERNEL(nucleus_stream_many_xf, SUFFIX, InT, kSChunk, true, true, false, 8)                                   \
+  MS_STREAM_KERNEL(largek_stream, SUFFIX, InT, kSChunk, true, false, true, 1)                                            \
+  MS_STREAM_KERNEL(largek_stream_xf, SUFFIX, InT, kSChunk, true, true, true, 1)                                          \
   MS_MIXED_KERNEL(mixed_stream, SUFFIX, InT, false)                                                                      \
   MS_MIXED_KERNEL(mixed_stream_xf, SUFFIX, InT, true)                                                                    \
   static hipError_t launch_stream##SUFFIX(const SampleArgs* a, const InlineParams* table, int which, hipStream_t stream) { \
     const dim3 block(which == 0 ? kTopkBlock : kNucleusBlock);                                                           \
     const dim3 grid = which == 0 && a->rows_first ? dim3(a->rows, a->chunks) : dim3(a->chunks, a->rows);                 \
-    const bool xf = a->xf.active();                                                                                      \
+    const bool xf = a->xf.active(), many = a->rows * static_cast<long long>(a->chunks) > kCus;                           \
     if (which == 0 && a->emit_topk == kEmitArgmax && !table) {                                                           \
       auto* f = xf ? MS_OF_CHUNK(argmax_stream_xf, SUFFIX, _kernel, a) : MS_OF_CHUNK(argmax_stream, SUFFIX, _kernel, a); \
       hipLaunchKernelGGL(f, grid, block, 0, stream, *a);                                                                 \
     } else if (table) {                                                                                                  \
       auto* f = which == 0   ? (xf ? MS_OF_CHUNK(sample_fused_xf, SUFFIX, _rows_kernel, a)                               \
                                    : MS_OF_CHUNK(sample_fused, SUFFIX, _rows_kernel, a))                                 \
-                : which == 1 ? (xf ? nucleus_stream_xf##SUFFIX##_rows_kernel : nucleus_stream##SUFFIX##_rows_kernel)     \
+                : which == 1 ? (many ? (xf ? nucleus_stream_many_xf##SUFFIX##_rows_kernel : nucleus_stream_many##SUFFIX##_rows_kernel) \
+                                     : (xf ? nucleus_stream_xf##SUFFIX##_rows_kernel : nucleus_stream##SUFFIX##_rows_kernel)) \
                 : which == 3 ? (xf ? mixed_stream_xf##SUFFIX##_rows_kernel : mixed_stream##SUFFIX##_rows_kernel)         \
                              : (xf ? largek_stream_xf##SUFFIX##_rows_kernel : largek_stream##SUFFIX##_rows_kernel);      \
       hipLaunchKernelGGL(f, grid, block, 0, stream, *a, *table);                                                         \
     } else {                                                                                                             \
       auto* f = which == 0   ? (xf ? MS_OF_CHUNK(sample_fused_xf, SUFFIX, _kernel, a)                                    \
                                    : MS_OF_CHUNK(sample_fused, SUFFIX, _kernel, a))                                      \
-                : which == 1 ? (xf ? nucleus_stream_xf##SUFFIX##_kernel : nucleus_stream##SUFFIX##_kernel)               \
+                : which == 1 ? (many ? (xf ? nucleus_stream_many_xf##SUFFIX##_kernel : nucleus_stream_many##SUFFIX##_kernel) \
+                                     : (xf ? nucleus_stream_xf##SUFFIX##_kernel : nucleus_stream##SUFFIX##_kernel))      \
                 : which == 3 ? (xf ? mixed_stream_xf##SUFFIX##_kernel : mixed_stream##SUFFIX##_kernel)                   \
                              : (xf ? largek_stream_xf##SUFFIX##_kernel : largek_stream##SUFFIX##_kernel);                \
       hipLaunchKernelGGL(f, grid, block, 0, stream, *a);                                                                 \

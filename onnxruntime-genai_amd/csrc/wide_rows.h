@@ -189,8 +189,10 @@ __device__ __forceinline__ double2* wide_masses(const SampleArgs& a, const WideA
   return reinterpret_cast<double2*>(a.big + static_cast<size_t>(row) * a.big_stride + static_cast<size_t>(w.chunks) * (kWideBlock / 2));
 }
 
+// (Eight waves a SIMD: two workgroups a CU.  With 66 registers instead of 64 it was one: 256 x 128256 fp16, all launches, 158.7 -> 132.3 us,
+// 64 x 201088 104.5 -> 94.3, 64 x 128256 55.3 -> 50.6; 16 rows as before.)
 template <typename InT, bool INLINE>
-__global__ __launch_bounds__(kWideBlock) void wide_count_kernel(const SampleArgs a, const typename WideTable<INLINE>::type, const WideArgs w) {
+__global__ __launch_bounds__(kWideBlock, 8) void wide_count_kernel(const SampleArgs a, const typename WideTable<INLINE>::type, const WideArgs w) {
   __shared__ uint32_t hist[kWideBuckets + 1];
   __shared__ double mass[kWideBuckets];
   __shared__ uint64_t exp_tab[32];
