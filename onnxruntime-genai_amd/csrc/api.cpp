@@ -487,6 +487,7 @@ int SampleImpl(mi355x_search_ctx* ctx, hipStream_t s, const void* logits, const 
     const bool nucleus = p.k <= 1 && !whole, large_k = p.k > 1 && kk > 64 && kk <= ms::kLargeKMax;
     if (nucleus && vocab > 64) any_nucleus = true;
     if (large_k && vocab > 64) any_large_k = true;
+    if (large_k && kk > 4 * ms::kLargeKOneOffer) a.all_offers = 1;
     if (whole && wide_fits) any_wide = true;
     else if (vocab > 64 && (!fits || whole || (p.k > 1 && kk > ms::kLargeKMax))) any_exact = true;
     else if (!((nucleus || large_k) && fits)) any_other = true;
@@ -679,6 +680,7 @@ int mi355x_topk_scores(mi355x_search_ctx* ctx, void* stream, const void* logits,
   const bool large_k = fits && k > 64 && k <= ms::kLargeKMax;
   const bool exact = vocab > 64 && (!fits || k > ms::kLargeKMax);
   a.exact_kernel = exact ? ms::kExactRows : 0;
+  a.all_offers = k > 4 * ms::kLargeKOneOffer ? 1 : 0;
   PlanStream(ctx, &a, !large_k);
   HIP_TRY(ms_launch_sample(&a, nullptr, !large_k && !exact, false, large_k, s, nullptr));
   return MI355X_OK;

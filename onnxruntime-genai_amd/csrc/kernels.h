@@ -36,6 +36,7 @@ constexpr int kModeTopkLarge = 3;  // 64 < k <= kLargeKMax: streamed and finishe
 // each beyond that (about 1.1 k elements reach the k-th best of those 4096).
 constexpr int kLargeKMax = 8192;
 constexpr int kLargeKOneOffer = 512;  // up to here one offer per thread is enough
+constexpr int kFourOffers = 1, kAllOffers = 2;  // which offers a streaming kernel has code for (the last need a register each)
 
 // Heterogeneous (k, p, T) of a batch of at most kInlineParamRows rows travel inside the kernel
 // arguments, as a second argument of kernel variants of their own, so that no copy to the device
@@ -51,6 +52,7 @@ struct SampleArgs {
   int64_t row_stride;
   int rows, vocab, chunks;
   int chunk_room, chunk_elems;  // top-k and argmax rows: logits a workgroup of the kernel has room for, and those of a chunk (a multiple of 64)
+  int all_offers;       // not 0: some row of large k takes all of its elements for offers
   int rows_first;       // ... not 0: workgroups are numbered chunk by chunk, the rows of one chunk side by side
   int dtype;            // MI355X_F32 / MI355X_F16 / MI355X_BF16 (0 counts as fp32)
   Xform xf;

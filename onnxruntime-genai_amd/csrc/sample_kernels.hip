@@ -1994,8 +1994,6 @@ __global__ __launch_bounds__(kFinishBlock) void exact_rows_rows_kernel(const Sam
 
 }  // namespace ms
 
-MS_STREAM_KERNELS(, float)  // the fp32 streaming kernels live here, next to the finish kernels
-
 extern "C" hipError_t ms_launch_sample(const ms::SampleArgs* a, const ms::InlineParams* table, bool any_other,
                                        bool any_nucleus, bool any_large_k, hipStream_t stream, const ms::WideArgs* wide) {
   const dim3 fgrid(a->rows), fblock(ms::kFinishBlock);

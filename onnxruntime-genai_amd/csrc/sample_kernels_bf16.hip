@@ -2,4 +2,4 @@
 // BFloat16ToFloat32 does, src/models/utils.cpp:84-86).
 #include "sample_stream.h"
 
-MS_STREAM_KERNELS(_bf16, ms::bf16_t)
+MS_STREAM_KERNELS(_bf16, ms::bf16_t, MS_NONE_OF_LARGE_K)

@@ -617,7 +617,8 @@ __device__ __forceinline__ void mask_registers(float (&v)[CHUNK / kSBlock], cons
 // Streaming pass of one (row, chunk) of a top-k<=64 or nucleus row.  Returns true when this workgroup
 // must run the general path for the row (it was the last to arrive and the fast path declined).
 // CHUNK: the logits the workgroup has room for.  A nucleus row's chunks have that many each, the others' chunk_elems.
-template <typename InT, int CHUNK, bool NUCLEUS, bool XFORM, bool LARGEK = false, bool ARGMAX = false>
+// LARGEK: kFourOffers for rows of k <= 4 * kLargeKOneOffer, kAllOffers for any k.
+template <typename InT, int CHUNK, bool NUCLEUS, bool XFORM, int LARGEK = 0, bool ARGMAX = false>
 __device__ __forceinline__ bool stream_row(const SampleArgs& a, int row, const void* row0, int chunk,
                                            mi355x_sample_params prm, FusedShared& sm) {
   constexpr int kSBlock = NUCLEUS ? kNucleusBlock : kTopkBlock;  // threads of this workgroup
@@ -957,7 +958,7 @@ __device__ __forceinline__ bool stream_row(const SampleArgs& a, int row, const v
     static_assert(kLargeKOneOffer <= kSBlock && 4 * kLargeKOneOffer <= 4 * kSBlock && kLargeKMax <= CHUNK && kSElems % 4 == 0,
                   "one offer per thread, four, or every element");
     static_assert(sizeof(sm.wave_list) >= kKthBinWords * sizeof(uint32_t) && kSBlock >= 256, "the selection's bins lie in the hit lists' LDS");
-    constexpr bool large_k = LARGEK;
+    constexpr bool large_k = LARGEK != 0;
     uint32_t cmax = 0u;
     float thr = -__builtin_inff();
     if constexpr (!LARGEK) {
@@ -1022,7 +1023,8 @@ __device__ __forceinline__ bool stream_row(const SampleArgs& a, int row, const v
           }
           return block_kth_largest<G>(best, kk, bins);
         };
-        kth = kk <= 4 * kLargeKOneOffer ? group_maxima(std::integral_constant<int, 4>{}) : group_maxima(std::integral_constant<int, kSElems>{});
+        if (LARGEK != kAllOffers || kk <= 4 * kLargeKOneOffer) kth = group_maxima(std::integral_constant<int, 4>{});
+        else kth = group_maxima(std::integral_constant<int, kSElems>{});
       }
       if (kth != 0u) thr = key_to_float(kth);
     }
@@ -1630,7 +1632,7 @@ __device__ __forceinline__ mi355x_sample_params args_up_front(const SampleArgs& 
   return q;
 }
 
-template <typename InT, int CHUNK, bool INLINE, bool NUCLEUS, bool XFORM, bool LARGEK = false, bool ARGMAX = false>
+template <typename InT, int CHUNK, bool INLINE, bool NUCLEUS, bool XFORM, int LARGEK = 0, bool ARGMAX = false>
 __device__ __forceinline__ void sample_fused_body(const SampleArgs& a) {
   const mi355x_sample_params uniform_prm = args_up_front<XFORM>(a);
   const int row = !NUCLEUS && a.rows_first ? blockIdx.x : blockIdx.y, chunk = !NUCLEUS && a.rows_first ? blockIdx.y : blockIdx.x;
@@ -1666,7 +1668,7 @@ __device__ __forceinline__ void sample_fused_body(const SampleArgs& a) {
 // candidate lists serve any k), and one finish launch ends them.  The modes' own kernels would follow each other on
 // the stream (12 + 42 + 39 us for top-k, nucleus and large-k rows of 64 x 128256), and side by side on streams forked
 // from the caller's the forks and joins cost the host 23 us each, more than the kernels they overlap take.
-template <typename InT, bool INLINE, bool XFORM>
+template <typename InT, bool INLINE, bool XFORM, int LARGEK>
 __device__ __forceinline__ void mixed_stream_body(const SampleArgs& a) {
   const mi355x_sample_params uniform_prm = args_up_front<XFORM>(a);
   const int row = blockIdx.y, chunk = blockIdx.x;
@@ -1678,9 +1680,9 @@ __device__ __forceinline__ void mixed_stream_body(const SampleArgs& a) {
     if constexpr (XFORM) {
       if (a.xf.mask && a.row_done && a.row_done[row] != 0u) return;  // finished by the sparse-mask kernel
     }
-    stream_row<InT, kSChunk, true, XFORM, false>(a, row, row0, chunk, prm, sm);
+    stream_row<InT, kSChunk, true, XFORM>(a, row, row0, chunk, prm, sm);
   } else if (mode == kModeTopkLarge) {
-    stream_row<InT, kSChunk, true, XFORM, true>(a, row, row0, chunk, prm, sm);
+    stream_row<InT, kSChunk, true, XFORM, LARGEK>(a, row, row0, chunk, prm, sm);
   }
 }
 
@@ -1701,68 +1703,86 @@ __device__ __forceinline__ void mixed_stream_body(const SampleArgs& a) {
     sample_fused_body<InT, CHUNK, true, NUCLEUS, XFORM, LARGEK>(a);                                                      \
   }
 
-#define MS_MIXED_KERNEL(NAME, SUFFIX, InT, XFORM)                                                                        \
-  __global__ __launch_bounds__(kNucleusBlock) void NAME##SUFFIX##_kernel(const SampleArgs a) {                           \
-    mixed_stream_body<InT, false, XFORM>(a);                                                                             \
+#define MS_MIXED_KERNEL(NAME, SUFFIX, InT, XFORM, LARGEK, WAVES)                                                                        \
+  __global__ __launch_bounds__(kNucleusBlock, WAVES) void NAME##SUFFIX##_kernel(const SampleArgs a) {                           \
+    mixed_stream_body<InT, false, XFORM, LARGEK>(a);                                                                             \
   }                                                                                                                      \
-  __global__ __launch_bounds__(kNucleusBlock) void NAME##SUFFIX##_rows_kernel(const SampleArgs a, const InlineParams) {  \
-    mixed_stream_body<InT, true, XFORM>(a);                                                                              \
+  __global__ __launch_bounds__(kNucleusBlock, WAVES) void NAME##SUFFIX##_rows_kernel(const SampleArgs a, const InlineParams) {  \
+    mixed_stream_body<InT, true, XFORM, LARGEK>(a);                                                                              \
   }
 
 #define MS_SMALL_K_KERNELS(SUFFIX, InT, CHUNK)                                                                           \
-  MS_STREAM_KERNEL(sample_fused, SUFFIX, InT, CHUNK, false, false, false, 1)                                                \
-  MS_STREAM_KERNEL(sample_fused_xf, SUFFIX, InT, CHUNK, false, true, false, 1)                                              \
+  MS_STREAM_KERNEL(sample_fused, SUFFIX, InT, CHUNK, false, false, 0, 1)                                                \
+  MS_STREAM_KERNEL(sample_fused_xf, SUFFIX, InT, CHUNK, false, true, 0, 1)                                              \
   __global__ __launch_bounds__(kTopkBlock) void argmax_stream##SUFFIX##_kernel(const SampleArgs a) {                     \
-    sample_fused_body<InT, CHUNK, false, false, false, false, true>(a);                                                  \
+    sample_fused_body<InT, CHUNK, false, false, false, 0, true>(a);                                                  \
   }                                                                                                                      \
   __global__ __launch_bounds__(kTopkBlock) void argmax_stream_xf##SUFFIX##_kernel(const SampleArgs a) {                  \
-    sample_fused_body<InT, CHUNK, false, false, true, false, true>(a);                                                   \
+    sample_fused_body<InT, CHUNK, false, false, true, 0, true>(a);                                                   \
   }
 
-// The kernel of a chunk size by its name.
+// The kernels of large-k rows and of rows in several modes fit two workgroups a CU as well where none of the rows takes all of its
+// elements for offers (32 registers) and the logits are fp32: 256 x 201088, k = 1000, both launches, 119.5 -> 93.8 us,
+// 128 x 128256 54.7 -> 46.6, with a penalty 59.6 -> 53.8.  For sixteen-bit logits they spill 25 registers and are slower by a third.
+#define MS_MANY_OF_LARGE_K(SUFFIX, InT)                                                                                  \
+  MS_STREAM_KERNEL(largek_stream_many, SUFFIX, InT, kSChunk, true, false, kFourOffers, 8)                                \
+  MS_STREAM_KERNEL(largek_stream_many_xf, SUFFIX, InT, kSChunk, true, true, kFourOffers, 8)                              \
+  MS_MIXED_KERNEL(mixed_stream_many, SUFFIX, InT, false, kFourOffers, 8)                                                 \
+  MS_MIXED_KERNEL(mixed_stream_many_xf, SUFFIX, InT, true, kFourOffers, 8)
+#define MS_SAME_KERNEL(NAME, SUFFIX, OTHER)                                                                              \
+  constexpr auto* NAME##SUFFIX##_kernel = &OTHER##SUFFIX##_kernel;                                                       \
+  constexpr auto* NAME##SUFFIX##_rows_kernel = &OTHER##SUFFIX##_rows_kernel;
+#define MS_NONE_OF_LARGE_K(SUFFIX, InT)                                                                                  \
+  MS_SAME_KERNEL(largek_stream_many, SUFFIX, largek_stream)                                                              \
+  MS_SAME_KERNEL(largek_stream_many_xf, SUFFIX, largek_stream_xf)                                                        \
+  MS_SAME_KERNEL(mixed_stream_many, SUFFIX, mixed_stream)                                                                \
+  MS_SAME_KERNEL(mixed_stream_many_xf, SUFFIX, mixed_stream_xf)
+
+// The kernel of a chunk size, and the one of nucleus, large-k or mixed rows, by its name.
 #define MS_OF_CHUNK(NAME, SUFFIX, KIND, a)                                                                               \
   ((a)->chunk_room == kSChunk / 4   ? NAME##SUFFIX##_quarter##KIND                                                       \
    : (a)->chunk_room == kSChunk / 2 ? NAME##SUFFIX##_half##KIND                                                          \
                                     : NAME##SUFFIX##KIND)
+#define MS_OF_MANY(NAME, SUFFIX, KIND, xf, many)                                                                         \
+  (many ? (xf ? NAME##_many_xf##SUFFIX##KIND : NAME##_many##SUFFIX##KIND) : (xf ? NAME##_xf##SUFFIX##KIND : NAME##SUFFIX##KIND))
 
 // Defines the streaming kernels of one element type and ms_launch_stream##SUFFIX, which launches the one a call needs:
 // which = 0 rows of every other mode (argmax calls: the argmax kernels), 1 nucleus rows, 2 rows with
 // 64 < k <= kLargeKMax, 3 a call's rows of all three kinds (1 to 3: chunks of kSChunk).
-#define MS_STREAM_KERNELS(SUFFIX, InT)                                                                                   \
+#define MS_STREAM_KERNELS(SUFFIX, InT, MANY_OF_LARGE_K)                                                                                   \
   namespace ms {                                                                                                         \
   MS_SMALL_K_KERNELS(SUFFIX, InT, kSChunk)                                                                               \
   MS_SMALL_K_KERNELS(SUFFIX##_half, InT, kSChunk / 2)                                                                    \
   MS_SMALL_K_KERNELS(SUFFIX##_quarter, InT, kSChunk / 4)                                                                 \
-  MS_STREAM_KERNEL(nucleus_stream, SUFFIX, InT, kSChunk, true, false, false, 1)                                          \
-  MS_STREAM_KERNEL(nucleus_stream_xf, SUFFIX, InT, kSChunk, true, true, false, 1)                                        \
-  MS_STREAM_KERNEL(nucleus_stream_many, SUFFIX, InT, kSChunk, true, false, false, 8)                                     \
-  MS_STREAM_KERNEL(nucleus_stream_many_xf, SUFFIX, InT, kSChunk, true, true, false, 8)                                   \
-  MS_STREAM_KERNEL(largek_stream, SUFFIX, InT, kSChunk, true, false, true, 1)                                            \
-  MS_STREAM_KERNEL(largek_stream_xf, SUFFIX, InT, kSChunk, true, true, true, 1)                                          \
-  MS_MIXED_KERNEL(mixed_stream, SUFFIX, InT, false)                                                                      \
-  MS_MIXED_KERNEL(mixed_stream_xf, SUFFIX, InT, true)                                                                    \
+  MS_STREAM_KERNEL(nucleus_stream, SUFFIX, InT, kSChunk, true, false, 0, 1)                                          \
+  MS_STREAM_KERNEL(nucleus_stream_xf, SUFFIX, InT, kSChunk, true, true, 0, 1)                                        \
+  MS_STREAM_KERNEL(nucleus_stream_many, SUFFIX, InT, kSChunk, true, false, 0, 8)                                     \
+  MS_STREAM_KERNEL(nucleus_stream_many_xf, SUFFIX, InT, kSChunk, true, true, 0, 8)                                   \
+  MS_STREAM_KERNEL(largek_stream, SUFFIX, InT, kSChunk, true, false, kAllOffers, 1)                                      \
+  MS_STREAM_KERNEL(largek_stream_xf, SUFFIX, InT, kSChunk, true, true, kAllOffers, 1)                                    \
+  MS_MIXED_KERNEL(mixed_stream, SUFFIX, InT, false, kAllOffers, 1)                                                       \
+  MS_MIXED_KERNEL(mixed_stream_xf, SUFFIX, InT, true, kAllOffers, 1)                                                     \
+  MANY_OF_LARGE_K(SUFFIX, InT)                                                                                           \
   static hipError_t launch_stream##SUFFIX(const SampleArgs* a, const InlineParams* table, int which, hipStream_t stream) { \
     const dim3 block(which == 0 ? kTopkBlock : kNucleusBlock);                                                           \
     const dim3 grid = which == 0 && a->rows_first ? dim3(a->rows, a->chunks) : dim3(a->chunks, a->rows);                 \
-    const bool xf = a->xf.active(), many = a->rows * static_cast<long long>(a->chunks) > kCus;                           \
+    const bool xf = a->xf.active(), many = a->rows * static_cast<long long>(a->chunks) > kCus, all = a->all_offers != 0; \
     if (which == 0 && a->emit_topk == kEmitArgmax && !table) {                                                           \
       auto* f = xf ? MS_OF_CHUNK(argmax_stream_xf, SUFFIX, _kernel, a) : MS_OF_CHUNK(argmax_stream, SUFFIX, _kernel, a); \
       hipLaunchKernelGGL(f, grid, block, 0, stream, *a);                                                                 \
     } else if (table) {                                                                                                  \
       auto* f = which == 0   ? (xf ? MS_OF_CHUNK(sample_fused_xf, SUFFIX, _rows_kernel, a)                               \
                                    : MS_OF_CHUNK(sample_fused, SUFFIX, _rows_kernel, a))                                 \
-                : which == 1 ? (many ? (xf ? nucleus_stream_many_xf##SUFFIX##_rows_kernel : nucleus_stream_many##SUFFIX##_rows_kernel) \
-                                     : (xf ? nucleus_stream_xf##SUFFIX##_rows_kernel : nucleus_stream##SUFFIX##_rows_kernel)) \
-                : which == 3 ? (xf ? mixed_stream_xf##SUFFIX##_rows_kernel : mixed_stream##SUFFIX##_rows_kernel)         \
-                             : (xf ? largek_stream_xf##SUFFIX##_rows_kernel : largek_stream##SUFFIX##_rows_kernel);      \
+                : which == 1 ? MS_OF_MANY(nucleus_stream, SUFFIX, _rows_kernel, xf, many)                                \
+                : which == 3 ? MS_OF_MANY(mixed_stream, SUFFIX, _rows_kernel, xf, many && !all)                           \
+                             : MS_OF_MANY(largek_stream, SUFFIX, _rows_kernel, xf, many && !all);                         \
       hipLaunchKernelGGL(f, grid, block, 0, stream, *a, *table);                                                         \
     } else {                                                                                                             \
       auto* f = which == 0   ? (xf ? MS_OF_CHUNK(sample_fused_xf, SUFFIX, _kernel, a)                                    \
                                    : MS_OF_CHUNK(sample_fused, SUFFIX, _kernel, a))                                      \
-                : which == 1 ? (many ? (xf ? nucleus_stream_many_xf##SUFFIX##_kernel : nucleus_stream_many##SUFFIX##_kernel) \
-                                     : (xf ? nucleus_stream_xf##SUFFIX##_kernel : nucleus_stream##SUFFIX##_kernel))      \
-                : which == 3 ? (xf ? mixed_stream_xf##SUFFIX##_kernel : mixed_stream##SUFFIX##_kernel)                   \
-                             : (xf ? largek_stream_xf##SUFFIX##_kernel : largek_stream##SUFFIX##_kernel);                \
+                : which == 1 ? MS_OF_MANY(nucleus_stream, SUFFIX, _kernel, xf, many)                                     \
+                : which == 3 ? MS_OF_MANY(mixed_stream, SUFFIX, _kernel, xf, many && !all)                                \
+                             : MS_OF_MANY(largek_stream, SUFFIX, _kernel, xf, many && !all);                              \
       hipLaunchKernelGGL(f, grid, block, 0, stream, *a);                                                                 \
     }                                                                                                                    \
     return hipGetLastError();                                                                                            \

@@ -1143,6 +1143,41 @@ def test_chunks_of_every_size(orc, rows, vocab, dtype):
         c.close()
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("processed", [False, True])
+def test_batches_of_more_workgroups_than_cus(orc, dtype, processed):
+    """Nucleus and large-k rows and rows in several modes are streamed by kernels of their own where there are more workgroups than CUs, and
+    where some k takes every element for an offer: 40 rows of seven chunks."""
+    say("many workgroups", dtype, processed)
+    rows, vocab, cap = 40, 201088, 4096
+    rng = np.random.default_rng(31)
+    x = (torch.randn(rows, vocab, generator=torch.Generator().manual_seed(32)) * 5).to(dtype)
+    hist = rng.integers(0, vocab, (rows, 90)).astype(np.int32)
+    u = rng.random(rows)
+    xf = pkg().LogitsXform(history=torch.from_numpy(hist).cuda(), repetition_penalty=1.2) if processed else None
+    c = pkg().SearchContext(rows, vocab)
+    checked = (0, 17, 39)
+    try:
+        want = {r: x[r].float().numpy() for r in checked}
+        if processed:
+            want = {r: orc.apply_repetition_penalty(want[r], hist[r], 1.2) for r in checked}
+        xd, ud = x.cuda(), torch.from_numpy(u).cuda()
+        several = [(0, 0.8, 1.0), (50, 0.9, 0.7), (300, 0.95, 1.0), (1000, 0.9, 1.0), (1, 0.0, 1.0)]
+        calls = [[one] * rows for one in ((0, 0.8, 1.0), (1000, 0.9, 1.0), (2048, 0.0, 1.0), (3000, 0.9, 1.0))]
+        calls += [[several[r % 5] for r in range(rows)], [several[r % 5] if r != 17 else (2500, 0.95, 1.0) for r in range(rows)]]
+        for params in calls:
+            tok, kc, ki, kp = c.sample(xd, ud, per_row=params, xf=xf, kept_capacity=cap)
+            tok, kc, ki, kp = tok.cpu().numpy(), kc.cpu().numpy(), ki.cpu().numpy(), kp.cpu().numpy()
+            for r in checked:
+                idx, probs = orc.sampled_categorical(want[r], *params[r])
+                n = min(len(idx), cap)
+                assert kc[r] == len(idx) and np.array_equal(ki[r, :n], idx[:n]), (params[r], r)
+                assert np.array_equal(bits(kp[r, :n]), bits(probs[:n])), (params[r], r)
+                assert tok[r] == idx[orc.discrete_draw(probs, u[r])], (params[r], r)
+    finally:
+        c.close()
+
+
 @pytest.mark.parametrize("hist_len", [1500, 2500, 3400, 5000])
 def test_sparse_mask_rows_with_thousands_of_distinct_history_ids(orc, hist_len):
     """Nucleus rows under a sparse grammar mask whose history holds more distinct ids than the sparse-mask kernel's
