@@ -122,6 +122,7 @@ struct mi355x_search_ctx {
   ms::WideRow* wide_rows{};
   uint32_t* wide_tile_start{};
   uint2* wide_cut_bucket{};
+  uint32_t* wide_rest{};
   int32_t* beam_row_tokens{};
   // Pinned host staging for the per-row parameters of more than 64 rows, which come in a caller's HOST array and do
   // not fit the kernel arguments: the call copies the array into a slot here and records a copy from the slot to the
@@ -302,7 +303,9 @@ int mi355x_search_create(int device, int max_rows, int max_vocab, mi355x_search_
   c->max_segs = (max_vocab + ms::kWideTile - 1) / ms::kWideTile;
   static_assert(ms::kWideTile <= ms::kSegElems, "room for either");
   ok(c->Alloc(&c->wide_rows, static_cast<size_t>(max_rows), false));
-  ok(c->Alloc(&c->wide_tile_start, static_cast<size_t>(max_rows) * (c->max_segs + 1), false));
+  const size_t tile_starts = static_cast<size_t>(max_rows) * (c->max_segs + 1);
+  ok(c->Alloc(&c->wide_tile_start, tile_starts + 2 + 3 * static_cast<size_t>(max_rows), false));  // (and what wide_rest counts)
+  if (c->wide_tile_start) c->wide_rest = c->wide_tile_start + tile_starts;
   ok(c->Alloc(&c->wide_cut_bucket, static_cast<size_t>(max_rows) * (c->max_segs + 1), false));
   ok(c->Alloc(&c->seg_max, static_cast<size_t>(max_rows) * c->max_segs, false));
   ok(c->Alloc(&c->seg_sum, static_cast<size_t>(max_rows) * c->max_segs, false));
@@ -536,7 +539,8 @@ int SampleImpl(mi355x_search_ctx* ctx, hipStream_t s, const void* logits, const 
   PlanStream(ctx, &a, !any_nucleus && !any_large_k);
   a.exact_kernel = (any_exact ? ms::kExactRows : 0) | (any_wide ? ms::kWideRows : 0);
   const ms::WideArgs wide{(vocab + ms::kWideChunk - 1) / ms::kWideChunk, tiles, ctx->wide_rows, ctx->wide_tile_start, ctx->wide_cut_bucket, ctx->seg_sum,
-                          ctx->seg_step, ctx->sub_step, ctx->sub_se, ctx->chunk_next, kept_ids == nullptr && kept_count == nullptr};
+                          ctx->seg_step, ctx->sub_step, ctx->sub_se, ctx->chunk_next, kept_ids == nullptr && kept_count == nullptr,
+                          {ctx->wide_rest, ctx->wide_rest + 1, ctx->wide_rest + 2, ctx->wide_rest + 2 + ctx->max_rows, ctx->wide_rest + 2 + 2 * static_cast<size_t>(ctx->max_rows)}};
   // a caller that bounds the number of allowed ids per row lets the sparse-mask kernel work alone
   if (xf && xf->mask && xf->mask_allowed_max > 0) {
     const int hist = a.xf.history_lens ? a.xf.history_stride : a.xf.history_len;

@@ -92,13 +92,21 @@ constexpr int kWideTile = 3072;       // keys after which a new tile begins, wit
 constexpr int kWideBucketMax = 1024;  // keys of a bucket that a tile takes whole
 constexpr int kWideMaxTiles = 192;    // tiles of the longest row (589824 logits)
 constexpr int kWideMinVocab = 4096;   // shorter rows are a single workgroup's work anyway
-constexpr uint32_t kWideDeclined = 1, kWideGivenBack = 2, kWidePicked = 3;
+constexpr int kWideRestBlocks = 256;  // workgroups that do what a pick left: one a CU
+constexpr uint32_t kWideDeclined = 1, kWideGivenBack = 2;
 struct WideRow {
   uint32_t n, tiles;  // listed keys, their tiles
   uint32_t declined;  // kWideDeclined: the row is not one for this path; kWideGivenBack: a tile of it found so (other tiles
-                      // of that launch go on: one that returned would leave those behind it waiting for its sum);
-                      // kWidePicked: wide_pick has found its token
+                      // of that launch go on: one that returned would leave those behind it waiting for its sum)
   float top;          // the row's maximum
+};
+// The rows a pick gave back, and how far the work on them is (wide_rest_kernel).
+struct WideRest {
+  uint32_t* count;      // of listed rows
+  uint32_t* ticket;     // the next piece of work
+  uint32_t* rows;       // [rows]
+  uint32_t* scattered;  // [rows]: chunks done
+  uint32_t* ranked;     // [rows]: tiles done
 };
 struct WideArgs {
   int chunks, max_tiles;
@@ -110,7 +118,8 @@ struct WideArgs {
   int4* sub_step;
   int* sub_se;
   u64* best_below;       // [rows]: the best element past the list, 0: none
-  int pick;              // the token alone is asked for: wide_pick runs
+  int pick;              // the token alone is asked for: wide_pick and wide_rest run
+  WideRest rest;
 };
 struct NoTable {};
 template <bool INLINE>

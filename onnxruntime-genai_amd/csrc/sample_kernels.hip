@@ -2071,6 +2071,12 @@ extern "C" hipError_t ms_sample_init() {
                           reinterpret_cast<const void*>(ms::wide_pick_kernel<uint16_t, true>),
                           reinterpret_cast<const void*>(ms::wide_pick_kernel<ms::bf16_t, false>),
                           reinterpret_cast<const void*>(ms::wide_pick_kernel<ms::bf16_t, true>),
+                          reinterpret_cast<const void*>(ms::wide_rest_kernel<float, false>),
+                          reinterpret_cast<const void*>(ms::wide_rest_kernel<float, true>),
+                          reinterpret_cast<const void*>(ms::wide_rest_kernel<uint16_t, false>),
+                          reinterpret_cast<const void*>(ms::wide_rest_kernel<uint16_t, true>),
+                          reinterpret_cast<const void*>(ms::wide_rest_kernel<ms::bf16_t, false>),
+                          reinterpret_cast<const void*>(ms::wide_rest_kernel<ms::bf16_t, true>),
                           reinterpret_cast<const void*>(ms::wide_scatter_kernel<float, false>),
                           reinterpret_cast<const void*>(ms::wide_scatter_kernel<float, true>),
                           reinterpret_cast<const void*>(ms::wide_scatter_kernel<uint16_t, false>),

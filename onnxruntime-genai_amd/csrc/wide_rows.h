@@ -8,8 +8,8 @@
 // every step but the last is spread over the GPU, in five launches (16 x 128256 fp16: 557 -> 59 us per
 // step on the same rows again and 66 on rows that come from memory: 4.7 + 4.7 + 11.5 + 21.6 + 20 us by a trace; every
 // one of them is a chain of dependent phases of a few barriers each, no launch moves more than 33 MB).  Rows whose token
-// alone is asked for need no order: for p = 1 a launch between 2 and 3 picks it from the histogram (wide_pick_kernel), and
-// the launches behind it find nothing to do for 99.7 % of such rows.
+// alone is asked for need no order: for p = 1 a launch behind 2 picks it from the histogram (wide_pick_kernel), and
+// one launch does 3 to 5 for the rows it gives back (wide_rest_kernel), 0.3 % of such rows.
 //   1. wide_max:     the maximum of every chunk of kWideChunk logits.
 //   2. wide_count:   a histogram per chunk over kWideBuckets buckets, linear in the score below the row's maximum down
 //                    to the depth past which no element can lie inside the kept set.
@@ -41,7 +41,6 @@ namespace ms {
 constexpr int kWideBlock = 1024;
 constexpr int kWidePer = kWideChunk / kWideBlock;  // logits per thread
 constexpr int kWideRankBlock = 512;
-constexpr int kWideRankPer = kSegElems / kWideRankBlock;
 static_assert(kWideTile + kWideBucketMax <= kSegElems, "a tile fits the segment its step record describes");
 
 // Rows of this kind: every element counts, whatever k says (k <= 1) and however large p is.
@@ -158,13 +157,18 @@ __global__ __launch_bounds__(kWideBlock) void wide_max_kernel(const SampleArgs a
   __shared__ uint32_t red[16];
   const WideShare mine = wide_share(w.chunks);
   const int chunk = mine.item, row = mine.row, tid = threadIdx.x;
+  if (blockIdx.x == 0 && tid == 0) *w.rest.count = *w.rest.ticket = 0u;
   if (row >= a.rows || !wide_row(row_params<INLINE>(a, row))) return;
   float v[kWidePer];
   wide_load<InT>(static_cast<const InT*>(row_start<INLINE>(a, row, sizeof(InT))), a.vocab, chunk, v);
-  // (this launch is the first of its sequence: it also marks the sums of the row's tiles as not written)
+  // (this launch is the first of its sequence: it also marks the sums of the row's tiles as not written, and the row's counts of
+  // what wide_rest has done)
   if (chunk == 0) {
     for (int t = tid; t < w.max_tiles; t += kWideBlock) store_sum_bits(w.tile_sum + static_cast<size_t>(row) * w.max_tiles + t, kSumNotReady);
-    if (tid == 0) w.best_below[row] = 0;
+    if (tid == 0) {
+      w.best_below[row] = 0;
+      w.rest.scattered[row] = w.rest.ranked[row] = 0u;
+    }
   }
   float m = -__builtin_inff();
 #pragma unroll
@@ -256,8 +260,8 @@ __global__ __launch_bounds__(kWideBlock, 8) void wide_count_kernel(const SampleA
 // of rows of 128256 and 201088 logits, which go the long way behind this.  (Masses as whole numbers of 2^-43, whose rounding
 // such rows of a few heavy tokens notice: twice as many.)  One workgroup per row: it adds the chunks' histograms up,
 // finds the bucket and looks the row through once more for its keys.  A trace of 16 x 128256 fp16: 3.2 (maximum) + 7.1
-// (counts and masses, 4.8 without these) + 19.2 + 10.5 us, the last for the three launches that find nothing to do; steps
-// 62.9 -> 35.1 us, 64 x 128256 fp16 142 -> 58, 1 x 128256 fp32 50 -> 29, 24 x 201088 bf16 129 -> 51.  A compare of every logit with the two
+// (counts and masses, 4.8 without these) + 19.2 us and what wide_rest takes to find nothing to do; steps, with three launches in its
+// place, 62.9 -> 35.1 us, 64 x 128256 fp16 142 -> 58, 1 x 128256 fp32 50 -> 29, 24 x 201088 bf16 129 -> 51.  A compare of every logit with the two
 // buckets and a load of four chunks at a time instead of eight ahead: 23.0 us for this launch.
 template <typename InT, bool INLINE>
 __global__ __launch_bounds__(kWideBlock) void wide_pick_kernel(const SampleArgs a, const typename WideTable<INLINE>::type, const WideArgs w) {
@@ -270,8 +274,9 @@ __global__ __launch_bounds__(kWideBlock) void wide_pick_kernel(const SampleArgs 
   const mi355x_sample_params prm = row_params<INLINE>(a, row);
   if (!wide_row(prm)) return;
   const uint32_t rmax = wide_row_max(a, w, row);
+  auto give_back = [&] { w.rest.rows[atomicAdd(w.rest.count, 1u)] = static_cast<uint32_t>(row); };
   if (rmax == 0xffffffffu || !(prm.p == 1.0f)) {
-    if (tid == 0) w.rows[row].declined = 0u;
+    if (tid == 0) give_back();
     return;
   }
   // The first of the row's chunks are requested now: they are looked through last.
@@ -312,7 +317,7 @@ __global__ __launch_bounds__(kWideBlock) void wide_pick_kernel(const SampleArgs 
     wave_counts[wave] = n_inc;
   }
   if (__syncthreads_or(nan)) {  // (one that is kept makes all weights NaN: the long way)
-    if (tid == 0) w.rows[row].declined = 0u;
+    if (tid == 0) give_back();
     return;
   }
   const double ws = wave_prefix_sum<double>(lane < 16 ? em::as_double(sh.sums[lane]) : 0.0);
@@ -406,12 +411,12 @@ __global__ __launch_bounds__(kWideBlock) void wide_pick_kernel(const SampleArgs 
     }
   }
   if (tid == 0) {
-    w.rows[row].declined = id != kNoPick ? kWidePicked : 0u;
     if (id != kNoPick) {
       *row_outputs(a, row).token = static_cast<int32_t>(id);
       atomicAdd(a.fallback_rows, 1u);  // (a row of the exact path, spread over the GPU)
     } else {
       atomicAdd(a.fallback_rows + 3, 1u);
+      give_back();
     }
   }
 }
@@ -423,20 +428,13 @@ struct WideScatterShared {
   u64 keys[kWideChunk];
   uint32_t place[kWideBuckets];  // the bucket's next place in keys
   uint32_t shift[kWideBuckets];  // what takes a place in keys to one in the row's buffer
+  uint32_t wave_sums[16], wave_own[16];
+  u64 red64[16];
 };
 template <typename InT, bool INLINE>
-__global__ __launch_bounds__(kWideBlock) void wide_scatter_kernel(const SampleArgs a, const typename WideTable<INLINE>::type, const WideArgs w) {
-  extern __shared__ u64 lds_keys[];
-  WideScatterShared& sh = *reinterpret_cast<WideScatterShared*>(lds_keys);
-  __shared__ uint32_t wave_sums[16], wave_own[16];
-  __shared__ u64 red64[16];
-  const WideShare mine = wide_share(w.chunks);
-  const int chunk = mine.item, row = mine.row, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  if (row >= a.rows) return;
-  const mi355x_sample_params prm = row_params<INLINE>(a, row);
-  if (!wide_row(prm)) return;
+__device__ __forceinline__ void wide_scatter_chunk(const SampleArgs& a, const WideArgs& w, int row, int chunk, mi355x_sample_params prm, WideScatterShared& sh) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   WideRow* const info = w.rows + row;
-  if (w.pick != 0 && info->declined == kWidePicked) return;
   const uint32_t rmax = wide_row_max(a, w, row);
   if (rmax == 0xffffffffu) {
     if (chunk == 0 && tid == 0) *info = WideRow{0u, 0u, kWideDeclined, 0.0f};
@@ -465,11 +463,11 @@ __global__ __launch_bounds__(kWideBlock) void wide_scatter_kernel(const SampleAr
   const uint32_t own0 = own & 0xffffu, own1 = own >> 16;
   const uint32_t inc = wave_prefix_sum<uint32_t>(all0 + all1), own_inc = wave_prefix_sum<uint32_t>(own0 + own1);
   if (lane == 63) {
-    wave_sums[wave] = inc;
-    wave_own[wave] = own_inc;
+    sh.wave_sums[wave] = inc;
+    sh.wave_own[wave] = own_inc;
   }
   __syncthreads();
-  const uint32_t ws = wave_prefix_sum<uint32_t>(lane < 16 ? wave_sums[lane] : 0u), wo = wave_prefix_sum<uint32_t>(lane < 16 ? wave_own[lane] : 0u);
+  const uint32_t ws = wave_prefix_sum<uint32_t>(lane < 16 ? sh.wave_sums[lane] : 0u), wo = wave_prefix_sum<uint32_t>(lane < 16 ? sh.wave_own[lane] : 0u);
   const uint32_t n = wave_read_lane(ws, 15), n_own = wave_read_lane(wo, 15);
   const uint32_t start0 = (wave > 0 ? wave_read_lane(ws, wave - 1) : 0u) + inc - (all0 + all1), start1 = start0 + all0;
   const uint32_t here0 = (wave > 0 ? wave_read_lane(wo, wave - 1) : 0u) + own_inc - (own0 + own1), here1 = here0 + own0;
@@ -516,7 +514,7 @@ __global__ __launch_bounds__(kWideBlock) void wide_scatter_kernel(const SampleAr
     if (b < static_cast<uint32_t>(kWideBuckets)) sh.keys[atomicAdd(&sh.place[b], 1u)] = k;
     else if (v[e] == v[e]) below = k > below ? k : below;
   }
-  below = block_max<u64>(below, red64, false);  // (its barrier: the keys are in their places)
+  below = block_max<u64>(below, sh.red64, false);  // (its barrier: the keys are in their places)
   if (tid == 0 && below != 0) atomicMax(reinterpret_cast<unsigned long long*>(w.best_below + row), static_cast<unsigned long long>(below));
   u64* const keys = a.big2 + static_cast<size_t>(row) * a.big_stride;
 #pragma unroll
@@ -529,9 +527,21 @@ __global__ __launch_bounds__(kWideBlock) void wide_scatter_kernel(const SampleAr
   }
 }
 
+template <typename InT, bool INLINE>
+__global__ __launch_bounds__(kWideBlock) void wide_scatter_kernel(const SampleArgs a, const typename WideTable<INLINE>::type, const WideArgs w) {
+  extern __shared__ u64 lds_keys[];
+  const WideShare mine = wide_share(w.chunks);
+  if (mine.row >= a.rows) return;
+  const mi355x_sample_params prm = row_params<INLINE>(a, mine.row);
+  if (!wide_row(prm)) return;
+  wide_scatter_chunk<InT, INLINE>(a, w, mine.row, mine.item, prm, *reinterpret_cast<WideScatterShared*>(lds_keys));
+}
+
 constexpr int kWideSubBuckets = 4096;
 
-struct WideRankShared {  // 50 KB: three workgroups a CU
+template <int BLOCK>
+struct WideRankShared {  // 50 KB: three workgroups of 512 threads a CU
+  static constexpr int kWaves = BLOCK / 64;
   union {
     u64 keys[kSegElems];                  // by bucket, then in rank order with the exponentials in the score half
     uint32_t first_key[kWideSubBuckets];  // while the keys are counted: the score of the first key of a bucket
@@ -539,29 +549,30 @@ struct WideRankShared {  // 50 KB: three workgroups a CU
   uint32_t start[kWideSubBuckets + 1];
   uint32_t mixed[kWideSubBuckets / 32];  // buckets that hold more than one score
   uint64_t exp_tab[32];
-  uint32_t red[8], red2[8];
-  double dred[8];
-  Step wave_tot[8];
-  u64 low[8], high[8];     // a cut bucket's extremes
+  uint32_t red[kWaves], red2[kWaves];
+  double dred[kWaves];
+  Step wave_tot[kWaves];
+  u64 low[kWaves], high[kWaves];  // a cut bucket's extremes
   uint32_t pick[2], fill;  // the selection's digit and the rank inside it; the next free place in keys
 };
 
 // The key of rank r (from 0, best first) among the m distinct keys at src, whose lowest and highest are given: a
 // selection by twelve bits at a time below the bits all keys share.  (Two or three passes over the bucket: its keys
 // differ in the lower bits of their scores, or in their ids alone.)  Ends with a barrier.
-__device__ __forceinline__ u64 wide_select_key(const u64* src, uint32_t m, uint32_t r, u64 lowest, u64 highest, WideRankShared& sh) {
+template <int BLOCK>
+__device__ __forceinline__ u64 wide_select_key(const u64* src, uint32_t m, uint32_t r, u64 lowest, u64 highest, WideRankShared<BLOCK>& sh) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  constexpr int kDigitBits = 12, kPer = (1 << kDigitBits) / kWideRankBlock;
+  constexpr int kDigitBits = 12, kPer = (1 << kDigitBits) / BLOCK;
   static_assert(1 << kDigitBits == kWideSubBuckets, "the counts take the sub-buckets' place");
   int open = 64 - __clzll(static_cast<long long>(lowest ^ highest));  // bits still to be decided
   u64 prefix = open < 64 ? highest >> open : 0;
   while (open > 0) {
     const int take = open < kDigitBits ? open : kDigitBits, above = open;
     open -= take;
-    for (int d = tid; d < kWideSubBuckets; d += kWideRankBlock) sh.start[d] = 0u;
+    for (int d = tid; d < kWideSubBuckets; d += BLOCK) sh.start[d] = 0u;
     __syncthreads();
 #pragma unroll 4
-    for (uint32_t i = tid; i < m; i += kWideRankBlock) {
+    for (uint32_t i = tid; i < m; i += BLOCK) {
       const u64 k = src[i];
       if ((above < 64 ? k >> above : 0) == prefix) atomicAdd(&sh.start[(k >> open) & ((1u << take) - 1u)], 1u);
     }
@@ -575,7 +586,7 @@ __device__ __forceinline__ u64 wide_select_key(const u64* src, uint32_t m, uint3
     const uint32_t inc = wave_prefix_sum<uint32_t>(local);
     if (lane == 63) sh.red[wave] = inc;
     __syncthreads();
-    const uint32_t ws = wave_prefix_sum<uint32_t>(lane < kWideRankBlock / 64 ? sh.red[lane] : 0u);
+    const uint32_t ws = wave_prefix_sum<uint32_t>(lane < BLOCK / 64 ? sh.red[lane] : 0u);
     uint32_t before = (wave > 0 ? wave_read_lane(ws, wave - 1) : 0u) + inc - local;
 #pragma unroll
     for (int j = 0; j < kPer; ++j) {
@@ -602,8 +613,9 @@ __device__ __forceinline__ u64 wide_select_key(const u64* src, uint32_t m, uint3
 // fp32 rows of sigma 1 at T = 25 take 1014 us a step against 1154 on the exact path, 24 x 128256 at T = 40 368 against
 // 602, one 208 against 537; with all of a row in one or two buckets 24 x 128256 took 1400 to 1800 against 620 to 930.)
 constexpr uint32_t kWideSelectMax = 32768;
+template <int BLOCK>
 __device__ __forceinline__ bool wide_gather_cut(const u64* list, uint32_t first, uint32_t n, uint2 head, uint2 tail, bool order_ties,
-                                                WideRankShared& sh) {
+                                                WideRankShared<BLOCK>& sh) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const uint32_t end = first + n;
   uint32_t done = first;  // the tile's places up to here have their keys
@@ -612,14 +624,14 @@ __device__ __forceinline__ bool wide_gather_cut(const u64* list, uint32_t first,
     const uint2 bucket = side == 0 ? head : tail;
     if (bucket.y == 0u || (side == 1 && bucket.x < done)) continue;  // (a tile inside one bucket has its only share already)
     const uint32_t from = side == 0 ? first : bucket.x, to = bucket.y < end ? bucket.y : end;
-    for (uint32_t i = done + tid; i < from; i += kWideRankBlock) sh.keys[i - first] = list[i];  // the buckets between the two
+    for (uint32_t i = done + tid; i < from; i += BLOCK) sh.keys[i - first] = list[i];  // the buckets between the two
     done = to;
     const u64* const src = list + bucket.x;
     const uint32_t m = bucket.y - bucket.x;
     if (m > kWideSelectMax) {  // (all of its tiles together see whether it has one score)
       int differs = order_ties ? 1 : 0;
       const uint32_t score = key64_okey(src[0]);
-      for (uint32_t i = from + tid; i < to && !order_ties; i += kWideRankBlock) {
+      for (uint32_t i = from + tid; i < to && !order_ties; i += BLOCK) {
         const u64 k = list[i];
         sh.keys[i - first] = k;
         differs |= key64_okey(k) != score ? 1 : 0;
@@ -629,7 +641,7 @@ __device__ __forceinline__ bool wide_gather_cut(const u64* list, uint32_t first,
     }
     u64 highest = 0, below = 0;  // (below: complement of the lowest)
 #pragma unroll 4
-    for (uint32_t i = tid; i < m; i += kWideRankBlock) {
+    for (uint32_t i = tid; i < m; i += BLOCK) {
       const u64 k = src[i];
       highest = k > highest ? k : highest;
       below = ~k > below ? ~k : below;
@@ -642,10 +654,10 @@ __device__ __forceinline__ bool wide_gather_cut(const u64* list, uint32_t first,
     }
     if (tid == 0) sh.fill = from - first;
     __syncthreads();
-    highest = row16_max<u64>(lane < kWideRankBlock / 64 ? sh.high[lane] : 0);
-    const u64 lowest = ~row16_max<u64>(lane < kWideRankBlock / 64 ? sh.low[lane] : 0);
+    highest = row16_max<u64>(lane < BLOCK / 64 ? sh.high[lane] : 0);
+    const u64 lowest = ~row16_max<u64>(lane < BLOCK / 64 ? sh.low[lane] : 0);
     if (!order_ties && key64_okey(lowest) == key64_okey(highest)) {
-      for (uint32_t i = from + tid; i < to; i += kWideRankBlock) sh.keys[i - first] = list[i];
+      for (uint32_t i = from + tid; i < to; i += BLOCK) sh.keys[i - first] = list[i];
     } else {
       u64 best = highest, last = lowest;
 #pragma unroll 1
@@ -655,14 +667,14 @@ __device__ __forceinline__ bool wide_gather_cut(const u64* list, uint32_t first,
         if (e == 0) best = key;
         else last = key;
       }
-      for (uint32_t i = tid; i < m; i += kWideRankBlock) {
+      for (uint32_t i = tid; i < m; i += BLOCK) {
         const u64 k = src[i];
         if (k <= best && k >= last) sh.keys[atomicAdd(&sh.fill, 1u)] = k;
       }
     }
     __syncthreads();
   }
-  for (uint32_t i = done + tid; i < end; i += kWideRankBlock) sh.keys[i - first] = list[i];
+  for (uint32_t i = done + tid; i < end; i += BLOCK) sh.keys[i - first] = list[i];
   __syncthreads();
   return true;
 }
@@ -672,16 +684,12 @@ __device__ __forceinline__ bool wide_gather_cut(const u64* list, uint32_t first,
 // 190 and 188 us a step for runs of up to 270 ties, 195 and 202 for runs of up to 400, 208 and 594 for runs of 1600.)
 constexpr uint32_t kWideRankCap = 256;
 
-template <bool INLINE>
-__global__ __launch_bounds__(kWideRankBlock) void wide_rank_kernel(const SampleArgs a, const typename WideTable<INLINE>::type, const WideArgs w) {
-  __shared__ WideRankShared sh;
-  const WideShare mine_of_rows = wide_share(w.max_tiles);
-  const int t = mine_of_rows.item, row = mine_of_rows.row, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  if (row >= a.rows) return;
-  const mi355x_sample_params prm = row_params<INLINE>(a, row);
-  if (!wide_row(prm)) return;
+template <int BLOCK>
+__device__ __forceinline__ void wide_rank_tile(const SampleArgs& a, const WideArgs& w, int row, int t, mi355x_sample_params prm, WideRankShared<BLOCK>& sh) {
+  constexpr int kPerThread = kSegElems / BLOCK;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const WideRow info = w.rows[row];
-  if (info.declined == kWideDeclined || info.declined == kWidePicked || static_cast<uint32_t>(t) >= info.tiles) return;
+  if (info.declined == kWideDeclined || static_cast<uint32_t>(t) >= info.tiles) return;
   const uint32_t* const tile = w.tile_start + static_cast<size_t>(row) * (w.max_tiles + 1) + t;
   const uint32_t first = tile[0], n = tile[1] - first;
   const u64* const keys = a.big2 + static_cast<size_t>(row) * a.big_stride;
@@ -689,13 +697,13 @@ __global__ __launch_bounds__(kWideRankBlock) void wide_rank_kernel(const SampleA
   const uint2 head = cut[0], tail = cut[1];
   const bool order_ties = a.kept_ids != nullptr;
   const u64* const src = keys + first;
-  u64 k[kWideRankPer];
+  u64 k[kPerThread];
 #pragma unroll
-  for (int r = 0; r < kWideRankPer; ++r) {
-    const uint32_t i = static_cast<uint32_t>(r * kWideRankBlock + tid);
+  for (int r = 0; r < kPerThread; ++r) {
+    const uint32_t i = static_cast<uint32_t>(r * BLOCK + tid);
     k[r] = i < n ? src[i] : 0;
   }
-  for (int b = tid; b <= kWideSubBuckets; b += kWideRankBlock) sh.start[b] = 0u;
+  for (int b = tid; b <= kWideSubBuckets; b += BLOCK) sh.start[b] = 0u;
   if (tid < kWideSubBuckets / 32) sh.mixed[tid] = 0u;
   if (tid >= 64 && tid < 96) sh.exp_tab[tid - 64] = em::exp2_tab(static_cast<uint32_t>(tid - 64));
   if (__builtin_expect((head.y | tail.y) != 0u, 0)) {  // (its code lies behind the kernel's: in line it makes every row's launch 0.7 us longer)
@@ -708,15 +716,15 @@ __global__ __launch_bounds__(kWideRankBlock) void wide_rank_kernel(const SampleA
       return;
     }
 #pragma unroll
-    for (int r = 0; r < kWideRankPer; ++r) {
-      const uint32_t i = static_cast<uint32_t>(r * kWideRankBlock + tid);
+    for (int r = 0; r < kPerThread; ++r) {
+      const uint32_t i = static_cast<uint32_t>(r * BLOCK + tid);
       k[r] = i < n ? sh.keys[i] : 0;
     }
-    for (int b = tid; b <= kWideSubBuckets; b += kWideRankBlock) sh.start[b] = 0u;
+    for (int b = tid; b <= kWideSubBuckets; b += BLOCK) sh.start[b] = 0u;
   }
   uint32_t hi = 0u, lo = 0xffffffffu;
 #pragma unroll
-  for (int r = 0; r < kWideRankPer; ++r) {
+  for (int r = 0; r < kPerThread; ++r) {
     const uint32_t o = key64_okey(k[r]);
     hi = o > hi ? o : hi;
     if (k[r] != 0) lo = o < lo ? o : lo;
@@ -728,8 +736,8 @@ __global__ __launch_bounds__(kWideRankBlock) void wide_rank_kernel(const SampleA
     sh.red2[wave] = lo;
   }
   __syncthreads();
-  hi = row16_max<uint32_t>(lane < kWideRankBlock / 64 ? sh.red[lane] : 0u);
-  lo = ~row16_max<uint32_t>(lane < kWideRankBlock / 64 ? ~sh.red2[lane] : 0u);
+  hi = row16_max<uint32_t>(lane < BLOCK / 64 ? sh.red[lane] : 0u);
+  lo = ~row16_max<uint32_t>(lane < BLOCK / 64 ? ~sh.red2[lane] : 0u);
   const float top = key_to_float(hi), span = top - key_to_float(lo);
   const float scale = span > 0.0f ? static_cast<float>(kWideSubBuckets) / span : 0.0f;
   auto bucket_of = [=](u64 key) {
@@ -737,9 +745,9 @@ __global__ __launch_bounds__(kWideRankBlock) void wide_rank_kernel(const SampleA
     bf = bf < static_cast<float>(kWideSubBuckets - 1) ? bf : static_cast<float>(kWideSubBuckets - 1);
     return bf > 0.0f ? static_cast<uint32_t>(bf) : 0u;
   };
-  uint32_t slot[kWideRankPer];
+  uint32_t slot[kPerThread];
 #pragma unroll
-  for (int r = 0; r < kWideRankPer; ++r) {
+  for (int r = 0; r < kPerThread; ++r) {
     if (k[r] != 0) {
       const uint32_t b = bucket_of(k[r]);
       slot[r] = atomicAdd(&sh.start[b], 1u);
@@ -748,7 +756,7 @@ __global__ __launch_bounds__(kWideRankBlock) void wide_rank_kernel(const SampleA
   }
   __syncthreads();
 #pragma unroll
-  for (int r = 0; r < kWideRankPer; ++r) {
+  for (int r = 0; r < kPerThread; ++r) {
     if (k[r] != 0 && slot[r] != 0u) {
       const uint32_t b = bucket_of(k[r]);
       if (sh.first_key[b] != key64_okey(k[r])) atomicOr(&sh.mixed[b >> 5], 1u << (b & 31u));
@@ -756,7 +764,7 @@ __global__ __launch_bounds__(kWideRankBlock) void wide_rank_kernel(const SampleA
   }
   bool crowded;  // some bucket holds more than kWideRankCap keys
   {  // the buckets' first places: eight consecutive buckets per thread
-    constexpr int kPer = kWideSubBuckets / kWideRankBlock;
+    constexpr int kPer = kWideSubBuckets / BLOCK;
     constexpr uint32_t kCrowded = 1u << 31;
     uint32_t cnt[kPer], local = 0u, most = 0u;
 #pragma unroll
@@ -769,7 +777,7 @@ __global__ __launch_bounds__(kWideRankBlock) void wide_rank_kernel(const SampleA
     const bool crowded_wave = __ballot(most > kWideRankCap) != 0;
     if (lane == 63) sh.red[wave] = inc | (crowded_wave ? kCrowded : 0u);
     __syncthreads();
-    const uint32_t of_wave = lane < kWideRankBlock / 64 ? sh.red[lane] : 0u;
+    const uint32_t of_wave = lane < BLOCK / 64 ? sh.red[lane] : 0u;
     crowded = __ballot((of_wave & kCrowded) != 0u) != 0;
     const uint32_t ws = wave_prefix_sum<uint32_t>(of_wave & ~kCrowded);
     uint32_t c = (wave > 0 ? wave_read_lane(ws, wave - 1) : 0u) + inc - local;
@@ -778,11 +786,11 @@ __global__ __launch_bounds__(kWideRankBlock) void wide_rank_kernel(const SampleA
       sh.start[tid * kPer + i] = c;
       c += cnt[i];
     }
-    if (tid == kWideRankBlock - 1) sh.start[kWideSubBuckets] = c;
+    if (tid == BLOCK - 1) sh.start[kWideSubBuckets] = c;
   }
   __syncthreads();
 #pragma unroll
-  for (int r = 0; r < kWideRankPer; ++r)
+  for (int r = 0; r < kPerThread; ++r)
     if (k[r] != 0) sh.keys[sh.start[bucket_of(k[r])] + slot[r]] = k[r];
   __syncthreads();
   // Ranks, place by place (the lanes of a wave then look at the same few buckets).  A bucket of one score is in order
@@ -792,8 +800,8 @@ __global__ __launch_bounds__(kWideRankBlock) void wide_rank_kernel(const SampleA
   if (__builtin_expect(crowded, 0)) {
     int too_full = 0;
 #pragma unroll
-    for (int r = 0; r < kWideRankPer; ++r) {
-      const uint32_t p = static_cast<uint32_t>(r * kWideRankBlock + tid);
+    for (int r = 0; r < kPerThread; ++r) {
+      const uint32_t p = static_cast<uint32_t>(r * BLOCK + tid);
       if (p < n) {
         const uint32_t b = bucket_of(sh.keys[p]);
         if (sh.start[b + 1u] - sh.start[b] > kWideRankCap && must_rank(b)) too_full = 1;
@@ -804,10 +812,10 @@ __global__ __launch_bounds__(kWideRankBlock) void wide_rank_kernel(const SampleA
     by_network = __syncthreads_or(too_full) != 0;
     if (by_network) block_sort_desc(sh.keys, kSegElems);
   }
-  uint32_t fin[kWideRankPer];
+  uint32_t fin[kPerThread];
 #pragma unroll
-  for (int r = 0; r < kWideRankPer; ++r) {
-    const uint32_t p = static_cast<uint32_t>(r * kWideRankBlock + tid);
+  for (int r = 0; r < kPerThread; ++r) {
+    const uint32_t p = static_cast<uint32_t>(r * BLOCK + tid);
     k[r] = 0;
     fin[r] = p;
     if (p < n) {
@@ -827,7 +835,7 @@ __global__ __launch_bounds__(kWideRankBlock) void wide_rank_kernel(const SampleA
   auto lds_tab = [=](uint32_t i) { return tab[i]; };
   double part = 0.0;
 #pragma unroll
-  for (int r = 0; r < kWideRankPer; ++r) {
+  for (int r = 0; r < kPerThread; ++r) {
     const float e = k[r] != 0 ? em::expf_core((key_to_float(key64_okey(k[r])) - info.top) * inv_temp, lds_tab) : 0.0f;
     part += static_cast<double>(e);
     sh.keys[exp_slot(fin[r])] = (static_cast<u64>(__float_as_uint(e)) << 32) | (k[r] & 0xffffffffull);  // (zeros past the tile's end)
@@ -835,19 +843,19 @@ __global__ __launch_bounds__(kWideRankBlock) void wide_rank_kernel(const SampleA
   part = wave_sum<double>(part);
   if (lane == 0) sh.dred[wave] = part;
   __syncthreads();
-  const double own = wave_read_lane(row_scan_add(lane < kWideRankBlock / 64 ? sh.dred[lane] : 0.0), kWideRankBlock / 64 - 1);
+  const double own = wave_read_lane(row_scan_add(lane < BLOCK / 64 ? sh.dred[lane] : 0.0), BLOCK / 64 - 1);
   double* const sums = w.tile_sum + static_cast<size_t>(row) * w.max_tiles;
   if (tid == 0) store_sum_bits(sums + t, static_cast<unsigned long long>(__double_as_longlong(own)));
   u64* const dst = a.big + static_cast<size_t>(row) * a.big_stride + first;
 #pragma unroll
-  for (int r = 0; r < kWideRankPer; ++r) {
-    const uint32_t p = static_cast<uint32_t>(r * kWideRankBlock + tid);
+  for (int r = 0; r < kPerThread; ++r) {
+    const uint32_t p = static_cast<uint32_t>(r * BLOCK + tid);
     if (p < n) dst[p] = sh.keys[exp_slot(p)];
   }
   // the exact sum's step record, as in seqsum_exp_step_body: the sums of the tiles before this one tell the binade
   double before = 0.0;
   bool gave_up = false;
-  for (int s = tid; s < t; s += kWideRankBlock) {
+  for (int s = tid; s < t; s += BLOCK) {
     unsigned long long bits = load_sum_bits(sums + s);
     for (int spins = 0; bits == kSumNotReady && spins < a.poll_limit; ++spins) {
       __builtin_amdgcn_s_sleep(1);
@@ -860,7 +868,7 @@ __global__ __launch_bounds__(kWideRankBlock) void wide_rank_kernel(const SampleA
   before = wave_sum<double>(before);
   if (lane == 0) sh.dred[wave] = before;
   __syncthreads();
-  before = wave_read_lane(row_scan_add(lane < kWideRankBlock / 64 ? sh.dred[lane] : 0.0), kWideRankBlock / 64 - 1);
+  before = wave_read_lane(row_scan_add(lane < BLOCK / 64 ? sh.dred[lane] : 0.0), BLOCK / 64 - 1);
   const size_t rec_at = static_cast<size_t>(row) * w.max_tiles + t;
   int4* const rec = w.tile_step + rec_at;
   if (gave_up) {
@@ -871,24 +879,25 @@ __global__ __launch_bounds__(kWideRankBlock) void wide_rank_kernel(const SampleA
     }
     return;
   }
-  float ev[kWideRankPer];
+  float ev[kPerThread];
 #pragma unroll
-  for (int j = 0; j < kWideRankPer; ++j)
-    ev[j] = __uint_as_float(static_cast<uint32_t>(sh.keys[exp_slot(static_cast<uint32_t>(tid * kWideRankPer + j))] >> 32));
+  for (int j = 0; j < kPerThread; ++j)
+    ev[j] = __uint_as_float(static_cast<uint32_t>(sh.keys[exp_slot(static_cast<uint32_t>(tid * kPerThread + j))] >> 32));
   const float lo_f = __double2float_rd(before * (1.0 - seq_drift(static_cast<int>(first))));
   const float hi_f = __double2float_ru((before + own) * (1.0 + seq_drift(static_cast<int>(first + n))));
   const int se = seq_decompose(lo_f).se;
   const bool known = lo_f > 0.0f && hi_f < 3.0e38f && seq_decompose(hi_f).se == se;
   if (!known) {
-    // powers of two may fall inside the tile: records per part of 64 elements, eight lanes each
-    constexpr int kPartLanes = kWalkPart / kWideRankPer;
-    static_assert(kPartLanes == 8 && kSegSubs * kPartLanes == kWideRankBlock, "a part is eight lanes");
+    // powers of two may fall inside the tile: records per part of 64 elements, eight or sixteen lanes each
+    constexpr int kPartLanes = kWalkPart / kPerThread;
+    static_assert((kPartLanes == 8 || kPartLanes == 16) && kSegSubs * kPartLanes == BLOCK, "a part is eight or sixteen lanes");
     double mine = 0.0;
 #pragma unroll
-    for (int j = 0; j < kWideRankPer; ++j) mine += static_cast<double>(ev[j]);
+    for (int j = 0; j < kPerThread; ++j) mine += static_cast<double>(ev[j]);
     mine += __longlong_as_double(static_cast<long long>(lane_xor64<1>(static_cast<u64>(__double_as_longlong(mine)))));
     mine += __longlong_as_double(static_cast<long long>(lane_xor64<2>(static_cast<u64>(__double_as_longlong(mine)))));
     mine += __longlong_as_double(static_cast<long long>(lane_xor64<4>(static_cast<u64>(__double_as_longlong(mine)))));
+    if constexpr (kPartLanes == 16) mine += __longlong_as_double(static_cast<long long>(lane_xor64<8>(static_cast<u64>(__double_as_longlong(mine)))));
     const int part_i = tid / kPartLanes;
     const double upto = wave_prefix_sum<double>((lane & (kPartLanes - 1)) == 0 ? mine : 0.0);
     __syncthreads();
@@ -904,11 +913,11 @@ __global__ __launch_bounds__(kWideRankBlock) void wide_rank_kernel(const SampleA
     if (!(plo > 0.0f && phi < 3.0e38f && pse_end <= pse + 1)) pse = -1;  // the walk adds this part itself
     Step lo_step{0u, 0u}, hi_step{0u, 0u};
     if (pse >= 0) {
-      lo_step = seq_compose_run(ev, kWideRankPer, pse);
-      hi_step = seq_compose_run(ev, kWideRankPer, pse + 1);
+      lo_step = seq_compose_run(ev, kPerThread, pse);
+      hi_step = seq_compose_run(ev, kPerThread, pse + 1);
     }
-    lo_step = oct_scan_steps(lo_step);
-    hi_step = oct_scan_steps(hi_step);
+    lo_step = group_scan_steps<kPartLanes>(lo_step);
+    hi_step = group_scan_steps<kPartLanes>(hi_step);
     if ((lane & (kPartLanes - 1)) == kPartLanes - 1) {
       const size_t at = rec_at * kSegSubs + part_i;
       w.sub_step[at] = make_int4(static_cast<int>(lo_step.d0), static_cast<int>(lo_step.d1), static_cast<int>(hi_step.d0),
@@ -918,14 +927,24 @@ __global__ __launch_bounds__(kWideRankBlock) void wide_rank_kernel(const SampleA
     if (tid == 0) *rec = make_int4(0, 0, -2, 0);
     return;
   }
-  const Step inc = wave_scan_steps(seq_compose_run(ev, kWideRankPer, se));
+  const Step inc = wave_scan_steps(seq_compose_run(ev, kPerThread, se));
   if (lane == 63) sh.wave_tot[wave] = inc;
   __syncthreads();
   if (tid == 0) {
     Step s = sh.wave_tot[0];
-    for (int w = 1; w < kWideRankBlock / 64; ++w) s = step_compose(s, sh.wave_tot[w]);
+    for (int w = 1; w < BLOCK / 64; ++w) s = step_compose(s, sh.wave_tot[w]);
     *rec = make_int4(static_cast<int>(s.d0), static_cast<int>(s.d1), se, 0);
   }
+}
+
+template <bool INLINE>
+__global__ __launch_bounds__(kWideRankBlock) void wide_rank_kernel(const SampleArgs a, const typename WideTable<INLINE>::type, const WideArgs w) {
+  __shared__ WideRankShared<kWideRankBlock> sh;
+  const WideShare mine = wide_share(w.max_tiles);
+  if (mine.row >= a.rows) return;
+  const mi355x_sample_params prm = row_params<INLINE>(a, mine.row);
+  if (!wide_row(prm)) return;
+  wide_rank_tile<kWideRankBlock>(a, w, mine.row, mine.item, prm, sh);
 }
 
 // The tiles of a row as the walk reads them.
@@ -1197,22 +1216,89 @@ __device__ __forceinline__ bool wide_finish_row(const SampleArgs& a, const WideA
   return true;
 }
 
+struct WideFinishReds {
+  SeqShared seq;
+  uint32_t red32[16];
+  u64 red64[16];
+};
 template <bool INLINE>
-__global__ __launch_bounds__(kFinishBlock) void wide_finish_kernel(const SampleArgs a, const typename WideTable<INLINE>::type, const WideArgs w) {
-  extern __shared__ u64 lds_keys[];
-  __shared__ SeqShared seqsh;
-  __shared__ uint32_t red32[16];
-  __shared__ u64 red64[16];
-  const int row = blockIdx.x;
-  const mi355x_sample_params prm = row_params<INLINE>(a, row);
-  if (!wide_row(prm) || w.rows[row].declined == kWidePicked) return;
-  if (wide_finish_row<INLINE>(a, w, row, prm, *reinterpret_cast<WideFinishShared*>(lds_keys), seqsh)) {
+__device__ __forceinline__ void wide_finish_or_sort(const SampleArgs& a, const WideArgs& w, int row, mi355x_sample_params prm, u64* lds, WideFinishReds& reds) {
+  if (wide_finish_row<INLINE>(a, w, row, prm, *reinterpret_cast<WideFinishShared*>(lds), reds.seq)) {
     if (threadIdx.x == 0) atomicAdd(a.fallback_rows, 1u);  // (a row of the exact path, spread over the GPU)
     return;
   }
   __syncthreads();
-  general_row<AnyDtype, SortWithTile, 8>(a, row, row_start<INLINE>(a, row, dtype_bytes(a.dtype)), prm, a.big + static_cast<size_t>(row) * a.big_stride, seqsh,
-                                         SortWithTile{a.big2 + static_cast<size_t>(row) * a.big_stride, lds_keys, red32, red64});
+  general_row<AnyDtype, SortWithTile, 8>(a, row, row_start<INLINE>(a, row, dtype_bytes(a.dtype)), prm, a.big + static_cast<size_t>(row) * a.big_stride, reds.seq,
+                                         SortWithTile{a.big2 + static_cast<size_t>(row) * a.big_stride, lds, reds.red32, reds.red64});
+}
+
+template <bool INLINE>
+__global__ __launch_bounds__(kFinishBlock) void wide_finish_kernel(const SampleArgs a, const typename WideTable<INLINE>::type, const WideArgs w) {
+  extern __shared__ u64 lds_keys[];
+  __shared__ WideFinishReds reds;
+  const int row = blockIdx.x;
+  const mi355x_sample_params prm = row_params<INLINE>(a, row);
+  if (!wide_row(prm)) return;
+  wide_finish_or_sort<INLINE>(a, w, row, prm, lds_keys, reds);
+}
+
+// What wide_scatter, wide_rank and wide_finish do, in one launch, for the rows that wide_pick has listed: seldom any, and
+// then the launch is all there is to pay.  (Means over 24 inputs, three launches that mostly find nothing to do and this one:
+// 16 x 128256 fp16 39.2 -> 33.9 us a step, 64 x 128256 68.9 -> 57.3, 1 x 128256 fp32 30.6 -> 26.3, 256 x 32064 fp32 73.3 -> 62.5; a single
+// row that is given back 57.8 -> 58.1.  Batches of which every row is given back pay for it, with one workgroup a CU and a hand-over per
+// tile: 16 x 128256 of N(0, 0.02^2) 812 -> 870, 64 x 128256 1208 -> 1432, 256 x 32064 with a NaN in every row 168 -> 287.  With every wave
+// writing the caches back and invalidating them, not one, that was 2364, and the single row 102.)
+// The chunks of all rows and their tiles behind them are numbered; every workgroup takes the next number until none is left,
+// and finishes the listed row of its own index.  Tiles wait for chunks, which have lower numbers: workgroups that run have
+// taken these, and wait for nothing.  A finish waits with no number in hand.  So every wait ends, however many workgroups
+// the GPU has room for.  (The finish is not numbered as well, in one loop with the rest: what the compiler then keeps in registers
+// over the loop takes all 128 of them and 700 bytes of scratch.)
+template <typename InT, bool INLINE>
+__global__ __launch_bounds__(kWideBlock) void wide_rest_kernel(const SampleArgs a, const typename WideTable<INLINE>::type, const WideArgs w) {
+  extern __shared__ u64 lds_keys[];
+  __shared__ WideFinishReds reds;
+  __shared__ uint32_t next;
+  static_assert(kWideBlock == kFinishBlock && sizeof(WideRankShared<kWideBlock>) <= kFinishLds, "one shape for all three");
+  const uint32_t listed = *w.rest.count;
+  if (listed == 0u) return;
+  const uint32_t chunks = static_cast<uint32_t>(w.chunks), tiles = static_cast<uint32_t>(w.max_tiles);
+  auto take = [&] {
+    __syncthreads();
+    if (threadIdx.x == 0) next = atomicAdd(w.rest.ticket, 1u);
+    __syncthreads();
+    return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(next));
+  };
+  auto listed_row = [&](uint32_t i) { return static_cast<int>(__builtin_amdgcn_readfirstlane(w.rest.rows[i])); };
+  // One wave waits and invalidates, one writes back: the caches are the CU's and the XCD's.
+  auto wait_for = [](const uint32_t* count, uint32_t all) {
+    if (threadIdx.x == 0) {
+      while (__hip_atomic_load(count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < all) __builtin_amdgcn_s_sleep(2);
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    }
+    __syncthreads();
+  };
+  auto done = [](uint32_t* count) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // every wave's own stores are in the XCD's L2 ...
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);  // ... and one of them has it written back
+  };
+  uint32_t item = take();
+  for (; item < listed * chunks; item = take()) {
+    const int row = listed_row(item / chunks);
+    wide_scatter_chunk<InT, INLINE>(a, w, row, static_cast<int>(item % chunks), row_params<INLINE>(a, row), *reinterpret_cast<WideScatterShared*>(lds_keys));
+    done(w.rest.scattered + row);
+  }
+  for (; item < listed * (chunks + tiles); item = take()) {
+    const uint32_t i = item - listed * chunks;
+    const int row = listed_row(i / tiles);
+    wait_for(w.rest.scattered + row, chunks);
+    wide_rank_tile<kWideBlock>(a, w, row, static_cast<int>(i % tiles), row_params<INLINE>(a, row), *reinterpret_cast<WideRankShared<kWideBlock>*>(lds_keys));
+    done(w.rest.ranked + row);
+  }
+  if (blockIdx.x >= listed) return;
+  const int row = listed_row(blockIdx.x);
+  wait_for(w.rest.ranked + row, tiles);
+  wide_finish_or_sort<INLINE>(a, w, row, row_params<INLINE>(a, row), lds_keys, reds);
 }
 
 template <bool INLINE>
@@ -1223,12 +1309,18 @@ hipError_t launch_wide(const SampleArgs& a, const typename WideTable<INLINE>::ty
     typedef decltype(elt) InT;
     hipLaunchKernelGGL((wide_max_kernel<InT, INLINE>), grid, block, 0, stream, a, table, w);
     hipLaunchKernelGGL((wide_count_kernel<InT, INLINE>), grid, block, 0, stream, a, table, w);
-    if (w.pick != 0) hipLaunchKernelGGL((wide_pick_kernel<InT, INLINE>), dim3(a.rows), block, kFinishLds, stream, a, table, w);
-    hipLaunchKernelGGL((wide_scatter_kernel<InT, INLINE>), grid, block, sizeof(WideScatterShared), stream, a, table, w);
+    if (w.pick != 0) {
+      hipLaunchKernelGGL((wide_pick_kernel<InT, INLINE>), dim3(a.rows), block, kFinishLds, stream, a, table, w);
+      const int items = a.rows * w.max_tiles, most = a.rows > kWideRestBlocks ? a.rows : kWideRestBlocks;  // (a workgroup per row at least)
+      hipLaunchKernelGGL((wide_rest_kernel<InT, INLINE>), dim3(items < most ? items : most), block, kFinishLds, stream, a, table, w);
+    } else {
+      hipLaunchKernelGGL((wide_scatter_kernel<InT, INLINE>), grid, block, sizeof(WideScatterShared), stream, a, table, w);
+    }
   };
   if (a.dtype == MI355X_F16) passes(uint16_t{});
   else if (a.dtype == MI355X_BF16) passes(bf16_t{});
   else passes(float{});
+  if (w.pick != 0) return hipGetLastError();
   hipLaunchKernelGGL(wide_rank_kernel<INLINE>, dim3(w.max_tiles * rows8), dim3(kWideRankBlock), 0, stream, a, table, w);
   hipLaunchKernelGGL(wide_finish_kernel<INLINE>, dim3(a.rows), dim3(kFinishBlock), kFinishLds, stream, a, table, w);
   return hipGetLastError();

@@ -1731,6 +1731,41 @@ def test_whole_vocabulary_draws_on_the_edges_of_their_guard_bands(ctx, orc, voca
     assert np.array_equal(tokens_only(ctx, x, us, 0, 1.0, t), orc.sample_batch(x.astype(np.float32), 0, 1.0, t, us))
 
 
+@pytest.mark.parametrize("rows,vocab,dtype", [(1, 4099, torch.float32), (9, 50257, torch.float16), (40, 20011, torch.bfloat16), (300, 4099, torch.float32)])
+def test_rows_given_back_by_the_pick_are_finished_in_one_launch(orc, rows, vocab, dtype):
+    """Temperature-only rows that the pick gives back, their draws on cumulative values: one of them, some among others, all, and more
+    than there are workgroups at once; eagerly and from a graph that is replayed with eager calls between."""
+    say("rows given back", rows, vocab, dtype)
+    ctx = pkg().SearchContext(rows, vocab)
+    rng = np.random.default_rng(rows)
+    x = (2.0 * rng.standard_normal((rows, vocab))).astype(np.float32)
+    if rows == 40:
+        x[4, :] = -1e38
+        x[5, 11] = np.inf
+    xd = torch.from_numpy(x).cuda().to(dtype)
+    xw = xd.float().cpu().numpy()
+    u = rng.random(rows)
+    open_draws = [r for r in range(0, rows, 1 if rows in (1, 300) else 3) if r not in (4, 5)]
+    for r in open_draws:
+        _, probs = orc.sampled_categorical(xw[r], 0, 1.0, 0.9)
+        cp = np.cumsum(np.asarray(probs, np.float64))
+        u[r] = cp[int(rng.integers(len(cp) // 100, len(cp) // 2))] / cp[-1]
+    ud = torch.from_numpy(u).cuda()
+    want = orc.sample_batch(xw, 0, 1.0, 0.9, u)
+    for _ in range(3):
+        assert np.array_equal(ctx.sample(xd, ud, k=0, p=1.0, temperature=0.9).cpu().numpy(), want)
+    out = torch.zeros(rows, dtype=torch.int32, device="cuda")
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        ctx.sample(xd, ud, k=0, p=1.0, temperature=0.9, out=out)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        assert np.array_equal(out.cpu().numpy(), want)
+        assert np.array_equal(ctx.sample(xd, ud, k=0, p=1.0, temperature=0.9).cpu().numpy(), want)
+    ctx.close()
+
+
 def crowded_rows(name, rng, rows, vocab):
     """Rows of which many ids share a score, or lie so close together that a bucket of the row's histogram (a 2048th of
     about thirty temperatures) holds more of them than a tile takes whole: (logits, element type, temperatures)."""
