@@ -1045,6 +1045,42 @@ __device__ __noinline__ uint32_t wide_tie_id(const u64* list, int run_lo, int ru
   return block_tie_id(run, pos - run_lo, key64_okey(whole_key(pos)), [=](int i) { return whole_key(run_lo + i); }, table);
 }
 
+// The position the reference's own operations end on (block_discrete_draw's replay), run by one wave: the additions are one
+// chain in the reference's order, the loads, conversions and quotients of 64 weights at a time lie beside it.  (One lane
+// that loads, divides and adds in turn: 13.4 -> 1.57 ms for 128256 elements, 21.2 -> 2.4 for 201088, 0.90 -> 0.16 for 8000: 6 ns
+// an element and pass.)
+__device__ __noinline__ int wide_replay(const u64* list, int listed, float e_below, float scale, int keep, double u) {
+  const int lane = lane_id();
+  auto weight = [=](int i) {
+    const float e = i < listed ? __uint_as_float(static_cast<uint32_t>(list[i < keep ? i : 0] >> 32)) : e_below;
+    return i < keep ? e * scale : 0.0f;  // (what is added behind the last weight changes nothing)
+  };
+  double sum = 0.0;
+  float w = weight(lane);
+  for (int i0 = 0; i0 < keep; i0 += 64) {
+    const double x = static_cast<double>(w);
+    w = weight(i0 + 64 + lane);
+#pragma unroll
+    for (int l = 0; l < 64; ++l) sum += wave_read_lane(x, l);
+  }
+  double cp = 0.0;
+  w = weight(lane);
+  for (int i0 = 0; i0 < keep; i0 += 64) {
+    const double x = static_cast<double>(w) / sum, start = cp;
+    w = weight(i0 + 64 + lane);
+#pragma unroll
+    for (int l = 0; l < 64; ++l) cp += wave_read_lane(x, l);
+    if (cp >= u) {  // one of these, or the last one, whose value is forced to one
+      cp = start;
+      for (int l = 0; l < 64 && i0 + l < keep - 1; ++l) {
+        cp += wave_read_lane(x, l);
+        if (cp >= u) return i0 + l;
+      }
+    }
+  }
+  return keep - 1;
+}
+
 // Runs by the whole workgroup; false: the row needs the exact path.
 template <bool INLINE>
 __device__ __forceinline__ bool wide_finish_row(const SampleArgs& a, const WideArgs& w, int row, mi355x_sample_params prm, WideFinishShared& sh, SeqShared& seqsh) {
@@ -1138,8 +1174,20 @@ __device__ __forceinline__ bool wide_finish_row(const SampleArgs& a, const WideA
         if (lane == 0) sh.weight[t] = s;
       }
       __syncthreads();
-      pos = wide_draw([=](int i) { return static_cast<double>(exps(i) * scale); }, keep, used, u, 16.0 * keep * 1.1102230246251565e-16, sh, seqsh);
-      if (pos < 0) pos = block_discrete_draw<4>(keep, [=](int i) { return exps(i) * scale; }, u, seqsh);  // (replays the reference's own operations)
+      // The reference's sum and its cumulative value have `keep` roundings of 2^-53 each at most, the quotients one; here every
+      // value comes from a tree of fewer than 256.  (A band of 16 keep of them takes seven times as many rows the long way, 5.8e-5 of
+      // those of 128256 elements and 1.4e-4 of 201088: 0.8 and 3 us a row and step at what that took.  24 x 201088 bf16, 24 inputs of
+      // which one has such a row: 1858 -> 51 us.)
+      pos = wide_draw([=](int i) { return static_cast<double>(exps(i) * scale); }, keep, used, u, (2.25 * keep + 512.0) * 1.1102230246251565e-16, sh, seqsh);
+      if (pos < 0) {
+        if (wave == 0) {
+          const int p = wide_replay(list, n, e_below, scale, keep, u);
+          if (lane == 0) seqsh.bcast_i = p;
+        }
+        __syncthreads();
+        pos = seqsh.bcast_i;
+        __syncthreads();
+      }
     }
   }
   const RowOutputs out = row_outputs(a, row);

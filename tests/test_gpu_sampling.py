@@ -1731,6 +1731,25 @@ def test_whole_vocabulary_draws_on_the_edges_of_their_guard_bands(ctx, orc, voca
     assert np.array_equal(tokens_only(ctx, x, us, 0, 1.0, t), orc.sample_batch(x.astype(np.float32), 0, 1.0, t, us))
 
 
+@pytest.mark.parametrize("vocab,sigma,t", [(4097, 2.0, 1.0), (4160, 0.5, 1.0), (50257, 3.0, 1.0), (128256, 2.0, 0.8)])
+def test_whole_vocabulary_draws_that_replay_the_sums(ctx, orc, vocab, sigma, t):
+    """Draws on the reference's cumulative values, at the first, at both ends of a wave's 64 and at the last ones, and beside them at
+    distances inside, at the edge of and beyond the band (2.25 n + 512) 2^-53, within which the reference's own sums are replayed."""
+    say("replayed draws", vocab)
+    rng = np.random.default_rng(vocab)
+    base = (rng.standard_normal(vocab) * sigma).astype(np.float32)
+    _, probs = orc.sampled_categorical(base, 0, 1.0, t)
+    w = np.asarray(probs, np.float64)
+    cp = np.cumsum(w / np.cumsum(w)[-1])
+    band = (2.25 * len(cp) + 512) * 2.0 ** -53
+    us = []
+    for j in sorted({0, 1, 63, 64, 127, len(cp) // 3, len(cp) // 2 | 63, len(cp) - 66, len(cp) - 3, len(cp) - 2}):
+        us += [cp[j], np.nextafter(cp[j], 0.0), np.nextafter(cp[j], 1.0)] + [cp[j] + s * f * band for s in (-1, 1) for f in (0.1, 0.99, 1.01, 8.0)]
+    us = np.array([v for v in us if 0.0 <= v < 1.0], np.float64)
+    x = np.tile(base, (len(us), 1))
+    assert np.array_equal(tokens_only(ctx, x, us, 0, 1.0, t), orc.sample_batch(x, 0, 1.0, t, us))
+
+
 @pytest.mark.parametrize("rows,vocab,dtype", [(1, 4099, torch.float32), (9, 50257, torch.float16), (40, 20011, torch.bfloat16), (300, 4099, torch.float32)])
 def test_rows_given_back_by_the_pick_are_finished_in_one_launch(orc, rows, vocab, dtype):
     """Temperature-only rows that the pick gives back, their draws on cumulative values: one of them, some among others, all, and more
