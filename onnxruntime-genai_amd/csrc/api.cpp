@@ -474,7 +474,7 @@ int SampleImpl(mi355x_search_ctx* ctx, hipStream_t s, const void* logits, const 
                int32_t* kept_count, int32_t* kept_ids, float* kept_probs, int kept_capacity, bool kept_pad) {
   ms::SampleArgs a{};
   if (int r = MakeXform(ctx, xf, rows, vocab, s, &a.xf)) return r;
-  bool any_nucleus = false, any_other = false, any_large_k = false, any_exact = false, any_wide = false;
+  bool any_nucleus = false, any_other = false, any_large_k = false, any_exact = false, any_wide = false, any_pick = false;
   ms::InlineParams table{};
   bool use_table = false;
   // Sampling from the whole vocabulary is spread over the GPU wherever its kernels can take the row as it lies: no
@@ -491,8 +491,10 @@ int SampleImpl(mi355x_search_ctx* ctx, hipStream_t s, const void* logits, const 
     if (nucleus && vocab > 64) any_nucleus = true;
     if (large_k && vocab > 64) any_large_k = true;
     if (large_k && kk > 4 * ms::kLargeKOneOffer) a.all_offers = 1;
-    if (whole && wide_fits) any_wide = true;
-    else if (vocab > 64 && (!fits || whole || (p.k > 1 && kk > ms::kLargeKMax))) any_exact = true;
+    if (whole && wide_fits) {
+      any_wide = true;
+      any_pick |= p.p == 1.0f;  // (a pick gives back what lies above one: p = 1.5, 256 x 32064 fp32 279 us with a pick, 151 without)
+    } else if (vocab > 64 && (!fits || whole || (p.k > 1 && kk > ms::kLargeKMax))) any_exact = true;
     else if (!((nucleus || large_k) && fits)) any_other = true;
     return MI355X_OK;
   };
@@ -539,7 +541,7 @@ int SampleImpl(mi355x_search_ctx* ctx, hipStream_t s, const void* logits, const 
   PlanStream(ctx, &a, !any_nucleus && !any_large_k);
   a.exact_kernel = (any_exact ? ms::kExactRows : 0) | (any_wide ? ms::kWideRows : 0);
   const ms::WideArgs wide{(vocab + ms::kWideChunk - 1) / ms::kWideChunk, tiles, ctx->wide_rows, ctx->wide_tile_start, ctx->wide_cut_bucket, ctx->seg_sum,
-                          ctx->seg_step, ctx->sub_step, ctx->sub_se, ctx->chunk_next, kept_ids == nullptr && kept_count == nullptr,
+                          ctx->seg_step, ctx->sub_step, ctx->sub_se, ctx->chunk_next, any_pick && kept_ids == nullptr && kept_count == nullptr,
                           {ctx->wide_rest, ctx->wide_rest + 1, ctx->wide_rest + 2, ctx->wide_rest + 2 + ctx->max_rows, ctx->wide_rest + 2 + 2 * static_cast<size_t>(ctx->max_rows)}};
   // a caller that bounds the number of allowed ids per row lets the sparse-mask kernel work alone
   if (xf && xf->mask && xf->mask_allowed_max > 0) {
