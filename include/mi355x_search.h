@@ -388,8 +388,10 @@ int mi355x_search_set_poll_limit(mi355x_search_ctx* ctx, int polls);
 /* The exact sums of long rows (mi355x_softmax, mi355x_beam_select from 16384 logits per row on) have a bounded
  * wait of their own: a 4096-logit segment's workgroup polls, under the same limit, for the sums of the row's
  * earlier segments, which workgroups of the same launch publish.  A wait that gives up costs time only: the
- * segment is then added element by element, and the result is the same.  *segments = how many segments that has
- * happened to on this context (synchronises `stream`; no counterpart in the reference). */
+ * segment is then added element by element, and the result is the same.  The tiles of a row that samples from the
+ * whole vocabulary wait in the same way for the sums of the tiles before them and for the row's keys (then the exact
+ * path finishes the row).  *segments = how many segments and tiles that has happened to on this context
+ * (synchronises `stream`; no counterpart in the reference). */
 int mi355x_search_sum_waits_gave_up(mi355x_search_ctx* ctx, void* stream, unsigned* segments);
 
 #ifdef __cplusplus

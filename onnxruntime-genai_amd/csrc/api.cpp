@@ -294,7 +294,7 @@ int mi355x_search_create(int device, int max_rows, int max_vocab, mi355x_search_
   ok(c->Alloc(&c->big, static_cast<size_t>(max_rows) * c->big_stride, false));
   ok(c->Alloc(&c->big2, static_cast<size_t>(max_rows) * c->big_stride, false));
   ok(c->Alloc(&c->row_done, static_cast<size_t>(max_rows), true));
-  ok(c->Alloc(&c->fallback_rows, 4, true));  // [0] rows finished by the exact path, [1] a wait gave up, [2] exact-sum segments whose wait gave up, [3] rows given back by a pick
+  ok(c->Alloc(&c->fallback_rows, 4, true));  // [0] rows finished by the exact path, [1] a wait gave up, [2] exact-sum segments and tiles whose wait gave up, [3] rows given back by a pick
   ok(c->Alloc(&c->ban, static_cast<size_t>(max_rows) * ((max_vocab - 1) / 32 + 1), false));
   ok(c->Alloc(&c->params_dev, static_cast<size_t>(max_rows), false));
   ok(c->Alloc(&c->beam_row_scores, static_cast<size_t>(max_rows) * ms::kBeamMaxCand, false));
@@ -304,8 +304,8 @@ int mi355x_search_create(int device, int max_rows, int max_vocab, mi355x_search_
   static_assert(ms::kWideTile <= ms::kSegElems, "room for either");
   ok(c->Alloc(&c->wide_rows, static_cast<size_t>(max_rows), false));
   const size_t tile_starts = static_cast<size_t>(max_rows) * (c->max_segs + 1);
-  ok(c->Alloc(&c->wide_tile_start, tile_starts + 2 + 3 * static_cast<size_t>(max_rows), false));  // (and what wide_rest counts)
-  if (c->wide_tile_start) c->wide_rest = c->wide_tile_start + tile_starts;
+  ok(c->Alloc(&c->wide_tile_start, tile_starts, false));
+  ok(c->Alloc(&c->wide_rest, 2 + static_cast<size_t>(max_rows) * (2 + ms::kRestStride), false));
   ok(c->Alloc(&c->wide_cut_bucket, static_cast<size_t>(max_rows) * (c->max_segs + 1), false));
   ok(c->Alloc(&c->seg_max, static_cast<size_t>(max_rows) * c->max_segs, false));
   ok(c->Alloc(&c->seg_sum, static_cast<size_t>(max_rows) * c->max_segs, false));

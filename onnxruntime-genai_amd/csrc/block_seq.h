@@ -106,15 +106,6 @@ __device__ __forceinline__ Step oct_scan_steps(Step x) {
   return x;
 }
 
-// Over groups of eight or sixteen lanes: the last lane of each ends with the composition of its group.
-template <int LANES>
-__device__ __forceinline__ Step group_scan_steps(Step x) {
-  static_assert(LANES == 8 || LANES == 16, "within a row of sixteen lanes");
-  x = oct_scan_steps(x);
-  if constexpr (LANES == 16) x = step_compose(step_from_below<0x118, 0xf>(x), x);  // row_shr:8
-  return x;
-}
-
 __device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) { return ~wave_max<uint32_t>(~v); }
 
 // Fetches the ITEMS consecutive addends thread t owns in the window [w0, wend): indices

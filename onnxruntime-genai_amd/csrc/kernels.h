@@ -92,7 +92,6 @@ constexpr int kWideTile = 3072;       // keys after which a new tile begins, wit
 constexpr int kWideBucketMax = 1024;  // keys of a bucket that a tile takes whole
 constexpr int kWideMaxTiles = 192;    // tiles of the longest row (589824 logits)
 constexpr int kWideMinVocab = 4096;   // shorter rows are a single workgroup's work anyway
-constexpr int kWideRestBlocks = 256;  // workgroups that do what a pick left: one a CU
 constexpr uint32_t kWideDeclined = 1, kWideGivenBack = 2;
 struct WideRow {
   uint32_t n, tiles;  // listed keys, their tiles
@@ -101,12 +100,13 @@ struct WideRow {
   float top;          // the row's maximum
 };
 // The rows a pick gave back, and how far the work on them is (wide_rest_kernel).
+constexpr int kRestStride = 32;  // words from one row's count to the next: a line of memory
 struct WideRest {
-  uint32_t* count;      // of listed rows
-  uint32_t* ticket;     // the next piece of work
-  uint32_t* rows;       // [rows]
-  uint32_t* scattered;  // [rows]: chunks done
-  uint32_t* ranked;     // [rows]: tiles done
+  uint32_t* sorted;     // how many are listed to be sorted ...
+  uint32_t* exact;      // ... and for the exact path
+  uint32_t* rows;       // [rows]: the first from the front, the second from the back
+  uint32_t* gave_up;    // [rows]: not 0, a tile's wait for the row's chunks gave up
+  uint32_t* scattered;  // [rows][kRestStride]: chunks done
 };
 struct WideArgs {
   int chunks, max_tiles;
@@ -118,7 +118,7 @@ struct WideArgs {
   int4* sub_step;
   int* sub_se;
   u64* best_below;       // [rows]: the best element past the list, 0: none
-  int pick;              // the token alone is asked for: wide_pick and wide_rest run
+  int pick;              // the token alone is asked for: wide_pick runs, and wide_rest and wide_finish for the rows it gives back
   WideRest rest;
 };
 struct NoTable {};

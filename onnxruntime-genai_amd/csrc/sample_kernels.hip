@@ -2071,19 +2071,13 @@ extern "C" hipError_t ms_sample_init() {
                           reinterpret_cast<const void*>(ms::wide_pick_kernel<uint16_t, true>),
                           reinterpret_cast<const void*>(ms::wide_pick_kernel<ms::bf16_t, false>),
                           reinterpret_cast<const void*>(ms::wide_pick_kernel<ms::bf16_t, true>),
-                          reinterpret_cast<const void*>(ms::wide_rest_kernel<float, false>),
-                          reinterpret_cast<const void*>(ms::wide_rest_kernel<float, true>),
-                          reinterpret_cast<const void*>(ms::wide_rest_kernel<uint16_t, false>),
-                          reinterpret_cast<const void*>(ms::wide_rest_kernel<uint16_t, true>),
-                          reinterpret_cast<const void*>(ms::wide_rest_kernel<ms::bf16_t, false>),
-                          reinterpret_cast<const void*>(ms::wide_rest_kernel<ms::bf16_t, true>),
                           reinterpret_cast<const void*>(ms::wide_scatter_kernel<float, false>),
                           reinterpret_cast<const void*>(ms::wide_scatter_kernel<float, true>),
                           reinterpret_cast<const void*>(ms::wide_scatter_kernel<uint16_t, false>),
                           reinterpret_cast<const void*>(ms::wide_scatter_kernel<uint16_t, true>),
                           reinterpret_cast<const void*>(ms::wide_scatter_kernel<ms::bf16_t, false>),
                           reinterpret_cast<const void*>(ms::wide_scatter_kernel<ms::bf16_t, true>)};
-  static_assert(sizeof(ms::WideScatterShared) <= ms::kFinishLds, "one limit for all");
+  static_assert(sizeof(ms::WideScatterWhole) <= ms::kFinishLds, "one limit for all");
   for (const void* f : finish) {
     const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, ms::kFinishLds);
     if (e != hipSuccess) return e;

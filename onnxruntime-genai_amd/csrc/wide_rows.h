@@ -8,8 +8,8 @@
 // every step but the last is spread over the GPU, in five launches (16 x 128256 fp16: 557 -> 59 us per
 // step on the same rows again and 66 on rows that come from memory: 4.7 + 4.7 + 11.5 + 21.6 + 20 us by a trace; every
 // one of them is a chain of dependent phases of a few barriers each, no launch moves more than 33 MB).  Rows whose token
-// alone is asked for need no order: for p = 1 a launch behind 2 picks it from the histogram (wide_pick_kernel), and
-// one launch does 3 to 5 for the rows it gives back (wide_rest_kernel), 0.3 % of such rows.
+// alone is asked for need no order: for p = 1 a launch behind 2 picks it from the histogram (wide_pick_kernel), one launch does
+// 3 and 4 for the rows it gives back (wide_rest_kernel), 0.3 % of such rows, and 5 finishes these.
 //   1. wide_max:     the maximum of every chunk of kWideChunk logits.
 //   2. wide_count:   a histogram per chunk over kWideBuckets buckets, linear in the score below the row's maximum down
 //                    to the depth past which no element can lie inside the kept set.
@@ -65,13 +65,13 @@ __device__ __forceinline__ WideShare wide_share(int per_row) {
   return WideShare{xcd + 8 * (slot / per_row), slot % per_row};
 }
 
-// The kWidePer logits of thread t in a chunk, in loads of 16 bytes; ids past the vocabulary are NaN.
-template <typename InT>
-__device__ __forceinline__ void wide_load(const InT* row, int V, int chunk, float (&v)[kWidePer]) {
+// The logits of thread t of BLOCK in a chunk, in loads of 16 bytes; ids past the vocabulary are NaN.
+template <typename InT, int BLOCK = kWideBlock>
+__device__ __forceinline__ void wide_load(const InT* row, int V, int chunk, float (&v)[kWideChunk / BLOCK]) {
   constexpr int VEC = 16 / static_cast<int>(sizeof(InT));
 #pragma unroll
-  for (int j = 0; j < kWidePer / VEC; ++j) {
-    const int i0 = chunk * kWideChunk + (j * kWideBlock + static_cast<int>(threadIdx.x)) * VEC;
+  for (int j = 0; j < kWideChunk / BLOCK / VEC; ++j) {
+    const int i0 = chunk * kWideChunk + (j * BLOCK + static_cast<int>(threadIdx.x)) * VEC;
     if (i0 + VEC <= V) {
       if constexpr (VEC == 4) {
         const v4f_any q = *reinterpret_cast<const v4f_any*>(row + i0);
@@ -134,10 +134,10 @@ struct WideRaw {
     }
   }
 };
-template <typename InT>
+template <typename InT, int BLOCK = kWideBlock>
 __device__ __forceinline__ int wide_index(int chunk, int e) {
   constexpr int VEC = 16 / static_cast<int>(sizeof(InT));
-  return chunk * kWideChunk + ((e / VEC) * kWideBlock + static_cast<int>(threadIdx.x)) * VEC + e % VEC;
+  return chunk * kWideChunk + ((e / VEC) * BLOCK + static_cast<int>(threadIdx.x)) * VEC + e % VEC;
 }
 
 // The row's maximum as the chunks left it (0xffffffff where the row is not one for this path).
@@ -157,17 +157,17 @@ __global__ __launch_bounds__(kWideBlock) void wide_max_kernel(const SampleArgs a
   __shared__ uint32_t red[16];
   const WideShare mine = wide_share(w.chunks);
   const int chunk = mine.item, row = mine.row, tid = threadIdx.x;
-  if (blockIdx.x == 0 && tid == 0) *w.rest.count = *w.rest.ticket = 0u;
+  if (blockIdx.x == 0 && tid == 0) *w.rest.sorted = *w.rest.exact = 0u;
   if (row >= a.rows || !wide_row(row_params<INLINE>(a, row))) return;
   float v[kWidePer];
   wide_load<InT>(static_cast<const InT*>(row_start<INLINE>(a, row, sizeof(InT))), a.vocab, chunk, v);
-  // (this launch is the first of its sequence: it also marks the sums of the row's tiles as not written, and the row's counts of
-  // what wide_rest has done)
+  // (this launch is the first of its sequence: it also marks the sums of the row's tiles as not written, and none of its chunks as
+  // scattered by wide_rest)
   if (chunk == 0) {
     for (int t = tid; t < w.max_tiles; t += kWideBlock) store_sum_bits(w.tile_sum + static_cast<size_t>(row) * w.max_tiles + t, kSumNotReady);
     if (tid == 0) {
       w.best_below[row] = 0;
-      w.rest.scattered[row] = w.rest.ranked[row] = 0u;
+      w.rest.scattered[row * kRestStride] = w.rest.gave_up[row] = 0u;
     }
   }
   float m = -__builtin_inff();
@@ -175,6 +175,29 @@ __global__ __launch_bounds__(kWideBlock) void wide_max_kernel(const SampleArgs a
   for (int e = 0; e < kWidePer; ++e) m = fmaxf(m, v[e]);
   const uint32_t k = block_max<uint32_t>(order_key(m), red, false);
   if (tid == 0) a.chunk_max[static_cast<size_t>(row) * w.chunks + chunk] = k;
+}
+
+// What one workgroup writes and others of the same launch read (HANDED) goes past the caches of the CUs and the XCDs in both
+// directions; what the next launch reads need not.  (Plain stores and loads, with the caches written back by every chunk's workgroup and
+// invalidated by every tile's: wide_rest of 64 x 128256 rows 33 us longer, of 256 x 32064 34.)
+template <bool HANDED, typename T>
+__device__ __forceinline__ void wide_put(T* p, T v) {
+  if constexpr (HANDED) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  else *p = v;
+}
+template <bool HANDED, typename T>
+__device__ __forceinline__ T wide_get(const T* p) {
+  if constexpr (HANDED) return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  else return *p;
+}
+template <bool HANDED>
+__device__ __forceinline__ void wide_put(uint2* p, uint2 v) {
+  wide_put<HANDED>(reinterpret_cast<u64*>(p), static_cast<u64>(v.x) | (static_cast<u64>(v.y) << 32));
+}
+template <bool HANDED>
+__device__ __forceinline__ uint2 wide_get(const uint2* p) {
+  const u64 v = wide_get<HANDED>(reinterpret_cast<const u64*>(p));
+  return make_uint2(static_cast<uint32_t>(v), static_cast<uint32_t>(v >> 32));
 }
 
 // Bucket of a score: a non-increasing function of it (every operation is monotone), kWideBuckets and up for what lies
@@ -260,8 +283,8 @@ __global__ __launch_bounds__(kWideBlock, 8) void wide_count_kernel(const SampleA
 // of rows of 128256 and 201088 logits, which go the long way behind this.  (Masses as whole numbers of 2^-43, whose rounding
 // such rows of a few heavy tokens notice: twice as many.)  One workgroup per row: it adds the chunks' histograms up,
 // finds the bucket and looks the row through once more for its keys.  A trace of 16 x 128256 fp16: 3.2 (maximum) + 7.1
-// (counts and masses, 4.8 without these) + 19.2 us and what wide_rest takes to find nothing to do; steps, with three launches in its
-// place, 62.9 -> 35.1 us, 64 x 128256 fp16 142 -> 58, 1 x 128256 fp32 50 -> 29, 24 x 201088 bf16 129 -> 51.  A compare of every logit with the two
+// (counts and masses, 4.8 without these) + 19.2 us and what wide_rest and wide_finish take to find nothing to do; steps, with three
+// launches in their place, 62.9 -> 35.1 us, 64 x 128256 fp16 142 -> 58, 1 x 128256 fp32 50 -> 29, 24 x 201088 bf16 129 -> 51.  A compare of every logit with the two
 // buckets and a load of four chunks at a time instead of eight ahead: 23.0 us for this launch.
 template <typename InT, bool INLINE>
 __global__ __launch_bounds__(kWideBlock) void wide_pick_kernel(const SampleArgs a, const typename WideTable<INLINE>::type, const WideArgs w) {
@@ -274,9 +297,14 @@ __global__ __launch_bounds__(kWideBlock) void wide_pick_kernel(const SampleArgs 
   const mi355x_sample_params prm = row_params<INLINE>(a, row);
   if (!wide_row(prm)) return;
   const uint32_t rmax = wide_row_max(a, w, row);
-  auto give_back = [&] { w.rest.rows[atomicAdd(w.rest.count, 1u)] = static_cast<uint32_t>(row); };
+  // (rows to be sorted are listed from the front, those of the exact path from the back)
+  auto give_back = [&](bool exact) {
+    const uint32_t i = atomicAdd(exact ? w.rest.exact : w.rest.sorted, 1u);
+    w.rest.rows[exact ? static_cast<uint32_t>(a.rows) - 1u - i : i] = static_cast<uint32_t>(row);
+    atomicAdd(a.fallback_rows + 3, 1u);
+  };
   if (rmax == 0xffffffffu || !(prm.p == 1.0f)) {
-    if (tid == 0) give_back();
+    if (tid == 0) give_back(rmax == 0xffffffffu);
     return;
   }
   // The first of the row's chunks are requested now: they are looked through last.
@@ -317,7 +345,7 @@ __global__ __launch_bounds__(kWideBlock) void wide_pick_kernel(const SampleArgs 
     wave_counts[wave] = n_inc;
   }
   if (__syncthreads_or(nan)) {  // (one that is kept makes all weights NaN: the long way)
-    if (tid == 0) give_back();
+    if (tid == 0) give_back(false);
     return;
   }
   const double ws = wave_prefix_sum<double>(lane < 16 ? em::as_double(sh.sums[lane]) : 0.0);
@@ -415,24 +443,27 @@ __global__ __launch_bounds__(kWideBlock) void wide_pick_kernel(const SampleArgs 
       *row_outputs(a, row).token = static_cast<int32_t>(id);
       atomicAdd(a.fallback_rows, 1u);  // (a row of the exact path, spread over the GPU)
     } else {
-      atomicAdd(a.fallback_rows + 3, 1u);
-      give_back();
+      give_back(false);
     }
   }
 }
 
 // The keys go to LDS in bucket order first and from there to memory, so that neighbouring lanes write neighbouring
 // places (eight keys a bucket and chunk at 128256 logits).  Written straight from the registers every lane's 8 bytes
-// are a line of their own: 8.3 of the 17.9 us the launch took at 16 x 128256.
+// are a line of their own: 8.3 of the 17.9 us the launch took at 16 x 128256.  ROOM: the keys LDS has room for; a chunk of more goes
+// through it in several parts.
+template <int BLOCK, int ROOM>
 struct WideScatterShared {
-  u64 keys[kWideChunk];
-  uint32_t place[kWideBuckets];  // the bucket's next place in keys
-  uint32_t shift[kWideBuckets];  // what takes a place in keys to one in the row's buffer
-  uint32_t wave_sums[16], wave_own[16];
-  u64 red64[16];
+  u64 keys[ROOM];
+  uint32_t place[kWideBuckets];  // the bucket's next place among the chunk's keys
+  uint32_t shift[kWideBuckets];  // what takes a place among these to one in the row's buffer
+  uint32_t wave_sums[BLOCK / 64], wave_own[BLOCK / 64];
+  u64 red64[BLOCK / 64];
 };
-template <typename InT, bool INLINE>
-__device__ __forceinline__ void wide_scatter_chunk(const SampleArgs& a, const WideArgs& w, int row, int chunk, mi355x_sample_params prm, WideScatterShared& sh) {
+template <typename InT, bool INLINE, bool HANDED, int BLOCK, int ROOM>
+__device__ __forceinline__ void wide_scatter_chunk(const SampleArgs& a, const WideArgs& w, int row, int chunk, mi355x_sample_params prm, WideScatterShared<BLOCK, ROOM>& sh) {
+  constexpr int kElems = kWideChunk / BLOCK;
+  constexpr int kWords = kWideBlock / BLOCK;  // of two buckets each, a thread
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   WideRow* const info = w.rows + row;
   const uint32_t rmax = wide_row_max(a, w, row);
@@ -440,41 +471,62 @@ __device__ __forceinline__ void wide_scatter_chunk(const SampleArgs& a, const Wi
     if (chunk == 0 && tid == 0) *info = WideRow{0u, 0u, kWideDeclined, 0.0f};
     return;
   }
-  float v[kWidePer];
-  wide_load<InT>(static_cast<const InT*>(row_start<INLINE>(a, row, sizeof(InT))), a.vocab, chunk, v);
-  // the thread's two buckets: keys in the whole row, in the chunks before this one, and in this one
-  uint32_t all0 = 0u, all1 = 0u, before0 = 0u, before1 = 0u, own = 0u;
-  const uint32_t* h = reinterpret_cast<const uint32_t*>(a.big + static_cast<size_t>(row) * a.big_stride) + tid;
-  for (int c0 = 0; c0 < w.chunks; c0 += 8) {
-    uint32_t pair[8];
+  float v[kElems];
+  wide_load<InT, BLOCK>(static_cast<const InT*>(row_start<INLINE>(a, row, sizeof(InT))), a.vocab, chunk, v);
+  // the thread's buckets: keys in the whole row, in the chunks before this one, and in this one
+  uint32_t all[2 * kWords], before[2 * kWords], own[2 * kWords];
 #pragma unroll
-    for (int c = 0; c < 8; ++c) pair[c] = c0 + c < w.chunks ? h[static_cast<size_t>(c0 + c) * kWideBlock] : 0u;
+  for (int b = 0; b < 2 * kWords; ++b) all[b] = before[b] = own[b] = 0u;
+  const uint32_t* h = reinterpret_cast<const uint32_t*>(a.big + static_cast<size_t>(row) * a.big_stride) + tid * kWords;
+  for (int c0 = 0; c0 < w.chunks; c0 += 8) {
+    uint32_t pair[8][kWords];
+#pragma unroll
+    for (int c = 0; c < 8; ++c)
+#pragma unroll
+      for (int q = 0; q < kWords; ++q) pair[c][q] = c0 + c < w.chunks ? h[static_cast<size_t>(c0 + c) * kWideBlock + q] : 0u;
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
-      all0 += pair[c] & 0xffffu;
-      all1 += pair[c] >> 16;
-      if (c0 + c < chunk) {
-        before0 += pair[c] & 0xffffu;
-        before1 += pair[c] >> 16;
+#pragma unroll
+      for (int q = 0; q < kWords; ++q) {
+        const uint32_t n0 = pair[c][q] & 0xffffu, n1 = pair[c][q] >> 16;
+        all[2 * q] += n0;
+        all[2 * q + 1] += n1;
+        if (c0 + c < chunk) {
+          before[2 * q] += n0;
+          before[2 * q + 1] += n1;
+        }
+        if (c0 + c == chunk) {
+          own[2 * q] = n0;
+          own[2 * q + 1] = n1;
+        }
       }
-      own = c0 + c == chunk ? pair[c] : own;
     }
   }
-  const uint32_t own0 = own & 0xffffu, own1 = own >> 16;
-  const uint32_t inc = wave_prefix_sum<uint32_t>(all0 + all1), own_inc = wave_prefix_sum<uint32_t>(own0 + own1);
+  uint32_t all_sum = 0u, own_sum = 0u;
+#pragma unroll
+  for (int b = 0; b < 2 * kWords; ++b) {
+    all_sum += all[b];
+    own_sum += own[b];
+  }
+  const uint32_t inc = wave_prefix_sum<uint32_t>(all_sum), own_inc = wave_prefix_sum<uint32_t>(own_sum);
   if (lane == 63) {
     sh.wave_sums[wave] = inc;
     sh.wave_own[wave] = own_inc;
   }
   __syncthreads();
-  const uint32_t ws = wave_prefix_sum<uint32_t>(lane < 16 ? sh.wave_sums[lane] : 0u), wo = wave_prefix_sum<uint32_t>(lane < 16 ? sh.wave_own[lane] : 0u);
-  const uint32_t n = wave_read_lane(ws, 15), n_own = wave_read_lane(wo, 15);
-  const uint32_t start0 = (wave > 0 ? wave_read_lane(ws, wave - 1) : 0u) + inc - (all0 + all1), start1 = start0 + all0;
-  const uint32_t here0 = (wave > 0 ? wave_read_lane(wo, wave - 1) : 0u) + own_inc - (own0 + own1), here1 = here0 + own0;
-  sh.place[2 * tid] = here0;
-  sh.place[2 * tid + 1] = here1;
-  sh.shift[2 * tid] = start0 + before0 - here0;
-  sh.shift[2 * tid + 1] = start1 + before1 - here1;
+  const uint32_t ws = wave_prefix_sum<uint32_t>(lane < BLOCK / 64 ? sh.wave_sums[lane] : 0u), wo = wave_prefix_sum<uint32_t>(lane < BLOCK / 64 ? sh.wave_own[lane] : 0u);
+  const uint32_t n = wave_read_lane(ws, BLOCK / 64 - 1), n_own = wave_read_lane(wo, BLOCK / 64 - 1);
+  const uint32_t start = (wave > 0 ? wave_read_lane(ws, wave - 1) : 0u) + inc - all_sum;
+  {
+    uint32_t at = start, here = (wave > 0 ? wave_read_lane(wo, wave - 1) : 0u) + own_inc - own_sum;
+#pragma unroll
+    for (int b = 0; b < 2 * kWords; ++b) {
+      sh.place[2 * kWords * tid + b] = here;
+      sh.shift[2 * kWords * tid + b] = at + before[b] - here;
+      at += all[b];
+      here += own[b];
+    }
+  }
   if (chunk == 0) {
     // Tile t begins with the first bucket that starts at or after t * kWideTile: a bucket's start and the one before
     // it enclose the multiples it is the first after.  (The first bucket starts tile 0; an empty tile begins where
@@ -485,48 +537,77 @@ __device__ __forceinline__ void wide_scatter_chunk(const SampleArgs& a, const Wi
     auto enclose = [&](uint32_t prev, uint32_t at) {
       for (uint32_t t = prev / kWideTile + 1u; t <= at / kWideTile; ++t) {
         const bool inside = at - prev > static_cast<uint32_t>(kWideBucketMax) && t * kWideTile < at;
-        tile[t] = inside ? t * kWideTile : at;
-        cut[t] = inside ? make_uint2(prev, at) : make_uint2(0u, 0u);
+        wide_put<HANDED>(tile + t, inside ? t * kWideTile : at);
+        wide_put<HANDED>(cut + t, inside ? make_uint2(prev, at) : make_uint2(0u, 0u));
       }
     };
     if (tid == 0) {
-      tile[0] = 0u;
-      cut[0] = make_uint2(0u, 0u);
+      wide_put<HANDED>(tile, 0u);
+      wide_put<HANDED>(cut, make_uint2(0u, 0u));
     }
-    enclose(start0, start1);  // (the start after the last bucket's is n)
-    enclose(start1, start1 + all1);
+    uint32_t at = start;
+#pragma unroll
+    for (int b = 0; b < 2 * kWords; ++b) {  // (the start after the last bucket's is n)
+      enclose(at, at + all[b]);
+      at += all[b];
+    }
     const uint32_t tiles = (n + kWideTile - 1u) / kWideTile;
     if (tid == 0) {
       if (n % kWideTile != 0u) {  // (where n is a multiple itself, it is enclosed above)
-        tile[tiles] = n;
-        cut[tiles] = make_uint2(0u, 0u);
+        wide_put<HANDED>(tile + tiles, n);
+        wide_put<HANDED>(cut + tiles, make_uint2(0u, 0u));
       }
-      *info = WideRow{n, tiles, 0u, key_to_float(rmax)};
+      wide_put<HANDED>(&info->n, n);
+      wide_put<HANDED>(&info->tiles, tiles);
+      wide_put<HANDED>(&info->declined, 0u);
+      wide_put<HANDED>(&info->top, key_to_float(rmax));
     }
   }
   __syncthreads();
   const WideBuckets bucket_of(key_to_float(rmax), wide_depth(prm, a.vocab));
-  u64 below = 0;
-#pragma unroll
-  for (int e = 0; e < kWidePer; ++e) {
-    const uint32_t b = bucket_of(v[e]);
-    const u64 k = make_key64(order_key(v[e]), static_cast<uint32_t>(wide_index<InT>(chunk, e)));
-    if (b < static_cast<uint32_t>(kWideBuckets)) sh.keys[atomicAdd(&sh.place[b], 1u)] = k;
-    else if (v[e] == v[e]) below = k > below ? k : below;
-  }
-  below = block_max<u64>(below, sh.red64, false);  // (its barrier: the keys are in their places)
-  if (tid == 0 && below != 0) atomicMax(reinterpret_cast<unsigned long long*>(w.best_below + row), static_cast<unsigned long long>(below));
   u64* const keys = a.big2 + static_cast<size_t>(row) * a.big_stride;
+  u64 below = 0;
+  constexpr uint32_t kLeftOut = 0xffffffffu;
+  uint32_t place[kElems];
 #pragma unroll
-  for (int e = 0; e < kWidePer; ++e) {
-    const uint32_t p = static_cast<uint32_t>(e * kWideBlock + tid);
-    if (p < n_own) {
-      const u64 k = sh.keys[p];
-      keys[p + sh.shift[bucket_of(key_to_float(key64_okey(k)))]] = k;
+  for (int e = 0; e < kElems; ++e) {
+    const uint32_t b = bucket_of(v[e]);
+    place[e] = kLeftOut;
+    if (b < static_cast<uint32_t>(kWideBuckets)) {
+      place[e] = atomicAdd(&sh.place[b], 1u);
+    } else if (v[e] == v[e]) {
+      const u64 k = make_key64(order_key(v[e]), static_cast<uint32_t>(wide_index<InT, BLOCK>(chunk, e)));
+      below = k > below ? k : below;
+    }
+  }
+#pragma unroll
+  for (uint32_t from = 0u; from < static_cast<uint32_t>(kWideChunk); from += ROOM) {
+    if (from != 0u) {
+      if (n_own <= from) break;
+      __syncthreads();
+    }
+#pragma unroll
+    for (int e = 0; e < kElems; ++e)
+      if (place[e] - from < static_cast<uint32_t>(ROOM))
+        sh.keys[place[e] - from] = make_key64(order_key(v[e]), static_cast<uint32_t>(wide_index<InT, BLOCK>(chunk, e)));
+    if (from == 0u) {
+      below = block_max<u64>(below, sh.red64, false);  // (its barrier: the keys are in their places)
+      if (tid == 0 && below != 0) atomicMax(reinterpret_cast<unsigned long long*>(w.best_below + row), static_cast<unsigned long long>(below));
+    } else {
+      __syncthreads();
+    }
+#pragma unroll
+    for (int e = 0; e < ROOM / BLOCK; ++e) {
+      const uint32_t p = static_cast<uint32_t>(e * BLOCK + tid);
+      if (from + p < n_own) {
+        const u64 k = sh.keys[p];
+        wide_put<HANDED>(keys + (from + p + sh.shift[bucket_of(key_to_float(key64_okey(k)))]), k);
+      }
     }
   }
 }
 
+typedef WideScatterShared<kWideBlock, kWideChunk> WideScatterWhole;
 template <typename InT, bool INLINE>
 __global__ __launch_bounds__(kWideBlock) void wide_scatter_kernel(const SampleArgs a, const typename WideTable<INLINE>::type, const WideArgs w) {
   extern __shared__ u64 lds_keys[];
@@ -534,14 +615,13 @@ __global__ __launch_bounds__(kWideBlock) void wide_scatter_kernel(const SampleAr
   if (mine.row >= a.rows) return;
   const mi355x_sample_params prm = row_params<INLINE>(a, mine.row);
   if (!wide_row(prm)) return;
-  wide_scatter_chunk<InT, INLINE>(a, w, mine.row, mine.item, prm, *reinterpret_cast<WideScatterShared*>(lds_keys));
+  wide_scatter_chunk<InT, INLINE, false, kWideBlock, kWideChunk>(a, w, mine.row, mine.item, prm, *reinterpret_cast<WideScatterWhole*>(lds_keys));
 }
 
 constexpr int kWideSubBuckets = 4096;
 
-template <int BLOCK>
-struct WideRankShared {  // 50 KB: three workgroups of 512 threads a CU
-  static constexpr int kWaves = BLOCK / 64;
+struct WideRankShared {  // 50 KB: three workgroups a CU
+  static constexpr int kWaves = kWideRankBlock / 64;
   union {
     u64 keys[kSegElems];                  // by bucket, then in rank order with the exponentials in the score half
     uint32_t first_key[kWideSubBuckets];  // while the keys are counted: the score of the first key of a bucket
@@ -559,20 +639,19 @@ struct WideRankShared {  // 50 KB: three workgroups of 512 threads a CU
 // The key of rank r (from 0, best first) among the m distinct keys at src, whose lowest and highest are given: a
 // selection by twelve bits at a time below the bits all keys share.  (Two or three passes over the bucket: its keys
 // differ in the lower bits of their scores, or in their ids alone.)  Ends with a barrier.
-template <int BLOCK>
-__device__ __forceinline__ u64 wide_select_key(const u64* src, uint32_t m, uint32_t r, u64 lowest, u64 highest, WideRankShared<BLOCK>& sh) {
+__device__ __forceinline__ u64 wide_select_key(const u64* src, uint32_t m, uint32_t r, u64 lowest, u64 highest, WideRankShared& sh) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  constexpr int kDigitBits = 12, kPer = (1 << kDigitBits) / BLOCK;
+  constexpr int kDigitBits = 12, kPer = (1 << kDigitBits) / kWideRankBlock;
   static_assert(1 << kDigitBits == kWideSubBuckets, "the counts take the sub-buckets' place");
   int open = 64 - __clzll(static_cast<long long>(lowest ^ highest));  // bits still to be decided
   u64 prefix = open < 64 ? highest >> open : 0;
   while (open > 0) {
     const int take = open < kDigitBits ? open : kDigitBits, above = open;
     open -= take;
-    for (int d = tid; d < kWideSubBuckets; d += BLOCK) sh.start[d] = 0u;
+    for (int d = tid; d < kWideSubBuckets; d += kWideRankBlock) sh.start[d] = 0u;
     __syncthreads();
 #pragma unroll 4
-    for (uint32_t i = tid; i < m; i += BLOCK) {
+    for (uint32_t i = tid; i < m; i += kWideRankBlock) {
       const u64 k = src[i];
       if ((above < 64 ? k >> above : 0) == prefix) atomicAdd(&sh.start[(k >> open) & ((1u << take) - 1u)], 1u);
     }
@@ -586,7 +665,7 @@ __device__ __forceinline__ u64 wide_select_key(const u64* src, uint32_t m, uint3
     const uint32_t inc = wave_prefix_sum<uint32_t>(local);
     if (lane == 63) sh.red[wave] = inc;
     __syncthreads();
-    const uint32_t ws = wave_prefix_sum<uint32_t>(lane < BLOCK / 64 ? sh.red[lane] : 0u);
+    const uint32_t ws = wave_prefix_sum<uint32_t>(lane < kWideRankBlock / 64 ? sh.red[lane] : 0u);
     uint32_t before = (wave > 0 ? wave_read_lane(ws, wave - 1) : 0u) + inc - local;
 #pragma unroll
     for (int j = 0; j < kPer; ++j) {
@@ -613,9 +692,8 @@ __device__ __forceinline__ u64 wide_select_key(const u64* src, uint32_t m, uint3
 // fp32 rows of sigma 1 at T = 25 take 1014 us a step against 1154 on the exact path, 24 x 128256 at T = 40 368 against
 // 602, one 208 against 537; with all of a row in one or two buckets 24 x 128256 took 1400 to 1800 against 620 to 930.)
 constexpr uint32_t kWideSelectMax = 32768;
-template <int BLOCK>
 __device__ __forceinline__ bool wide_gather_cut(const u64* list, uint32_t first, uint32_t n, uint2 head, uint2 tail, bool order_ties,
-                                                WideRankShared<BLOCK>& sh) {
+                                                WideRankShared& sh) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const uint32_t end = first + n;
   uint32_t done = first;  // the tile's places up to here have their keys
@@ -624,14 +702,14 @@ __device__ __forceinline__ bool wide_gather_cut(const u64* list, uint32_t first,
     const uint2 bucket = side == 0 ? head : tail;
     if (bucket.y == 0u || (side == 1 && bucket.x < done)) continue;  // (a tile inside one bucket has its only share already)
     const uint32_t from = side == 0 ? first : bucket.x, to = bucket.y < end ? bucket.y : end;
-    for (uint32_t i = done + tid; i < from; i += BLOCK) sh.keys[i - first] = list[i];  // the buckets between the two
+    for (uint32_t i = done + tid; i < from; i += kWideRankBlock) sh.keys[i - first] = list[i];  // the buckets between the two
     done = to;
     const u64* const src = list + bucket.x;
     const uint32_t m = bucket.y - bucket.x;
     if (m > kWideSelectMax) {  // (all of its tiles together see whether it has one score)
       int differs = order_ties ? 1 : 0;
       const uint32_t score = key64_okey(src[0]);
-      for (uint32_t i = from + tid; i < to && !order_ties; i += BLOCK) {
+      for (uint32_t i = from + tid; i < to && !order_ties; i += kWideRankBlock) {
         const u64 k = list[i];
         sh.keys[i - first] = k;
         differs |= key64_okey(k) != score ? 1 : 0;
@@ -641,7 +719,7 @@ __device__ __forceinline__ bool wide_gather_cut(const u64* list, uint32_t first,
     }
     u64 highest = 0, below = 0;  // (below: complement of the lowest)
 #pragma unroll 4
-    for (uint32_t i = tid; i < m; i += BLOCK) {
+    for (uint32_t i = tid; i < m; i += kWideRankBlock) {
       const u64 k = src[i];
       highest = k > highest ? k : highest;
       below = ~k > below ? ~k : below;
@@ -654,10 +732,10 @@ __device__ __forceinline__ bool wide_gather_cut(const u64* list, uint32_t first,
     }
     if (tid == 0) sh.fill = from - first;
     __syncthreads();
-    highest = row16_max<u64>(lane < BLOCK / 64 ? sh.high[lane] : 0);
-    const u64 lowest = ~row16_max<u64>(lane < BLOCK / 64 ? sh.low[lane] : 0);
+    highest = row16_max<u64>(lane < kWideRankBlock / 64 ? sh.high[lane] : 0);
+    const u64 lowest = ~row16_max<u64>(lane < kWideRankBlock / 64 ? sh.low[lane] : 0);
     if (!order_ties && key64_okey(lowest) == key64_okey(highest)) {
-      for (uint32_t i = from + tid; i < to; i += BLOCK) sh.keys[i - first] = list[i];
+      for (uint32_t i = from + tid; i < to; i += kWideRankBlock) sh.keys[i - first] = list[i];
     } else {
       u64 best = highest, last = lowest;
 #pragma unroll 1
@@ -667,14 +745,14 @@ __device__ __forceinline__ bool wide_gather_cut(const u64* list, uint32_t first,
         if (e == 0) best = key;
         else last = key;
       }
-      for (uint32_t i = tid; i < m; i += BLOCK) {
+      for (uint32_t i = tid; i < m; i += kWideRankBlock) {
         const u64 k = src[i];
         if (k <= best && k >= last) sh.keys[atomicAdd(&sh.fill, 1u)] = k;
       }
     }
     __syncthreads();
   }
-  for (uint32_t i = done + tid; i < end; i += BLOCK) sh.keys[i - first] = list[i];
+  for (uint32_t i = done + tid; i < end; i += kWideRankBlock) sh.keys[i - first] = list[i];
   __syncthreads();
   return true;
 }
@@ -684,29 +762,32 @@ __device__ __forceinline__ bool wide_gather_cut(const u64* list, uint32_t first,
 // 190 and 188 us a step for runs of up to 270 ties, 195 and 202 for runs of up to 400, 208 and 594 for runs of 1600.)
 constexpr uint32_t kWideRankCap = 256;
 
-template <int BLOCK>
-__device__ __forceinline__ void wide_rank_tile(const SampleArgs& a, const WideArgs& w, int row, int t, mi355x_sample_params prm, WideRankShared<BLOCK>& sh) {
-  constexpr int kPerThread = kSegElems / BLOCK;
+template <bool HANDED>
+__device__ __forceinline__ void wide_rank_tile(const SampleArgs& a, const WideArgs& w, int row, int t, mi355x_sample_params prm, WideRankShared& sh) {
+  constexpr int kPerThread = kSegElems / kWideRankBlock;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const WideRow info = w.rows[row];
+  const WideRow* const of_row = w.rows + row;
+  const WideRow info{wide_get<HANDED>(&of_row->n), wide_get<HANDED>(&of_row->tiles), wide_get<HANDED>(&of_row->declined), wide_get<HANDED>(&of_row->top)};
   if (info.declined == kWideDeclined || static_cast<uint32_t>(t) >= info.tiles) return;
   const uint32_t* const tile = w.tile_start + static_cast<size_t>(row) * (w.max_tiles + 1) + t;
-  const uint32_t first = tile[0], n = tile[1] - first;
+  const uint32_t first = wide_get<HANDED>(tile), n = wide_get<HANDED>(tile + 1) - first;
   const u64* const keys = a.big2 + static_cast<size_t>(row) * a.big_stride;
   const uint2* const cut = w.cut_bucket + static_cast<size_t>(row) * (w.max_tiles + 1) + t;
-  const uint2 head = cut[0], tail = cut[1];
+  const uint2 head = wide_get<HANDED>(cut), tail = wide_get<HANDED>(cut + 1);
   const bool order_ties = a.kept_ids != nullptr;
   const u64* const src = keys + first;
   u64 k[kPerThread];
 #pragma unroll
   for (int r = 0; r < kPerThread; ++r) {
-    const uint32_t i = static_cast<uint32_t>(r * BLOCK + tid);
-    k[r] = i < n ? src[i] : 0;
+    const uint32_t i = static_cast<uint32_t>(r * kWideRankBlock + tid);
+    k[r] = i < n ? wide_get<HANDED>(src + i) : 0;
   }
-  for (int b = tid; b <= kWideSubBuckets; b += BLOCK) sh.start[b] = 0u;
+  for (int b = tid; b <= kWideSubBuckets; b += kWideRankBlock) sh.start[b] = 0u;
   if (tid < kWideSubBuckets / 32) sh.mixed[tid] = 0u;
   if (tid >= 64 && tid < 96) sh.exp_tab[tid - 64] = em::exp2_tab(static_cast<uint32_t>(tid - 64));
   if (__builtin_expect((head.y | tail.y) != 0u, 0)) {  // (its code lies behind the kernel's: in line it makes every row's launch 0.7 us longer)
+    // (A cut bucket's keys are read by all of its tiles, several times each: from the XCD's cache, once a wave has invalidated it.)
+    if (HANDED && tid == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     __syncthreads();  // (the gather uses the table as well)
     if (!wide_gather_cut(keys, first, n, head, tail, order_ties, sh)) {
       if (tid == 0) {
@@ -717,10 +798,10 @@ __device__ __forceinline__ void wide_rank_tile(const SampleArgs& a, const WideAr
     }
 #pragma unroll
     for (int r = 0; r < kPerThread; ++r) {
-      const uint32_t i = static_cast<uint32_t>(r * BLOCK + tid);
+      const uint32_t i = static_cast<uint32_t>(r * kWideRankBlock + tid);
       k[r] = i < n ? sh.keys[i] : 0;
     }
-    for (int b = tid; b <= kWideSubBuckets; b += BLOCK) sh.start[b] = 0u;
+    for (int b = tid; b <= kWideSubBuckets; b += kWideRankBlock) sh.start[b] = 0u;
   }
   uint32_t hi = 0u, lo = 0xffffffffu;
 #pragma unroll
@@ -736,8 +817,8 @@ __device__ __forceinline__ void wide_rank_tile(const SampleArgs& a, const WideAr
     sh.red2[wave] = lo;
   }
   __syncthreads();
-  hi = row16_max<uint32_t>(lane < BLOCK / 64 ? sh.red[lane] : 0u);
-  lo = ~row16_max<uint32_t>(lane < BLOCK / 64 ? ~sh.red2[lane] : 0u);
+  hi = row16_max<uint32_t>(lane < kWideRankBlock / 64 ? sh.red[lane] : 0u);
+  lo = ~row16_max<uint32_t>(lane < kWideRankBlock / 64 ? ~sh.red2[lane] : 0u);
   const float top = key_to_float(hi), span = top - key_to_float(lo);
   const float scale = span > 0.0f ? static_cast<float>(kWideSubBuckets) / span : 0.0f;
   auto bucket_of = [=](u64 key) {
@@ -764,7 +845,7 @@ __device__ __forceinline__ void wide_rank_tile(const SampleArgs& a, const WideAr
   }
   bool crowded;  // some bucket holds more than kWideRankCap keys
   {  // the buckets' first places: eight consecutive buckets per thread
-    constexpr int kPer = kWideSubBuckets / BLOCK;
+    constexpr int kPer = kWideSubBuckets / kWideRankBlock;
     constexpr uint32_t kCrowded = 1u << 31;
     uint32_t cnt[kPer], local = 0u, most = 0u;
 #pragma unroll
@@ -777,7 +858,7 @@ __device__ __forceinline__ void wide_rank_tile(const SampleArgs& a, const WideAr
     const bool crowded_wave = __ballot(most > kWideRankCap) != 0;
     if (lane == 63) sh.red[wave] = inc | (crowded_wave ? kCrowded : 0u);
     __syncthreads();
-    const uint32_t of_wave = lane < BLOCK / 64 ? sh.red[lane] : 0u;
+    const uint32_t of_wave = lane < kWideRankBlock / 64 ? sh.red[lane] : 0u;
     crowded = __ballot((of_wave & kCrowded) != 0u) != 0;
     const uint32_t ws = wave_prefix_sum<uint32_t>(of_wave & ~kCrowded);
     uint32_t c = (wave > 0 ? wave_read_lane(ws, wave - 1) : 0u) + inc - local;
@@ -786,7 +867,7 @@ __device__ __forceinline__ void wide_rank_tile(const SampleArgs& a, const WideAr
       sh.start[tid * kPer + i] = c;
       c += cnt[i];
     }
-    if (tid == BLOCK - 1) sh.start[kWideSubBuckets] = c;
+    if (tid == kWideRankBlock - 1) sh.start[kWideSubBuckets] = c;
   }
   __syncthreads();
 #pragma unroll
@@ -801,7 +882,7 @@ __device__ __forceinline__ void wide_rank_tile(const SampleArgs& a, const WideAr
     int too_full = 0;
 #pragma unroll
     for (int r = 0; r < kPerThread; ++r) {
-      const uint32_t p = static_cast<uint32_t>(r * BLOCK + tid);
+      const uint32_t p = static_cast<uint32_t>(r * kWideRankBlock + tid);
       if (p < n) {
         const uint32_t b = bucket_of(sh.keys[p]);
         if (sh.start[b + 1u] - sh.start[b] > kWideRankCap && must_rank(b)) too_full = 1;
@@ -815,7 +896,7 @@ __device__ __forceinline__ void wide_rank_tile(const SampleArgs& a, const WideAr
   uint32_t fin[kPerThread];
 #pragma unroll
   for (int r = 0; r < kPerThread; ++r) {
-    const uint32_t p = static_cast<uint32_t>(r * BLOCK + tid);
+    const uint32_t p = static_cast<uint32_t>(r * kWideRankBlock + tid);
     k[r] = 0;
     fin[r] = p;
     if (p < n) {
@@ -843,19 +924,19 @@ __device__ __forceinline__ void wide_rank_tile(const SampleArgs& a, const WideAr
   part = wave_sum<double>(part);
   if (lane == 0) sh.dred[wave] = part;
   __syncthreads();
-  const double own = wave_read_lane(row_scan_add(lane < BLOCK / 64 ? sh.dred[lane] : 0.0), BLOCK / 64 - 1);
+  const double own = wave_read_lane(row_scan_add(lane < kWideRankBlock / 64 ? sh.dred[lane] : 0.0), kWideRankBlock / 64 - 1);
   double* const sums = w.tile_sum + static_cast<size_t>(row) * w.max_tiles;
   if (tid == 0) store_sum_bits(sums + t, static_cast<unsigned long long>(__double_as_longlong(own)));
   u64* const dst = a.big + static_cast<size_t>(row) * a.big_stride + first;
 #pragma unroll
   for (int r = 0; r < kPerThread; ++r) {
-    const uint32_t p = static_cast<uint32_t>(r * BLOCK + tid);
+    const uint32_t p = static_cast<uint32_t>(r * kWideRankBlock + tid);
     if (p < n) dst[p] = sh.keys[exp_slot(p)];
   }
   // the exact sum's step record, as in seqsum_exp_step_body: the sums of the tiles before this one tell the binade
   double before = 0.0;
   bool gave_up = false;
-  for (int s = tid; s < t; s += BLOCK) {
+  for (int s = tid; s < t; s += kWideRankBlock) {
     unsigned long long bits = load_sum_bits(sums + s);
     for (int spins = 0; bits == kSumNotReady && spins < a.poll_limit; ++spins) {
       __builtin_amdgcn_s_sleep(1);
@@ -868,7 +949,7 @@ __device__ __forceinline__ void wide_rank_tile(const SampleArgs& a, const WideAr
   before = wave_sum<double>(before);
   if (lane == 0) sh.dred[wave] = before;
   __syncthreads();
-  before = wave_read_lane(row_scan_add(lane < BLOCK / 64 ? sh.dred[lane] : 0.0), BLOCK / 64 - 1);
+  before = wave_read_lane(row_scan_add(lane < kWideRankBlock / 64 ? sh.dred[lane] : 0.0), kWideRankBlock / 64 - 1);
   const size_t rec_at = static_cast<size_t>(row) * w.max_tiles + t;
   int4* const rec = w.tile_step + rec_at;
   if (gave_up) {
@@ -888,16 +969,15 @@ __device__ __forceinline__ void wide_rank_tile(const SampleArgs& a, const WideAr
   const int se = seq_decompose(lo_f).se;
   const bool known = lo_f > 0.0f && hi_f < 3.0e38f && seq_decompose(hi_f).se == se;
   if (!known) {
-    // powers of two may fall inside the tile: records per part of 64 elements, eight or sixteen lanes each
+    // powers of two may fall inside the tile: records per part of 64 elements, eight lanes each
     constexpr int kPartLanes = kWalkPart / kPerThread;
-    static_assert((kPartLanes == 8 || kPartLanes == 16) && kSegSubs * kPartLanes == BLOCK, "a part is eight or sixteen lanes");
+    static_assert(kPartLanes == 8 && kSegSubs * kPartLanes == kWideRankBlock, "a part is eight lanes");
     double mine = 0.0;
 #pragma unroll
     for (int j = 0; j < kPerThread; ++j) mine += static_cast<double>(ev[j]);
     mine += __longlong_as_double(static_cast<long long>(lane_xor64<1>(static_cast<u64>(__double_as_longlong(mine)))));
     mine += __longlong_as_double(static_cast<long long>(lane_xor64<2>(static_cast<u64>(__double_as_longlong(mine)))));
     mine += __longlong_as_double(static_cast<long long>(lane_xor64<4>(static_cast<u64>(__double_as_longlong(mine)))));
-    if constexpr (kPartLanes == 16) mine += __longlong_as_double(static_cast<long long>(lane_xor64<8>(static_cast<u64>(__double_as_longlong(mine)))));
     const int part_i = tid / kPartLanes;
     const double upto = wave_prefix_sum<double>((lane & (kPartLanes - 1)) == 0 ? mine : 0.0);
     __syncthreads();
@@ -916,8 +996,8 @@ __device__ __forceinline__ void wide_rank_tile(const SampleArgs& a, const WideAr
       lo_step = seq_compose_run(ev, kPerThread, pse);
       hi_step = seq_compose_run(ev, kPerThread, pse + 1);
     }
-    lo_step = group_scan_steps<kPartLanes>(lo_step);
-    hi_step = group_scan_steps<kPartLanes>(hi_step);
+    lo_step = oct_scan_steps(lo_step);
+    hi_step = oct_scan_steps(hi_step);
     if ((lane & (kPartLanes - 1)) == kPartLanes - 1) {
       const size_t at = rec_at * kSegSubs + part_i;
       w.sub_step[at] = make_int4(static_cast<int>(lo_step.d0), static_cast<int>(lo_step.d1), static_cast<int>(hi_step.d0),
@@ -932,19 +1012,19 @@ __device__ __forceinline__ void wide_rank_tile(const SampleArgs& a, const WideAr
   __syncthreads();
   if (tid == 0) {
     Step s = sh.wave_tot[0];
-    for (int w = 1; w < BLOCK / 64; ++w) s = step_compose(s, sh.wave_tot[w]);
+    for (int w = 1; w < kWideRankBlock / 64; ++w) s = step_compose(s, sh.wave_tot[w]);
     *rec = make_int4(static_cast<int>(s.d0), static_cast<int>(s.d1), se, 0);
   }
 }
 
 template <bool INLINE>
 __global__ __launch_bounds__(kWideRankBlock) void wide_rank_kernel(const SampleArgs a, const typename WideTable<INLINE>::type, const WideArgs w) {
-  __shared__ WideRankShared<kWideRankBlock> sh;
+  __shared__ WideRankShared sh;
   const WideShare mine = wide_share(w.max_tiles);
   if (mine.row >= a.rows) return;
   const mi355x_sample_params prm = row_params<INLINE>(a, mine.row);
   if (!wide_row(prm)) return;
-  wide_rank_tile<kWideRankBlock>(a, w, mine.row, mine.item, prm, sh);
+  wide_rank_tile<false>(a, w, mine.row, mine.item, prm, sh);
 }
 
 // The tiles of a row as the walk reads them.
@@ -1270,8 +1350,8 @@ struct WideFinishReds {
   u64 red64[16];
 };
 template <bool INLINE>
-__device__ __forceinline__ void wide_finish_or_sort(const SampleArgs& a, const WideArgs& w, int row, mi355x_sample_params prm, u64* lds, WideFinishReds& reds) {
-  if (wide_finish_row<INLINE>(a, w, row, prm, *reinterpret_cast<WideFinishShared*>(lds), reds.seq)) {
+__device__ __forceinline__ void wide_finish_or_sort(const SampleArgs& a, const WideArgs& w, int row, mi355x_sample_params prm, bool exact, u64* lds, WideFinishReds& reds) {
+  if (!exact && wide_finish_row<INLINE>(a, w, row, prm, *reinterpret_cast<WideFinishShared*>(lds), reds.seq)) {
     if (threadIdx.x == 0) atomicAdd(a.fallback_rows, 1u);  // (a row of the exact path, spread over the GPU)
     return;
   }
@@ -1284,69 +1364,75 @@ template <bool INLINE>
 __global__ __launch_bounds__(kFinishBlock) void wide_finish_kernel(const SampleArgs a, const typename WideTable<INLINE>::type, const WideArgs w) {
   extern __shared__ u64 lds_keys[];
   __shared__ WideFinishReds reds;
-  const int row = blockIdx.x;
+  int row = blockIdx.x;
+  bool exact = false;
+  if (w.pick != 0) {  // a row that the pick has given back
+    const uint32_t sorted = *w.rest.sorted, i = blockIdx.x;
+    if (i >= sorted + *w.rest.exact) return;
+    exact = i >= sorted;
+    row = static_cast<int>(__builtin_amdgcn_readfirstlane(w.rest.rows[exact ? static_cast<uint32_t>(a.rows) - 1u - (i - sorted) : i]));
+    exact |= w.rest.gave_up[row] != 0u;
+  }
   const mi355x_sample_params prm = row_params<INLINE>(a, row);
   if (!wide_row(prm)) return;
-  wide_finish_or_sort<INLINE>(a, w, row, prm, lds_keys, reds);
+  wide_finish_or_sort<INLINE>(a, w, row, prm, exact, lds_keys, reds);
 }
 
-// What wide_scatter, wide_rank and wide_finish do, in one launch, for the rows that wide_pick has listed: seldom any, and
-// then the launch is all there is to pay.  (Means over 24 inputs, three launches that mostly find nothing to do and this one:
-// 16 x 128256 fp16 39.2 -> 33.9 us a step, 64 x 128256 68.9 -> 57.3, 1 x 128256 fp32 30.6 -> 26.3, 256 x 32064 fp32 73.3 -> 62.5; a single
-// row that is given back 57.8 -> 58.1.  Batches of which every row is given back pay for it, with one workgroup a CU and a hand-over per
-// tile: 16 x 128256 of N(0, 0.02^2) 812 -> 870, 64 x 128256 1208 -> 1432, 256 x 32064 with a NaN in every row 168 -> 287.  With every wave
-// writing the caches back and invalidating them, not one, that was 2364, and the single row 102.)
-// The chunks of all rows and their tiles behind them are numbered; every workgroup takes the next number until none is left,
-// and finishes the listed row of its own index.  Tiles wait for chunks, which have lower numbers: workgroups that run have
-// taken these, and wait for nothing.  A finish waits with no number in hand.  So every wait ends, however many workgroups
-// the GPU has room for.  (The finish is not numbered as well, in one loop with the rest: what the compiler then keeps in registers
-// over the loop takes all 128 of them and 700 bytes of scratch.)
+// What wide_scatter and wide_rank do, in one launch, for the rows that wide_pick has listed: seldom any, and then two launches that find
+// nothing to do are all there is to pay, not three.  Both parts are workgroups of 512 threads of which three fit a CU (a chunk's keys go
+// through LDS in two halves), in front the chunks of all listed rows, behind them their tiles, a row's all with indices of one remainder
+// (see wide_share).  A tile waits for its row's chunks, whose workgroups have started before its own and wait for nothing; a wait that
+// gives up leaves the row to the exact path, in the launch behind this one.  The polls are rare and a row's count has a line of memory to
+// itself: 500 waiting workgroups that polled sixteen counts in one line every 0.1 us took the launch from 40 to 60 us.
+// us a step, three launches behind the pick -> this one and the finish: no row given back 1 x 128256 fp32 29.3 -> 28.0, 16 x 128256 fp16
+// 37.3 -> 33.9, 64 x 128256 57.6 -> 48.1, 256 x 32064 fp32 54.8 -> 46.3; one row of one given back 83.9 -> 88.9; a NaN in every row
+// 16 x 128256 fp32 85.7 -> 92.8, 64 x 128256 174 -> 162, 256 x 32064 163 -> 156; near-flat rows 16 x 128256 766 -> 781, 64 x 128256
+// 1166 -> 1171, 256 x 32064 425 -> 386.  The worst of 70 such batches: four rows of 128256 with open draws, 87.8 -> 100.5.
+// (All in one launch of a workgroup a CU, the finish with it, is 2 to 4 us faster where nothing is given back, and up to 1.75 times as
+// slow in batches of which every row is: 64 x 128256 with a NaN in each 304, near-flat 1390, 256 x 32064 286 and 604.)
+constexpr int kWideRestRoom = kWideChunk / 2;
 template <typename InT, bool INLINE>
-__global__ __launch_bounds__(kWideBlock) void wide_rest_kernel(const SampleArgs a, const typename WideTable<INLINE>::type, const WideArgs w) {
-  extern __shared__ u64 lds_keys[];
-  __shared__ WideFinishReds reds;
-  __shared__ uint32_t next;
-  static_assert(kWideBlock == kFinishBlock && sizeof(WideRankShared<kWideBlock>) <= kFinishLds, "one shape for all three");
-  const uint32_t listed = *w.rest.count;
-  if (listed == 0u) return;
-  const uint32_t chunks = static_cast<uint32_t>(w.chunks), tiles = static_cast<uint32_t>(w.max_tiles);
-  auto take = [&] {
+__global__ __launch_bounds__(kWideRankBlock, 6) void wide_rest_kernel(const SampleArgs a, const typename WideTable<INLINE>::type, const WideArgs w) {
+  __shared__ union {
+    WideScatterShared<kWideRankBlock, kWideRestRoom> scatter;
+    WideRankShared rank;
+  } sh;
+  __shared__ bool all_there;
+  static_assert(3 * (sizeof(sh) + 1280) <= 160 * 1024, "three workgroups a CU");
+  const int sorted = static_cast<int>(*w.rest.sorted);
+  const int xcd = static_cast<int>(blockIdx.x) & 7, slot = static_cast<int>(blockIdx.x) >> 3;
+  if (xcd >= sorted) return;
+  const int rows = (sorted - xcd + 7) >> 3, of_chunks = rows * w.chunks;  // of the listed rows whose work has these indices
+  if (slot >= of_chunks + rows * w.max_tiles) return;
+  const bool ranks = slot >= of_chunks;
+  const int at = ranks ? slot - of_chunks : slot, per_row = ranks ? w.max_tiles : w.chunks, i = xcd + 8 * (at / per_row), item = at % per_row;
+  const int row = static_cast<int>(__builtin_amdgcn_readfirstlane(w.rest.rows[i]));
+  const mi355x_sample_params prm = row_params<INLINE>(a, row);
+  uint32_t* const scattered = w.rest.scattered + row * kRestStride;
+  if (!ranks) {
+    wide_scatter_chunk<InT, INLINE, true, kWideRankBlock, kWideRestRoom>(a, w, row, item, prm, sh.scatter);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // every wave's own stores are done
     __syncthreads();
-    if (threadIdx.x == 0) next = atomicAdd(w.rest.ticket, 1u);
-    __syncthreads();
-    return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(next));
-  };
-  auto listed_row = [&](uint32_t i) { return static_cast<int>(__builtin_amdgcn_readfirstlane(w.rest.rows[i])); };
-  // One wave waits and invalidates, one writes back: the caches are the CU's and the XCD's.
-  auto wait_for = [](const uint32_t* count, uint32_t all) {
-    if (threadIdx.x == 0) {
-      while (__hip_atomic_load(count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < all) __builtin_amdgcn_s_sleep(2);
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    if (threadIdx.x == 0) __hip_atomic_fetch_add(scattered, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return;
+  }
+  if (threadIdx.x == 0) {
+    const uint32_t chunks = static_cast<uint32_t>(w.chunks);
+    uint32_t n = __hip_atomic_load(scattered, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int polls = 0; n < chunks && polls < a.poll_limit; ++polls) {
+      __builtin_amdgcn_s_sleep(8);
+      n = __hip_atomic_load(scattered, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    __syncthreads();
-  };
-  auto done = [](uint32_t* count) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // every wave's own stores are in the XCD's L2 ...
-    __syncthreads();
-    if (threadIdx.x == 0) __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);  // ... and one of them has it written back
-  };
-  uint32_t item = take();
-  for (; item < listed * chunks; item = take()) {
-    const int row = listed_row(item / chunks);
-    wide_scatter_chunk<InT, INLINE>(a, w, row, static_cast<int>(item % chunks), row_params<INLINE>(a, row), *reinterpret_cast<WideScatterShared*>(lds_keys));
-    done(w.rest.scattered + row);
+    all_there = n >= chunks;
+    if (n < chunks) {
+      w.rest.gave_up[row] = 1u;
+      store_sum_bits(w.tile_sum + static_cast<size_t>(row) * w.max_tiles + item, 0ull);  // (other tiles of the row wait for one)
+      atomicAdd(a.fallback_rows + 2, 1u);
+    }
   }
-  for (; item < listed * (chunks + tiles); item = take()) {
-    const uint32_t i = item - listed * chunks;
-    const int row = listed_row(i / tiles);
-    wait_for(w.rest.scattered + row, chunks);
-    wide_rank_tile<kWideBlock>(a, w, row, static_cast<int>(i % tiles), row_params<INLINE>(a, row), *reinterpret_cast<WideRankShared<kWideBlock>*>(lds_keys));
-    done(w.rest.ranked + row);
-  }
-  if (blockIdx.x >= listed) return;
-  const int row = listed_row(blockIdx.x);
-  wait_for(w.rest.ranked + row, tiles);
-  wide_finish_or_sort<INLINE>(a, w, row, row_params<INLINE>(a, row), lds_keys, reds);
+  __syncthreads();
+  if (!all_there) return;
+  wide_rank_tile<true>(a, w, row, item, prm, sh.rank);
 }
 
 template <bool INLINE>
@@ -1359,17 +1445,15 @@ hipError_t launch_wide(const SampleArgs& a, const typename WideTable<INLINE>::ty
     hipLaunchKernelGGL((wide_count_kernel<InT, INLINE>), grid, block, 0, stream, a, table, w);
     if (w.pick != 0) {
       hipLaunchKernelGGL((wide_pick_kernel<InT, INLINE>), dim3(a.rows), block, kFinishLds, stream, a, table, w);
-      const int items = a.rows * w.max_tiles, most = a.rows > kWideRestBlocks ? a.rows : kWideRestBlocks;  // (a workgroup per row at least)
-      hipLaunchKernelGGL((wide_rest_kernel<InT, INLINE>), dim3(items < most ? items : most), block, kFinishLds, stream, a, table, w);
+      hipLaunchKernelGGL((wide_rest_kernel<InT, INLINE>), dim3((w.chunks + w.max_tiles) * rows8), dim3(kWideRankBlock), 0, stream, a, table, w);
     } else {
-      hipLaunchKernelGGL((wide_scatter_kernel<InT, INLINE>), grid, block, sizeof(WideScatterShared), stream, a, table, w);
+      hipLaunchKernelGGL((wide_scatter_kernel<InT, INLINE>), grid, block, sizeof(WideScatterWhole), stream, a, table, w);
     }
   };
   if (a.dtype == MI355X_F16) passes(uint16_t{});
   else if (a.dtype == MI355X_BF16) passes(bf16_t{});
   else passes(float{});
-  if (w.pick != 0) return hipGetLastError();
-  hipLaunchKernelGGL(wide_rank_kernel<INLINE>, dim3(w.max_tiles * rows8), dim3(kWideRankBlock), 0, stream, a, table, w);
+  if (w.pick == 0) hipLaunchKernelGGL(wide_rank_kernel<INLINE>, dim3(w.max_tiles * rows8), dim3(kWideRankBlock), 0, stream, a, table, w);
   hipLaunchKernelGGL(wide_finish_kernel<INLINE>, dim3(a.rows), dim3(kFinishBlock), kFinishLds, stream, a, table, w);
   return hipGetLastError();
 }

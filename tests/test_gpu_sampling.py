@@ -1751,7 +1751,7 @@ def test_whole_vocabulary_draws_that_replay_the_sums(ctx, orc, vocab, sigma, t):
 
 
 @pytest.mark.parametrize("rows,vocab,dtype", [(1, 4099, torch.float32), (9, 50257, torch.float16), (40, 20011, torch.bfloat16), (300, 4099, torch.float32)])
-def test_rows_given_back_by_the_pick_are_finished_in_one_launch(orc, rows, vocab, dtype):
+def test_rows_given_back_by_the_pick_are_sorted_and_finished(orc, rows, vocab, dtype):
     """Temperature-only rows that the pick gives back, their draws on cumulative values: one of them, some among others, all, and more
     than there are workgroups at once; eagerly and from a graph that is replayed with eager calls between."""
     say("rows given back", rows, vocab, dtype)
@@ -1771,18 +1771,108 @@ def test_rows_given_back_by_the_pick_are_finished_in_one_launch(orc, rows, vocab
         u[r] = cp[int(rng.integers(len(cp) // 100, len(cp) // 2))] / cp[-1]
     ud = torch.from_numpy(u).cuda()
     want = orc.sample_batch(xw, 0, 1.0, 0.9, u)
+    back = len(open_draws) + (2 if rows == 40 else 0)  # (a row of maxima that are not ordinary numbers is given back as well)
+
+    def given_back(step):
+        before = ctx.picks_given_back()
+        step()
+        return ctx.picks_given_back() - before
+
     for _ in range(3):
-        assert np.array_equal(ctx.sample(xd, ud, k=0, p=1.0, temperature=0.9).cpu().numpy(), want)
+        got = []
+        assert given_back(lambda: got.append(ctx.sample(xd, ud, k=0, p=1.0, temperature=0.9).cpu().numpy())) >= back
+        assert np.array_equal(got[0], want)
     out = torch.zeros(rows, dtype=torch.int32, device="cuda")
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
         ctx.sample(xd, ud, k=0, p=1.0, temperature=0.9, out=out)
     for _ in range(3):
         out.zero_()
-        graph.replay()
+        assert given_back(graph.replay) >= back
         assert np.array_equal(out.cpu().numpy(), want)
         assert np.array_equal(ctx.sample(xd, ud, k=0, p=1.0, temperature=0.9).cpu().numpy(), want)
     ctx.close()
+
+
+@pytest.mark.parametrize("rows,vocab,dtype", [(1, 4099, torch.bfloat16), (9, 50257, torch.float32), (40, 20011, torch.float16), (300, 4099, torch.float32)])
+def test_rows_given_back_by_the_pick_whose_waits_give_up(orc, rows, vocab, dtype):
+    """The tiles of a row that the pick gives back wait for the row's chunks; a wait that gives up -- forced with a poll limit of 0 -- leaves
+    the row to the exact path, with the same token, and the next call is as before."""
+    say("waits of rows given back", rows, vocab, dtype)
+    ctx = pkg().SearchContext(rows, vocab)
+    rng = np.random.default_rng(vocab)
+    xd = torch.from_numpy((2.0 * rng.standard_normal((rows, vocab))).astype(np.float32)).cuda().to(dtype)
+    xw = xd.float().cpu().numpy()
+    u = rng.random(rows)
+    for r in range(rows):
+        _, probs = orc.sampled_categorical(xw[r], 0, 1.0, 0.9)
+        cp = np.cumsum(np.asarray(probs, np.float64))
+        u[r] = cp[int(rng.integers(len(cp) // 100, len(cp) // 2))] / cp[-1]
+    ud = torch.from_numpy(u).cuda()
+    want = orc.sample_batch(xw, 0, 1.0, 0.9, u)
+    for limit in (1 << 21, 0, 1 << 21):
+        ctx.set_poll_limit(limit)
+        before, back = ctx.sum_waits_gave_up(), ctx.picks_given_back()
+        for _ in range(3):
+            assert np.array_equal(ctx.sample(xd, ud, k=0, p=1.0, temperature=0.9).cpu().numpy(), want), limit
+        assert ctx.picks_given_back() - back >= 3 * rows
+        assert (ctx.sum_waits_gave_up() > before) == (limit == 0)
+    ctx.close()
+
+
+@pytest.mark.parametrize("rows,vocab,dtype", [(24, 50257, torch.float16), (100, 4099, torch.float32), (60, 20011, torch.bfloat16)])
+def test_whole_vocabulary_rows_of_p_one_and_above_among_others(orc, rows, vocab, dtype):
+    """Rows of p = 1 that are picked or given back, rows of p above one (all of them given back), a row whose maximum is not finite, and rows
+    of other modes between them, in one call: more than one row of each kind, by the argument table and (100 rows) by the device's."""
+    say("p of one and above", rows, vocab, dtype)
+    ctx = pkg().SearchContext(rows, vocab)
+    rng = np.random.default_rng(rows)
+    x = (2.0 * rng.standard_normal((rows, vocab))).astype(np.float32)
+    if dtype != torch.float16:  # (whose values all are ordinary)
+        x[6] = -1e38
+    xd = torch.from_numpy(x).cuda().to(dtype)
+    xw = xd.float().cpu().numpy()
+    kinds = [(0, 1.0, 0.9), (50, 0.9, 0.7), (1, 2.0, 1.1), (0, 1.0, 0.9), (0, 0.9, 1.0), (200, 0.95, 1.0), (0, 1.0, 0.4), (0, 1.5, 0.8)]
+    params = [kinds[r % len(kinds)] for r in range(rows)]
+    u = rng.random(rows)
+    for r in range(3, rows, len(kinds)):  # the open draws
+        _, probs = orc.sampled_categorical(xw[r], *params[r])
+        cp = np.cumsum(np.asarray(probs, np.float64))
+        u[r] = cp[int(rng.integers(len(cp) // 100, len(cp) // 2))] / cp[-1]
+    want = np.array([orc.sample_batch(xw[r:r + 1], *params[r], u[r:r + 1])[0] for r in range(rows)])
+    ud = torch.from_numpy(u).cuda()
+    for _ in range(3):
+        before = ctx.picks_given_back()
+        assert np.array_equal(ctx.sample(xd, ud, per_row=params).cpu().numpy(), want)
+        assert ctx.picks_given_back() - before >= sum(p > 1.0 for _, p, _ in params) + len(range(3, rows, len(kinds)))
+    above = [(k, 1.5 if p == 1.0 else p, t) for k, p, t in params]  # (no row to pick from: no pick)
+    want = np.array([orc.sample_batch(xw[r:r + 1], *above[r], u[r:r + 1])[0] for r in range(rows)])
+    assert np.array_equal(ctx.sample(xd, ud, per_row=above).cpu().numpy(), want)
+    ctx.close()
+
+
+@pytest.mark.parametrize("rows,vocab", [(64, 128256), (256, 32064)])
+def test_batches_of_which_every_row_is_given_back_are_spread_over_the_gpu(rows, vocab):
+    """A NaN in every row sends all of them past the pick: the step takes about as long as where the kept set is asked for and no pick is
+    tried.  Sorted and finished by one workgroup a CU the rows took 1.75 times as long."""
+    say("time of batches given back", rows, vocab)
+    ctx = pkg().SearchContext(rows, vocab)
+    g = torch.Generator(device="cuda").manual_seed(vocab)
+    x = torch.randn(rows, vocab, generator=g, device="cuda") * 3
+    x[:, 7] = float("nan")
+    u = torch.rand(rows, generator=g, device="cuda", dtype=torch.float64)
+    best = {}
+    for kept in (0, 8):
+        for _ in range(8):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            for _ in range(8):
+                ctx.sample(x, u, k=0, p=1.0, temperature=1.0, kept_capacity=kept)
+            end.record()
+            end.synchronize()
+            best[kept] = min(best.get(kept, 1e9), start.elapsed_time(end))
+    ctx.close()
+    assert best[0] < 1.4 * best[8], best
 
 
 def crowded_rows(name, rng, rows, vocab):
