@@ -86,8 +86,6 @@ struct ScorerHost {
   void GiveBackWord(int word) { used.fetch_and(~(uint64_t{1} << word)); }
 };
 
-constexpr int kPlanBlocks = ms::kCus;  // a workgroup per CU
-
 struct mi355x_search_ctx {
   int device{};
   int max_rows{}, max_vocab{}, max_chunks{};
@@ -210,45 +208,15 @@ int ms_make_xform(mi355x_search_ctx* ctx, const mi355x_logits_xform* in, int row
   return MI355X_OK;
 }
 
-// How the rows of a call are cut into chunks, a workgroup each.  small_k: every row is one of top-k (k <= 64) or argmax.
-//
-// A workgroup spends some ten vector instructions on every logit it has room for and a fixed time on selecting and
-// handing over, so chunks are short while the GPU has a CU for each of them (8192, then 16384 logits) and long beyond:
-// twice the workgroups select twice as often.  us, chunks of 32768 -> as chosen, 1 / 8 / 32 rows: argmax of 128256 fp32
-// logits 5.2 -> 4.0, 5.5 -> 4.3, 6.3 -> 5.6, with a penalty over 256 ids 7.5 -> 5.4, 7.7 -> 5.7, 8.2 -> 7.2; top-k of 32064 with the
-// penalty 11.1 -> 8.3, 11.2 -> 8.7, 11.7 -> 9.0; of 151936 fp16 9.1 -> 8.3, 9.7 -> 8.7, 10.2 (as before).  The lines:
-//  * Top-k lists are merged four at a time by a wave, more through LDS: 7 of 8192 instead of 4 of 16384 logits, 1 x 50257 fp32 7.1 -> 7.7.
-//  * More workgroups than CUs, sixteen-bit top-k rows: 16384, whose kernel takes half the registers, so that two fit a CU
-//    (256 x 201088 55.2 -> 42.4, 64 x 151936 16.6 -> 14.6), but 32768 while that is a workgroup per CU (64 x 128256 10.3 against 11.3).
-//  * Argmax of more workgroups than CUs: 16384 up to two per CU (64 x 50257 fp16 7.2 -> 5.3) and where those of 32768 do not all run at
-//    once either (256 x 201088 fp16 23.7 -> 21.8, fp32 34.0 -> 33.0); in between some shapes gain and others lose (64 x 151936 fp16 0.91,
-//    128 x 128256 fp16 1.13).  Sixteen-bit rows with logits processing lose (256 x 128256 22.5 -> 25.9).
-//  * Numbered row by row, rows of an even number of chunks have their finishing workgroups on every other XCD, those of eight on one:
-//    many workgroups are numbered chunk by chunk (256 x 128256 fp16 36.1 -> 28.4, fp32 27.7 -> 26.8); few start and end in order with their
-//    rows side by side (64 x 128256 fp32 11.5, against 12.1).
-//  * A last chunk of few logits has them in few lanes, whose maxima bound nothing: rows are cut evenly then (64 x 50257 fp16 in chunks
-//    of 16384 24.2 -> 9.0, 64 x 33000 in chunks of 32768 23.5 -> 9.5).
+// small_k: every row is one of top-k (k <= 64) or argmax.
 void PlanStream(const mi355x_search_ctx* ctx, ms::SampleArgs* a, bool small_k) {
-  const long long rows = a->rows;
-  const bool argmax = a->emit_topk == ms::kEmitArgmax, wide = a->dtype == MI355X_F32 || a->dtype == 0;
-  auto chunks_of = [&](int room) { return (a->vocab + room - 1) / room; };
-  const int quarters = chunks_of(ms::kSChunk / 4), halves = chunks_of(ms::kSChunk / 2), wholes = chunks_of(ms::kSChunk);
-  const int most = argmax ? 64 : ms::kStreamMaxChunks;  // lists a finishing workgroup takes
-  int room = ms::kSChunk;
-  if (small_k) {
-    if (quarters == 1 || (quarters <= most && (argmax || quarters <= 4 || halves > 4) && rows * quarters <= kPlanBlocks)) room = ms::kSChunk / 4;
-    else if (halves == 1 || (halves <= most && rows * halves <= kPlanBlocks)) room = ms::kSChunk / 2;
-    else if (argmax ? (wide || !a->xf.active()) && ((rows * halves <= 2 * kPlanBlocks && wholes > 1) || rows * wholes > 2 * kPlanBlocks)
-                    : !wide && rows * wholes > kPlanBlocks) room = halves <= most ? ms::kSChunk / 2 : ms::kSChunk;
-    if (static_cast<size_t>(rows) * chunks_of(room) > ctx->cand_lists) room = ms::kSChunk;
-  }
-  a->chunk_room = a->chunk_elems = room;
-  a->chunks = chunks_of(room);
-  if (!small_k) return;
-  const long long many = argmax ? (room < ms::kSChunk ? kPlanBlocks : 2 * kPlanBlocks) : 4 * kPlanBlocks - 1;
-  a->rows_first = rows * a->chunks > many ? 1 : 0;
-  const int last = a->vocab - (a->chunks - 1) * room;
-  if (last < room / 4) a->chunk_elems = ((a->vocab + a->chunks - 1) / a->chunks + 63) & ~63;
+  const bool sixteen_bit = a->dtype == MI355X_F16 || a->dtype == MI355X_BF16;
+  const ms::StreamPlan plan =
+      ms::plan_stream({a->rows, a->vocab, small_k, a->emit_topk == ms::kEmitArgmax, sixteen_bit, a->xf.active()}, ctx->cand_lists);
+  a->chunk_room = plan.room;
+  a->chunk_elems = plan.elems;
+  a->chunks = plan.chunks;
+  a->rows_first = plan.rows_first ? 1 : 0;
 }
 
 extern "C" {
@@ -281,10 +249,8 @@ int mi355x_search_create(int device, int max_rows, int max_vocab, mi355x_search_
   auto ok = [&](hipError_t r) {
     if (e == hipSuccess) e = r;
   };
-  size_t sc = static_cast<size_t>(max_rows) * ((max_vocab + ms::kSChunk / 2 - 1) / (ms::kSChunk / 2));
-  if (sc < static_cast<size_t>(kPlanBlocks)) sc = kPlanBlocks;  // (what PlanStream asks for at most)
-  c->cand_lists = sc;
-  ok(c->Alloc(&c->cand_small, sc * ms::kSmallCap, true));  // all-zero between launches
+  c->cand_lists = ms::stream_lists(max_rows, max_vocab);
+  ok(c->Alloc(&c->cand_small, c->cand_lists * ms::kSmallCap, true));  // all-zero between launches
   ok(c->Alloc(&c->chunk_cnt, rc, true));
   ok(c->Alloc(&c->chunk_max, rc, true));
   ok(c->Alloc(&c->chunk_thr, rc, true));

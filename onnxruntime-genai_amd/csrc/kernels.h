@@ -2,16 +2,15 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include "device_utils.h"
+#include "stream_plan.h"
 
 namespace ms {
 
 // Shape of the fused sampling kernel: 512 threads x 16 float4 = one 32K-logit chunk per workgroup, or 8 or 4 float4
-// where the GPU has a CU for more workgroups than that makes (PlanStream has the rule and the figures).
+// where the GPU has a CU for more workgroups than that makes (plan_stream has the rule and the figures).
 // Many logits per lane keep the per-wave selection overhead small against the streaming work, few
 // chunks per row keep the finishing merge shallow (a 128K vocabulary is four sorted lists, two merge
 // levels), and thread t's float4s (t, t+512, t+1024, ...) make every wave an even sample of the chunk.
-constexpr int kCus = 256;             // of the GPU
-constexpr int kSChunk = 32768;        // logits per workgroup of the streaming kernels; those of top-k and argmax rows also come for 16384 and 8192
 constexpr int kTopkBlock = 512;       // threads of a workgroup that streams a top-k row (16 128-bit loads each) ...
 constexpr int kNucleusBlock = 1024;   // ... and a nucleus row (8 each: lighter threads, twice the waves in flight)
 constexpr int kSMaxWaves = 16;
@@ -20,8 +19,6 @@ constexpr int kSMaxWaves = 16;
 constexpr int kDefaultPollLimit = 1 << 21;
 constexpr int kSmallCap = 64;        // sorted candidates a chunk publishes on the k<=64 path
 constexpr int kListCap = 128;        // candidates a chunk can hold before its sort
-constexpr int kStreamMaxChunks = 16;  // whose lists a finishing workgroup merges
-constexpr int kStreamMaxVocab = kStreamMaxChunks * kSChunk;  // longer rows take the exact path
 constexpr int kNucleusCap = 16384;   // sorted nucleus candidates held in LDS by the finish kernel
 constexpr int kFinishBlock = 1024;
 

@@ -1,7 +1,7 @@
 // Streaming kernels of the sampling path (templates; a source file per element type instantiates them).
 //
 // sample_fused_kernel (top-k rows, k <= 64; one launch per step): every workgroup (512 threads x 16, 32 or 64
-// logits, see StreamPlan) streams one chunk of one row with 128-bit non-temporal loads, logits processing
+// logits, see stream_plan.h) streams one chunk of one row with 128-bit non-temporal loads, logits processing
 // fused, keeps the chunk's best 64 candidates and publishes them sorted; the workgroup of a row's last
 // chunk polls for the other chunks' lists, merges them four at a time (bitonic merges in registers)
 // and runs the reference's scalar epilogue (softmax over the k, nucleus cut, categorical draw) in rank
