@@ -45,9 +45,11 @@ inline size_t stream_lists(int max_rows, int max_vocab) {
 //  * Argmax of more workgroups than CUs: 16384 up to two per CU (64 x 50257 fp16 7.2 -> 5.3) and where those of 32768 do not all run at
 //    once either (256 x 201088 fp16 23.7 -> 21.8, fp32 34.0 -> 33.0); in between some shapes gain and others lose (64 x 151936 fp16 0.91,
 //    128 x 128256 fp16 1.13).  Sixteen-bit rows with logits processing lose (256 x 128256 22.5 -> 25.9).
-//  * Numbered row by row, rows of an even number of chunks have their finishing workgroups on every other XCD, those of eight on one:
-//    many workgroups are numbered chunk by chunk (256 x 128256 fp16 36.1 -> 28.4, fp32 27.7 -> 26.8); few start and end in order with their
-//    rows side by side (64 x 128256 fp32 11.5, against 12.1).
+//  * Numbered row by row, rows of an even number of chunks have their finishing workgroups on every other XCD, those of four on two, of
+//    eight on one: many workgroups are numbered chunk by chunk (256 x 128256 fp16 36.1 -> 28.4, fp32 27.7 -> 26.8); few start and end in order with
+//    their rows side by side (64 x 128256 fp32 11.5, against 12.1).  Short chunks of top-k rows, four or eight (or twelve, or sixteen) a row, from
+//    two workgroups per CU on: 100 x 128256 fp16 19.2 -> 17.0, with a penalty 25.7 -> 22.2, 130 x 65536 15.3 -> 13.7, 200 x 50257 18.8 -> 16.7; with ten or
+//    thirteen chunks a row they stay (60 x 151936 14.8 against 15.0, with a penalty 18.7 against 19.3).
 //  * A last chunk of few logits has them in few lanes, whose maxima bound nothing: rows are cut evenly then (64 x 50257 fp16 in chunks
 //    of 16384 24.2 -> 9.0, 64 x 33000 in chunks of 32768 23.5 -> 9.5).
 inline StreamPlan plan_stream(const StreamCall& call, size_t lists) {
@@ -66,7 +68,9 @@ inline StreamPlan plan_stream(const StreamCall& call, size_t lists) {
   else if (halves == 1 || (halves <= most && (rows * halves <= kCus || many_halves))) room = half;
   if (static_cast<size_t>(rows) * static_cast<size_t>(chunks_of(room)) > lists) room = whole;
   StreamPlan plan{room, room, chunks_of(room), false};
-  const long long in_order = call.argmax ? (room < whole ? kCus : 2 * kCus) : 4 * kCus - 1;  // workgroups that are numbered row by row
+  const long long in_order = call.argmax                                ? (room < whole ? kCus : 2 * kCus)
+                             : room < whole && plan.chunks % 4 == 0 ? 2 * kCus
+                                                                    : 4 * kCus - 1;  // workgroups that are numbered row by row
   plan.rows_first = rows * plan.chunks > in_order;
   const int last = call.vocab - (plan.chunks - 1) * room;
   if (last < room / 4) plan.elems = ((call.vocab + plan.chunks - 1) / plan.chunks + 63) & ~63;

@@ -17,6 +17,8 @@ static void check(const ms::StreamCall& call) {
   else if (static_cast<size_t>(call.rows) * static_cast<size_t>(p.chunks) > lists) wrong = "more lists than the context has";
   else if (call.vocab <= ms::kStreamMaxVocab && p.chunks > (call.argmax ? ms::kArgmaxMaxChunks : ms::kStreamMaxChunks)) wrong = "more lists than a row may have";
   else if (!call.small_k && (p.room != ms::kSChunk || p.elems != ms::kSChunk || p.rows_first)) wrong = "kernels of other rows have one chunk size and order";
+  else if (call.small_k && !call.argmax && p.room < ms::kSChunk && p.chunks % 4 == 0 && call.rows * p.chunks > 2 * ms::kCus && !p.rows_first)
+    wrong = "the workgroups that finish many rows are on two of the eight XCDs, or on one";
   if (wrong && ++failures <= 20)
     std::printf("%lld x %d small_k %d argmax %d sixteen_bit %d processed %d: %s (room %d, elems %d, chunks %d)\n", call.rows, call.vocab, call.small_k,
                 call.argmax, call.sixteen_bit, call.processed, wrong, p.room, p.elems, p.chunks);
