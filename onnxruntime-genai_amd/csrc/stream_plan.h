@@ -9,6 +9,7 @@ constexpr int kCus = 256;             // of the GPU
 constexpr int kSChunk = 32768;        // logits per workgroup of the streaming kernels; those of top-k and argmax rows also come for 16384 and 8192
 constexpr int kStreamMaxChunks = 16;  // whose lists a finishing workgroup merges ...
 constexpr int kArgmaxMaxChunks = 64;  // ... or whose best elements, a lane each
+constexpr int kEvenLanes = 384;       // a top-k row whose last chunk has elements for fewer lanes (4, or 8 of sixteen bits, each) is cut evenly
 constexpr int kStreamMaxVocab = kStreamMaxChunks * kSChunk;  // longer rows take the exact path
 
 struct StreamPlan {
@@ -51,7 +52,10 @@ inline size_t stream_lists(int max_rows, int max_vocab) {
 //    two workgroups per CU on: 100 x 128256 fp16 19.2 -> 17.0, with a penalty 25.7 -> 22.2, 130 x 65536 15.3 -> 13.7, 200 x 50257 18.8 -> 16.7; with ten or
 //    thirteen chunks a row they stay (60 x 151936 14.8 against 15.0, with a penalty 18.7 against 19.3).
 //  * A last chunk of few logits has them in few lanes, whose maxima bound nothing: rows are cut evenly then (64 x 50257 fp16 in chunks
-//    of 16384 24.2 -> 9.0, 64 x 33000 in chunks of 32768 23.5 -> 9.5).
+//    of 16384 24.2 -> 9.0, 64 x 33000 in chunks of 32768 23.5 -> 9.5).  The line is at 384 lanes, six of a workgroup's eight waves.  Top-50 of
+//    50 x 98304 and a last chunk of 258 lanes, whose fifth wave has two of them, as it is and evenly: fp32 29.5 and 13.4 us, fp16 32.2 and 13.7;
+//    of 300 to 512 lanes 12.8 and 13.5, 13.0 and 13.6, since no chunk of an even cut is whole (64 x 100000 fp32 with a penalty, 424 lanes,
+//    13.2 and 14.0).  Argmax rows, which need no bound, are cut evenly for a last chunk of under a quarter (50 x 98304 and 1700 more 7.3 and 7.0).
 inline StreamPlan plan_stream(const StreamCall& call, size_t lists) {
   const long long rows = call.rows;
   auto chunks_of = [&](int room) { return static_cast<int>((static_cast<long long>(call.vocab) + room - 1) / room); };
@@ -68,12 +72,13 @@ inline StreamPlan plan_stream(const StreamCall& call, size_t lists) {
   else if (halves == 1 || (halves <= most && (rows * halves <= kCus || many_halves))) room = half;
   if (static_cast<size_t>(rows) * static_cast<size_t>(chunks_of(room)) > lists) room = whole;
   StreamPlan plan{room, room, chunks_of(room), false};
-  const long long in_order = call.argmax                                ? (room < whole ? kCus : 2 * kCus)
-                             : room < whole && plan.chunks % 4 == 0 ? 2 * kCus
-                                                                    : 4 * kCus - 1;  // workgroups that are numbered row by row
+  long long in_order = 4 * kCus - 1;  // workgroups that are numbered row by row
+  if (call.argmax) in_order = room < whole ? kCus : 2 * kCus;
+  else if (room < whole && plan.chunks % 4 == 0) in_order = 2 * kCus;
   plan.rows_first = rows * plan.chunks > in_order;
   const int last = call.vocab - (plan.chunks - 1) * room;
-  if (last < room / 4) plan.elems = ((call.vocab + plan.chunks - 1) / plan.chunks + 63) & ~63;
+  const int short_of = call.argmax ? room / 4 : (call.sixteen_bit ? 8 : 4) * kEvenLanes;
+  if (last < short_of) plan.elems = ((call.vocab + plan.chunks - 1) / plan.chunks + 63) & ~63;
   return plan;
 }
 

@@ -17,6 +17,10 @@ static void check(const ms::StreamCall& call) {
   else if (static_cast<size_t>(call.rows) * static_cast<size_t>(p.chunks) > lists) wrong = "more lists than the context has";
   else if (call.vocab <= ms::kStreamMaxVocab && p.chunks > (call.argmax ? ms::kArgmaxMaxChunks : ms::kStreamMaxChunks)) wrong = "more lists than a row may have";
   else if (!call.small_k && (p.room != ms::kSChunk || p.elems != ms::kSChunk || p.rows_first)) wrong = "kernels of other rows have one chunk size and order";
+  else if (call.small_k && !call.argmax && p.chunks > 1 && call.vocab - (p.chunks - 1) * p.elems < (call.sixteen_bit ? 8 : 4) * 384)
+    wrong = "a last chunk of few lanes";
+  else if (call.small_k && !call.argmax && call.vocab - (p.chunks - 1) * p.room >= (call.sixteen_bit ? 8 : 4) * 384 && p.elems != p.room)
+    wrong = "no chunk is whole, though the last one has lanes enough";
   else if (call.small_k && !call.argmax && p.room < ms::kSChunk && p.chunks % 4 == 0 && call.rows * p.chunks > 2 * ms::kCus && !p.rows_first)
     wrong = "the workgroups that finish many rows are on two of the eight XCDs, or on one";
   if (wrong && ++failures <= 20)

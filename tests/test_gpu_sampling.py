@@ -1100,7 +1100,8 @@ def test_logits_processing_on_rows_of_any_alignment_and_end(ctx, orc, vocab):
 
 
 @pytest.mark.parametrize("rows,vocab", [(1, 8191), (300, 8193), (3, 16383), (5, 16385), (2, 32770), (40, 33000), (9, 49161), (130, 50257),
-                                        (16, 131072), (4, 131073), (90, 98400), (1, 262144), (2, 262145), (1, 524288)])
+                                        (16, 131072), (4, 131073), (90, 98400), (50, 99839), (50, 99840), (50, 101375), (50, 101376), (1, 262144), (2, 262145),
+                                        (1, 524288)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 def test_chunks_of_every_size(orc, rows, vocab, dtype):
     """Rows of top-k and argmax calls are cut into chunks of 8192, 16384 or 32768 logits, or evenly where the last one would be short, by
