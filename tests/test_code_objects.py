@@ -14,6 +14,7 @@ import __graft_entry__ as ge
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 OBJDUMP = "/opt/rocm/llvm/bin/llvm-objdump"
+READELF = "/opt/rocm/llvm/bin/llvm-readelf"
 COPY = re.compile(r"^(v_mov_b32_e32|v_mov_b64_e32|v_accvgpr_\w+|scratch_load_\w+) (v\d+|v\[\d+:\d+\]|a\d+), (v\d+|v\[\d+:\d+\]|a\d+|off|s\d+|s\[\d+:\d+\])\b")
 SETS_LANES = re.compile(r"^s_\w+ exec\b|saveexec")
 LEAVES = re.compile(r"^s_(branch|cbranch|endpgm|setpc|barrier)")
@@ -97,3 +98,20 @@ def test_lanes_are_on_where_registers_are_copied_behind_conditional_code(tmp_pat
             wrong += [(name, hex(address), text) for address, text in misplaced_copies(code)]
     assert kernels >= 60 and branches > 10000, (kernels, branches)
     assert not wrong, wrong[:8]
+
+
+@pytest.mark.skipif(not os.path.exists(READELF), reason="no reader of the kernels' notes")
+def test_kernels_for_two_workgroups_a_cu_have_the_registers_for_it(tmp_path):
+    """Kernels that a call chooses when it has more workgroups than CUs, because two of them fit one: of 1024 threads with 64 vector and 80
+    scalar registers and half of the LDS at most.  (Three registers more in the walk over a row's segments were 9 % of a softmax of 257 rows.)"""
+    ge.ensure_built()
+    seen = {}
+    for path in code_objects(os.path.join(ROOT, "onnxruntime-genai_amd", "libmi355x_search.so"), str(tmp_path)):
+        notes = subprocess.run([READELF, "--notes", path], check=True, text=True, stdout=subprocess.PIPE).stdout
+        for kernel in notes.split("  - .agpr_count:")[1:]:
+            of = {key: value for key, value in re.findall(r"\.(\w+):\s+(\S+)", kernel)}
+            if re.match(r"_ZN2ms\d+(\w+_many\w*_kernel|seqsum_walk_kernelI\w+Li8E|wide_count_kernel)", of["name"]):
+                seen[of["name"]] = [int(of[key]) for key in ("max_flat_workgroup_size", "vgpr_count", "sgpr_count", "group_segment_fixed_size")]
+    assert sum("seqsum_walk" in name for name in seen) == 3 and sum("_many" in name for name in seen) >= 12, sorted(seen)
+    wrong = {name: n for name, n in seen.items() if n[0] != 1024 or n[1] > 64 or n[2] > 80 or n[3] > 80 * 1024}
+    assert not wrong, wrong

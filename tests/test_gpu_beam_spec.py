@@ -113,6 +113,39 @@ def test_softmax_of_long_rows_with_masked_infinite_and_nan_logits(ctx, orc, voca
             assert np.array_equal(bits(got[number]), bits(want[number])), r
 
 
+@pytest.mark.parametrize("rows,vocab", [(256, 16384), (257, 16384), (300, 20481), (600, 16385)])
+def test_softmax_of_more_rows_than_cus(orc, rows, vocab):
+    """The walk over a row's segments has a kernel of its own for more rows than CUs: batches on both sides of that line."""
+    say("softmax, many rows", rows, vocab)
+    c = pkg().SearchContext(rows, vocab)
+    x = (np.random.default_rng(rows).standard_normal((rows, vocab)) * 3).astype(np.float32)
+    x[rows - 1] = -7.25  # (powers of two in every segment)
+    sm = c.softmax(torch.from_numpy(x.copy()).cuda(), 0.8, log=False).cpu().numpy()
+    lsm = c.softmax(torch.from_numpy(x.copy()).cuda(), 0.8, log=True).cpu().numpy()
+    c.close()
+    for r in {0, 100, 255, rows - 2, rows - 1}:
+        assert np.array_equal(bits(sm[r]), bits(orc.softmax(x[r], 0.8))), r
+        assert np.array_equal(bits(lsm[r]), bits(orc.log_softmax(x[r], 0.8))), r
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_beams_of_more_rows_than_cus(dtype):
+    """The same for beam selection in every element type: 65 entries of four beams, and the same entries a few at a time."""
+    say("beams, many rows", dtype)
+    batch, beams, vocab = 65, 4, 16390
+    c = pkg().SearchContext(batch * beams, vocab)
+    g = torch.Generator(device="cuda").manual_seed(65)
+    x = (torch.randn(batch * beams, vocab, generator=g, device="cuda") * 3).to(dtype)
+    scores = -5.0 * torch.rand(batch * beams, generator=g, device="cuda")
+    got = [t.cpu().numpy().reshape(batch, -1) for t in c.beam_select(x, batch, beams, scores)]
+    for first in range(0, batch, 13):
+        rows = slice(first * beams, (first + 13) * beams)
+        few = [t.cpu().numpy().reshape(13, -1) for t in c.beam_select(x[rows], 13, beams, scores[rows])]
+        assert np.array_equal(bits(got[0][first:first + 13]), bits(few[0]))
+        assert np.array_equal(got[1][first:first + 13], few[1]) and np.array_equal(got[2][first:first + 13], few[2])
+    c.close()
+
+
 def test_log_softmax_extreme_rows(ctx, orc):
     """Sums that start subnormal, cross many binades, or hit exact ties in the running sum."""
     say("softmax extreme")
