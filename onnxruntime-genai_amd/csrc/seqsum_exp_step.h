@@ -66,7 +66,7 @@ __device__ __forceinline__ double seq_drift(int count) {
 // on the segment's elements v (as loaded: zeros past the end of the row) that would otherwise wait for a launch of
 // its own.
 // Bound by the chain from the loads over the exponentials, the exchange of the sums and the composition to the record, with a
-// third of the time spent issuing vector instructions: exponentials side by side (wave_expf) and a thread's sixteen elements in a row, so that
+// third of the time spent issuing vector instructions (two thirds with the lists of the beam search): exponentials side by side (wave_expf) and a thread's sixteen elements in a row, so that
 // neither a transposition through LDS nor a copy of the exponentials in memory is needed (the walk computes the few it
 // looks at once more, and takes 1 us longer), took the launch from 12.3 to 8.7 us at 16 x 151936 fp32 (9.7 MB, in the cache by
 // then), with the lists of the beam search from 20.4 to 17.1 at 32 x 151936 fp16 and from 11.4 to 8.9 at 8 x 51865.

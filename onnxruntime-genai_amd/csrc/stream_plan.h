@@ -42,10 +42,12 @@ inline size_t stream_lists(int max_rows, int max_vocab) {
 // penalty 11.1 -> 8.3, 11.2 -> 8.7, 11.7 -> 9.0; of 151936 fp16 9.1 -> 8.3, 9.7 -> 8.7, 10.2 (as before).  The lines:
 //  * Top-k lists are merged four at a time by a wave, more through LDS: 7 of 8192 instead of 4 of 16384 logits, 1 x 50257 fp32 7.1 -> 7.7.
 //  * More workgroups than CUs, sixteen-bit top-k rows: 16384, whose kernel takes half the registers, so that two fit a CU
-//    (256 x 201088 55.2 -> 42.4, 64 x 151936 16.6 -> 14.6), but 32768 while that is a workgroup per CU (64 x 128256 10.3 against 11.3).
+//    (256 x 201088 55.2 -> 42.4, 64 x 151936 16.6 -> 14.6, with a penalty over 128 ids 69.5 -> 53.6 and 20.7 -> 18.9), but 32768 while that is
+//    a workgroup per CU (64 x 128256 10.3 against 11.3, with the penalty 12.6 against 13.5).
 //  * Argmax of more workgroups than CUs: 16384 up to two per CU (64 x 50257 fp16 7.2 -> 5.3) and where those of 32768 do not all run at
-//    once either (256 x 201088 fp16 23.7 -> 21.8, fp32 34.0 -> 33.0); in between some shapes gain and others lose (64 x 151936 fp16 0.91,
-//    128 x 128256 fp16 1.13).  Sixteen-bit rows with logits processing lose (256 x 128256 22.5 -> 25.9).
+//    once either (256 x 201088 fp16 23.8 -> 22.5, bf16 22.7 -> 22.4, fp32 with a penalty 40.1 -> 37.5; 200 x 151936 bf16, whose 1000 of 32768 fill the
+//    GPU just twice, 14.8 -> 15.3); in between some shapes gain and others lose (64 x 151936 fp16 0.91, 128 x 128256 fp16 1.13).  Sixteen-bit
+//    rows with logits processing lose (256 x 128256 22.5 -> 25.9).
 //  * Numbered row by row, rows of an even number of chunks have their finishing workgroups on every other XCD, those of four on two, of
 //    eight on one: many workgroups are numbered chunk by chunk (256 x 128256 fp16 36.1 -> 28.4, fp32 27.7 -> 26.8); few start and end in order with
 //    their rows side by side (64 x 128256 fp32 11.5, against 12.1).  Short chunks of top-k rows, four or eight (or twelve, or sixteen) a row, from
